@@ -1785,6 +1785,47 @@ def test_config5_fused_experts_decode_regime(device, T):
     assert rep["matched"] >= 0.999 and rep["max_rel_to_sigma"] <= 0.1, rep
 
 
+@pytest.mark.parametrize("T,H,I,E,k,dtype,skew", [
+    (1, 640, 384, 40, 8, torch.bfloat16, 0),      # sum form; K tails of one and of three steps (5 and 3 K steps)
+    (2, 512, 1408, 64, 6, torch.float16, 0),      # sum form, two tokens
+    (3, 128, 128, 3, 2, torch.bfloat16, 0),       # one K step; more slots than experts
+    (16, 1152, 256, 64, 4, torch.float16, 0),     # 16 rows held, row-per-slot form
+    (40, 256, 640, 33, 5, torch.bfloat16, 0),     # an expert count over one mask word
+    (48, 256, 256, 40, 6, torch.bfloat16, 48),    # every token also to one expert: more rows than are held, several tiles
+    (150, 384, 384, 64, 6, torch.bfloat16, 0),    # two tiles of 16 rows
+    (5, 7168, 256, 16, 8, torch.bfloat16, 0),     # a long K: more than one batch of activations, fewer rows held
+])
+def test_decoding_moe_layer_gives_the_bits_of_the_row_tiled_layer(device, T, H, I, E, k, dtype, skew):
+    """The layer on the weight-streaming kernels (few rows per expert) against the row-tiled kernels called one by one: K blocks
+    are added in the same order with the same fused multiply-adds and both quantizations round alike, so the bits agree;
+    first call, repeated call, ids as int32 and int64."""
+    from tilegym_amd.ops import fused_moe, moe_interface
+
+    g = _g(1000 * T + H + E)
+    hidden = torch.randn(T, H, generator=g).to(dtype).to(device)
+    hidden[0, :128] = 0                             # (an all-zero group: scale 1)
+    w1q, w1s = R.quantize_weight_128x128(torch.randn(E * 2 * I, H, generator=g) * 0.1)
+    w2q, w2s = R.quantize_weight_128x128(torch.randn(E * H, I, generator=g) * 0.1)
+    w1q, w1s = w1q.reshape(E, 2 * I, H).to(device), w1s.reshape(E, 2 * I // 128, H // 128).to(device)
+    w2q, w2s = w2q.reshape(E, H, I).to(device), w2s.reshape(E, H // 128, I // 128).to(device)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+    if skew:
+        ids = torch.where(ids == E - 1, ids[:, :1], ids)
+        ids[:skew, 0] = E - 1
+    ids = ids.to(device)
+    tw = torch.softmax(torch.randn(T, k, generator=g), dim=-1).to(device)
+    try:
+        moe_interface.USE_ONE_CALL_LAYER = False
+        want = fused_moe(hidden, w1q, w2q, tw, ids, w1_scale=w1s, w2_scale=w2s)
+    finally:
+        moe_interface.USE_ONE_CALL_LAYER = True
+    for again in (ids, ids.to(torch.int32), ids):
+        _lib.workspace_for(hidden.device, 1 << 20).fill_(0xAB)
+        got = fused_moe(hidden, w1q, w2q, tw, again, w1_scale=w1s, w2_scale=w2s)
+        assert _lib.last_config()["KERNEL_NAME"] == "stream"
+        assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
 def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_path):
     """A table written by tilegym_amd.tune (here: by hand, and by tune_shape on a small shape) decides the schedule of calls
     that bring no kernel_configs; explicit kernel_configs still win; unloading the table restores the automatic choice."""

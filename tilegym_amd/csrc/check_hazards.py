@@ -48,7 +48,7 @@ VGPR_SPILL_LIMITS = {"fp8_gemm_tile256_kernel": 0, "fp8_gemm_bs256_kernelILi0ELb
                      "fp8_gemm_bs256_kernelILi1ELb0E": 17, "fp8_gemm_bs256_kernelILi1ELb1E": 0}
 # translation units with inline-assembly memory instructions
 DEFAULT_SOURCES = ["fp8_gemm_tile_pt.hip", "fp8_gemm_tile256.hip", "fp8_gemm_tile_bs.hip", "fp8_gemm_tile_bs256.hip",
-                   "fp8_gemm_tile_grouped.hip", "fp8_gemm_tile_list.hip", "fp8_gemm_stream.hip"]
+                   "fp8_gemm_tile_grouped.hip", "fp8_gemm_tile_list.hip", "fp8_gemm_stream.hip", "fp8_moe_decode.hip"]
 
 
 def scalar_regs(tok):

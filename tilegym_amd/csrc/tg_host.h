@@ -17,6 +17,19 @@ struct GenericParams {
     int rows;                // row slots to visit (M, or the sorted-slot capacity in gather mode)
 };
 
+// One GEMM of the decoding MoE layer (fp8_moe_decode.h): 16-bit activation rows, expert weights with 128 x 128 block scales.
+struct MoeDecodeParams {
+    const void* x;             // first GEMM: (tokens, K), slot s reads row s / top_k; second: (slots, K)
+    const uint8_t* w;          // (E, N, K) e4m3
+    const float* ws;           // (E, nblocks, kblocks)
+    const float* topk_weights; // (slots); second GEMM only
+    const void* ids;           // (slots) int32 or int64 expert ids
+    void* out;                 // first GEMM: (slots, inter); second: (slots, N), or with the sum (tokens, N)
+    int ids_are_i64, slots, top_k, E, N, K, inter, kblocks, nblocks;
+    int row_cap;               // activation rows held at a time: a power of two, at most 32
+    int wscale_cap;            // floats of LDS for a segment's weight scales, a multiple of 64
+};
+
 struct TileShape { int bm, bn; };
 
 // Launchers return hipErrorInvalidConfiguration when the combination is not instantiated.
@@ -40,6 +53,15 @@ int compute_units();
 hipError_t run_tile_block_dense(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 hipError_t run_tile_moe_act(int bm, const GemmParams& p, int gx, hipStream_t s);
 hipError_t run_tile_block_grouped(int bm, int bn, int group, const GemmParams& p, int gx, hipStream_t s);
+// The two GEMMs of the decoding MoE layer: out = T(silu(gate) * up) resp. out = T(result x routed weight).  `up` selects the
+// first.  The `fits` forms say (from the sizes in p alone) whether the layer is one for these kernels: few enough rows per
+// expert, and row buffers that fit in LDS.
+constexpr int kMoeDecodeSlots = 2048;
+bool moe_decode_fits(MoeDecodeParams p, bool up, int tokens);
+hipError_t run_moe_decode(MoeDecodeParams p, bool up, bool is_bf16, int tokens, hipStream_t s);
+// the second GEMM with the sum over a token's slots in the same launch: out (tokens, N)
+bool moe_decode_sum_fits(const MoeDecodeParams& p, int tokens);
+hipError_t run_moe_decode_sum(const MoeDecodeParams& p, bool is_bf16, int tokens, hipStream_t s);
 // up to kListMax per-tensor NT problems in one launch (tile 256x256, 128x128 or 64x128)
 hipError_t run_tile_list(int bm, int bn, const GemmList& gl, int gx, hipStream_t s);
 hipError_t run_skinny(int mt, int rg, int nw, bool blockscale, const GemmParams& p, int gx, int gy, hipStream_t s);

@@ -1613,9 +1613,28 @@ int32_t tg_fp8_group_gemm(const tg_tensor* const* c, const tg_tensor* const* a, 
 
 namespace {
 struct MoeLayout {
-    int64_t sorted_ids, expert_ids, post, cumsum, max_count, xq, xs, q2, s2, c3, total;  // byte offsets
+    int64_t sorted_ids, expert_ids, post, cumsum, max_count, xq, xs, q2, s2, act, c3, total;  // byte offsets
     int64_t cap, nblk;
 };
+// Few rows per expert: the layer streams the experts' weights (fp8_moe_decode.h) instead of padding every expert to a row
+// tile.  Sizes only; the two GEMMs' parameters.
+struct MoeDecode {
+    tg::MoeDecodeParams up, down;
+    bool takes;
+};
+MoeDecode moe_decode(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I) {
+    MoeDecode d{};
+    if (T <= 0 || T * k > tg::kMoeDecodeSlots || E > 512 || H % 128 != 0 || I % 128 != 0 || H > 65536 || I > 65536) return d;
+    d.up.slots = d.down.slots = (int)(T * k);
+    d.up.top_k = d.down.top_k = (int)k;
+    d.up.E = d.down.E = (int)E;
+    d.up.N = (int)(2 * I); d.up.K = (int)H; d.up.inter = (int)I;
+    d.up.kblocks = (int)(H / 128); d.up.nblocks = (int)(2 * I / 128);
+    d.down.N = (int)H; d.down.K = (int)I;
+    d.down.kblocks = (int)(I / 128); d.down.nblocks = (int)(H / 128);
+    d.takes = tg::moe_decode_fits(d.up, true, (int)T) && tg::moe_decode_fits(d.down, false, (int)T);
+    return d;
+}
 MoeLayout moe_layout(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I, int64_t block_m, int64_t elem16) {
     MoeLayout l{};
     auto take = [&](int64_t bytes) { const int64_t at = l.total; l.total += (bytes + 255) / 256 * 256; return at; };
@@ -1630,6 +1649,8 @@ MoeLayout moe_layout(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I, int6
     l.xs = take(T * (H / 128) * 4);
     l.q2 = take(T * k * I);
     l.s2 = take(T * k * cdiv(I, 128) * 4);
+    // (the decoding form keeps the activations between its GEMMs as 16-bit values)
+    l.act = moe_decode(T, k, E, H, I).takes ? take(T * k * I * elem16) : 0;
     l.c3 = take(T * k * H * elem16);
     return l;
 }
@@ -1689,6 +1710,46 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
                     (long long)l.total);
     if (workspace->ptr % 256 != 0) return fail(TG_ERR_INVALID, "workspace must be 256-byte aligned");
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace->ptr);
+    if (MoeDecode d = moe_decode(T, k, E, H, I); d.takes) {
+        for (const tg_tensor* t : {out, hidden, w1, w2, w1_scale, w2_scale, topk_weights, topk_ids})
+            if (!contiguous(t)) return fail(TG_ERR_INVALID, "all tensors must be contiguous");
+        if (topk_ids->dtype != TG_I32 && topk_ids->dtype != TG_I64) return fail(TG_ERR_DTYPE, "topk_ids must be int32 or int64");
+        if (w1->dtype != TG_F8E4M3FN || w2->dtype != TG_F8E4M3FN) return fail(TG_ERR_DTYPE, "w1 and w2 must be float8_e4m3fn (dtype code 7)");
+        if (w1_scale->dtype != TG_F32 || w2_scale->dtype != TG_F32) return fail(TG_ERR_DTYPE, "w1_scale and w2_scale must be f32");
+        if (w1_scale->shape[0] != E || w1_scale->shape[1] != 2 * I / 128 || w1_scale->shape[2] != H / 128)
+            return fail(TG_ERR_INVALID, "w1_scale must be (%lld, %lld, %lld)", (long long)E, (long long)(2 * I / 128), (long long)(H / 128));
+        if (w2_scale->shape[0] != E || w2_scale->shape[1] != H / 128 || w2_scale->shape[2] != I / 128)
+            return fail(TG_ERR_INVALID, "w2_scale must be (%lld, %lld, %lld)", (long long)E, (long long)(H / 128), (long long)(I / 128));
+        for (const tg_tensor* t : {out, hidden, w1, w2})
+            if (!aligned16(t->ptr)) return fail(TG_ERR_INVALID, "out, hidden, w1 and w2 must be 16-byte aligned");
+        DeviceGuard guard(device_id);
+        if (!guard.ok) return fail(TG_ERR_DEVICE, "cannot use HIP device %d", device_id);
+        hipStream_t stream = reinterpret_cast<hipStream_t>(hip_stream);
+        const bool bf16 = hidden->dtype == TG_BF16;
+        d.up.x = reinterpret_cast<const void*>(hidden->ptr);
+        d.up.w = reinterpret_cast<const uint8_t*>(w1->ptr);
+        d.up.ws = reinterpret_cast<const float*>(w1_scale->ptr);
+        d.up.ids = d.down.ids = reinterpret_cast<const void*>(topk_ids->ptr);
+        d.up.ids_are_i64 = d.down.ids_are_i64 = topk_ids->dtype == TG_I64;
+        d.up.out = ws + l.act;
+        d.down.x = ws + l.act;
+        d.down.w = reinterpret_cast<const uint8_t*>(w2->ptr);
+        d.down.ws = reinterpret_cast<const float*>(w2_scale->ptr);
+        d.down.topk_weights = reinterpret_cast<const float*>(topk_weights->ptr);
+        remember(Schedule{3, -1, -1, 1, -1, -1, -1});
+        hipError_t e = tg::run_moe_decode(d.up, true, bf16, (int)T, stream);
+        if (e == hipSuccess && tg::moe_decode_sum_fits(d.down, (int)T)) {
+            d.down.out = reinterpret_cast<void*>(out->ptr);
+            e = tg::run_moe_decode_sum(d.down, bf16, (int)T, stream);
+        } else if (e == hipSuccess) {
+            d.down.out = ws + l.c3;
+            e = tg::run_moe_decode(d.down, false, bf16, (int)T, stream);
+            if (e == hipSuccess)
+                e = tg::run_moe_sum(ws + l.c3, reinterpret_cast<void*>(out->ptr), bf16 ? tg::OUT_BF16 : tg::OUT_F16, T, (int)k, (int)H, stream);
+        }
+        if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "decoding MoE launch failed: %s", hipGetErrorString(e));
+        return TG_OK;
+    }
     const tg_tensor sorted_ids = describe(ws, l.sorted_ids, TG_I32, {l.cap});
     const tg_tensor expert_ids = describe(ws, l.expert_ids, TG_I32, {l.nblk});
     const tg_tensor post = describe(ws, l.post, TG_I32, {1});
