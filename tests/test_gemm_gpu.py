@@ -1785,6 +1785,17 @@ def test_config5_fused_experts_decode_regime(device, T):
     assert rep["matched"] >= 0.999 and rep["max_rel_to_sigma"] <= 0.1, rep
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 16, 128), (96, 144, 256), (130, 272, 1040), (65, 4112, 4096), (300, 128, 200), (20, 4080, 1008)])
+def test_kn_weights_give_the_bits_of_nk_weights(device, M, N, K):
+    """(K, N) weights go through the 16-byte transpose: edges of its 128 x 128 tiles in both directions, a padded K (rows of the
+    copy longer than K: 1040, 200, 1008 are no multiples of 128), against the same weight handed over as (N, K)."""
+    g = _g(M + N + K)
+    a, b = fp8_randn((M, K), g).to(device), fp8_randn((N, K), g, 0.3).to(device)
+    want = matmul(a, b, trans_b=True, out_dtype=torch.float32)
+    got = matmul(a, b.view(torch.uint8).t().contiguous().view(FP8), out_dtype=torch.float32)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("T,H,I,E,k,dtype,skew", [
     (1, 640, 384, 40, 8, torch.bfloat16, 0),      # sum form; K tails of one and of three steps (5 and 3 K steps)
     (2, 512, 1408, 64, 6, torch.float16, 0),      # sum form, two tokens
