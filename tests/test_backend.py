@@ -206,3 +206,25 @@ def test_recorded_schedule_table_round_trip(tmp_path):
     assert [c for c in tune.candidates(1, 4096, 4096, False) if c["KERNEL"] == "tiled"] == []
     assert {"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 256, "SPLIT_K": 1} in tune.candidates(4096, 4096, 4096, True)
     assert tune._parse_shape("8,4096,11008,block") == (8, 4096, 11008, True) and tune._parse_shape("8,4096,11008") == (8, 4096, 11008, False)
+
+
+def test_native_binding_declines_host_tensors_and_odd_arguments():
+    """The native call paths take plain device calls only; anything else is left to the Python implementations (None / False),
+    which convert or raise."""
+    import torch
+
+    from tilegym_amd import _lib
+
+    _lib.load()
+    n, f8 = _lib.native, torch.float8_e4m3fn
+    a, b, s = torch.zeros(4, 128, dtype=f8), torch.zeros(8, 128, dtype=f8), torch.ones(1)
+    assert n.matmul(a, b, False, True, s, s, 1.0, torch.bfloat16) is None
+    assert n.matmul("a", b, False, True, None, None, 1.0, None) is None
+    assert n.gemm(torch.zeros(4, 8), a, b, s, None, False, True, 1.0, 0.0, True) is False
+    assert n.block_matmul(a, b, torch.ones(4, 1), torch.ones(1, 1), torch.float32) is None
+    assert n.act_quant(torch.zeros(4, 128), 128, 0.0, 0) is None
+    assert n.ragged_matmul(a, b.reshape(1, 8, 128), torch.ones(4, 1), torch.ones(1, 1, 1), torch.tensor([0, 4], dtype=torch.int32), None) is None
+    assert n.fused_moe(torch.zeros(2, 128), b, b, s, s, None, None, False, 512) is None
+    for call in (lambda: n.matmul(a, b), lambda: n.act_quant(a)):
+        with pytest.raises(TypeError):
+            call()

@@ -1785,6 +1785,35 @@ def test_config5_fused_experts_decode_regime(device, T):
     assert rep["matched"] >= 0.999 and rep["max_rel_to_sigma"] <= 0.1, rep
 
 
+def test_native_binding_agrees_with_the_general_path(device):
+    """The same call through the native module and, by an option it leaves to Python, through the general path: number
+    scales, 3-D activations, f16 scales (converted in Python), empty problems, and the errors both raise."""
+    g = _g(77)
+    a, b = fp8_randn((6, 256), g).to(device), fp8_randn((24, 256), g, 0.1).to(device)
+    s = torch.tensor([0.5], device=device)
+    want = matmul(a, b, trans_b=True, scale_a=s, scale_b=0.25, out_dtype=torch.float32, kernel_configs={})
+    for sa in (s, 0.5, s.to(torch.float16), s.double()):
+        assert torch.equal(matmul(a, b, trans_b=True, scale_a=sa, scale_b=0.25, out_dtype=torch.float32), want)
+    kw = dict(trans_a=True, trans_b=True, scale_a=s, scale_b=0.25, out_dtype=torch.float32)
+    at = a.t().contiguous()
+    assert torch.equal(matmul(at, b, **kw), matmul(at, b, kernel_configs={}, **kw))
+    assert matmul(a[:0], b, trans_b=True).shape == (0, 24)
+    As, Bs = torch.rand(6, 2, generator=g).to(device), torch.rand(1, 2, generator=g).to(device)
+    want = w8a8_block_fp8_matmul(a, b, As, Bs, None, torch.float32, kernel_configs={})
+    got = w8a8_block_fp8_matmul(a.view(2, 3, 256), b, As.view(2, 3, 2), Bs, [128, 128], torch.float32)
+    assert got.shape == (2, 3, 24) and torch.equal(got.view(6, 24), want)
+    assert torch.equal(w8a8_block_fp8_matmul(a, b, As.half(), Bs, None, torch.float32),
+                       w8a8_block_fp8_matmul(a, b, As.half().float(), Bs, None, torch.float32))
+    with pytest.raises(AssertionError):
+        matmul(a, b[:, :128].contiguous(), trans_b=True)
+    with pytest.raises(AssertionError):
+        matmul(a, b.t(), out_dtype=torch.float32)
+    with pytest.raises(NotImplementedError):
+        matmul(a, b, trans_b=True, out_dtype=torch.float64)
+    with pytest.raises(_lib.TileGymHipError):
+        _lib.fp8_gemm(torch.empty(6, 23, device=device), a, b)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 16, 128), (96, 144, 256), (130, 272, 1040), (65, 4112, 4096), (300, 128, 200), (20, 4080, 1008)])
 def test_kn_weights_give_the_bits_of_nk_weights(device, M, N, K):
     """(K, N) weights go through the 16-byte transpose: edges of its 128 x 128 tiles in both directions, a padded K (rows of the

@@ -1,5 +1,7 @@
-"""ctypes binding of libtilegym_hip.so: tensor descriptors, return-code checks, workspaces.
+"""Binding of libtilegym_hip.so: tensor descriptors, return-code checks, workspaces.
 
+Ordinary calls of the operators go through the extension module ``_native`` (csrc/binding.cpp), which checks, allocates and
+calls the C ABI in native code; everything else -- schedule overrides, unusual layouts, the helpers -- through ctypes here.
 This is the only module that touches the shared library.  It never falls back to another
 implementation: if the library is missing or a call fails, it raises.
 
@@ -11,7 +13,6 @@ from __future__ import annotations
 
 import ctypes
 import struct
-import weakref
 import os
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -64,6 +65,9 @@ class TileGymHipError(RuntimeError):
 
 
 _lib = None
+native = None  # the extension module, once load() has run
+_NATIVE_ENTRY_POINTS = ("tg_fp8_gemm", "tg_fp8_gemm_workspace_bytes", "tg_fp8_ragged_gemm", "tg_fp8_quant_group", "tg_fp8_fused_moe",
+                        "tg_fp8_fused_moe_workspace_bytes")
 
 
 def lib_path() -> str:
@@ -138,8 +142,27 @@ def load():
     L.tg_diag_mfma.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, P, ctypes.c_int32, ctypes.c_uint64]
     if L.tg_abi_version() != 1:
         raise RuntimeError(f"libtilegym_hip.so ABI version {L.tg_abi_version()} != 1")
+    try:
+        from . import _native
+    except ImportError as e:
+        raise RuntimeError(f"tilegym_amd/_native.so cannot be loaded ({e}); build it with `python -m tilegym_amd.build`. "
+                           f"There is no fallback implementation.") from e
+    _native.set_up({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _NATIVE_ENTRY_POINTS}, _workspaces,
+                   workspace_for, check_rc)
+    global native
+    native = _native
     _lib = L
     return L
+
+
+def loaded() -> bool:
+    """Load the library if it is not; True (a missing one raises)."""
+    return _lib is not None or load() is not None
+
+
+def fast_path() -> bool:
+    """Whether a dense call without kernel_configs may go straight to the native module: no schedule table to look up."""
+    return loaded() and not schedules_recorded()
 
 
 def make_tensor_desc(t: Optional[torch.Tensor]) -> Optional[TgTensor]:
@@ -303,40 +326,7 @@ def _stream_handle(t: torch.Tensor) -> int:
 
 
 # ---------------------------------------------------------------------------- raw calls
-# tg_fp8_gemm is called with the same weights, and often with the same activation and output buffers, over and over by
-# a decode loop, and building six descriptors, the cfg array and the workspace size costs more host time (~15 us) than a
-# small decode kernel runs (6 - 20 us).  Two caches take most of that away:
-#   * per call: the prepared arguments of a call whose five tensors are the very objects of an earlier call, keyed by
-#     their identities.  A hit is checked on every use (weak references to the tensors, their data pointers, shapes and strides),
-#     so a tensor that was freed, resized or given new storage is described afresh; a key whose entry keeps failing that
-#     check (Python hands the address of a freed tensor object to the next one, so fresh outputs repeat ids) is marked
-#     volatile and no longer kept;
-#   * per weight: the descriptors of b and scale_b, keyed and checked the same way, for calls whose activations and
-#     outputs are fresh tensors every time; and the workspace size per (M, N, K, trans_b).
-_gemm_calls: Dict[tuple, object] = {}
-_weight_descs: Dict[int, tuple] = {}
-_ws_bytes: Dict[tuple, int] = {}
 _CACHE_MAX = 4096
-_VOLATILE = object()
-
-
-def _same(ref, ptr, t) -> bool:
-    return (t is None) if ref is None else (ref() is t and t.data_ptr() == ptr)
-
-
-def _weight_desc(t):
-    """Descriptor of a long-lived tensor (None -> None), cached by identity and checked against the object's current
-    storage, shape and strides."""
-    if t is None:
-        return None
-    hit = _weight_descs.get(id(t))
-    if hit is not None and hit[0]() is t and t.data_ptr() == hit[1] and t.shape == hit[2] and t.stride() == hit[3]:
-        return hit[4]
-    d = _desc(t)
-    if len(_weight_descs) >= _CACHE_MAX:
-        _weight_descs.clear()
-    _weight_descs[id(t)] = (weakref.ref(t), t.data_ptr(), t.shape, t.stride(), d)
-    return d
 
 
 # ---- recorded schedules: TILEGYM_HIP_TUNE names a JSON file written by ``python -m tilegym_amd.tune`` that maps
@@ -348,8 +338,7 @@ _tune_table: Optional[Dict[tuple, dict]] = None
 
 
 def load_tune_table(path: Optional[str] = None) -> Dict[tuple, dict]:
-    """(Re)load the schedule table from ``path`` (default: the file TILEGYM_HIP_TUNE names; no file -> empty table) and forget
-    the prepared calls that were made under the previous one."""
+    """(Re)load the schedule table from ``path`` (default: the file TILEGYM_HIP_TUNE names; no file -> empty table)."""
     global _tune_table
     import json
     path = path if path is not None else os.environ.get(TUNE_ENV)
@@ -360,9 +349,12 @@ def load_tune_table(path: Optional[str] = None) -> Dict[tuple, dict]:
         for e in doc.get("entries", []):
             table[(int(e["M"]), int(e["N"]), int(e["K"]), bool(e.get("block_scaled", False)))] = dict(e["kernel_configs"])
     _tune_table = table
-    _gemm_calls.clear()
-    _ws_bytes.clear()
     return table
+
+
+def schedules_recorded() -> bool:
+    """Whether a table of recorded schedules is loaded (then calls without kernel_configs look their shape up in it)."""
+    return bool(_tune_table if _tune_table is not None else load_tune_table())
 
 
 def _tuned_cfg(M: int, N: int, K: int, block_scaled: bool):
@@ -375,90 +367,29 @@ def _tuned_cfg(M: int, N: int, K: int, block_scaled: bool):
     return _cfg(None)
 
 
-def _gemm_constants(a, b, scale_b, trans_a, trans_b, use_workspace):
-    M = a.shape[1] if trans_a else a.shape[0]
-    K = a.shape[0] if trans_a else a.shape[1]
-    N = b.shape[0] if trans_b else b.shape[1]
-    cfg, ncfg = _tuned_cfg(M, N, K, scale_b is not None and scale_b.numel() > 1)
-    ws_bytes = 0
-    if use_workspace and M > 0 and N > 0 and K > 0:
-        key = (M, N, K, trans_b, cfg is _cfg(None)[0])
-        ws_bytes = _ws_bytes.get(key) if key[4] else None   # (a recorded schedule may ask for another split)
-        if ws_bytes is None:
-            if len(_ws_bytes) >= _CACHE_MAX:
-                _ws_bytes.clear()
-            ws_bytes = workspace_bytes(M, N, K, trans_b, cfg, ncfg)
-            if key[4]:
-                _ws_bytes[key] = ws_bytes
-    return cfg, ncfg, ws_bytes
-
-
-def _prepared_gemm(c, a, b, scale_a, scale_b, trans_a, trans_b, use_workspace):
-    """(argument references, cfg, ncfg, device index, workspace bytes, device, keep-alive) of a call without kernel_configs."""
-    key = (id(c), id(a), id(b), id(scale_a), id(scale_b), trans_a, trans_b, use_workspace)
-    hit = _gemm_calls.get(key)
-    if hit is not None and hit is not _VOLATILE:
-        refs, ptrs, shapes = hit[0], hit[1], hit[2]
-        if (_same(refs[0], ptrs[0], c) and _same(refs[1], ptrs[1], a) and _same(refs[2], ptrs[2], b)
-                and _same(refs[3], ptrs[3], scale_a) and _same(refs[4], ptrs[4], scale_b)
-                and c.shape == shapes[0] and a.shape == shapes[1] and b.shape == shapes[2]
-                and c.stride() == shapes[3] and a.stride() == shapes[4] and b.stride() == shapes[5]):
-            return hit[3]
-        hit[4][0] += 1
-    dev = _device_index(a)
-    cfg, ncfg, ws_bytes = _gemm_constants(a, b, scale_b, trans_a, trans_b, use_workspace)
-    if hit is _VOLATILE or (hit is not None and hit[4][0] >= 2):
-        _gemm_calls[key] = _VOLATILE
-        descs = (_desc(c), _desc(a), _weight_desc(b), _desc(scale_a), _weight_desc(scale_b))
-        return tuple(_ref(d) for d in descs), cfg, ncfg, dev, ws_bytes, a.device, descs
-    tensors = (c, a, b, scale_a, scale_b)
-    descs = (_desc(c), _desc(a), _weight_desc(b), _desc(scale_a), _weight_desc(scale_b))
-    prepared = (tuple(_ref(d) for d in descs), cfg, ncfg, dev, ws_bytes, a.device, descs)
-    if len(_gemm_calls) >= _CACHE_MAX:
-        _gemm_calls.clear()
-    _gemm_calls[key] = (tuple(None if t is None else weakref.ref(t) for t in tensors),
-                        tuple(0 if t is None else t.data_ptr() for t in tensors),
-                        (c.shape, a.shape, b.shape, c.stride(), a.stride(), b.stride()), prepared,
-                        hit[4] if hit is not None else [0])
-    return prepared
-
-
 def release_call_caches() -> None:
-    """Forget every prepared call and cached descriptor (they hold no tensor alive; this only frees the bookkeeping)."""
-    _gemm_calls.clear()
-    _weight_descs.clear()
-    _ws_bytes.clear()
+    """Forget the sizes kept per layer shape (bookkeeping only: nothing about tensors is kept)."""
+    _moe_ws_bytes.clear()
 
 
 def fp8_gemm(c, a, b, scale_a=None, scale_b=None, trans_a=False, trans_b=True, alpha=1.0, beta=0.0,
              kernel_configs=None, use_workspace=True) -> None:
     L = _lib if _lib is not None else load()
-    if kernel_configs is None:
-        refs, cfg, ncfg, dev, ws_bytes, device, _ = _prepared_gemm(c, a, b, scale_a, scale_b, bool(trans_a), bool(trans_b),
-                                                                   bool(use_workspace))
-        stream = _raw_stream(dev)
-        dws = None
-        if ws_bytes > 0:
-            dws = _ref(_weight_desc(workspace_for(device, ws_bytes, dev, stream)))
-        rc = L.tg_fp8_gemm(refs[0], refs[1], refs[2], refs[3], refs[4], 1 if trans_a else 0, 1 if trans_b else 0,
-                           alpha if type(alpha) is float else float(alpha), beta if type(beta) is float else float(beta),
-                           dws, cfg, ncfg, dev, stream)
-        if rc != 0:
-            check_rc(rc, "tg_fp8_gemm")
+    trans_a, trans_b = bool(trans_a), bool(trans_b)
+    if (kernel_configs is None and not schedules_recorded()
+            and native.gemm(c, a, b, scale_a, scale_b, trans_a, trans_b, float(alpha), float(beta), bool(use_workspace))):
         return
     dev = _device_index(a)
-    cfg, ncfg = make_cfg(kernel_configs)
     M = a.shape[1] if trans_a else a.shape[0]
     K = a.shape[0] if trans_a else a.shape[1]
     N = b.shape[0] if trans_b else b.shape[1]
+    cfg, ncfg = (make_cfg(kernel_configs) if kernel_configs is not None
+                 else _tuned_cfg(M, N, K, scale_b is not None and scale_b.numel() > 1))
     ws = None
     if use_workspace and M > 0 and N > 0 and K > 0:
         ws = workspace_for(a.device, workspace_bytes(M, N, K, trans_b, cfg, ncfg))
-    dc, da, db = _desc(c), _desc(a), _desc(b)
-    dsa, dsb, dws = _desc(scale_a), _desc(scale_b), _desc(ws)
-    rc = L.tg_fp8_gemm(_ref(dc), _ref(da), _ref(db), _ref(dsa), _ref(dsb), int(bool(trans_a)),
-                       int(bool(trans_b)), float(alpha), float(beta), _ref(dws), cfg, ncfg, dev,
-                       _stream_handle(a))
+    rc = L.tg_fp8_gemm(_desc(c), _desc(a), _desc(b), _desc(scale_a), _desc(scale_b), int(trans_a), int(trans_b), float(alpha), float(beta),
+                       _desc(ws), cfg, ncfg, dev, _stream_handle(a))
     check_rc(rc, "tg_fp8_gemm")
 
 
@@ -483,7 +414,7 @@ def fp8_ragged_gemm(c, a, b, a_scale, b_scale, m_indptr, kernel_configs=None) ->
     L = load()
     dev = _device_index(a)
     cfg, ncfg = _cfg(kernel_configs)
-    rc = L.tg_fp8_ragged_gemm(_desc(c), _desc(a), _weight_desc(b), _desc(a_scale), _weight_desc(b_scale), _desc(m_indptr),
+    rc = L.tg_fp8_ragged_gemm(_desc(c), _desc(a), _desc(b), _desc(a_scale), _desc(b_scale), _desc(m_indptr),
                               cfg, ncfg, dev, _stream_handle(a))
     check_rc(rc, "tg_fp8_ragged_gemm")
 
@@ -493,7 +424,7 @@ def fp8_moe_gemm(c, a, b, a_scale, b_scale, topk_weights, sorted_token_ids, expe
     L = load()
     dev = _device_index(a)
     cfg, ncfg = _cfg(kernel_configs)
-    rc = L.tg_fp8_moe_gemm(_desc(c), _desc(a), _weight_desc(b), _desc(a_scale), _weight_desc(b_scale), _desc(topk_weights),
+    rc = L.tg_fp8_moe_gemm(_desc(c), _desc(a), _desc(b), _desc(a_scale), _desc(b_scale), _desc(topk_weights),
                            _desc(sorted_token_ids), _desc(expert_ids), _desc(num_tokens_post_padded),
                            int(bool(mul_routed_weight)), int(top_k), int(block_m), cfg, ncfg, dev, _stream_handle(a))
     check_rc(rc, "tg_fp8_moe_gemm")
@@ -514,7 +445,7 @@ def fp8_moe_gemm_silu_quant(a, b, a_scale, b_scale, sorted_token_ids, expert_ids
     inter = b.shape[1] // 2
     q = torch.empty((num_valid, inter), dtype=torch.float8_e4m3fn, device=a.device)
     scales = torch.empty((num_valid, inter // 128), dtype=torch.float32, device=a.device)
-    rc = L.tg_fp8_moe_gemm_silu_quant(_desc(q), _desc(scales), _desc(a), _weight_desc(b), _desc(a_scale), _weight_desc(b_scale),
+    rc = L.tg_fp8_moe_gemm_silu_quant(_desc(q), _desc(scales), _desc(a), _desc(b), _desc(a_scale), _desc(b_scale),
                                       _desc(sorted_token_ids), _desc(expert_ids), _desc(num_tokens_post_padded),
                                       int(top_k), int(block_m), _DTYPE_CODES[act_dtype], dev, _stream_handle(a))
     check_rc(rc, "tg_fp8_moe_gemm_silu_quant")
@@ -697,8 +628,8 @@ def fp8_fused_moe(out, hidden, w1, w2, w1_scale, w2_scale, topk_weights, topk_id
         need = _moe_ws_bytes[key] = int(L.tg_fp8_fused_moe_workspace_bytes(T, k, E, H, two_i // 2, block_m))
     stream = _raw_stream(dev)
     ws = workspace_for(hidden.device, need, dev, stream)
-    rc = L.tg_fp8_fused_moe(_desc(out), _desc(hidden), _weight_desc(w1), _weight_desc(w2), _weight_desc(w1_scale),
-                            _weight_desc(w2_scale), _desc(topk_weights), _desc(topk_ids), _weight_desc(ws), int(block_m), dev, stream)
+    rc = L.tg_fp8_fused_moe(_desc(out), _desc(hidden), _desc(w1), _desc(w2), _desc(w1_scale),
+                            _desc(w2_scale), _desc(topk_weights), _desc(topk_ids), _desc(ws), int(block_m), dev, stream)
     if rc != 0:
         check_rc(rc, "tg_fp8_fused_moe")
 

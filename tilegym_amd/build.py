@@ -1,4 +1,5 @@
-"""Build recipe for libtilegym_hip.so (hipcc, gfx950).  Cross-compiles without a GPU."""
+"""Build recipe for libtilegym_hip.so (hipcc, gfx950) and the Python binding _native.so (g++ against the installed torch).
+Cross-compiles without a GPU."""
 
 from __future__ import annotations
 
@@ -8,10 +9,11 @@ import subprocess
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(_HERE, "libtilegym_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 
 def build(force: bool = True, jobs: int = 8, verbose: bool = False, check: bool = False) -> str:
-    """Compile every HIP translation unit and link the shared library in-tree.
+    """Compile every HIP translation unit and link the shared library and the binding in-tree.
 
     ``force=True`` rebuilds all objects (``make -B``); returns the library path.  ``check=True`` also runs
     ``make check``: the kernels' assembly against the hardware rules around their inline-assembly loads
@@ -23,9 +25,10 @@ def build(force: bool = True, jobs: int = 8, verbose: bool = False, check: bool 
     if verbose or res.returncode != 0:
         print(res.stdout)
     if res.returncode != 0:
-        raise RuntimeError("hipcc build of libtilegym_hip.so failed (see output above)")
-    if not os.path.exists(LIB_PATH):
-        raise RuntimeError(f"build finished but {LIB_PATH} is missing")
+        raise RuntimeError("build of libtilegym_hip.so / _native.so failed (see output above)")
+    for path in (LIB_PATH, NATIVE_PATH):
+        if not os.path.exists(path):
+            raise RuntimeError(f"build finished but {path} is missing")
     if check:
         res = subprocess.run(["make", "-C", CSRC, "check"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         if verbose or res.returncode != 0:

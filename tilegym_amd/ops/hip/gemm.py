@@ -39,8 +39,13 @@ def _split_scale(scale, alpha: float):
 
 @register_impl("matmul", backend="hip")
 def matmul(a, b, trans_a=None, trans_b=None, static_persistent=None, use_tma=None, **kwargs):
-    trans_a = bool(trans_a) if trans_a is not None else False
-    trans_b = bool(trans_b) if trans_b is not None else False
+    trans_a = bool(trans_a)
+    trans_b = bool(trans_b)
+    if kwargs.get("kernel_configs") is None and _lib.fast_path():
+        c = _lib.native.matmul(a, b, trans_a, trans_b, kwargs.get("scale_a"), kwargs.get("scale_b"), float(kwargs.get("alpha", 1.0)),
+                               kwargs.get("out_dtype"))
+        if c is not None:
+            return c
     _require_fp8(a, b)
     if a.dim() != 2 or b.dim() != 2:
         raise ValueError("matmul expects 2-D operands")
@@ -99,6 +104,11 @@ def gemm_alpha_beta(a, b, c, trans_a=False, trans_b=True, alpha=1.0, beta=0.0, n
 def w8a8_block_fp8_matmul(A, B, As, Bs, block_size: Optional[Sequence[int]] = None,
                           output_dtype: torch.dtype = torch.float32, **kwargs):
     """Block-scaled FP8 GEMM (src/tilegym/suites/unsloth/cutile/fp8.py:388-446)."""
+    if ((block_size is None or (len(block_size) == 2 and block_size[0] == 128 and block_size[1] == 128))
+            and kwargs.get("kernel_configs") is None and _lib.fast_path()):
+        C = _lib.native.block_matmul(A, B, As, Bs, output_dtype)
+        if C is not None:
+            return C
     if block_size is None:
         block_n, block_k = 128, 128
     else:
@@ -138,6 +148,10 @@ def ragged_block_scaled_bmm(a, b, a_scale, b_scale, m_indptr, max_m, max_m_devic
     ``max_m`` / ``max_m_device`` bound the reference's uniform tile walk; the expert-offset
     launch here reads the segment sizes on the device, so both are accepted and unused."""
     assert transpose_a == False and transpose_b == True, "Only NT layout is supported"  # noqa: E712
+    if not kwargs and _lib.loaded():
+        c = _lib.native.ragged_matmul(a, b, a_scale, b_scale, m_indptr, out_dtype)
+        if c is not None:
+            return c
     assert a.is_contiguous(), "A matrix must be contiguous"
     assert b.is_contiguous(), "B matrix must be contiguous"
     assert a_scale is None or a_scale.is_contiguous(), "A scale matrix must be contiguous"

@@ -33,6 +33,10 @@ def _require_device(x: torch.Tensor, what: str, group: int) -> None:
 def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-token 1 x block_size quantization; all-zero block -> scale 1.0
     (src/tilegym/suites/unsloth/cutile/fp8.py:370-385)."""
+    if block_size in _GROUPS and _lib.loaded():
+        out = _lib.native.act_quant(x, block_size, 0.0, 0)
+        if out is not None:
+            return out
     assert x.shape[-1] % block_size == 0, "last dim must be divisible by block_size"
     _require_device(x, "act_quant", block_size)
     return _lib.fp8_quant_group(x, block_size, 0.0, 0)
