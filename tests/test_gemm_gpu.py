@@ -1825,6 +1825,26 @@ def test_kn_weights_give_the_bits_of_nk_weights(device, M, N, K):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (16, 48, 256), (17, 4112, 384), (33, 80, 640), (64, 144, 1152), (65, 208, 128), (100, 2064, 1024),
+                                   (256, 1040, 512), (512, 64, 512), (64, 16400, 1152)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32, FP8])
+def test_kn_weights_read_as_they_lie(device, M, N, K, out_dtype):
+    """(K, N) weights that the narrow tiles turn inside LDS: columns and rows that end inside a tile, fewer K steps than waves.
+    The same tile asked for by name works on the (N, K) copy: the same products added in the same order, so the bits agree."""
+    g = _g(M * 3 + N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.3)
+    kn = b.view(torch.uint8).t().contiguous().view(FP8).to(device)
+    kw = dict(scale_a=0.25, scale_b=0.5, out_dtype=out_dtype)
+    got = matmul(a.to(device), kn, **kw)
+    cfg = _lib.last_config()
+    assert cfg["KERNEL_NAME"] == "tiled" and cfg["BLOCK_N"] <= 64
+    kc = {"KERNEL": "tiled", "BLOCK_M": cfg["BLOCK_M"], "BLOCK_N": cfg["BLOCK_N"]}
+    want = matmul(a.to(device), kn, kernel_configs=kc, **kw)
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    if out_dtype is torch.bfloat16:
+        check(got, R.ref_gemm_per_tensor(a, b, 0.25, 0.5, trans_b=True))
+
+
 @pytest.mark.parametrize("T,H,I,E,k,dtype,skew", [
     (1, 640, 384, 40, 8, torch.bfloat16, 0),      # sum form; K tails of one and of three steps (5 and 3 K steps)
     (2, 512, 1408, 64, 6, torch.float16, 0),      # sum form, two tokens

@@ -19,9 +19,9 @@ int compute_units() {
 }
 
 hipError_t run_tile256(const GemmParams& p, int gx, hipStream_t s) { return launch_tile256(p, gx, compute_units(), s); }
-hipError_t run_tile_mid(int bm, int bn, const GemmParams& p, hipStream_t s) {
-    if (bn == 64) return launch_tile_mid<64, 64, 2>(p, s);
-    return bm == 32 ? launch_tile_mid<32, 32, 4>(p, s) : launch_tile_mid<64, 32, 3>(p, s);
+hipError_t run_tile_mid(int bm, int bn, bool kn, const GemmParams& p, hipStream_t s) {
+    if (bn == 64) return launch_tile_mid<64, 64, 2>(p, kn, s);
+    return bm == 32 ? launch_tile_mid<32, 32, 4>(p, kn, s) : launch_tile_mid<64, 32, 3>(p, kn, s);
 }
 
 }  // namespace tg

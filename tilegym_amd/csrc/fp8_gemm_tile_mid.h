@@ -22,13 +22,28 @@
 // bytes of 16 rows where a direct load fetches 128 bytes of 8; eight waves per workgroup splitting K eight ways with
 // half the stages each: 2 - 8 % slower.
 // Slab layout, swizzles and fragment addressing are those of fp8_gemm_tile.h.
+//
+// KN: the weight is (K, N), a K step of it 128 rows of BN bytes.  They are staged as they lie and turned on the way out of LDS
+// (ds_read_b64_tr_b8: 16 lanes fetch 8 K rows x 16 columns and each gets 8 K bytes of one column), so no (N, K) copy is made.
+// The fragments hold the same K bytes in the same places: the bits of the (N, K) form.
+// Bound by the cache lines a compute unit takes in: a load instruction touches 16 or 32 lines (64 or 32 bytes of each) where the
+// (N, K) form's touches 8, so a K step takes two to three times as long, and what pays for it is the copy that is not made.
+// Copy + GEMM -> this, us: 28672 x 4096 weight M = 1 64.5 -> 35.6, M = 64 67.8 -> 40.9; 12288 x 5120 M = 16 40.0 -> 25.0; 6144 x 4096
+// M = 64 21.0 -> 18.6; 1024 x 1024 M = 256 7.8 -> 5.3; 4096 x 4096 M = 256 19.1 -> 18.1 (M = 64: 15.2 against 16.0, copied).  Tiles in
+// the order of the workgroups instead of neighbours on one XCD: 5 - 25 % slower (28672 x 4096: 42.9 at M = 1).
 #pragma once
 
 #include "fp8_gemm_tile.h"
 
 namespace tg {
 
-template <int BM, int BN, int STAGES>
+// Bytes of the (K, N) slab that 16 lanes turn: lane i of them fetches 8 bytes of K row i / 2, columns 8 (i % 2) ..., and receives
+// column i of the 8 rows.
+__device__ __forceinline__ v2i lds_read_transposed_8x16(uint32_t address) {
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(uintptr_t)address);
+}
+
+template <int BM, int BN, int STAGES, bool KN>
 __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NW = 4;
@@ -45,12 +60,15 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = p.K;
-    const int n0 = (int)blockIdx.x * BN, m0 = (int)blockIdx.y * BM;
+    // (KN: neighbouring tiles share the 128-byte lines of a K row, so they go to one XCD's L2)
+    const int n0 = (KN ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x) * BN, m0 = (int)blockIdx.y * BM;
     const int rows_valid = min(BM, p.M - m0);
     // this wave's K steps: a contiguous share
     const int ks = (int)((int64_t)p.kblocks * wave / NW), ks_end = (int)((int64_t)p.kblocks * (wave + 1) / NW);
     const int nsteps = ks_end - ks;
 
+    // KN: spreads the 8 rows x 16 bytes that two groups of 16 lanes fetch at once over all banks
+    auto kn_swz = [](int r) { return BN == 64 ? ((r >> 2) & 1) | ((r >> 3) & 2) : (r >> 4) & 1; };
     const int lrow = lane >> 3;
     const int lj = (lane & 7) ^ swz16(lrow);
     uint32_t a_off[A_IT], b_off[B_IT];
@@ -61,6 +79,12 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
     }
 #pragma unroll
     for (int i = 0; i < B_IT; ++i) {
+        if constexpr (KN) {
+            // LDS position lane * 16 of load i: K row r, 16-byte place q, which holds chunk q ^ kn_swz(r) (columns past N repeat the last ones)
+            const int r = i * (1024 / BN) + lane / (BN / 16), q = lane % (BN / 16);
+            b_off[i] = (uint32_t)r * (uint32_t)p.N + min(n0 + ((q ^ kn_swz(r)) << 4), p.N - 16);
+            continue;
+        }
         const int br = i * 8 + lrow;
         const int ljb = (lane & 7) ^ swz_w(((i & 1) << 3) | lrow);
         b_off[i] = (uint32_t)min(n0 + br, p.N - 1) * (uint32_t)K + ljb * 16;
@@ -72,7 +96,10 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
         const int k0 = kstep * kKBlock;
         const uint32_t dst = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-        for (int i = 0; i < B_IT; ++i) direct_load_b128_nt(rsrc_b, dst + BM * kKBlock + i * 1024, b_off[i], k0);
+        for (int i = 0; i < B_IT; ++i) {
+            if constexpr (KN) direct_load_b128(rsrc_b, dst + BM * kKBlock + i * 1024, b_off[i], k0 * p.N);
+            else direct_load_b128_nt(rsrc_b, dst + BM * kKBlock + i * 1024, b_off[i], k0);
+        }
 #pragma unroll
         for (int i = 0; i < A_IT; ++i) direct_load_b128(rsrc_a, dst + i * 1024, a_off[i], k0);
     };
@@ -106,6 +133,18 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
         v8i af[TM], wf[TN];
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) {
+            if constexpr (KN) {
+                // columns tn * 16 + li; K bytes lg * 16 ... + 15 and 64 + lg * 16 ... + 15, eight at a time
+                const uint32_t slab = lds0 + stage * STAGE_BYTES + BM * kKBlock;
+                v2i part[4];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const int r = (h >> 1) * 64 + lg * 16 + (h & 1) * 8 + (li >> 1);
+                    part[h] = lds_read_transposed_8x16(slab + r * BN + ((tn ^ kn_swz(r)) << 4) + (li & 1) * 8);
+                }
+                wf[tn] = v8i{part[0][0], part[0][1], part[1][0], part[1][1], part[2][0], part[2][1], part[3][0], part[3][1]};
+                continue;
+            }
             const uint8_t* b = base + ((tn >> 1) * 32 + (tn & 1) * 4) * kKBlock;
             wf[tn] = join(*reinterpret_cast<const v4i*>(b + wfrag0), *reinterpret_cast<const v4i*>(b + wfrag1));
         }
@@ -147,11 +186,15 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
     for (int u = wave; u < TM * (TN / 2); u += NW) {
         const int tm = u / (TN / 2), tp = u % (TN / 2);
         const int rt = tm * 16 + li;
-        v4f s0 = red[((0 * TN + 2 * tp) * TM + tm) * 64 + lane], s1 = red[((0 * TN + 2 * tp + 1) * TM + tm) * 64 + lane];
+        // the lane's eight columns are one of its own registers in both tiles of the pair; KN, where tile t holds columns
+        // 16 t ..., two neighbouring lane groups of one tile
+        const int at0 = KN ? ((2 * tp + (lg >> 1)) * TM + tm) * 64 + (lg & 1) * 32 + li : (2 * tp * TM + tm) * 64 + lane;
+        const int at1 = KN ? at0 + 16 : at0 + TM * 64;
+        v4f s0 = red[at0], s1 = red[at1];
 #pragma unroll
         for (int w = 1; w < NW; ++w) {
-            s0 += red[((w * TN + 2 * tp) * TM + tm) * 64 + lane];
-            s1 += red[((w * TN + 2 * tp + 1) * TM + tm) * 64 + lane];
+            s0 += red[w * TN * TM * 64 + at0];
+            s1 += red[w * TN * TM * 64 + at1];
         }
         const int c = col + tp * 32;
         if (rt < rows_valid && c < p.N) store8(p.C, p.out_type, m0 + rt, c, p.N, p.ldc, s0 * scale, s1 * scale, p.beta, vec_ok);
@@ -160,8 +203,13 @@ __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmPar
 }
 
 template <int BM, int BN, int STAGES>
-inline hipError_t launch_tile_mid(const GemmParams& p, hipStream_t stream) {
-    hipLaunchKernelGGL((fp8_gemm_tile_mid_kernel<BM, BN, STAGES>), dim3((p.N + BN - 1) / BN, (p.M + BM - 1) / BM, 1), dim3(256, 1, 1), 0, stream, p);
+inline hipError_t launch_tile_mid(const GemmParams& p, bool kn, hipStream_t stream) {
+    // (K, N): 16-byte pieces of whole K rows, 32-bit offsets
+    if (kn && (p.N < 16 || p.N % 16 != 0 || p.K % kKBlock != 0 || (int64_t)p.N * p.K >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
+    if (kn)
+        hipLaunchKernelGGL((fp8_gemm_tile_mid_kernel<BM, BN, STAGES, true>), dim3((p.N + BN - 1) / BN, (p.M + BM - 1) / BM, 1), dim3(256, 1, 1), 0, stream, p);
+    else
+        hipLaunchKernelGGL((fp8_gemm_tile_mid_kernel<BM, BN, STAGES, false>), dim3((p.N + BN - 1) / BN, (p.M + BM - 1) / BM, 1), dim3(256, 1, 1), 0, stream, p);
     return hipGetLastError();
 }
 

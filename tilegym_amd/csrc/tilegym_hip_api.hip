@@ -546,6 +546,41 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     return s;
 }
 
+// No kernel, tile, split or wave count asked for.
+bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
+    for (int slot : {TG_CFG_KERNEL, TG_CFG_BLOCK_M, TG_CFG_BLOCK_N, TG_CFG_SPLIT_K, TG_CFG_ROW_GROUPS, TG_CFG_WAVES})
+        if (cfg_get(cfg, ncfg, slot) >= 0) return false;
+    return true;
+}
+
+// A per-tensor (K, N) weight: whether the narrow tiles read it as it lies, and with which tile; else it is copied to (N, K)
+// first and any kernel takes it.  Costs in us like tile_cost_us's, fitted by hand to 8 weights x 12 row counts (1 ... 512), both
+// ways measured: a direct tile's K step takes 0.39 - 0.45 us whatever the grid; the copy 3 us + 0.36 us per MB, and up to
+// 64 rows copy and GEMM together 7 us + 0.5 us per MB.  Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 against
+// 65.4; 1024 x 1024: 5.2 against 7.7), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied;
+// 2048 x 6144: 20.7 against 16.4), and so are most from 256 rows on (6144 x 4096 at M = 256: 28.3 direct, 24.9 copied).
+constexpr TileCost kKnTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
+constexpr float kKnMargin = 1.05f, kCopyUs = 3.0f, kCopyUsPerMB = 0.36f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
+bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, int* bm, int* bn) {
+    if (M > 512 || N % 16 != 0 || K % 128 != 0) return false;
+    const int64_t kblocks = K / 128;
+    const float mb = (float)(N * K) * 1e-6f;
+    float best = 0.f;
+    *bm = -1;
+    for (const TileCost& t : kKnTiles) {
+        const float tiles = (float)(cdiv(M, t.bm) * cdiv(N, t.bn));   // one workgroup per compute unit
+        const float us = (tiles > 256.f ? tiles / 256.f : 1.f) * ((float)kblocks * t.alone + t.fixed);
+        if (*bm < 0 || us < best) { best = us; *bm = t.bm; *bn = t.bn; }
+    }
+    if (M <= 64) return best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
+    int nk_bm = -1, nk_bn = -1, nk_split = 1;
+    pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, &nk_bm, &nk_bn, &nk_split);
+    float nk = 0.f;
+    for (const TileCost& t : kPerTensorTiles)
+        if (t.bm == nk_bm && t.bn == nk_bn) nk = tile_cost_us(t, M, N, kblocks, nk_split);
+    return best * kKnMargin <= nk + kCopyUs + kCopyUsPerMB * mb;
+}
+
 struct Resolved {
     int64_t M, N, K;
     bool block_scaled;
@@ -870,10 +905,14 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     const uint8_t* Bnt = reinterpret_cast<const uint8_t*>(b->ptr);
     bool b_is_nk = trans_b != 0;
     const int want_kernel = cfg_get(cfg, ncfg, TG_CFG_KERNEL);
+    bool direct_kn = false;   // a (K, N) weight read as it lies by the narrow tiles
+    int kn_bm = -1, kn_bn = -1;
     if (!b_is_nk && !trans_a && want_kernel != 0 && K > 0) {
         // (K,N) weights: make a K-contiguous copy at the tail of the workspace when it fits
         const int64_t need = (N * K + 255) / 256 * 256;
-        if (ws_free >= need) {
+        direct_kn = ws_free >= need && !static_scratch && !block_scaled && M * K < kOffsetLimit && N * K < kOffsetLimit && aligned16(a->ptr) && aligned16(b->ptr) &&
+                    nothing_forced(cfg, ncfg) && pick_kn_tile(M, N, K, ws_free - need, &kn_bm, &kn_bn);
+        if (!direct_kn && ws_free >= need) {
             uint8_t* bt = ws + ws_bytes - need;
             bt = reinterpret_cast<uint8_t*>(reinterpret_cast<uintptr_t>(bt) & ~(uintptr_t)15);
             if (bt >= ws_cursor) {
@@ -888,7 +927,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
 
     const bool fast_layout = !trans_a && b_is_nk && (K % 16) == 0 && aligned16(a->ptr) &&
                              aligned16(reinterpret_cast<uint64_t>(Bnt)) && N * K < kOffsetLimit && (!block_scaled || std_blocks);
-    Schedule s = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free);
+    Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free);
     if (static_scratch) {
         // same schedule as tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split
         const Schedule full = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, INT64_MAX / 2);
@@ -991,7 +1030,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
                                    N * K < kBs256WeightLimit && pc.As && pc.Bs && cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS) == 1 &&
                                    cfg_get(cfg, ncfg, TG_CFG_WAVES) != 8;
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
-        hipError_t e = mid ? tg::run_tile_mid(s.bm, s.bn, pc, stream)
+        hipError_t e = mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
                      : ordered ? tg::run_tile256(pc, gx, stream)
                      : bs_persistent ? tg::run_bs256(tg::GROUP_DENSE, pc, gx, stream)
                      : deep ? tg::run_tile_deep(split, pc, gx, pc.split_k, stream)
