@@ -1845,6 +1845,20 @@ def test_kn_weights_read_as_they_lie(device, M, N, K, out_dtype):
         check(got, R.ref_gemm_per_tensor(a, b, 0.25, 0.5, trans_b=True))
 
 
+@pytest.mark.parametrize("rows", [8191, 8192, 8195])
+def test_quantizer_with_one_and_four_groups_per_lane(device, rows):
+    """67 M elements are the line between the quantizer's two forms; a tensor on either side of it, and one whose last workgroup
+    is not full, against the same rows in pieces small enough for the other form."""
+    from tilegym_amd.quant import act_quant
+
+    x = torch.randn(rows, 8192, generator=torch.Generator(device=device).manual_seed(rows), device=device).to(torch.bfloat16)
+    x[3, 128:256] = 0
+    q, s = act_quant(x, 128)
+    for lo in range(0, rows, 4096):
+        qp, sp = act_quant(x[lo:lo + 4096], 128)
+        assert torch.equal(q[lo:lo + 4096].view(torch.uint8), qp.view(torch.uint8)) and torch.equal(s[lo:lo + 4096], sp)
+
+
 @pytest.mark.parametrize("T,H,I,E,k,dtype,skew", [
     (1, 640, 384, 40, 8, torch.bfloat16, 0),      # sum form; K tails of one and of three steps (5 and 3 K steps)
     (2, 512, 1408, 64, 6, torch.float16, 0),      # sum form, two tokens

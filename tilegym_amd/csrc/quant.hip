@@ -19,18 +19,18 @@
 // row-major layout and the column-major ones of per_token_group_quant_8bit.py:185-204.
 //
 // HBM-bound: group_size / 8 lanes own one group at a time (8 elements = one 16-byte load of bf16/f16 per
-// lane, two for fp32) and four groups in all, whose loads are issued together; the maximum is reduced over
+// lane, two for fp32), one or four groups in all (kQuantFewWorkgroups), whose loads are issued together; the maximum is reduced over
 // those lanes with cross-lane shuffles, every lane writes 8 bytes of codes and the first lane of the group
 // the scale.  The divisions go through ScaleDivider (bit-equal to the IEEE division).
 #include "quant_device.h"
 
 namespace tg {
 
-template <typename T, int LPG, bool STRIDED, bool I8>
+template <typename T, int LPG, bool STRIDED, bool I8, int G>
 __global__ void __launch_bounds__(256) act_quant_group_kernel(const T* __restrict__ x, uint8_t* __restrict__ q,
                                                              float* __restrict__ scales, int64_t groups, float eps,
                                                              int rule, uint32_t groups_per_row, int64_t s_row, int64_t s_col) {
-    act_quant_group_body<T, LPG, STRIDED, I8>(x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col, (int64_t)blockIdx.x,
+    act_quant_group_body<T, LPG, STRIDED, I8, G>(x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col, (int64_t)blockIdx.x,
                                               (int)threadIdx.x);
 }
 
@@ -140,19 +140,29 @@ __global__ void __launch_bounds__(256) moe_sum_kernel(const T* __restrict__ x, T
     *reinterpret_cast<vecT*>(out + idx) = __builtin_convertvector(acc, vecT);
 }
 
+template <typename T, int LPG, int G>
+static void launch_act_quant_g(const T* x, uint8_t* q, bool i8, float* scales, int64_t groups, float eps, int rule, bool strided,
+                               uint32_t groups_per_row, int64_t s_row, int64_t s_col, hipStream_t s) {
+    constexpr int per_wg = (256 / LPG) * G;
+    const dim3 grid((unsigned)((groups + per_wg - 1) / per_wg)), block(256);
+    if (strided && i8)
+        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, true, true, G>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+    else if (strided)
+        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, true, false, G>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+    else if (i8)
+        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, false, true, G>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+    else
+        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, false, false, G>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+}
+
 template <typename T, int LPG>
 static void launch_act_quant(const T* x, uint8_t* q, bool i8, float* scales, int64_t groups, float eps, int rule, bool strided,
                              uint32_t groups_per_row, int64_t s_row, int64_t s_col, hipStream_t s) {
     constexpr int per_wg = (256 / LPG) * kQuantGroupsPerLane;
-    const dim3 grid((unsigned)((groups + per_wg - 1) / per_wg)), block(256);
-    if (strided && i8)
-        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, true, true>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
-    else if (strided)
-        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, true, false>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
-    else if (i8)
-        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, false, true>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+    if (groups < kQuantFewWorkgroups * per_wg)
+        launch_act_quant_g<T, LPG, 1>(x, q, i8, scales, groups, eps, rule, strided, groups_per_row, s_row, s_col, s);
     else
-        hipLaunchKernelGGL((act_quant_group_kernel<T, LPG, false, false>), grid, block, 0, s, x, q, scales, groups, eps, rule, groups_per_row, s_row, s_col);
+        launch_act_quant_g<T, LPG, kQuantGroupsPerLane>(x, q, i8, scales, groups, eps, rule, strided, groups_per_row, s_row, s_col, s);
 }
 
 template <typename T>

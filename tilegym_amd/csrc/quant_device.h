@@ -28,6 +28,11 @@ __device__ __forceinline__ v8f_q load8<float>(const float* p) {
 // kQuantGroupsPerLane groups per lane, all loads issued before the first use (one 16-byte load per lane
 // leaves too few bytes in flight per wave for an HBM-bound kernel).
 constexpr int kQuantGroupsPerLane = 4;
+// One group per lane below this many workgroups of four (67 M elements): four are worked through one after the other, and more
+// waves hide more.  Kernel with launch, four -> one, bf16 in groups of 128: 16 x 5120 4.1 -> 2.2 us, 256 x 4096 4.3 -> 2.5,
+// 1024 x 4096 6.4 -> 4.8, 4096 x 5120 19.9 -> 15.8, 4096 x 12288 36.5 -> 35.4; 8192 x 14336 70.8 -> 76.4 and 32000 x 16384
+// 281 -> 307 with one, so four from there on.  Groups of 16, 4096 x 8192: 21.0 -> 18.5; f32 30.4 -> 28.9.
+constexpr int64_t kQuantFewWorkgroups = 1 << 13;
 
 enum QuantRule { QUANT_ZERO_TO_ONE = 0, QUANT_EPS = 1, QUANT_EPS_POW2 = 2 };
 
@@ -38,12 +43,12 @@ enum QuantRule { QUANT_ZERO_TO_ONE = 0, QUANT_EPS = 1, QUANT_EPS_POW2 = 2 };
 // [-128, 127] and converted as a float -> integer cast does (toward zero).
 // (body of 256-thread block `block`, thread `tid` of it: the kernel below runs it as such, the MoE preparation kernel
 // runs four such blocks per 1024-thread workgroup)
-template <typename T, int LPG, bool STRIDED, bool I8>
+template <typename T, int LPG, bool STRIDED, bool I8, int G = kQuantGroupsPerLane>
 __device__ __forceinline__ void act_quant_group_body(const T* __restrict__ x, uint8_t* __restrict__ q,
                                                      float* __restrict__ scales, int64_t groups, float eps,
                                                      int rule, uint32_t groups_per_row, int64_t s_row, int64_t s_col,
                                                      const int64_t block, const int tid) {
-    constexpr int G = kQuantGroupsPerLane, GS = 8 * LPG, PASS = 256 / LPG;
+    constexpr int GS = 8 * LPG, PASS = 256 / LPG;
     constexpr float QMAX = I8 ? 127.0f : 448.0f, QMIN = I8 ? -128.0f : -448.0f;
     const int sub = tid & (LPG - 1);
     const int64_t g0 = block * (PASS * G) + (tid / LPG);
