@@ -340,6 +340,10 @@ int32_t tg_diag_read(const tg_tensor* x, const tg_tensor* out, int32_t workgroup
                      uint64_t hip_stream);
 int32_t tg_diag_mfma(int32_t fmas, int32_t iters, int32_t workgroups, const tg_tensor* out, int32_t device_id, uint64_t hip_stream);
 
+/* Bytes of LDS that the largest launch of a tg_fp8_fused_moe layer of these sizes asks for when the layer takes its decoding
+ * form (few rows per expert); 0 when it does not.  Host arithmetic, no GPU needed.  Never more than a compute unit's 160 KiB. */
+int64_t tg_diag_moe_lds_bytes(int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t inter);
+
 #ifdef __cplusplus
 }
 #endif

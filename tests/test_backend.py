@@ -228,3 +228,17 @@ def test_native_binding_declines_host_tensors_and_odd_arguments():
     for call in (lambda: n.matmul(a, b), lambda: n.act_quant(a)):
         with pytest.raises(TypeError):
             call()
+
+
+@pytest.mark.parametrize("hidden,inter,experts,top_k", [(2048, 1408, 64, 6), (4096, 1536, 128, 8), (4096, 1408, 128, 8), (2048, 1024, 64, 8),
+                                                        (7168, 2048, 384, 8), (7168, 2048, 256, 8), (4096, 6400, 16, 2), (5120, 8192, 128, 1),
+                                                        (4096, 14336, 8, 2), (128, 128, 1, 1), (8192, 1024, 512, 4), (65536, 128, 512, 1)])
+def test_decoding_moe_layer_asks_for_no_more_lds_than_a_compute_unit_has(hidden, inter, experts, top_k):
+    """Every token count that the decoding form takes: the launches' dynamic LDS (the kernels have no static LDS, which the build
+    check asserts) fits the 160 KiB of a compute unit."""
+    from tilegym_amd import _lib
+
+    lds = _lib.load().tg_diag_moe_lds_bytes
+    asked = [lds(tokens, top_k, experts, hidden, inter) for tokens in range(1, 2048 // top_k + 2)]
+    assert max(asked) <= 160 * 1024 and asked[-1] == 0
+    assert asked[0] > 0 or hidden > 8192

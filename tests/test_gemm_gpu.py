@@ -1900,6 +1900,44 @@ def test_decoding_moe_layer_gives_the_bits_of_the_row_tiled_layer(device, T, H, 
         assert torch.isfinite(got.float()).all() and torch.equal(got, want)
 
 
+def _device_moe_layer(device, T, H, I, E, k, seed):
+    """An FP8 MoE layer made on the device: activations, weights with their scales, routing (even)."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    w1 = (torch.randn(E, 2 * I, H, generator=g, device=device, dtype=torch.float16) * 16).to(FP8)
+    w2 = (torch.randn(E, H, I, generator=g, device=device, dtype=torch.float16) * 16).to(FP8)
+    s1 = torch.rand(E, 2 * I // 128, H // 128, generator=g, device=device) * 4e-3 + 1e-3
+    s2 = torch.rand(E, H // 128, I // 128, generator=g, device=device) * 4e-3 + 1e-3
+    x = torch.randn(T, H, generator=g, device=device).to(torch.bfloat16)
+    tw, ids = torch.topk(torch.softmax(torch.randn(T, E, generator=g, device=device), dim=-1), k, dim=-1)
+    return x, w1, w2, s1, s2, tw, ids
+
+
+def _both_forms(x, w1, w2, s1, s2, tw, ids):
+    """(the layer as one call, the same on the row-tiled kernels called one by one, the kernel that the one call chose)"""
+    from tilegym_amd.ops import fused_moe, moe_interface
+
+    _lib.workspace_for(x.device, 1 << 20).fill_(0xFF)
+    got = fused_moe(x, w1, w2, tw, ids, w1_scale=s1, w2_scale=s2)
+    kernel = _lib.last_config()["KERNEL_NAME"]
+    try:
+        moe_interface.USE_ONE_CALL_LAYER = False
+        want = fused_moe(x, w1, w2, tw, ids, w1_scale=s1, w2_scale=s2)
+    finally:
+        moe_interface.USE_ONE_CALL_LAYER = True
+    return got, want, kernel
+
+
+@pytest.mark.parametrize("T,H,I,E,k", [(163, 2048, 1408, 64, 6), (164, 2048, 1408, 64, 6), (174, 2048, 1408, 64, 6), (175, 2048, 1408, 64, 6),
+                                       (108, 4096, 1536, 128, 8)])
+def test_decoding_moe_layer_where_its_lds_is_full(device, T, H, I, E, k):
+    """Layers whose decoding form asks for (almost) all of a compute unit's LDS, and the first size past the hand-over."""
+    layer = _device_moe_layer(device, T, H, I, E, k, seed=T)
+    got, want, kernel = _both_forms(*layer)
+    lds = _lib.load().tg_diag_moe_lds_bytes(T, k, E, H, I)
+    assert lds <= 160 * 1024 and kernel == ("stream" if lds else "tiled")
+    assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
 def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_path):
     """A table written by tilegym_amd.tune (here: by hand, and by tune_shape on a small shape) decides the schedule of calls
     that bring no kernel_configs; explicit kernel_configs still win; unloading the table restores the automatic choice."""

@@ -89,6 +89,15 @@ def test_spilled_registers_above_the_recorded_count_are_found(tmp_path):
     assert check_hazards.scan_spills(str(path)) == []
 
 
+def test_static_lds_of_a_kernel_that_uses_all_of_it_dynamically_is_found(tmp_path):
+    path = tmp_path / "k.s"
+    meta = "    .group_segment_fixed_size: {n}\n    .name:           _ZN2tg17moe_decode_kernelIDF16bLb1ELi2EEEvNS_15MoeDecodeParamsE\n"
+    path.write_text(meta.format(n=1024))
+    assert len(check_hazards.scan_static_lds(str(path))) == 1
+    path.write_text(meta.format(n=0) + meta.replace("moe_decode", "other").format(n=64))
+    assert check_hazards.scan_static_lds(str(path)) == []
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
 def test_no_kernel_breaks_either_rule():
     run = subprocess.run([sys.executable, os.path.join(CSRC, "check_hazards.py"), "--build"], capture_output=True, text=True,

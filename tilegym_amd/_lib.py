@@ -140,6 +140,8 @@ def load():
     L.tg_diag_read.argtypes = [P, P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint64]
     L.tg_diag_mfma.restype = ctypes.c_int32
     L.tg_diag_mfma.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, P, ctypes.c_int32, ctypes.c_uint64]
+    L.tg_diag_moe_lds_bytes.restype = ctypes.c_int64
+    L.tg_diag_moe_lds_bytes.argtypes = [ctypes.c_int64] * 5
     if L.tg_abi_version() != 1:
         raise RuntimeError(f"libtilegym_hip.so ABI version {L.tg_abi_version()} != 1")
     try:

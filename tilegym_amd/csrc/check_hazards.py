@@ -46,6 +46,9 @@ EARLY_USE_KNOWN = ("fp8_gemm_bs256_kernelILi0ELb1E", "fp8_gemm_bs256_kernelILi1E
 # 129 / 216 spilled registers, and 2.7 times the run time, when their second K step was made unconditional).
 VGPR_SPILL_LIMITS = {"fp8_gemm_tile256_kernel": 0, "fp8_gemm_bs256_kernelILi0ELb0E": 52, "fp8_gemm_bs256_kernelILi0ELb1E": 0,
                      "fp8_gemm_bs256_kernelILi1ELb0E": 17, "fp8_gemm_bs256_kernelILi1ELb1E": 0}
+# Kernels that are launched with as much dynamic LDS as a compute unit has: no static LDS beside it (the dynamic array is
+# 1024-byte aligned, so one static variable would take 1 KiB).
+NO_STATIC_LDS = ("moe_decode_kernel", "moe_decode_sum_kernel")
 # translation units with inline-assembly memory instructions
 DEFAULT_SOURCES = ["fp8_gemm_tile_pt.hip", "fp8_gemm_tile256.hip", "fp8_gemm_tile_bs.hip", "fp8_gemm_tile_bs256.hip",
                    "fp8_gemm_tile_grouped.hip", "fp8_gemm_tile_list.hip", "fp8_gemm_stream.hip", "fp8_moe_decode.hip"]
@@ -167,6 +170,21 @@ def scan_spills(path):
     return findings
 
 
+def scan_static_lds(path):
+    """kernels of NO_STATIC_LDS whose metadata reports static LDS."""
+    findings, size = [], 0
+    for raw in open(path):
+        line = raw.strip()
+        if line.startswith(".group_segment_fixed_size:"):   # (in front of the name: the metadata's keys are sorted)
+            size = int(line.split()[-1])
+        elif line.startswith(".name:"):
+            name = line.split()[-1]
+            if size and any(key in name for key in NO_STATIC_LDS):
+                findings.append(f"{os.path.basename(path)}: {name}: {size} bytes of static LDS")
+            size = 0
+    return findings
+
+
 def predecessors(insts, labels):
     preds = [[] for _ in insts]
     for i, (op, toks, _) in enumerate(insts):
@@ -228,7 +246,7 @@ def main(argv):
             return 2
     findings = []
     for f in files:
-        findings += scan(f) + scan_early_use(f) + scan_spills(f)
+        findings += scan(f) + scan_early_use(f) + scan_spills(f) + scan_static_lds(f)
     for line in findings:
         print(line)
     print(f"check_hazards: {len(files)} file(s), {len(findings)} finding(s)")

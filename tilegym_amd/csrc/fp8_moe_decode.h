@@ -119,9 +119,13 @@ __device__ __forceinline__ int decode_expert_id(const MoeDecodeParams& p, int sl
 // wave; 40 tokens: 59.4 / 60.1 / 60.2.)
 constexpr int kDecodeWaves = 5, kDecodeStages = 2, kDecodeQuantWaves = 4;
 
+// LDS of a compute unit.  The kernels below have no static LDS: a static variable in front of the 1024-byte aligned dynamic
+// array would take 1 KiB of it, whatever its size (the build check holds them to that).
+constexpr int kLdsBytes = 160 * 1024;
+
 // Dynamic LDS of moe_decode_kernel, in this order.
 struct MoeDecodeLds {
-    int ring, codes, scales, wscales, ids, list, weight, mask, total;  // byte offsets
+    int ring, codes, scales, wscales, ids, list, weight, mask, rows, total;  // byte offsets
     __host__ __device__ static MoeDecodeLds of(const MoeDecodeParams& p) {
         MoeDecodeLds l{};
         l.ring = 0;
@@ -132,7 +136,8 @@ struct MoeDecodeLds {
         l.list = l.ids + p.slots * 4;
         l.weight = l.list + p.slots * 4;
         l.mask = l.weight + p.slots * 4;
-        l.total = l.mask + (p.E + 31) / 32 * 4;
+        l.rows = l.mask + (p.E + 31) / 32 * 4;
+        l.total = l.rows + 4;
         return l;
     }
 };
@@ -154,7 +159,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     float* const s_weight = reinterpret_cast<float*>(lds + at.weight);     // second GEMM: routed weight of every slot
     int* const s_src = reinterpret_cast<int*>(lds + at.weight);            // first GEMM: the listed slots' rows of x
     uint32_t* const s_mask = reinterpret_cast<uint32_t*>(lds + at.mask);
-    __shared__ int s_rows;                      // rows of the segment's expert
+    int* const s_rows = reinterpret_cast<int*>(lds + at.rows);             // rows of the segment's expert
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -233,7 +238,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 }
                 rows += __popcll(m);
             }
-            if (qt == 0) s_rows = rows;
+            if (qt == 0) *s_rows = rows;
             // weight scales of the segment's block rows (UP: of the gate and of the up rows)
             const float* const ws = p.ws + (int64_t)e * p.nblocks * kblocks;
             const int nb0 = g0 * COLS / 128, nbs = (g1 * COLS - 1) / 128 - nb0 + 1;
@@ -318,7 +323,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
             if (r0 == 0) decode_barrier();
             for (int s = 0; s < STAGES && s < total; ++s) issue(s);
             decode_barrier();
-            rows = __builtin_amdgcn_readfirstlane(s_rows);
+            rows = __builtin_amdgcn_readfirstlane(*s_rows);
             const int rows_a = min(cap, rows - r0);
 
             // ---- this wave's groups
@@ -405,14 +410,17 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
 // to the 16-bit type as the row-per-slot form stores them, are added through LDS in slot order.
 constexpr int kDecodeSumRows = 8;
 constexpr int kDecodeSumStages = 3;
-inline int moe_decode_sum_lds(int top_k, int K) { return top_k * (kDecodeSumStages * kDecodeSumRows * kDecodePiece + (K + K / 32 + 255) / 256 * 256); }
+// Dynamic LDS of moe_decode_sum_kernel: every wave's ring, every wave's codes and scales, the slots' results.
+inline int moe_decode_sum_codes(int K) { return (K + K / 32 + 255) / 256 * 256; }
+inline int moe_decode_sum_lds(int top_k, int K) {
+    return top_k * (kDecodeSumStages * kDecodeSumRows * kDecodePiece + moe_decode_sum_codes(K) + kDecodeSumRows * 4);
+}
 
 template <typename T>
 __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodeParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int R = kDecodeSumRows, STAGES = kDecodeSumStages, BUF = R * kDecodePiece, LOADS = BUF / 1024, X_LOADS = 4;
     extern __shared__ __align__(1024) uint8_t lds[];
-    __shared__ float s_red[8 * R];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -421,8 +429,10 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
     const int npieces = (K + kDecodePiece - 1) / kDecodePiece;
     const int tail_steps = (K % kDecodePiece) / kKBlock;
     uint8_t* const my_ring = lds + wave * STAGES * BUF;
-    uint8_t* const my_codes = lds + p.top_k * STAGES * BUF + wave * ((K + K / 32 + 255) / 256 * 256);  // [K step][128 bytes]
-    float* const my_scale = reinterpret_cast<float*>(my_codes + K);                                    // [K step]
+    const int codes_bytes = (K + K / 32 + 255) / 256 * 256;
+    uint8_t* const my_codes = lds + p.top_k * STAGES * BUF + wave * codes_bytes;  // [K step][128 bytes]
+    float* const my_scale = reinterpret_cast<float*>(my_codes + K);               // [K step]
+    float* const s_red = reinterpret_cast<float*>(lds + p.top_k * (STAGES * BUF + codes_bytes));  // [slot][row]
     const int e = __builtin_amdgcn_readfirstlane(decode_expert_id(p, slot));
     const float weight = p.topk_weights[slot];
     v4f acc = v4f{0.f, 0.f, 0.f, 0.f};

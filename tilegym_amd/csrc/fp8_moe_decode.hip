@@ -7,8 +7,6 @@ namespace tg {
 
 namespace {
 
-constexpr int kLdsBytes = 160 * 1024 - 256;  // (a few static bytes beside the dynamic ones)
-
 // Fills in row_cap and wscale_cap; false when the layer is not one for this kernel.
 //
 // An expert with more than row_cap rows is streamed more than once, so the rows that the fullest expert is likely to get
@@ -55,6 +53,12 @@ bool decode_shape_ok(const MoeDecodeParams& p, bool up) {
 }  // namespace
 
 bool moe_decode_fits(MoeDecodeParams p, bool up, int tokens) { return decode_shape_ok(p, up) && decode_plan(p, up, tokens); }
+
+int64_t moe_decode_lds_bytes(MoeDecodeParams p, bool up, int tokens) {
+    return decode_shape_ok(p, up) && decode_plan(p, up, tokens) ? MoeDecodeLds::of(p).total : 0;
+}
+
+int64_t moe_decode_sum_lds_bytes(const MoeDecodeParams& p, int tokens) { return moe_decode_sum_fits(p, tokens) ? moe_decode_sum_lds(p.top_k, p.K) : 0; }
 
 hipError_t run_moe_decode(MoeDecodeParams p, bool up, bool is_bf16, int tokens, hipStream_t s) {
     if (!decode_shape_ok(p, up) || !decode_plan(p, up, tokens)) return hipErrorInvalidConfiguration;

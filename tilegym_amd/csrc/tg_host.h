@@ -62,6 +62,9 @@ bool moe_decode_fits(MoeDecodeParams p, bool up, int tokens);
 hipError_t run_moe_decode(MoeDecodeParams p, bool up, bool is_bf16, int tokens, hipStream_t s);
 // the second GEMM with the sum over a token's slots in the same launch: out (tokens, N)
 bool moe_decode_sum_fits(const MoeDecodeParams& p, int tokens);
+// LDS that the launches ask for (0: not one for these kernels)
+int64_t moe_decode_lds_bytes(MoeDecodeParams p, bool up, int tokens);
+int64_t moe_decode_sum_lds_bytes(const MoeDecodeParams& p, int tokens);
 hipError_t run_moe_decode_sum(const MoeDecodeParams& p, bool is_bf16, int tokens, hipStream_t s);
 // up to kListMax per-tensor NT problems in one launch (tile 256x256, 128x128 or 64x128)
 hipError_t run_tile_list(int bm, int bn, const GemmList& gl, int gx, hipStream_t s);

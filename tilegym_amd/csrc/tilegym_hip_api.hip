@@ -1,6 +1,7 @@
 // C ABI of libtilegym_hip.so (declared in include/tilegym_hip.h): argument validation on the
 // host, schedule selection, kernel launches.  No allocation, no synchronisation, no global
 // mutable state apart from two thread-local diagnostics (last error text, last schedule).
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1715,6 +1716,15 @@ int64_t tg_fp8_fused_moe_workspace_bytes(int64_t tokens, int64_t top_k, int64_t 
                                          int32_t block_m) {
     if (tokens < 0 || top_k < 1 || experts < 1 || hidden < 1 || inter < 1 || block_m < 1) return 0;
     return moe_layout(tokens, top_k, experts, hidden, inter, block_m, 2).total;
+}
+
+int64_t tg_diag_moe_lds_bytes(int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t inter) {
+    if (tokens < 0 || top_k < 1 || experts < 1 || hidden < 1 || inter < 1) return 0;
+    const MoeDecode d = moe_decode(tokens, top_k, experts, hidden, inter);
+    if (!d.takes) return 0;
+    const int T = (int)tokens;
+    const int64_t second = tg::moe_decode_sum_fits(d.down, T) ? tg::moe_decode_sum_lds_bytes(d.down, T) : tg::moe_decode_lds_bytes(d.down, false, T);
+    return std::max(tg::moe_decode_lds_bytes(d.up, true, T), second);
 }
 
 int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg_tensor* w1, const tg_tensor* w2,
