@@ -1938,6 +1938,20 @@ def test_decoding_moe_layer_where_its_lds_is_full(device, T, H, I, E, k):
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("T,H,I,k", [(1, 640, 128, 1), (1, 384, 640, 2), (16, 640, 128, 1), (16, 384, 640, 2)])
+def test_decoding_moe_layer_with_infinities_in_the_last_group(device, T, H, I, k):
+    """Rows whose last quantization group holds an infinity or a NaN, and a K that is no multiple of the 512 bytes of a piece: K steps
+    past the end add nothing, whatever the scale in front of them is, so the layer gives what the row-tiled kernels give."""
+    x, w1, w2, s1, s2, tw, ids = _device_moe_layer(device, T, H, I, 64, k, seed=H + T)
+    x[0, -1], x[T // 2, -3] = float("inf"), float("-inf")
+    x[T - 1, -128] = float("nan")
+    got, want, kernel = _both_forms(x, w1, w2, s1, s2, tw, ids)
+    assert kernel == "stream" and torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0))
+    if I == 128:
+        assert got[0].isinf().any()
+
+
 def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_path):
     """A table written by tilegym_amd.tune (here: by hand, and by tune_shape on a small shape) decides the schedule of calls
     that bring no kernel_configs; explicit kernel_configs still win; unloading the table restores the automatic choice."""

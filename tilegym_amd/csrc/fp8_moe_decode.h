@@ -336,7 +336,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 if (i + STAGES <= total) wait_vmcnt<(STAGES - 1) * LOADS>();
                 else wait_vmcnt<0>();
                 // Everything the piece needs is read at once: one LDS round trip per piece.  K steps past the end of K multiply
-                // zeros (their weight loads are out of range) with the last step's activations.
+                // zeros (their weight loads are out of range) with the last step's activations, and add the product under a scale
+                // of zero (the last step's may be infinite).
                 const uint8_t* wb = my_ring + stage * kDecodeBuf + li * kDecodePiece;
                 const float* ws = s_wscale + ((gc * COLS >> 7) - nb0) * (UP ? 2 : 1) * kblocks;
                 v8i wf[kDecodeSteps], af[MT][kDecodeSteps];
@@ -370,7 +371,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                     for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[mt][s], v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int s = 0; s < kDecodeSteps; ++s) {
-                        const float lo = as[mt][s] * bg[s], hi = UP ? as[mt][s] * bu[s] : lo;
+                        const bool inside = cc * kDecodeSteps + s < kblocks;
+                        const float lo = inside ? as[mt][s] * bg[s] : 0.f, hi = !UP ? lo : inside ? as[mt][s] * bu[s] : 0.f;
                         acc[mt] += part[s] * v4f{lo, lo, hi, hi};
                     }
                 }
@@ -507,8 +509,9 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
             for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[s], v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int s = 0; s < kDecodeSteps; ++s) {
-                const int kb = min(c * kDecodeSteps + s, kblocks - 1);
-                acc += part[s] * (sc[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), kb)));
+                const int kb = c * kDecodeSteps + s;   // (steps past the end of K add nothing: a scale of zero)
+                const float scale = sc[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), min(kb, kblocks - 1)));
+                acc += part[s] * (kb < kblocks ? scale : 0.f);
             }
         }
     }
