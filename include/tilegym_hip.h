@@ -291,6 +291,13 @@ int32_t tg_silu_mul_quant_1x128(const tg_tensor* q, const tg_tensor* scales, con
 int32_t tg_moe_sum(const tg_tensor* out, const tg_tensor* x, int32_t device_id, uint64_t hip_stream);
 
 /*
+ * tg_moe_sum over the slots that have an expert: out[t, :] = sum of x[t, j, :] over the j with 0 <= topk_ids[t, j] < num_experts.
+ * The other slots' rows, which the gather GEMMs leave unwritten, are not used.  topk_ids (T, top_k) int32 / int64, contiguous.
+ */
+int32_t tg_moe_sum_routed(const tg_tensor* out, const tg_tensor* x, const tg_tensor* topk_ids, int32_t num_experts, int32_t device_id,
+                          uint64_t hip_stream);
+
+/*
  * The FP8 MoE layer in one call: what src/tilegym/ops/moe_interface.py:116-322 (fused_experts_impl, use_fp8_w8a8) does
  * for one chunk of tokens, as the four launches tg_moe_align_quant_1x128 -> tg_fp8_moe_gemm_silu_quant -> tg_fp8_moe_gemm
  * (x routed weight) -> tg_moe_sum on the caller's stream, with every intermediate in `workspace`.  The results are the

@@ -1952,6 +1952,22 @@ def test_decoding_moe_layer_with_infinities_in_the_last_group(device, T, H, I, k
         assert got[0].isinf().any()
 
 
+@pytest.mark.parametrize("T,H,I,E,k", [(1, 256, 384, 64, 6), (16, 384, 256, 64, 6), (400, 256, 256, 16, 3), (9, 256, 256, 64, 1), (200, 256, 256, 4, 1)])
+def test_moe_slots_without_an_expert_add_nothing(device, T, H, I, E, k):
+    """Ids outside [0, E) in every form of the layer (one launch with the sum, decoding, row-tiled, call by call), whatever the
+    scratch memory and the slot's weight hold: what the same slots give with an expert of theirs and a weight of zero."""
+    x, w1, w2, s1, s2, tw, ids = _device_moe_layer(device, T, H, I, E, k, seed=T + k)
+    out_of = torch.rand(T, k, generator=torch.Generator(device=device).manual_seed(T), device=device) < 0.3
+    out_of[0, 0] = True
+    want = _both_forms(x, w1, w2, s1, s2, tw.masked_fill(out_of, 0.0), ids)[0]
+    assert torch.isfinite(want.float()).all()
+    for outside in (-1, E, E + 7):
+        torch.full((T, k, H), float("nan"), dtype=x.dtype, device=device)  # (freed: what the next allocation may find)
+        for dtype in (torch.int32, torch.int64):
+            for got in _both_forms(x, w1, w2, s1, s2, tw.masked_fill(out_of, float("inf")), ids.masked_fill(out_of, outside).to(dtype))[:2]:
+                assert torch.equal(got, want)
+
+
 def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_path):
     """A table written by tilegym_amd.tune (here: by hand, and by tune_shape on a small shape) decides the schedule of calls
     that bring no kernel_configs; explicit kernel_configs still win; unloading the table restores the automatic choice."""

@@ -128,6 +128,8 @@ def load():
     L.tg_silu_mul_quant_1x128.argtypes = [P, P, P, ctypes.c_int32, ctypes.c_uint64]
     L.tg_moe_sum.restype = ctypes.c_int32
     L.tg_moe_sum.argtypes = [P, P, ctypes.c_int32, ctypes.c_uint64]
+    L.tg_moe_sum_routed.restype = ctypes.c_int32
+    L.tg_moe_sum_routed.argtypes = [P, P, P, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint64]
     L.tg_fp8_fused_moe_workspace_bytes.restype = ctypes.c_int64
     L.tg_fp8_fused_moe_workspace_bytes.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int32]
     L.tg_fp8_fused_moe.restype = ctypes.c_int32
@@ -569,6 +571,14 @@ def moe_sum(x: torch.Tensor, out: torch.Tensor) -> None:
     L = load()
     rc = L.tg_moe_sum(_ref(_desc(out)), _ref(_desc(x)), _device_index(x), _stream_handle(x))
     check_rc(rc, "tg_moe_sum")
+
+
+def moe_sum_routed(x: torch.Tensor, out: torch.Tensor, topk_ids: torch.Tensor, num_experts: int) -> None:
+    """moe_sum over the slots whose id is in [0, num_experts) through tg_moe_sum_routed."""
+    L = load()
+    ids = topk_ids if topk_ids.dtype in (torch.int32, torch.int64) else topk_ids.to(torch.int64)
+    rc = L.tg_moe_sum_routed(_desc(out), _desc(x), _desc(ids), int(num_experts), _device_index(x), _stream_handle(x))
+    check_rc(rc, "tg_moe_sum_routed")
 
 
 def _desc_array(tensors):

@@ -336,8 +336,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 if (i + STAGES <= total) wait_vmcnt<(STAGES - 1) * LOADS>();
                 else wait_vmcnt<0>();
                 // Everything the piece needs is read at once: one LDS round trip per piece.  K steps past the end of K multiply
-                // zeros (their weight loads are out of range) with the last step's activations, and add the product under a scale
-                // of zero (the last step's may be infinite).
+                // zeros (their weight loads are out of range) with the last step's activations, under scales of zero (the last step's
+                // may be infinite).
                 const uint8_t* wb = my_ring + stage * kDecodeBuf + li * kDecodePiece;
                 const float* ws = s_wscale + ((gc * COLS >> 7) - nb0) * (UP ? 2 : 1) * kblocks;
                 v8i wf[kDecodeSteps], af[MT][kDecodeSteps];
@@ -364,6 +364,16 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 }
                 if (i + STAGES < total) issue(stage);
                 stage = stage + 1 == STAGES ? 0 : stage + 1;
+                if (tail_steps != 0 && cc == npieces - 1) {
+#pragma unroll
+                    for (int s = 1; s < kDecodeSteps; ++s) {
+                        const bool past = s >= tail_steps;
+                        bg[s] = past ? 0.f : bg[s];
+                        bu[s] = past ? 0.f : bu[s];
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) as[mt][s] = past ? 0.f : as[mt][s];
+                    }
+                }
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     v4f part[kDecodeSteps];
@@ -371,8 +381,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                     for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[mt][s], v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int s = 0; s < kDecodeSteps; ++s) {
-                        const bool inside = cc * kDecodeSteps + s < kblocks;
-                        const float lo = inside ? as[mt][s] * bg[s] : 0.f, hi = !UP ? lo : inside ? as[mt][s] * bu[s] : 0.f;
+                        const float lo = as[mt][s] * bg[s], hi = UP ? as[mt][s] * bu[s] : lo;
                         acc[mt] += part[s] * v4f{lo, lo, hi, hi};
                     }
                 }
@@ -413,7 +422,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
 constexpr int kDecodeSumRows = 8;
 constexpr int kDecodeSumStages = 3;
 // Dynamic LDS of moe_decode_sum_kernel: every wave's ring, every wave's codes and scales, the slots' results.
-inline int moe_decode_sum_codes(int K) { return (K + K / 32 + 255) / 256 * 256; }
+// (the scales of a piece's four K steps are read whole: three zeros behind the last one)
+__host__ __device__ inline int moe_decode_sum_codes(int K) { return (K + K / 32 + 12 + 255) / 256 * 256; }
 inline int moe_decode_sum_lds(int top_k, int K) {
     return top_k * (kDecodeSumStages * kDecodeSumRows * kDecodePiece + moe_decode_sum_codes(K) + kDecodeSumRows * 4);
 }
@@ -431,7 +441,7 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
     const int npieces = (K + kDecodePiece - 1) / kDecodePiece;
     const int tail_steps = (K % kDecodePiece) / kKBlock;
     uint8_t* const my_ring = lds + wave * STAGES * BUF;
-    const int codes_bytes = (K + K / 32 + 255) / 256 * 256;
+    const int codes_bytes = moe_decode_sum_codes(K);
     uint8_t* const my_codes = lds + p.top_k * STAGES * BUF + wave * codes_bytes;  // [K step][128 bytes]
     float* const my_scale = reinterpret_cast<float*>(my_codes + K);               // [K step]
     float* const s_red = reinterpret_cast<float*>(lds + p.top_k * (STAGES * BUF + codes_bytes));  // [slot][row]
@@ -477,6 +487,7 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
 #pragma unroll
         for (int j = 0; j < X_LOADS; ++j)
             if (j * 4 < kblocks) put(lane + j * 64, raw[j]);
+        if (lane < 3) my_scale[kblocks + lane] = 0.f;   // K steps past the end add nothing: both of their scales are zero
         for (int task = lane + X_LOADS * 64; task - lane < kblocks * 16; task += 64) {
             v4i v = v4i{0, 0, 0, 0};
             if (task < kblocks * 16) v = *reinterpret_cast<const v4i*>(reinterpret_cast<const uint8_t*>(p.x) + ((int64_t)slot * K + task * 8) * 2);
@@ -497,7 +508,7 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
                 const uint8_t* ab = my_codes + kb * kKBlock + lg * 16;   // (one row: the same in every column)
                 wf[s] = join(*reinterpret_cast<const v4i*>(wb + (((s * 8 + lg) ^ r) << 4)), *reinterpret_cast<const v4i*>(wb + (((s * 8 + 4 + lg) ^ r) << 4)));
                 af[s] = join(*reinterpret_cast<const v4i*>(ab), *reinterpret_cast<const v4i*>(ab + 64));
-                sc[s] = my_scale[kb];
+                sc[s] = my_scale[c * kDecodeSteps + s];
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);
 #pragma unroll
@@ -509,16 +520,15 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
             for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[s], v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int s = 0; s < kDecodeSteps; ++s) {
-                const int kb = c * kDecodeSteps + s;   // (steps past the end of K add nothing: a scale of zero)
-                const float scale = sc[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), min(kb, kblocks - 1)));
-                acc += part[s] * (kb < kblocks ? scale : 0.f);
+                // (at most 64 K steps; lanes past the last one hold zero)
+                acc += part[s] * (sc[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), c * kDecodeSteps + s)));
             }
         }
     }
     if (li == 0 && lg * 4 < R) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float v = acc[q] * weight;
+            float v = e >= 0 ? acc[q] * weight : 0.f;   // (a slot without an expert adds nothing, whatever its weight)
             asm("" : "+v"(v));  // (the product is rounded on its own before the conversion, as the stored form is)
             s_red[wave * R + lg * 4 + q] = (float)(T)v;
         }

@@ -24,6 +24,8 @@
 // the scale.  The divisions go through ScaleDivider (bit-equal to the IEEE division).
 #include "quant_device.h"
 
+#include <type_traits>
+
 namespace tg {
 
 template <typename T, int LPG, bool STRIDED, bool I8, int G>
@@ -127,16 +129,36 @@ __global__ void __launch_bounds__(256) silu_mul_quant_kernel(const T* __restrict
 }
 
 // out[t, :] = sum_j x[t, j, :]  (fp32 sum in slot order, rounded once), the top-k combine of
-// src/tilegym/ops/moe_interface.py:308-321.  H % 8 == 0.
-template <typename T>
-__global__ void __launch_bounds__(256) moe_sum_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t tokens, int top_k, int H) {
+// src/tilegym/ops/moe_interface.py:308-321.  H % 8 == 0.  IdT other than void: only the slots whose id is an expert; the
+// GEMMs wrote no row for the others.
+template <typename T, typename IdT>
+__global__ void __launch_bounds__(256) moe_sum_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t tokens, int top_k, int H,
+                                                      const IdT* __restrict__ ids, int E) {
     typedef T vecT __attribute__((ext_vector_type(8)));
     const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
     if (idx >= tokens * H) return;
     const int64_t t = idx / H;
     const int h = (int)(idx % H);
-    v8f_q acc = load8<T>(x + (t * top_k) * (int64_t)H + h);
-    for (int j = 1; j < top_k; ++j) acc += load8<T>(x + (t * top_k + j) * (int64_t)H + h);
+    // four slots' loads in flight at a time, added in slot order
+    v8f_q acc;
+    for (int j0 = 0; j0 < top_k; j0 += 4) {
+        v8f_q v[4];
+        bool use[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t slot = t * top_k + min(j0 + i, top_k - 1);
+            v[i] = load8<T>(x + slot * H + h);
+            use[i] = true;
+            if constexpr (!std::is_void_v<IdT>) use[i] = ids[slot] >= 0 && ids[slot] < E;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[i][q] = use[i] ? v[i][q] : 0.f;
+            if (j0 + i == 0) acc = v[i];
+            else if (j0 + i < top_k) acc += v[i];
+        }
+    }
     *reinterpret_cast<vecT*>(out + idx) = __builtin_convertvector(acc, vecT);
 }
 
@@ -224,16 +246,22 @@ hipError_t run_silu_mul_quant(const void* x, int x_type, uint8_t* q, float* scal
     return hipGetLastError();
 }
 
-hipError_t run_moe_sum(const void* x, void* out, int x_type, int64_t tokens, int top_k, int H, hipStream_t s) {
-    const int64_t n = tokens * H / 8;
-    if (n <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    if (x_type == OUT_BF16)
-        hipLaunchKernelGGL(moe_sum_kernel<__bf16>, grid, block, 0, s, (const __bf16*)x, (__bf16*)out, tokens, top_k, H);
-    else if (x_type == OUT_F16)
-        hipLaunchKernelGGL(moe_sum_kernel<_Float16>, grid, block, 0, s, (const _Float16*)x, (_Float16*)out, tokens, top_k, H);
+template <typename T>
+static void launch_moe_sum(const void* x, void* out, int64_t tokens, int top_k, int H, const void* ids, bool ids_are_i64, int E, hipStream_t s) {
+    const dim3 grid((unsigned)((tokens * H / 8 + 255) / 256)), block(256);
+    if (!ids)
+        hipLaunchKernelGGL((moe_sum_kernel<T, void>), grid, block, 0, s, (const T*)x, (T*)out, tokens, top_k, H, nullptr, 0);
+    else if (ids_are_i64)
+        hipLaunchKernelGGL((moe_sum_kernel<T, long long>), grid, block, 0, s, (const T*)x, (T*)out, tokens, top_k, H, (const long long*)ids, E);
     else
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL((moe_sum_kernel<T, int>), grid, block, 0, s, (const T*)x, (T*)out, tokens, top_k, H, (const int*)ids, E);
+}
+
+hipError_t run_moe_sum(const void* x, void* out, int x_type, int64_t tokens, int top_k, int H, const void* ids, bool ids_are_i64, int E, hipStream_t s) {
+    if (tokens * H / 8 <= 0) return hipSuccess;
+    if (x_type == OUT_BF16) launch_moe_sum<__bf16>(x, out, tokens, top_k, H, ids, ids_are_i64, E, s);
+    else if (x_type == OUT_F16) launch_moe_sum<_Float16>(x, out, tokens, top_k, H, ids, ids_are_i64, E, s);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

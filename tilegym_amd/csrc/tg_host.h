@@ -97,7 +97,8 @@ hipError_t run_weight_dequant(const uint8_t* x, const float* sc, void* y, int y_
 // q, scales <- quantize_1x128(round16(silu(x[:, :I]) * x[:, I:]));  x (rows, 2I) bf16/f16, I % 8 == 0
 hipError_t run_silu_mul_quant(const void* x, int x_type, uint8_t* q, float* scales, int64_t rows, int I, hipStream_t s);
 // out (tokens, H) <- sum over the top_k axis of x (tokens, top_k, H); bf16/f16, H % 8 == 0
-hipError_t run_moe_sum(const void* x, void* out, int x_type, int64_t tokens, int top_k, int H, hipStream_t s);
+// ids: null, or (tokens, top_k) expert ids; slots whose id is outside [0, E) then count as zeros
+hipError_t run_moe_sum(const void* x, void* out, int x_type, int64_t tokens, int top_k, int H, const void* ids, bool ids_are_i64, int E, hipStream_t s);
 // dst (cols, rows) <- transpose of src (rows, cols), one byte per element
 // dst (cols x ld) = transpose of src (rows x cols), zero beyond `rows` in every dst row
 hipError_t run_transpose_u8(const uint8_t* src, uint8_t* dst, int rows, int cols, int ld, hipStream_t s);

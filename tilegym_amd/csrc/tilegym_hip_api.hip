@@ -1547,10 +1547,17 @@ int32_t tg_silu_mul_quant_1x128(const tg_tensor* q, const tg_tensor* scales, con
     return TG_OK;
 }
 
-int32_t tg_moe_sum(const tg_tensor* out, const tg_tensor* x, int32_t device_id, uint64_t hip_stream) {
+static int32_t moe_sum(const tg_tensor* out, const tg_tensor* x, const tg_tensor* ids, int32_t num_experts, int32_t device_id, uint64_t hip_stream) {
     g_err[0] = 0;
     int32_t rc;
     if ((rc = check_tensor(x, "x", 3)) || (rc = check_tensor(out, "out", 2))) return rc;
+    if (ids) {
+        if ((rc = check_tensor(ids, "topk_ids", 2))) return rc;
+        if (ids->dtype != TG_I32 && ids->dtype != TG_I64) return fail(TG_ERR_DTYPE, "topk_ids must be int32 or int64");
+        if (ids->shape[0] != x->shape[0] || ids->shape[1] != x->shape[1] || !contiguous(ids))
+            return fail(TG_ERR_INVALID, "topk_ids must be contiguous (%lld, %lld)", (long long)x->shape[0], (long long)x->shape[1]);
+        if (num_experts < 1) return fail(TG_ERR_INVALID, "num_experts must be positive");
+    }
     const int x_type = io_type_of(x->dtype);
     if ((x_type != tg::OUT_BF16 && x_type != tg::OUT_F16) || out->dtype != x->dtype)
         return fail(TG_ERR_DTYPE, "x and out must both be bf16 or both f16");
@@ -1562,9 +1569,20 @@ int32_t tg_moe_sum(const tg_tensor* out, const tg_tensor* x, int32_t device_id, 
     DeviceGuard guard(device_id);
     if (!guard.ok) return fail(TG_ERR_DEVICE, "cannot use HIP device %d", device_id);
     hipError_t e = tg::run_moe_sum(reinterpret_cast<const void*>(x->ptr), reinterpret_cast<void*>(out->ptr), x_type, T, (int)k, (int)H,
+                                   ids ? reinterpret_cast<const void*>(ids->ptr) : nullptr, ids && ids->dtype == TG_I64, num_experts,
                                    reinterpret_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "moe_sum launch failed: %s", hipGetErrorString(e));
     return TG_OK;
+}
+
+int32_t tg_moe_sum(const tg_tensor* out, const tg_tensor* x, int32_t device_id, uint64_t hip_stream) {
+    return moe_sum(out, x, nullptr, 0, device_id, hip_stream);
+}
+
+int32_t tg_moe_sum_routed(const tg_tensor* out, const tg_tensor* x, const tg_tensor* topk_ids, int32_t num_experts, int32_t device_id,
+                          uint64_t hip_stream) {
+    if (!topk_ids) return fail(TG_ERR_NULL, "topk_ids: null tensor descriptor");
+    return moe_sum(out, x, topk_ids, num_experts, device_id, hip_stream);
 }
 
 int32_t tg_fp8_group_gemm(const tg_tensor* const* c, const tg_tensor* const* a, const tg_tensor* const* b,
@@ -1794,7 +1812,8 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
             d.down.out = ws + l.c3;
             e = tg::run_moe_decode(d.down, false, bf16, (int)T, stream);
             if (e == hipSuccess)
-                e = tg::run_moe_sum(ws + l.c3, reinterpret_cast<void*>(out->ptr), bf16 ? tg::OUT_BF16 : tg::OUT_F16, T, (int)k, (int)H, stream);
+                e = tg::run_moe_sum(ws + l.c3, reinterpret_cast<void*>(out->ptr), bf16 ? tg::OUT_BF16 : tg::OUT_F16, T, (int)k, (int)H, d.up.ids,
+                                    d.up.ids_are_i64, (int)E, stream);
         }
         if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "decoding MoE launch failed: %s", hipGetErrorString(e));
         return TG_OK;
@@ -1820,7 +1839,7 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
     if ((rc = tg_fp8_moe_gemm(&c3_rows, &q2, w2, &s2, w2_scale, &weights_flat, &sorted_ids, &expert_ids, &post, 1, 1, block_m, nullptr, 0,
                               device_id, hip_stream)))
         return rc;
-    return tg_moe_sum(out, &c3, device_id, hip_stream);
+    return tg_moe_sum_routed(out, &c3, topk_ids, (int32_t)E, device_id, hip_stream);
 }
 
 }  // extern "C"

@@ -67,7 +67,8 @@ def fused_experts_impl(
 
     hidden_states (T, H): bf16 / f16 (quantized 1 x 128 on the device here), or e4m3fn together with
     a1_scale (T, H/128).  w1 (E, 2I, H) and w2 (E, H, I) e4m3fn with w1_scale (E, 2I/128, H/128) and
-    w2_scale (E, H/128, ceil(I/128)).  Returns (T, H) bf16 for bf16 input, else f16.
+    w2_scale (E, H/128, ceil(I/128)).  A slot whose id is outside [0, E) (an expert of another rank, say) adds nothing.
+    Returns (T, H) bf16 for bf16 input, else f16.
 
     Two deliberate differences from the reference's FP8 branch: the activation between the GEMMs is
     re-quantized 1 x 128 with its own scales (the reference casts it to fp8 under an all-ones a2_scale,
@@ -159,10 +160,11 @@ def fused_experts_impl(
             q2, s2 = _lib.silu_mul_quant_1x128(c1.view(n * top_k, N))
         invoke_fused_moe_kernel(q2, w2, c3, s2, w2_scale, weights, ids, sorted_ids, expert_ids, post,
                                 True, 1, config, compute_type=out_dtype, use_fp8_w8a8=True)
+        # (slots whose id is no expert have no row in c3 and add nothing)
         if top_k == 1:
-            out[lo:hi] = c3[:, 0]
+            out[lo:hi] = c3[:, 0].masked_fill((ids < 0) | (ids >= E), 0.0)
         else:
-            _lib.moe_sum(c3, out[lo:hi])
+            _lib.moe_sum_routed(c3, out[lo:hi], ids, E)
     return out
 
 
