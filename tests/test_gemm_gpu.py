@@ -1952,6 +1952,25 @@ def test_decoding_moe_layer_with_infinities_in_the_last_group(device, T, H, I, k
         assert got[0].isinf().any()
 
 
+@pytest.mark.parametrize("T", [1, 16])
+def test_decoding_moe_layer_with_a_misaligned_weight(device, T):
+    """A w2 off a 16-byte boundary is taken (on the row-tiled form), any other such operand refused as it is there."""
+    from tilegym_amd.ops import fused_moe
+
+    def shifted(t):
+        raw = torch.empty(t.numel() * t.element_size() + 16, dtype=torch.uint8, device=device)[8:-8]
+        return raw.copy_(t.view(torch.uint8).reshape(-1)).view(t.dtype).view(t.shape)
+
+    x, w1, w2, s1, s2, tw, ids = _device_moe_layer(device, T, 256, 384, 16, 2, seed=T)
+    want = fused_moe(x, w1, w2, tw, ids, w1_scale=s1, w2_scale=s2)
+    assert _lib.last_config()["KERNEL_NAME"] == "stream"
+    got = fused_moe(x, w1, shifted(w2), tw, ids, w1_scale=s1, w2_scale=s2)
+    assert (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()   # (bf16 results of sums in another order)
+    for bad in ((shifted(x), w1), (x, shifted(w1))):
+        with pytest.raises(_lib.TileGymHipError, match="16-byte"):
+            fused_moe(*bad, w2, tw, ids, w1_scale=s1, w2_scale=s2)
+
+
 @pytest.mark.parametrize("T,H,I,E,k", [(1, 256, 384, 64, 6), (16, 384, 256, 64, 6), (400, 256, 256, 16, 3), (9, 256, 256, 64, 1), (200, 256, 256, 4, 1)])
 def test_moe_slots_without_an_expert_add_nothing(device, T, H, I, E, k):
     """Ids outside [0, E) in every form of the layer (one launch with the sum, decoding, row-tiled, call by call), whatever the
