@@ -1865,8 +1865,8 @@ def test_quantizer_with_one_and_four_groups_per_lane(device, rows):
     (3, 128, 128, 3, 2, torch.bfloat16, 0),       # one K step; more slots than experts
     (16, 1152, 256, 64, 4, torch.float16, 0),     # 16 rows held, row-per-slot form
     (40, 256, 640, 33, 5, torch.bfloat16, 0),     # an expert count over one mask word
-    (48, 256, 256, 40, 6, torch.bfloat16, 48),    # every token also to one expert: more rows than are held, several tiles
-    (150, 384, 384, 64, 6, torch.bfloat16, 0),    # two tiles of 16 rows
+    (44, 256, 256, 40, 6, torch.bfloat16, 44),    # every token also to one expert: more rows than are held, several passes
+    (75, 384, 384, 64, 6, torch.bfloat16, 0),     # seven rows per expert on average
     (5, 7168, 256, 16, 8, torch.bfloat16, 0),     # a long K: more than one batch of activations, fewer rows held
 ])
 def test_decoding_moe_layer_gives_the_bits_of_the_row_tiled_layer(device, T, H, I, E, k, dtype, skew):
@@ -1927,10 +1927,10 @@ def _both_forms(x, w1, w2, s1, s2, tw, ids):
     return got, want, kernel
 
 
-@pytest.mark.parametrize("T,H,I,E,k", [(163, 2048, 1408, 64, 6), (164, 2048, 1408, 64, 6), (174, 2048, 1408, 64, 6), (175, 2048, 1408, 64, 6),
-                                       (108, 4096, 1536, 128, 8)])
+@pytest.mark.parametrize("T,H,I,E,k", [(12, 4864, 384, 16, 2), (33, 4736, 384, 64, 8), (75, 4608, 768, 64, 6), (11, 4096, 6400, 16, 2),
+                                       (75, 2048, 1408, 64, 6), (76, 2048, 1408, 64, 6)])
 def test_decoding_moe_layer_where_its_lds_is_full(device, T, H, I, E, k):
-    """Layers whose decoding form asks for (almost) all of a compute unit's LDS, and the first size past the hand-over."""
+    """Layers whose decoding form asks for (almost) all of a compute unit's LDS, and both sides of the line between the forms."""
     layer = _device_moe_layer(device, T, H, I, E, k, seed=T)
     got, want, kernel = _both_forms(*layer)
     lds = _lib.load().tg_diag_moe_lds_bytes(T, k, E, H, I)
@@ -1950,6 +1950,30 @@ def test_decoding_moe_layer_with_infinities_in_the_last_group(device, T, H, I, k
     assert torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0))
     if I == 128:
         assert got[0].isinf().any()
+
+
+@pytest.mark.parametrize("T,E,k,routing", [(1, 64, 6, "duplicates"), (5, 200, 8, "duplicates"), (40, 64, 6, "same"), (70, 64, 6, "same"),
+                                           (100, 130, 6, "one"), (100, 130, 6, "far"), (60, 200, 4, "half"), (256, 512, 4, "far"),
+                                           (90, 33, 2, "half")])
+def test_decoding_moe_layer_with_more_rows_than_are_held(device, T, E, k, routing):
+    """Experts with more rows than a workgroup holds at a time, streamed once per pass: every token to the same experts, one or
+    several experts in every token (in the first and in the last of the mask's words), half of the batch alike, an id twice in a
+    token."""
+    x, w1, w2, s1, s2, tw, _ = _device_moe_layer(device, T, 384, 256, E, k, seed=T + E)
+    p = torch.rand(T, E, generator=torch.Generator(device=device).manual_seed(E), device=device)
+    if routing == "same":
+        p[:] = p[0].clone()
+    elif routing == "half":
+        p[T // 2:] = p[0].clone()
+    elif routing == "one":
+        p[:, 0] = 2.0
+    elif routing == "far":
+        p[:, E - 1], p[:, 65], p[T // 2:, 66] = 4.0, 3.0, 2.0
+    ids = p.topk(k, dim=1).indices
+    if routing == "duplicates":
+        ids[:] = ids[:, :1].clone()
+    got, want, kernel = _both_forms(x, w1, w2, s1, s2, tw, ids)
+    assert kernel == "stream" and torch.equal(got, want)
 
 
 @pytest.mark.parametrize("T", [1, 16])

@@ -6,14 +6,15 @@
 //   moe_decode_sum_kernel          the same and the sum over a token's slots in one launch, for very few slots
 //
 // Bound by the experts' weights out of HBM, 5.8 + 2.9 MB per expert at (hidden, inter) = (2048, 1408), and at one or two
-// tokens by the latency of the launches in a row.  Whole layer, 64 experts, top 6 (row-tiled form in brackets): 1 token 16.2 us
-// (35.0), 16 tokens 84 (112), 40 tokens 97 (123), 128 tokens 109 (126); at 40 tokens the first GEMM reads its weights at
-// 6.0 TB/s, 7.3 TB/s once the first pieces have arrived.  The row-tiled form of the layer pads every expert to 128 rows, needs
+// tokens by the latency of the launches in a row.  Whole layer, 64 experts, top 6 (row-tiled form in brackets): 1 token 16.1 us
+// (35.0), 16 tokens 75 (114), 40 tokens 95 (122), 64 tokens 99 (124); at 40 tokens the first GEMM reads its weights at
+// 6.0 TB/s.  The row-tiled form of the layer pads every expert to 128 rows, needs
 // moe_align and the quantizer in front and a sum behind, and leaves half of the chip without weights in flight.  Here:
-//   * No alignment launch.  The routing is a few hundred ids: every workgroup reads them all, marks the experts that have
-//     rows in an LDS bit mask and takes an equal share of (expert, group of columns) units -- contiguous, so that a
-//     workgroup meets one or two experts.  Every compute unit then takes in the same number of weight bytes whatever the
-//     routing is, which is what bounds the launch (about 27 bytes per nanosecond and compute unit).
+//   * No alignment launch.  The routing is a few hundred ids: every workgroup reads them all, counts the rows of every
+//     expert in LDS and takes an equal share of (expert, pass, group of columns) units -- contiguous, so that a workgroup
+//     meets one or two experts.  A pass is as many rows as are held at a time; an expert with more is streamed once per
+//     pass, and the passes are dealt like experts.  Every compute unit then takes in the same number of weight bytes whatever
+//     the routing is, which is what bounds the launch (about 27 bytes per nanosecond and compute unit).
 //   * No quantizer launch.  Four waves of a workgroup quantize the rows of its expert (a few rows; they come out of the L2)
 //     into LDS, in MFMA order, with the scales beside them, while the first weights are on their way to the others.
 //     The arithmetic is the quantizer's: the same bits.
@@ -125,7 +126,7 @@ constexpr int kLdsBytes = 160 * 1024;
 
 // Dynamic LDS of moe_decode_kernel, in this order.
 struct MoeDecodeLds {
-    int ring, codes, scales, wscales, ids, list, weight, mask, rows, total;  // byte offsets
+    int ring, codes, scales, wscales, ids, list, weight, count, rows, total;  // byte offsets
     __host__ __device__ static MoeDecodeLds of(const MoeDecodeParams& p) {
         MoeDecodeLds l{};
         l.ring = 0;
@@ -133,17 +134,16 @@ struct MoeDecodeLds {
         l.scales = l.codes + p.row_cap * p.K;
         l.wscales = l.scales + (p.row_cap * p.kblocks * 4 + 255) / 256 * 256;
         l.ids = l.wscales + p.wscale_cap * 4;
-        l.list = l.ids + p.slots * 4;
-        l.weight = l.list + p.slots * 4;
-        l.mask = l.weight + p.slots * 4;
-        l.rows = l.mask + (p.E + 31) / 32 * 4;
+        l.list = l.ids + p.slots * 2;
+        l.weight = l.list + p.slots * 2;
+        l.count = l.weight + p.slots * 4;
+        l.rows = l.count + (p.E + 1) / 2 * 4;
         l.total = l.rows + 4;
         return l;
     }
 };
 
-// MT: tiles of 16 activation rows (row_cap <= 16 MT)
-template <typename T, bool UP, int MT>
+template <typename T, bool UP>
 __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_decode_kernel(const MoeDecodeParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NW = kDecodeWaves, STAGES = kDecodeStages, NT = 64 * (NW + kDecodeQuantWaves), NTQ = 64 * kDecodeQuantWaves;
@@ -154,11 +154,11 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     uint8_t* const s_codes = lds + at.codes;    // [K step][row][128 bytes], chunk j of row r at j ^ (r % 8)
     float* const s_scale = reinterpret_cast<float*>(lds + at.scales);      // [K step][row]
     float* const s_wscale = reinterpret_cast<float*>(lds + at.wscales);    // [block row of the segment][gate, up][K step]
-    int* const s_ids = reinterpret_cast<int*>(lds + at.ids);
-    int* const s_list = reinterpret_cast<int*>(lds + at.list);             // the slots of the segment's expert
+    int16_t* const s_ids = reinterpret_cast<int16_t*>(lds + at.ids);
+    uint16_t* const s_list = reinterpret_cast<uint16_t*>(lds + at.list);   // the slots of the segment's expert
     float* const s_weight = reinterpret_cast<float*>(lds + at.weight);     // second GEMM: routed weight of every slot
-    int* const s_src = reinterpret_cast<int*>(lds + at.weight);            // first GEMM: the listed slots' rows of x
-    uint32_t* const s_mask = reinterpret_cast<uint32_t*>(lds + at.mask);
+    uint16_t* const s_src = reinterpret_cast<uint16_t*>(lds + at.weight);  // first GEMM: the listed slots' rows of x
+    uint32_t* const s_count = reinterpret_cast<uint32_t*>(lds + at.count); // rows of every expert, two 16-bit counts a word
     int* const s_rows = reinterpret_cast<int*>(lds + at.rows);             // rows of the segment's expert
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -166,55 +166,92 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     const int K = p.K, kblocks = p.kblocks, slots = p.slots, cap = p.row_cap;
     const int groups = (UP ? p.inter : p.N) / COLS;
 
-    // ---- the experts that have rows
-    const int words = (p.E + 31) / 32;
-    if (tid < words) s_mask[tid] = 0;           // (at most 16 words)
+    // ---- the experts' rows
+    if (tid < (p.E + 1) / 2) s_count[tid] = 0;  // (at most 256 words)
     __syncthreads();
     for (int i = tid; i < slots; i += NT) {
         const int e = decode_expert_id(p, i);
-        s_ids[i] = e;
+        s_ids[i] = (int16_t)e;
         if constexpr (!UP) s_weight[i] = p.topk_weights[i];
-        if (e >= 0) atomicOr(&s_mask[e >> 5], 1u << (e & 31));
+        if (e >= 0) atomicAdd(&s_count[e >> 1], 1u << ((e & 1) * 16));   // (at most 2048 slots: no carry into the other half)
     }
     __syncthreads();
-    int active = 0;
-    for (int i = 0; i < words; ++i) active += __popc(__builtin_amdgcn_readfirstlane((int)s_mask[i]));
+    auto rows_of = [&](int e) { return e < p.E ? (int)reinterpret_cast<const uint16_t*>(s_count)[e] : 0; };
+    const int cap_log2 = __builtin_ctz(cap);
+    int total_passes = 0;                       // one per expert that has rows; more for those with more than are held, if any
+    bool hot = false;
+    for (int base = 0; base < p.E; base += 64) {
+        const int c = rows_of(base + lane);
+        total_passes += __popcll(__ballot(c > 0));
+        hot |= __ballot(c > cap) != 0;
+    }
+    if (hot) {
+        total_passes = 0;
+        for (int base = 0; base < p.E; base += 64) total_passes += (rows_of(base + lane) + cap - 1) >> cap_log2;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) total_passes += __shfl_xor(total_passes, d);
+        total_passes = __builtin_amdgcn_readfirstlane(total_passes);
+    }
 
-    // ---- this workgroup's share of the active * groups units, in segments of one expert each.  When whole workgroups per
-    // expert leave few of them idle (one token, six experts: 42 of 256 for each) an expert's groups are dealt over its own
-    // workgroups, else the units are dealt over all of them, and a workgroup may meet two experts or more.
+    // ---- this workgroup's share of the total_passes * groups units, in segments of one pass each.  Either a pass's groups are
+    // dealt over workgroups of its own (one token, six experts: 42 of 256 for each), or the units are dealt over all of them
+    // and a workgroup may meet two passes or more: an equal share, but a second pass's preparation costs as much as streaming
+    // two groups and 40 K steps (about 3 us).  One expert in every token, 32 experts of (2048, 512), top 4, 48 tokens (33
+    // passes): 41.6 -> 32.7 us with 7 workgroups to each pass; 64 of (1024, 512), top 8, 56 tokens, half alike: 40.7 -> 35.6.
     const int grid = (int)gridDim.x, bid = (int)blockIdx.x;
     auto small_div = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };   // exact for x < 2^16
     int u_begin, u_end;
-    const int per = active > 0 ? small_div(grid, 1.0f / (float)active) : 0;              // workgroups per expert
-    if (per * active * 16 >= grid * 15) {
+    const int per = total_passes > 0 ? small_div(grid, 1.0f / (float)total_passes) : 0;  // workgroups per pass
+    if (per > 0 && groups * grid <= per * (total_passes * groups + (2 + 40 / kblocks) * grid)) {
         const float inv_per = 1.0f / (float)per;
         const int idx = small_div(bid, inv_per), part = bid - idx * per;
         u_begin = idx * groups + small_div(groups * part, inv_per);
         u_end = idx * groups + small_div(groups * (part + 1), inv_per);
-        if (idx >= active) u_begin = u_end = 0;
+        if (idx >= total_passes) u_begin = u_end = 0;
     } else {
-        const uint32_t units = (uint32_t)(active * groups);  // (below 2^20, and at most 1024 workgroups: 32 bits)
-        u_begin = (int)(units * (uint32_t)bid / (uint32_t)grid);
-        u_end = (int)(units * (uint32_t)(bid + 1) / (uint32_t)grid);
+        // units * bid / grid by quotient and remainder of units / grid: 32 bits suffice
+        const uint32_t units = (uint32_t)(total_passes * groups), q = units / (uint32_t)grid, r = units - q * (uint32_t)grid;
+        u_begin = (int)(q * (uint32_t)bid + r * (uint32_t)bid / (uint32_t)grid);
+        u_end = (int)(q * (uint32_t)(bid + 1) + r * (uint32_t)(bid + 1) / (uint32_t)grid);
     }
     u_begin = __builtin_amdgcn_readfirstlane(u_begin);
     u_end = __builtin_amdgcn_readfirstlane(u_end);
-    auto segment = [&](int u, int* e, int* g0, int* g1) {
+    // unit u -> its expert, the first of its rows and the groups [g0, g1) of the pass that are this workgroup's
+    auto segment = [&](int u, int* e, int* r0, int* g0, int* g1) {
         const int idx = __builtin_amdgcn_readfirstlane(u / groups);
         *g0 = u - idx * groups;
         *g1 = min(groups, *g0 + u_end - u);
-        int left = idx;   // the idx-th expert of the mask
+        int left = idx;
         *e = 0;
-        for (int i = 0; i < words; ++i) {
-            uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_mask[i]);
-            const int c = __popc(m);
-            if (left < c) {
-                for (; left > 0; --left) m &= m - 1;
-                *e = i * 32 + __builtin_ctz(m);
+        *r0 = 0;
+        for (int base = 0; base < p.E; base += 64) {
+            const int c = rows_of(base + lane);
+            if (!hot) {
+                // the left-th expert that has rows
+                const unsigned long long any = __ballot(c > 0);
+                if (left < __popcll(any)) {
+                    const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0));
+                    *e = base + __builtin_ctzll(__ballot(c > 0 && rank == left));
+                    break;
+                }
+                left -= __popcll(any);
+                continue;
+            }
+            const int mine = (c + cap - 1) >> cap_log2;
+            int incl = mine;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int below = __shfl_up(incl, d);
+                if (lane >= d) incl += below;
+            }
+            const unsigned long long past = __ballot(incl > left);
+            if (past != 0) {
+                const int at_lane = __builtin_ctzll(past);
+                *e = base + at_lane;
+                *r0 = (left - __builtin_amdgcn_readlane(incl - mine, at_lane)) * cap;
                 break;
             }
-            left -= c;
+            left -= __builtin_amdgcn_readlane(incl, 63);
         }
     };
 
@@ -223,8 +260,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
         const int qt = tid - 64 * NW;
         const float inv_kblocks = 1.0f / (float)kblocks, inv_top_k = 1.0f / (float)p.top_k;
         for (int u = u_begin; u < u_end;) {
-            int e, g0, g1;
-            segment(u, &e, &g0, &g1);
+            int e, r0, g0, g1;
+            segment(u, &e, &r0, &g0, &g1);
             u += g1 - g0;
             // the expert's slots, in ascending order (every one of these waves writes the same list)
             int rows = 0;
@@ -233,8 +270,8 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 const unsigned long long m = __ballot(mine);
                 if (mine) {
                     const int at_row = rows + __popcll(m & ((1ull << lane) - 1ull));
-                    s_list[at_row] = base + lane;
-                    if constexpr (UP) s_src[at_row] = small_div(base + lane, inv_top_k);
+                    s_list[at_row] = (uint16_t)(base + lane);
+                    if constexpr (UP) s_src[at_row] = (uint16_t)small_div(base + lane, inv_top_k);
                 }
                 rows += __popcll(m);
             }
@@ -248,36 +285,34 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                 const int nb = UP ? nb0 + (row >> 1) + ((row & 1) ? p.inter / 128 : 0) : nb0 + row;
                 s_wscale[i] = ws[nb * kblocks + kb];
             }
-            for (int r0 = 0; r0 < rows; r0 += cap) {
-                const int rows_a = min(cap, rows - r0);
-                const int n_x = rows_a * kblocks * 16;   // 16-byte pieces of activations: 16 to a group of 128
-                constexpr int BATCH = 8;
-                for (int first = qt; first - qt < n_x; first += BATCH * NTQ) {
-                    v4i raw[BATCH];
+            const int rows_a = min(cap, rows - r0);
+            const int n_x = rows_a * kblocks * 16;   // 16-byte pieces of activations: 16 to a group of 128
+            constexpr int BATCH = 8;
+            for (int first = qt; first - qt < n_x; first += BATCH * NTQ) {
+                v4i raw[BATCH];
 #pragma unroll
-                    for (int j = 0; j < BATCH; ++j) {
-                        const int task = min(first + j * NTQ, n_x - 16 + (lane & 15)), group = task >> 4;
-                        const int row = small_div(group, inv_kblocks), kb = group - row * kblocks;
-                        const int src = (UP ? s_src : s_list)[r0 + row];
-                        raw[j] = *reinterpret_cast<const v4i*>(reinterpret_cast<const T*>(p.x) + ((int64_t)src * K + kb * 128 + (task & 15) * 8));
-                    }
-                    // the first activations are requested before the weights: the compute unit takes its requests in order
-                    if (first == qt && r0 == 0) decode_barrier();
+                for (int j = 0; j < BATCH; ++j) {
+                    const int task = min(first + j * NTQ, n_x - 16 + (lane & 15)), group = task >> 4;
+                    const int row = small_div(group, inv_kblocks), kb = group - row * kblocks;
+                    const int src = (UP ? s_src : s_list)[r0 + row];
+                    raw[j] = *reinterpret_cast<const v4i*>(reinterpret_cast<const T*>(p.x) + ((int64_t)src * K + kb * 128 + (task & 15) * 8));
+                }
+                // the first activations are requested before the weights: the compute unit takes its requests in order
+                if (first == qt) decode_barrier();
 #pragma unroll
-                    for (int j = 0; j < BATCH; ++j) {
-                        const int task = first + j * NTQ, group = task >> 4, sub = task & 15;
-                        const int row = small_div(group, inv_kblocks), kb = group - row * kblocks;
-                        float sc;
-                        const v2i codes = quantize_lane<T>(raw[j], &sc);
-                        if (task < n_x) {
-                            *reinterpret_cast<v2i*>(s_codes + (kb * cap + row) * kKBlock + (((sub >> 1) ^ swz16(row)) << 4) + (sub & 1) * 8) = codes;
-                            if (sub == 0) s_scale[kb * cap + row] = sc;
-                        }
+                for (int j = 0; j < BATCH; ++j) {
+                    const int task = first + j * NTQ, group = task >> 4, sub = task & 15;
+                    const int row = small_div(group, inv_kblocks), kb = group - row * kblocks;
+                    float sc;
+                    const v2i codes = quantize_lane<T>(raw[j], &sc);
+                    if (task < n_x) {
+                        *reinterpret_cast<v2i*>(s_codes + (kb * cap + row) * kKBlock + (((sub >> 1) ^ swz16(row)) << 4) + (sub & 1) * 8) = codes;
+                        if (sub == 0) s_scale[kb * cap + row] = sc;
                     }
                 }
-                decode_barrier();   // the tile is ready
-                decode_barrier();   // ... and done with
             }
+            decode_barrier();   // the tile is ready
+            decode_barrier();   // ... and done with
         }
         return;
     }
@@ -299,118 +334,97 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     const uint32_t my_lds = lds_address(lds) + wave * STAGES * kDecodeBuf;
     const uint8_t* const my_ring = lds + wave * STAGES * kDecodeBuf;
     const int arow = li & (cap - 1);            // (columns past the rows of a tile repeat rows; they are not stored)
-    const uint32_t frag0 = arow * kKBlock + ((lg ^ swz16(arow)) << 4), frag1 = frag0 ^ 64;   // (16 rows on: 2 KiB)
+    const uint32_t frag0 = arow * kKBlock + ((lg ^ swz16(arow)) << 4), frag1 = frag0 ^ 64;
 
     for (int u = u_begin; u < u_end;) {
-        int e, g0, g1;
-        segment(u, &e, &g0, &g1);
+        int e, r0, g0, g1;
+        segment(u, &e, &r0, &g0, &g1);
         u += g1 - g0;
         const v4i rsrc_w = make_rsrc(p.w + (int64_t)e * p.N * K);
         const int nb0 = g0 * COLS / 128;
         const int total = max(0, (g1 - g0 - wave + NW - 1) / NW) * npieces;   // pieces of this wave
-        int r0 = 0, rows;
-        do {
-            // ---- the ring: as many pieces as it holds, before the activations are waited for
-            int gi = g0 + wave, ci = 0;
-            auto issue = [&](int stage) {
-                const int k0 = gi * (COLS * K) + ci * kDecodePiece;
-                const int valid = (tail_steps != 0 && ci == npieces - 1) ? tail_steps * 8 : 32;
+        // ---- the ring: as many pieces as it holds, before the activations are waited for
+        int gi = g0 + wave, ci = 0;
+        auto issue = [&](int stage) {
+            const int k0 = gi * (COLS * K) + ci * kDecodePiece;
+            const int valid = (tail_steps != 0 && ci == npieces - 1) ? tail_steps * 8 : 32;
 #pragma unroll
-                for (int i = 0; i < LOADS; ++i)
-                    direct_load_b128_nt(rsrc_w, my_lds + stage * kDecodeBuf + i * 1024, (pos ^ (2 * i + half)) < valid ? w_off[i] : kDecodeOutOfRange, k0);
-                if (++ci == npieces) { ci = 0; gi += NW; }
-            };
-            if (r0 == 0) decode_barrier();
-            for (int s = 0; s < STAGES && s < total; ++s) issue(s);
-            decode_barrier();
-            rows = __builtin_amdgcn_readfirstlane(*s_rows);
-            const int rows_a = min(cap, rows - r0);
+            for (int i = 0; i < LOADS; ++i)
+                direct_load_b128_nt(rsrc_w, my_lds + stage * kDecodeBuf + i * 1024, (pos ^ (2 * i + half)) < valid ? w_off[i] : kDecodeOutOfRange, k0);
+            if (++ci == npieces) { ci = 0; gi += NW; }
+        };
+        decode_barrier();
+        for (int s = 0; s < STAGES && s < total; ++s) issue(s);
+        decode_barrier();
+        const int rows_a = min(cap, __builtin_amdgcn_readfirstlane(*s_rows) - r0);
 
-            // ---- this wave's groups
-            int gc = g0 + wave, cc = 0;
-            v4f acc[MT];
+        // ---- this wave's groups
+        int gc = g0 + wave, cc = 0;
+        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+        int stage = 0;
+        for (int i = 0; i < total; ++i) {
+            if (i + STAGES <= total) wait_vmcnt<(STAGES - 1) * LOADS>();
+            else wait_vmcnt<0>();
+            // Everything the piece needs is read at once: one LDS round trip per piece.  K steps past the end of K multiply
+            // zeros (their weight loads are out of range) with the last step's activations, under scales of zero (the last step's
+            // may be infinite).
+            const uint8_t* wb = my_ring + stage * kDecodeBuf + li * kDecodePiece;
+            const float* ws = s_wscale + ((gc * COLS >> 7) - nb0) * (UP ? 2 : 1) * kblocks;
+            v8i wf[kDecodeSteps], af[kDecodeSteps];
+            float as[kDecodeSteps], bg[kDecodeSteps], bu[kDecodeSteps];
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[mt] = v4f{0.f, 0.f, 0.f, 0.f};
-            int stage = 0;
-            for (int i = 0; i < total; ++i) {
-                if (i + STAGES <= total) wait_vmcnt<(STAGES - 1) * LOADS>();
-                else wait_vmcnt<0>();
-                // Everything the piece needs is read at once: one LDS round trip per piece.  K steps past the end of K multiply
-                // zeros (their weight loads are out of range) with the last step's activations, under scales of zero (the last step's
-                // may be infinite).
-                const uint8_t* wb = my_ring + stage * kDecodeBuf + li * kDecodePiece;
-                const float* ws = s_wscale + ((gc * COLS >> 7) - nb0) * (UP ? 2 : 1) * kblocks;
-                v8i wf[kDecodeSteps], af[MT][kDecodeSteps];
-                float as[MT][kDecodeSteps], bg[kDecodeSteps], bu[kDecodeSteps];
+            for (int s = 0; s < kDecodeSteps; ++s) {
+                const int kb = min(cc * kDecodeSteps + s, kblocks - 1);
+                const uint8_t* ab = s_codes + kb * cap * kKBlock;
+                wf[s] = join(*reinterpret_cast<const v4i*>(wb + (((s * 8 + lg) ^ li) << 4)), *reinterpret_cast<const v4i*>(wb + (((s * 8 + 4 + lg) ^ li) << 4)));
+                af[s] = join(*reinterpret_cast<const v4i*>(ab + frag0), *reinterpret_cast<const v4i*>(ab + frag1));
+                as[s] = s_scale[kb * cap + arow];
+                bg[s] = ws[kb];
+                bu[s] = UP ? ws[kblocks + kb] : 0.f;
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the stage is free
 #pragma unroll
-                for (int s = 0; s < kDecodeSteps; ++s) {
-                    const int kb = min(cc * kDecodeSteps + s, kblocks - 1);
-                    const uint8_t* ab = s_codes + kb * cap * kKBlock;
-                    wf[s] = join(*reinterpret_cast<const v4i*>(wb + (((s * 8 + lg) ^ li) << 4)), *reinterpret_cast<const v4i*>(wb + (((s * 8 + 4 + lg) ^ li) << 4)));
+            for (int s = 0; s < kDecodeSteps; ++s) asm volatile("" : "+v"(wf[s]), "+v"(af[s]), "+v"(as[s]), "+v"(bg[s]), "+v"(bu[s]));
+            if (i + STAGES < total) issue(stage);
+            stage = stage + 1 == STAGES ? 0 : stage + 1;
+            if (tail_steps != 0 && cc == npieces - 1) {
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) {
-                        af[mt][s] = join(*reinterpret_cast<const v4i*>(ab + mt * 16 * kKBlock + frag0), *reinterpret_cast<const v4i*>(ab + mt * 16 * kKBlock + frag1));
-                        as[mt][s] = s_scale[kb * cap + mt * 16 + arow];
-                    }
-                    bg[s] = ws[kb];
-                    bu[s] = UP ? ws[kblocks + kb] : 0.f;
-                }
-                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the stage is free
-#pragma unroll
-                for (int s = 0; s < kDecodeSteps; ++s) {
-                    asm volatile("" : "+v"(wf[s]), "+v"(bg[s]), "+v"(bu[s]));
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(af[mt][s]), "+v"(as[mt][s]));
-                }
-                if (i + STAGES < total) issue(stage);
-                stage = stage + 1 == STAGES ? 0 : stage + 1;
-                if (tail_steps != 0 && cc == npieces - 1) {
-#pragma unroll
-                    for (int s = 1; s < kDecodeSteps; ++s) {
-                        const bool past = s >= tail_steps;
-                        bg[s] = past ? 0.f : bg[s];
-                        bu[s] = past ? 0.f : bu[s];
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) as[mt][s] = past ? 0.f : as[mt][s];
-                    }
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    v4f part[kDecodeSteps];
-#pragma unroll
-                    for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[mt][s], v4f{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                    for (int s = 0; s < kDecodeSteps; ++s) {
-                        const float lo = as[mt][s] * bg[s], hi = UP ? as[mt][s] * bu[s] : lo;
-                        acc[mt] += part[s] * v4f{lo, lo, hi, hi};
-                    }
-                }
-                if (++cc == npieces) {
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) {
-                        if (mt * 16 + li < rows_a) {
-                            const int slot = s_list[r0 + mt * 16 + li];
-                            if constexpr (UP) {
-                                typedef T vec2 __attribute__((ext_vector_type(2)));
-                                vec2 v;
-                                v[0] = (T)silu_mul_round<T>((float)(T)acc[mt][0], (float)(T)acc[mt][2]);
-                                v[1] = (T)silu_mul_round<T>((float)(T)acc[mt][1], (float)(T)acc[mt][3]);
-                                *reinterpret_cast<vec2*>(reinterpret_cast<T*>(p.out) + (int64_t)slot * p.inter + gc * COLS + lg * 2) = v;
-                            } else {
-                                typedef T vec4 __attribute__((ext_vector_type(4)));
-                                *reinterpret_cast<vec4*>(reinterpret_cast<T*>(p.out) + (int64_t)slot * p.N + gc * COLS + lg * 4) =
-                                    __builtin_convertvector(acc[mt] * s_weight[slot], vec4);
-                            }
-                        }
-                        acc[mt] = v4f{0.f, 0.f, 0.f, 0.f};
-                    }
-                    cc = 0;
-                    gc += NW;
+                for (int s = 1; s < kDecodeSteps; ++s) {
+                    const bool past = s >= tail_steps;
+                    as[s] = past ? 0.f : as[s];
+                    bg[s] = past ? 0.f : bg[s];
+                    bu[s] = past ? 0.f : bu[s];
                 }
             }
-            decode_barrier();
-            r0 += cap;
-        } while (r0 < rows);
+            v4f part[kDecodeSteps];
+#pragma unroll
+            for (int s = 0; s < kDecodeSteps; ++s) part[s] = mfma_e4m3(wf[s], af[s], v4f{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int s = 0; s < kDecodeSteps; ++s) {
+                const float lo = as[s] * bg[s], hi = UP ? as[s] * bu[s] : lo;
+                acc += part[s] * v4f{lo, lo, hi, hi};
+            }
+            if (++cc == npieces) {
+                if (li < rows_a) {
+                    const int slot = s_list[r0 + li];
+                    if constexpr (UP) {
+                        typedef T vec2 __attribute__((ext_vector_type(2)));
+                        vec2 v;
+                        v[0] = (T)silu_mul_round<T>((float)(T)acc[0], (float)(T)acc[2]);
+                        v[1] = (T)silu_mul_round<T>((float)(T)acc[1], (float)(T)acc[3]);
+                        *reinterpret_cast<vec2*>(reinterpret_cast<T*>(p.out) + (int64_t)slot * p.inter + gc * COLS + lg * 2) = v;
+                    } else {
+                        typedef T vec4 __attribute__((ext_vector_type(4)));
+                        *reinterpret_cast<vec4*>(reinterpret_cast<T*>(p.out) + (int64_t)slot * p.N + gc * COLS + lg * 4) =
+                            __builtin_convertvector(acc * s_weight[slot], vec4);
+                    }
+                }
+                acc = v4f{0.f, 0.f, 0.f, 0.f};
+                cc = 0;
+                gc += NW;
+            }
+        }
+        decode_barrier();
     }
 #endif
 }

@@ -10,38 +10,46 @@ namespace {
 // Fills in row_cap and wscale_cap; false when the layer is not one for this kernel.
 //
 // An expert with more than row_cap rows is streamed more than once, so the rows that the fullest expert is likely to get
-// decide: with m = slots / E rows on average and even routing about m + 3 sqrt(m).  Whole layer, (hidden, inter) =
-// (2048, 1408), 64 experts, top 6, against the row-tiled form: 1 token 16.2 us (35.0), 16 tokens 84 (112), 64 tokens
-// (m = 6) 99 (124); at 96 tokens (m = 9) 131 (125) with 16 rows held, so more rows are held from there on (two tiles of 16).
+// decide: with m = slots / E rows on average and even routing about m + 3 sqrt(m).  The line lies where a batch half of which
+// routes alike (padding rows, say) takes as long as on the row-tiled form.  Whole layer, 64 experts of (2048, 1408), top 6,
+// against that form (in brackets), us:
+//   tokens (m)    even routing   half alike     one expert in every token   all alike
+//   40 (3.8)       94 (122)       98 (118)      100 (122)                   43 (37)
+//   64 (6)         99 (124)      121 (122)      119 (123)                   56 (38)
+//   75 (7.0)      101 (125)      127 (124)      117 (125)                   51 (43)     <- the last one taken
+//   87 (8.2)      102 (125)      128 (126)      121 (126)                   72 (43)
+// and 128 experts of (4096, 1536), top 8: 80 (5) 382 (454), 420 (438), 426 (454), 137 (61); 96 (6) 390 (462), 445 (443), 421
+// (458), 175 (63); 130 (8.1) 401 (460), 494 (458), 429 (495), 251 (69).  32 rows held take even routing to 174 tokens (111
+// against 127 at 160), but an expert over the line then costs more than the rest saves (143 - 158 against 130 - 136).
+constexpr int kDecodeRows = 16;
+constexpr float kDecodeLikely = 15.0f;
 bool decode_plan(MoeDecodeParams& p, bool up, int tokens) {
     const int cols = up ? 8 : 16, groups = (up ? p.inter : p.N) / cols;
     const int nbs = (groups * cols + 127) / 128 + 1;   // block rows of a segment, at most
     p.wscale_cap = (nbs * (up ? 2 : 1) * p.kblocks + 63) / 64 * 64;
-    const float mean = (float)p.slots / (float)p.E, likely = fminf(mean + 3.0f * sqrtf(mean), (float)tokens);
-    const int most = likely < 18.0f ? 16 : 32;
     int cap = 1;
-    while (cap < tokens && cap < most) cap *= 2;
+    while (cap < tokens && cap < kDecodeRows) cap *= 2;
     while (cap > 1) {
         p.row_cap = cap;
         if (MoeDecodeLds::of(p).total <= kLdsBytes) break;
         cap /= 2;
     }
     p.row_cap = cap;
-    return MoeDecodeLds::of(p).total <= kLdsBytes && likely < (float)(cap + 2);
+    const float mean = (float)p.slots / (float)p.E, likely = mean + 3.0f * sqrtf(mean);
+    return MoeDecodeLds::of(p).total <= kLdsBytes && (tokens <= cap || likely < fminf((float)(cap + 2), kDecodeLikely));
 }
 
-template <typename T, bool UP, int MT>
+template <typename T, bool UP>
 hipError_t launch_decode(const MoeDecodeParams& p, hipStream_t s) {
     // one workgroup per compute unit: each takes an equal share of the weights
-    hipLaunchKernelGGL((moe_decode_kernel<T, UP, MT>), dim3((unsigned)compute_units()), dim3(64 * (kDecodeWaves + kDecodeQuantWaves)),
+    hipLaunchKernelGGL((moe_decode_kernel<T, UP>), dim3((unsigned)compute_units()), dim3(64 * (kDecodeWaves + kDecodeQuantWaves)),
                        (size_t)MoeDecodeLds::of(p).total, s, p);
     return hipGetLastError();
 }
 
 template <typename T>
 hipError_t dispatch_decode(const MoeDecodeParams& p, bool up, hipStream_t s) {
-    if (p.row_cap > 16) return up ? launch_decode<T, true, 2>(p, s) : launch_decode<T, false, 2>(p, s);
-    return up ? launch_decode<T, true, 1>(p, s) : launch_decode<T, false, 1>(p, s);
+    return up ? launch_decode<T, true>(p, s) : launch_decode<T, false>(p, s);
 }
 
 bool decode_shape_ok(const MoeDecodeParams& p, bool up) {

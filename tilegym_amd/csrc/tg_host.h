@@ -26,7 +26,7 @@ struct MoeDecodeParams {
     const void* ids;           // (slots) int32 or int64 expert ids
     void* out;                 // first GEMM: (slots, inter); second: (slots, N), or with the sum (tokens, N)
     int ids_are_i64, slots, top_k, E, N, K, inter, kblocks, nblocks;
-    int row_cap;               // activation rows held at a time: a power of two, at most 32
+    int row_cap;               // activation rows held at a time: a power of two, at most 16
     int wscale_cap;            // floats of LDS for a segment's weight scales, a multiple of 64
 };
 
