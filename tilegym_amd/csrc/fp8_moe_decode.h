@@ -199,14 +199,16 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     // two groups and 40 K steps (about 3 us).  One expert in every token, 32 experts of (2048, 512), top 4, 48 tokens (33
     // passes): 41.6 -> 32.7 us with 7 workgroups to each pass; 64 of (1024, 512), top 8, 56 tokens, half alike: 40.7 -> 35.6.
     const int grid = (int)gridDim.x, bid = (int)blockIdx.x;
-    auto small_div = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };   // exact for x < 2^16
+    // x / d from inv = 1 / d: two roundings move (x + 0.5) / d, which is 0.5 / d or more away from an integer, by less than
+    // (x + 0.5) / d * 2^-22, so exact for x < 2^21 (below: groups <= 8192 times fewer than 256 workgroups)
+    auto small_div = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
     int u_begin, u_end;
     const int per = total_passes > 0 ? small_div(grid, 1.0f / (float)total_passes) : 0;  // workgroups per pass
     if (per > 0 && groups * grid <= per * (total_passes * groups + (2 + 40 / kblocks) * grid)) {
         const float inv_per = 1.0f / (float)per;
         const int idx = small_div(bid, inv_per), part = bid - idx * per;
         u_begin = idx * groups + small_div(groups * part, inv_per);
-        u_end = idx * groups + small_div(groups * (part + 1), inv_per);
+        u_end = part == per - 1 ? (idx + 1) * groups : idx * groups + small_div(groups * (part + 1), inv_per);
         if (idx >= total_passes) u_begin = u_end = 0;
     } else {
         // units * bid / grid by quotient and remainder of units / grid: 32 bits suffice

@@ -1,6 +1,7 @@
 // Instantiations and launchers of the decoding MoE layer (fp8_moe_decode.h).
 #include "fp8_moe_decode.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace tg {
@@ -41,8 +42,8 @@ bool decode_plan(MoeDecodeParams& p, bool up, int tokens) {
 
 template <typename T, bool UP>
 hipError_t launch_decode(const MoeDecodeParams& p, hipStream_t s) {
-    // one workgroup per compute unit: each takes an equal share of the weights
-    hipLaunchKernelGGL((moe_decode_kernel<T, UP>), dim3((unsigned)compute_units()), dim3(64 * (kDecodeWaves + kDecodeQuantWaves)),
+    // one workgroup per compute unit: each takes an equal share of the weights (at most 256, for the kernel's 32-bit shares)
+    hipLaunchKernelGGL((moe_decode_kernel<T, UP>), dim3((unsigned)std::min(compute_units(), 256)), dim3(64 * (kDecodeWaves + kDecodeQuantWaves)),
                        (size_t)MoeDecodeLds::of(p).total, s, p);
     return hipGetLastError();
 }
