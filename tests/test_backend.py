@@ -242,3 +242,35 @@ def test_decoding_moe_layer_asks_for_no_more_lds_than_a_compute_unit_has(hidden,
     asked = [lds(tokens, top_k, experts, hidden, inter) for tokens in range(1, 2048 // top_k + 2)]
     assert max(asked) <= 160 * 1024 and asked[-1] == 0
     assert asked[0] > 0 or hidden > 8192
+
+
+def test_an_unusable_native_binding_leaves_the_ctypes_path():
+    """The binding depends on the torch it was compiled against; the library does not.  Without the binding load() warns, and calls
+    reach the library as they do with it (here: up to the check that refuses host tensors)."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import sys, warnings
+sys.modules["tilegym_amd._native"] = None   # import of the binding: ImportError
+import torch
+from tilegym_amd import _lib
+from tilegym_amd.ops import matmul
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    assert _lib.load().tg_abi_version() == 1
+assert any("_native.so" in str(w.message) for w in seen) and _lib.native is None
+assert not _lib.fast_path() and not _lib.native_path()
+a, b = torch.zeros(4, 128, dtype=torch.float8_e4m3fn), torch.zeros(8, 128, dtype=torch.float8_e4m3fn)
+try:
+    matmul(a, b, trans_b=True, out_dtype=torch.bfloat16)
+except RuntimeError as e:
+    assert "HIP device" in str(e), e
+else:
+    raise AssertionError("host tensors were taken")
+print("fine")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "fine" in run.stdout, run.stdout + run.stderr

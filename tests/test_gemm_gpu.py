@@ -1814,6 +1814,30 @@ def test_native_binding_agrees_with_the_general_path(device):
         _lib.fp8_gemm(torch.empty(6, 23, device=device), a, b)
 
 
+def test_calls_without_the_native_binding(device, monkeypatch):
+    """The same calls where the native module could not be imported: the ctypes path reaches the same kernels."""
+    from tilegym_amd.ops import fused_moe
+    from tilegym_amd.quant import act_quant
+
+    g = _g(78)
+    a, b = fp8_randn((6, 256), g).to(device), fp8_randn((128, 256), g, 0.1).to(device)
+    layer = _device_moe_layer(device, 3, 256, 128, 8, 2, seed=5)
+    indptr = torch.tensor([0, 2, 6], dtype=torch.int32, device=device)
+
+    def calls():
+        q, s = act_quant(layer[0], 128)
+        x, w1, w2, s1, s2, tw, ids = layer
+        return [matmul(a, b, trans_b=True, scale_a=0.5, out_dtype=torch.float32), matmul(a, b[:6].t().contiguous(), out_dtype=torch.bfloat16),
+                w8a8_block_fp8_matmul(q, b, s, s1[0, :1], [128, 128], torch.bfloat16), q.view(torch.uint8), s,
+                ragged_block_scaled_bmm(a, w1[:2], torch.ones(6, 2, device=device), s1[:2], indptr, 4),
+                fused_moe(x, w1, w2, tw, ids, w1_scale=s1, w2_scale=s2)]
+
+    want = calls()
+    monkeypatch.setattr(_lib, "native", None)
+    for got, w in zip(calls(), want):
+        assert torch.equal(got, w)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 16, 128), (96, 144, 256), (130, 272, 1040), (65, 4112, 4096), (300, 128, 200), (20, 4080, 1008)])
 def test_kn_weights_give_the_bits_of_nk_weights(device, M, N, K):
     """(K, N) weights go through the 16-byte transpose: edges of its 128 x 128 tiles in both directions, a padded K (rows of the

@@ -3,7 +3,8 @@
 Ordinary calls of the operators go through the extension module ``_native`` (csrc/binding.cpp), which checks, allocates and
 calls the C ABI in native code; everything else -- schedule overrides, unusual layouts, the helpers -- through ctypes here.
 This is the only module that touches the shared library.  It never falls back to another
-implementation: if the library is missing or a call fails, it raises.
+implementation: if the library is missing or a call fails, it raises.  (``_native`` is compiled against one torch; where
+another one cannot import it, load() warns and every call goes through ctypes: the same kernels, more host time.)
 
 The descriptor / return-code conventions follow the reference's own C-ABI precedent
 (src/tilegym/backend/cutile_rs/utils.py:268-290 ``make_tensor_desc``, :353-370 ``check_rc``).
@@ -14,6 +15,7 @@ from __future__ import annotations
 import ctypes
 import struct
 import os
+import warnings
 from typing import Dict, Optional, Sequence, Tuple
 
 import torch
@@ -65,7 +67,7 @@ class TileGymHipError(RuntimeError):
 
 
 _lib = None
-native = None  # the extension module, once load() has run
+native = None  # the extension module, once load() has run (still None where it cannot be imported)
 _NATIVE_ENTRY_POINTS = ("tg_fp8_gemm", "tg_fp8_gemm_workspace_bytes", "tg_fp8_ragged_gemm", "tg_fp8_quant_group", "tg_fp8_fused_moe",
                         "tg_fp8_fused_moe_workspace_bytes")
 
@@ -146,27 +148,28 @@ def load():
     L.tg_diag_moe_lds_bytes.argtypes = [ctypes.c_int64] * 5
     if L.tg_abi_version() != 1:
         raise RuntimeError(f"libtilegym_hip.so ABI version {L.tg_abi_version()} != 1")
+    global native
     try:
         from . import _native
     except ImportError as e:
-        raise RuntimeError(f"tilegym_amd/_native.so cannot be loaded ({e}); build it with `python -m tilegym_amd.build`. "
-                           f"There is no fallback implementation.") from e
-    _native.set_up({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _NATIVE_ENTRY_POINTS}, _workspaces,
-                   workspace_for, check_rc)
-    global native
-    native = _native
+        warnings.warn(f"tilegym_amd/_native.so cannot be imported ({e}): calls go through ctypes, at about twice the host time. "
+                      f"Build it against this torch with `python -m tilegym_amd.build`.", RuntimeWarning, stacklevel=2)
+    else:
+        _native.set_up({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _NATIVE_ENTRY_POINTS}, _workspaces,
+                       workspace_for, check_rc)
+        native = _native
     _lib = L
     return L
 
 
-def loaded() -> bool:
-    """Load the library if it is not; True (a missing one raises)."""
-    return _lib is not None or load() is not None
+def native_path() -> bool:
+    """Whether calls may go to the native module; loads the library if that has not been done (a missing one raises)."""
+    return (_lib is not None or load() is not None) and native is not None
 
 
 def fast_path() -> bool:
     """Whether a dense call without kernel_configs may go straight to the native module: no schedule table to look up."""
-    return loaded() and not schedules_recorded()
+    return native_path() and not schedules_recorded()
 
 
 def make_tensor_desc(t: Optional[torch.Tensor]) -> Optional[TgTensor]:
@@ -380,7 +383,7 @@ def fp8_gemm(c, a, b, scale_a=None, scale_b=None, trans_a=False, trans_b=True, a
              kernel_configs=None, use_workspace=True) -> None:
     L = _lib if _lib is not None else load()
     trans_a, trans_b = bool(trans_a), bool(trans_b)
-    if (kernel_configs is None and not schedules_recorded()
+    if (kernel_configs is None and native is not None and not schedules_recorded()
             and native.gemm(c, a, b, scale_a, scale_b, trans_a, trans_b, float(alpha), float(beta), bool(use_workspace))):
         return
     dev = _device_index(a)

@@ -148,7 +148,7 @@ def ragged_block_scaled_bmm(a, b, a_scale, b_scale, m_indptr, max_m, max_m_devic
     ``max_m`` / ``max_m_device`` bound the reference's uniform tile walk; the expert-offset
     launch here reads the segment sizes on the device, so both are accepted and unused."""
     assert transpose_a == False and transpose_b == True, "Only NT layout is supported"  # noqa: E712
-    if not kwargs and _lib.loaded():
+    if not kwargs and _lib.native_path():
         c = _lib.native.ragged_matmul(a, b, a_scale, b_scale, m_indptr, out_dtype)
         if c is not None:
             return c

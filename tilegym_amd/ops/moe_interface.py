@@ -79,7 +79,7 @@ def fused_experts_impl(
 
     if use_int8_w8a16 or not use_fp8_w8a8:
         raise NotImplementedError("the hip backend implements the use_fp8_w8a8 MoE path only")
-    if USE_ONE_CALL_LAYER and a1_scale is None and _lib.loaded():
+    if USE_ONE_CALL_LAYER and a1_scale is None and _lib.native_path():
         # the plain case of the one-call layer (below), taken in native code
         out = _lib.native.fused_moe(hidden_states, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, bool(inplace), _lib.MOE_ALIGN_MAX_EXPERTS)
         if out is not None:

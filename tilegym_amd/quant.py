@@ -33,7 +33,7 @@ def _require_device(x: torch.Tensor, what: str, group: int) -> None:
 def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-token 1 x block_size quantization; all-zero block -> scale 1.0
     (src/tilegym/suites/unsloth/cutile/fp8.py:370-385)."""
-    if block_size in _GROUPS and _lib.loaded():
+    if block_size in _GROUPS and _lib.native_path():
         out = _lib.native.act_quant(x, block_size, 0.0, 0)
         if out is not None:
             return out
