@@ -1840,13 +1840,15 @@ def test_calls_without_the_native_binding(device, monkeypatch):
 
 @pytest.mark.parametrize("M,N,K", [(70, 16, 128), (96, 144, 256), (130, 272, 1040), (65, 4112, 4096), (300, 128, 200), (20, 4080, 1008)])
 def test_kn_weights_give_the_bits_of_nk_weights(device, M, N, K):
-    """(K, N) weights go through the 16-byte transpose: edges of its 128 x 128 tiles in both directions, a padded K (rows of the
-    copy longer than K: 1040, 200, 1008 are no multiples of 128), against the same weight handed over as (N, K)."""
+    """(K, N) weights through the 16-byte transpose: edges of its 128 x 128 tiles in both directions, a padded K (rows of the copy
+    longer than K: 1040, 200, 1008 are no multiples of 128), against the same weight handed over as (N, K).  A kernel asked for by
+    name takes the copy; without one, the narrow tiles may read the weight as it lies."""
     g = _g(M + N + K)
     a, b = fp8_randn((M, K), g).to(device), fp8_randn((N, K), g, 0.3).to(device)
-    want = matmul(a, b, trans_b=True, out_dtype=torch.float32)
-    got = matmul(a, b.view(torch.uint8).t().contiguous().view(FP8), out_dtype=torch.float32)
-    assert torch.equal(got, want)
+    kn = b.view(torch.uint8).t().contiguous().view(FP8)
+    for kernel_configs in ({"KERNEL": "tiled"}, None):
+        want = matmul(a, b, trans_b=True, out_dtype=torch.float32, kernel_configs=kernel_configs)
+        assert torch.equal(matmul(a, kn, out_dtype=torch.float32, kernel_configs=kernel_configs), want)
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 128), (16, 48, 256), (17, 4112, 384), (33, 80, 640), (64, 144, 1152), (65, 208, 128), (100, 2064, 1024),
