@@ -437,11 +437,11 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
 // to the 16-bit type as the row-per-slot form stores them, are added through LDS in slot order.
 constexpr int kDecodeSumRows = 8;
 constexpr int kDecodeSumStages = 3;
-// Dynamic LDS of moe_decode_sum_kernel: every wave's ring, every wave's codes and scales, the slots' results.
+// Dynamic LDS of moe_decode_sum_kernel: every wave's ring (in the end its slot's results), every wave's codes and scales.
 // (the scales of a piece's four K steps are read whole: three zeros behind the last one)
 __host__ __device__ inline int moe_decode_sum_codes(int K) { return (K + K / 32 + 12 + 255) / 256 * 256; }
 inline int moe_decode_sum_lds(int top_k, int K) {
-    return top_k * (kDecodeSumStages * kDecodeSumRows * kDecodePiece + moe_decode_sum_codes(K) + kDecodeSumRows * 4);
+    return top_k * (kDecodeSumStages * kDecodeSumRows * kDecodePiece + moe_decode_sum_codes(K));
 }
 
 template <typename T>
@@ -460,7 +460,6 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
     const int codes_bytes = moe_decode_sum_codes(K);
     uint8_t* const my_codes = lds + p.top_k * STAGES * BUF + wave * codes_bytes;  // [K step][128 bytes]
     float* const my_scale = reinterpret_cast<float*>(my_codes + K);               // [K step]
-    float* const s_red = reinterpret_cast<float*>(lds + p.top_k * (STAGES * BUF + codes_bytes));  // [slot][row]
     const int e = __builtin_amdgcn_readfirstlane(decode_expert_id(p, slot));
     const float weight = p.topk_weights[slot];
     v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
@@ -546,13 +545,14 @@ __global__ void __launch_bounds__(512) moe_decode_sum_kernel(const MoeDecodePara
         for (int q = 0; q < 4; ++q) {
             float v = e >= 0 ? acc[q] * weight : 0.f;   // (a slot without an expert adds nothing, whatever its weight)
             asm("" : "+v"(v));  // (the product is rounded on its own before the conversion, as the stored form is)
-            s_red[wave * R + lg * 4 + q] = (float)(T)v;
+            reinterpret_cast<float*>(my_ring)[lg * 4 + q] = (float)(T)v;   // (the ring has been read to its end)
         }
     }
     __syncthreads();
     if (tid < R) {
-        float sum = s_red[tid];
-        for (int w = 1; w < p.top_k; ++w) sum += s_red[w * R + tid];
+        auto slot_result = [&](int w) { return reinterpret_cast<const float*>(lds + w * STAGES * BUF)[tid]; };
+        float sum = slot_result(0);
+        for (int w = 1; w < p.top_k; ++w) sum += slot_result(w);
         reinterpret_cast<T*>(p.out)[(int64_t)blockIdx.y * p.N + n0 + tid] = (T)sum;
     }
 #endif
