@@ -460,8 +460,7 @@ def main():
                 op = torch.ops.tilegym_hip.fp8_gemm_out
                 sh["eager_us_torch_op"] = round(_eager_us(lambda i, r=r: op(c0, r.a[i % r.copies], r.b[i % r.copies], r.sa, r.sb,
                                                                              False, True, 1.0, 0.0), 200, stream), 2)
-                # through the public op with a fresh output tensor per call (torch.empty included): the prepared-call
-                # cache of the binding cannot hit, only its per-weight descriptors do
+                # through the public op with a fresh output tensor per call (its allocation included)
                 from tilegym_amd.ops import matmul as op_matmul
                 sh["eager_us_fresh_output"] = round(_eager_us(lambda i, r=r: op_matmul(r.a[i % r.copies], r.b[i % r.copies], trans_b=True,
                                                                                    scale_a=r.sa, scale_b=r.sb, out_dtype=torch.bfloat16),

@@ -300,9 +300,10 @@ int32_t tg_moe_sum_routed(const tg_tensor* out, const tg_tensor* x, const tg_ten
 /*
  * The FP8 MoE layer in one call: what src/tilegym/ops/moe_interface.py:116-322 (fused_experts_impl, use_fp8_w8a8) does
  * for one chunk of tokens, as the four launches tg_moe_align_quant_1x128 -> tg_fp8_moe_gemm_silu_quant -> tg_fp8_moe_gemm
- * (x routed weight) -> tg_moe_sum on the caller's stream, with every intermediate in `workspace`.  The results are the
- * bits the four calls give one by one; what the call saves is the host time of four bindings and nine allocations, which at
- * one to sixteen tokens is more than the kernels run.
+ * (x routed weight) -> tg_moe_sum_routed on the caller's stream, with every intermediate in `workspace`; with few rows per
+ * expert (seven on average for ordinary sizes) as two or three launches that stream the weights of the experts that have rows.
+ * The results are the bits the four calls give one by one.  What the call saves is the host time of four bindings and nine
+ * allocations; the second form also saves the padding of every expert to a row tile.  Ids outside [0, E) add nothing.
  *   hidden (T, H) bf16 / f16, H % 128 == 0; w1 (E, 2I, H), w2 (E, H, I) e4m3fn with w1_scale (E, 2I/128, H/128) and
  *   w2_scale (E, H/128, ceil(I/128)) f32; topk_weights (T, k) f32 and topk_ids (T, k) int32 / int64, contiguous;
  *   out (T, H) of hidden's type.  E <= 512, 2I % 256 == 0, block_m 128 or 256 (the alignment block = the row tile of the

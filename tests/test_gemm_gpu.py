@@ -2056,7 +2056,7 @@ def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_
                        "us": 0.0, "auto_us": 0.0, "auto_schedule": {}}], path)
     try:
         _lib.load_tune_table(path)
-        for _ in range(2):                                             # the second call comes from the prepared-call cache
+        for _ in range(2):                                             # the table applies to every call
             _lib.fp8_gemm(c, a, b, sa, sb)
             got = _lib.last_config()
             assert (got["KERNEL_NAME"], got["ROW_GROUPS"], got["SPLIT_K"]) == ("stream", 4, 2), got
@@ -2073,9 +2073,9 @@ def test_recorded_schedule_is_used_when_no_kernel_configs_are_given(device, tmp_
 
 
 def test_prepared_call_cache_follows_the_tensors(device):
-    """The binding keeps the prepared arguments of a call by the identity of its tensors.  The same objects again: same
-    result; an operand given new storage, a resized output, fresh outputs whose Python ids repeat, a dead weight whose id
-    is taken over by another tensor: each described afresh, never the stale pointer."""
+    """The binding describes a call's tensors on every call.  The same objects again: same result; an operand given new storage, a
+    resized output, fresh outputs whose Python ids repeat, a dead weight whose id is taken over by another tensor: never a stale
+    pointer."""
     from tilegym_amd import _lib
 
     g = _g(123)

@@ -628,8 +628,9 @@ def fused_moe_ok(hidden, w1, w2, block_m: int) -> bool:
 
 
 def fp8_fused_moe(out, hidden, w1, w2, w1_scale, w2_scale, topk_weights, topk_ids, block_m: int) -> None:
-    """tg_fp8_fused_moe: the whole FP8 MoE layer (align + quantize, GEMM1 with the activation epilogue, GEMM2 x routed
-    weight, top-k sum) in one call, intermediates in the stream's scratch buffer."""
+    """tg_fp8_fused_moe: the whole FP8 MoE layer in one call, intermediates in the stream's scratch buffer: align + quantize, GEMM1
+    with the activation epilogue, GEMM2 x routed weight, top-k sum; with few rows per expert the decoding form's two or three
+    launches."""
     L = _lib if _lib is not None else load()
     dev = _device_index(hidden)
     T, H = hidden.shape

@@ -14,7 +14,7 @@
 //     expert in LDS and takes an equal share of (expert, pass, group of columns) units -- contiguous, so that a workgroup
 //     meets one or two experts.  A pass is as many rows as are held at a time; an expert with more is streamed once per
 //     pass, and the passes are dealt like experts.  Every compute unit then takes in the same number of weight bytes whatever
-//     the routing is, which is what bounds the launch (about 27 bytes per nanosecond and compute unit).
+//     the routing is, which is what bounds the launch (24 bytes per nanosecond and compute unit at 40 tokens).
 //   * No quantizer launch.  Four waves of a workgroup quantize the rows of its expert (a few rows; they come out of the L2)
 //     into LDS, in MFMA order, with the scales beside them, while the first weights are on their way to the others.
 //     The arithmetic is the quantizer's: the same bits.

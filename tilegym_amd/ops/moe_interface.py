@@ -43,8 +43,8 @@ def moe_align_block_size(
     raise NotImplementedError(f"moe_align_block_size is not implemented for this backend: {get_current_backend()}")
 
 
-# fused_experts_impl runs a layer that fits one chunk through tg_fp8_fused_moe (one call, same launches, same bits);
-# False: always call by call (what the tests compare the one-call form with)
+# fused_experts_impl runs a layer that fits one chunk through tg_fp8_fused_moe (one call, same bits: the row-tiled launches, or
+# with few rows per expert the decoding form); False: always call by call (what the tests compare the one-call form with)
 USE_ONE_CALL_LAYER = True
 
 
@@ -115,8 +115,8 @@ def fused_experts_impl(
     config = {"BLOCK_SIZE_M": 256 if (M * top_k) // max(E, 1) >= 96 else 128}
     fuse_act = _lib.moe_gemm_silu_quant_ok(w1, config["BLOCK_SIZE_M"]) and w1_scale is not None
     # One chunk of 16-bit activations with the fused activation epilogue: the whole layer is one call into the library
-    # (the same four launches, intermediates in the stream's scratch buffer): the host time of four bindings and nine
-    # allocations is more than the kernels run at decode sizes.
+    # (intermediates in the stream's scratch buffer): the host time of four bindings and nine allocations is more than the
+    # kernels run at decode sizes.
     if (USE_ONE_CALL_LAYER and fuse_act and w2_scale is not None and 0 < num_tokens <= CHUNK_SIZE and _lib.fused_moe_ok(hidden_states, w1, w2, config["BLOCK_SIZE_M"])
             and topk_ids.dtype in (torch.int32, torch.int64)):
         ids = topk_ids if topk_ids.is_contiguous() else topk_ids.contiguous()
