@@ -180,12 +180,13 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     const int cap_log2 = __builtin_ctz(cap);
     int total_passes = 0;                       // one per expert that has rows; more for those with more than are held, if any
     bool hot = false;
+#pragma unroll 1
     for (int base = 0; base < p.E; base += 64) {
         const int c = rows_of(base + lane);
         total_passes += __popcll(__ballot(c > 0));
         hot |= __ballot(c > cap) != 0;
     }
-    if (hot) {
+    if (__builtin_expect(hot, 0)) {
         total_passes = 0;
         for (int base = 0; base < p.E; base += 64) total_passes += (rows_of(base + lane) + cap - 1) >> cap_log2;
 #pragma unroll
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     // ---- this workgroup's share of the total_passes * groups units, in segments of one pass each.  Either a pass's groups are
     // dealt over workgroups of its own (one token, six experts: 42 of 256 for each), or the units are dealt over all of them
     // and a workgroup may meet two passes or more: an equal share, but a second pass's preparation costs as much as streaming
-    // two groups and 40 K steps (about 3 us).  One expert in every token, 32 experts of (2048, 512), top 4, 48 tokens (33
+    // pass_groups groups, two and 40 K steps (about 3 us).  One expert in every token, 32 experts of (2048, 512), top 4, 48 tokens (33
     // passes): 41.6 -> 32.7 us with 7 workgroups to each pass; 64 of (1024, 512), top 8, 56 tokens, half alike: 40.7 -> 35.6.
     const int grid = (int)gridDim.x, bid = (int)blockIdx.x;
     // x / d from inv = 1 / d: two roundings move (x + 0.5) / d, which is 0.5 / d or more away from an integer, by less than
@@ -204,7 +205,7 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
     auto small_div = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
     int u_begin, u_end;
     const int per = total_passes > 0 ? small_div(grid, 1.0f / (float)total_passes) : 0;  // workgroups per pass
-    if (per > 0 && groups * grid <= per * (total_passes * groups + (2 + 40 / kblocks) * grid)) {
+    if (per > 0 && groups * grid <= per * (total_passes * groups + p.pass_groups * grid)) {
         const float inv_per = 1.0f / (float)per;
         const int idx = small_div(bid, inv_per), part = bid - idx * per;
         u_begin = idx * groups + small_div(groups * part, inv_per);
@@ -226,10 +227,11 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
         int left = idx;
         *e = 0;
         *r0 = 0;
-        for (int base = 0; base < p.E; base += 64) {
-            const int c = rows_of(base + lane);
-            if (!hot) {
-                // the left-th expert that has rows
+        if (__builtin_expect(!hot, 1)) {
+            // the left-th expert that has rows
+#pragma unroll 1
+            for (int base = 0; base < p.E; base += 64) {
+                const int c = rows_of(base + lane);
                 const unsigned long long any = __ballot(c > 0);
                 if (left < __popcll(any)) {
                     const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0));
@@ -237,9 +239,11 @@ __global__ void __launch_bounds__(64 * (kDecodeWaves + kDecodeQuantWaves)) moe_d
                     break;
                 }
                 left -= __popcll(any);
-                continue;
             }
-            const int mine = (c + cap - 1) >> cap_log2;
+            return;
+        }
+        for (int base = 0; base < p.E; base += 64) {
+            const int mine = (rows_of(base + lane) + cap - 1) >> cap_log2;
             int incl = mine;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {

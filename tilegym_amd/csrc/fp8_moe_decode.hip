@@ -28,6 +28,7 @@ bool decode_plan(MoeDecodeParams& p, bool up, int tokens) {
     const int cols = up ? 8 : 16, groups = (up ? p.inter : p.N) / cols;
     const int nbs = (groups * cols + 127) / 128 + 1;   // block rows of a segment, at most
     p.wscale_cap = (nbs * (up ? 2 : 1) * p.kblocks + 63) / 64 * 64;
+    p.pass_groups = 2 + 40 / p.kblocks;
     int cap = 1;
     while (cap < tokens && cap < kDecodeRows) cap *= 2;
     while (cap > 1) {

@@ -28,6 +28,7 @@ struct MoeDecodeParams {
     int ids_are_i64, slots, top_k, E, N, K, inter, kblocks, nblocks;
     int row_cap;               // activation rows held at a time: a power of two, at most 16
     int wscale_cap;            // floats of LDS for a segment's weight scales, a multiple of 64
+    int pass_groups;           // what preparing the rows of one more pass costs, in groups of weight rows streamed
 };
 
 struct TileShape { int bm, bn; };
