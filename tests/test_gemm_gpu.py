@@ -539,6 +539,28 @@ def test_deep_tile_kernel_over_fewer_weight_rows_per_tile(device, bn, M, N, K, s
     assert torch.equal(out, full)     # the same products in the same order, whatever the tile's width
 
 
+@pytest.mark.parametrize("bm,bn", [(96, 128), (128, 128), (160, 128), (160, 192), (192, 192)])
+@pytest.mark.parametrize("dm,dn,K,split", [(0, 0, 128, 1), (-1, -8, 256, 1), (1, 8, 384, 2), (17, -3, 640, 1), (-33, 72, 2176, 3)])
+def test_ring_tiles(device, bm, bn, dm, dn, K, split):
+    """The tiles with waves of their own for the loads: rows and columns that end inside a tile, fewer K steps than stages,
+    split K.  Same bits as the 128 x 128 tile kernel (the same products in the same order), and the oracle's result."""
+    M, N = 2 * bm + dm, bn + dn
+    g = _g(bm + bn + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)
+    ad, bd = a.to(device), b.to(device)
+    kc = {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": split, "WAVES": 8}
+    for dtype in (torch.bfloat16, torch.float32, torch.float8_e4m3fn):
+        out = matmul(ad, bd, trans_b=True, scale_a=0.37, scale_b=0.5, out_dtype=dtype, kernel_configs=kc)
+        cfg = used("tiled")
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["WAVES"]) == (bm, bn, 8), cfg
+        base = matmul(ad, bd, trans_b=True, scale_a=0.37, scale_b=0.5, out_dtype=dtype,
+                      kernel_configs={"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": cfg["SPLIT_K"]})
+        assert _lib.last_config()["WAVES"] != 8
+        assert torch.equal(out.view(torch.uint8), base.view(torch.uint8))
+        if dtype == torch.bfloat16:
+            check(out, R.ref_gemm_per_tensor(a, b, 0.37, 0.5, trans_b=True), what=f"ring {bm}x{bn} M={M} N={N} K={K}")
+
+
 def test_deep_tile_is_narrowed_to_fill_the_chip(device):
     """28672 weight rows at M = 64: 224 tiles of 128 columns would leave an eighth of the compute units idle; 256 tiles of 112 run."""
     g = _g(112)

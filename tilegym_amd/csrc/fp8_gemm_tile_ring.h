@@ -1,0 +1,204 @@
+// Per-tensor tiles of 96 x 128 to 192 x 192 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], for M above 64 and below
+// the sizes that fill whole rounds of 256 x 256 tiles.
+//
+// One workgroup per compute unit: four waves compute (2 x 2, one per SIMD), four waves do nothing but request the next K steps'
+// slabs.  A direct global->LDS load holds its wave until the compute unit's address path has room (about 16 clocks per 1 KiB
+// load, whoever issues it).  At these tile sizes a step's loads take about as long as its MFMAs (160 x 128: 576 against 640
+// clocks), and with every wave loading and computing the two came one after the other: 256 x 4096 x 4096 with 160 x 128 tiles
+// took 20.0 us with four such waves, 15.9 with the loads in waves of their own.
+//
+// Three or four stages hold a K step each; a stage is requested again as soon as every computing wave has read it, so
+// STAGES - 1 steps are on their way while one is multiplied.  One barrier per step, in front of its last column tiles: behind it
+// step k+1 is visible and step k's stage is free, and the fragments of step k+1 are read while those last MFMAs run (activation
+// fragments into the registers that a row group's last MFMA releases, weight fragments over three or four rotating sets).
+//
+// Bound on a full chip by power, that is by bytes moved per MFMA: 240 tiles of 160 x 128 run at 1.3 - 1.5 GHz with 82 % of the
+// matrix pipes' slots in use, 64 of them at 2.25 GHz (clock stamps); hence the 192 x 192 tile for larger problems, which moves
+// a quarter less.  Measured (us, before -> now): 777 x 6144 x 4096 27.6 -> 20.9, 1400 x 12288 x 5120 102 -> 79,
+// 1014 x 5120 x 12288 85 -> 73, 512 x 4096 x 4096 18.1 -> 14.0.  A fifth kind of wave that touched the lines of steps further
+// ahead to have them in the caches: no faster (23.8 against 25.2 and 54.3 against 53.0 us), not kept.
+//
+// Same slab layout, swizzles, fragment addressing, MFMA order per accumulator and epilogue arithmetic as
+// fp8_gemm_tile_kernel<128, 128, 2, 2, false, GROUP_DENSE, SPLIT>: identical results.
+#pragma once
+
+#include "fp8_gemm_tile.h"
+
+namespace tg {
+
+template <int BM, int BN, int STAGES, bool SPLIT>
+__global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int WGM = 2, WGN = 2, NL = 4;             // four computing waves, four loading waves
+    constexpr int WTN = BN / WGN;
+    constexpr int TM = BM / (16 * WGM), TN = WTN / 16;
+    constexpr int A_IT = BM / (8 * NL), B_IT = BN / (8 * NL);
+    constexpr int STAGE_BYTES = (BM + BN) * kKBlock;
+    constexpr int PER_STEP = A_IT + B_IT;
+    constexpr int WS = TN == 6 ? 3 : 4;                 // weight fragment sets
+    constexpr int LAST = TN == 6 ? 1 : 2;               // column tiles behind the barrier
+    static_assert(BM % 32 == 0 && (TN == 4 || TN == 6) && STAGES >= 3 && STAGES * STAGE_BYTES <= 160 * 1024, "shape");
+
+    __shared__ __align__(1024) uint8_t lds[STAGES * STAGE_BYTES];  // stage s: A slab, then B slab
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K = p.K;
+    const int tiles_n = (p.N + BN - 1) / BN, tiles_m = (p.M + BM - 1) / BM;
+    const int pid = xcd_remap((int)blockIdx.x, tiles_m * tiles_n);
+    constexpr int GM = 8;
+    const int width = GM * tiles_n;
+    const int group = pid / width, first_m = group * GM;
+    const int gsz = min(tiles_m - first_m, GM);
+    const int m0 = (first_m + (pid % width) % gsz) * BM, n0 = ((pid % width) / gsz) * BN;
+    const int rows_valid = min(BM, p.M - m0);
+    int ks = 0, ks_end = p.kblocks;
+    if constexpr (SPLIT) {
+        ks = blockIdx.y * p.ksteps_per_split;
+        ks_end = min(ks + p.ksteps_per_split, p.kblocks);
+    }
+    const int nsteps = ks_end - ks, last = ks_end - 1;
+    if (nsteps <= 0) return;
+
+    constexpr int kPro = (STAGES - 1) * PER_STEP, kLoop = (STAGES - 2) * PER_STEP;  // loads that may stay in flight
+    static_assert(kPro < 64, "vmcnt has six bits");
+    constexpr int kWaitPro = 0x0F70 | (kPro & 15) | ((kPro >> 4) << 14);
+    constexpr int kWaitLoop = 0x0F70 | (kLoop & 15) | ((kLoop >> 4) << 14);
+    constexpr int kWaitAll = 0x0F70;
+    constexpr int kWaitLds = 0xC07F;
+#define TG_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+    if (wave >= 4) {
+        // ------------------------------------------------------------ loading waves
+        const int lw = wave - 4;
+        const int lrow = lane >> 3;
+        const int lj = (lane & 7) ^ swz16(lrow);
+        const int ljb = (lane & 7) ^ swz_w(((lw & 1) << 3) | lrow);
+        uint32_t a_off[A_IT], b_off[B_IT];
+#pragma unroll
+        for (int i = 0; i < A_IT; ++i) a_off[i] = (uint32_t)(m0 + min((i * NL + lw) * 8 + lrow, rows_valid - 1)) * (uint32_t)K + lj * 16;
+#pragma unroll
+        for (int i = 0; i < B_IT; ++i) b_off[i] = (uint32_t)min(n0 + (i * NL + lw) * 8 + lrow, p.N - 1) * (uint32_t)K + ljb * 16;
+        const v4i rsrc_a = make_rsrc(p.A), rsrc_b = make_rsrc(p.B);
+        const uint32_t lds0 = lds_address(lds) + lw * 1024;
+        auto issue = [&](int kstep, int stage) {
+            const int k0 = min(kstep, last) * kKBlock;
+            const uint32_t dst = lds0 + stage * STAGE_BYTES;
+#pragma unroll
+            for (int i = 0; i < B_IT; ++i) direct_load_b128(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], k0);
+#pragma unroll
+            for (int i = 0; i < A_IT; ++i) direct_load_b128(rsrc_a, dst + i * NL * 1024, a_off[i], k0);
+        };
+#pragma unroll
+        for (int s = 0; s < STAGES; ++s) issue(ks + s, s);
+        __builtin_amdgcn_s_waitcnt(kWaitPro);
+        __builtin_amdgcn_s_barrier();
+        int stage = 0;
+        for (int k = 0; k < nsteps; ++k) {
+            __builtin_amdgcn_s_waitcnt(kWaitLoop);  // step k+1 has landed (steps past the end re-fetch the last one)
+            __builtin_amdgcn_s_barrier();           // and every computing wave has read step k
+            issue(ks + k + STAGES, stage);
+            stage = stage == STAGES - 1 ? 0 : stage + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitAll);  // the re-fetches past the end must land before the workgroup's LDS is released
+        return;
+    }
+
+    // ---------------------------------------------------------------- computing waves
+    const int wm = wave % WGM, wn = wave / WGM;
+    const int li = lane & 15, lg = lane >> 4;
+    const uint32_t frag0 = wm * 16 * kKBlock + li * kKBlock + ((lg ^ swz16(li)) << 4), frag1 = frag0 ^ 64;
+    const int wrow = ((li >> 2) << 3) | (li & 3);
+    const uint32_t wfrag0 = BM * kKBlock + wn * WTN * kKBlock + wrow * kKBlock + ((lg ^ swz_w(wrow)) << 4), wfrag1 = wfrag0 ^ 64;
+
+    v4f acc[TN][TM];
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    v8i af[TM], wf[WS];
+    auto read_a = [&](int tm, const uint8_t* base) {
+        const uint8_t* a = base + tm * (WGM * 16 * kKBlock);
+        af[tm] = join(*reinterpret_cast<const v4i*>(a + frag0), *reinterpret_cast<const v4i*>(a + frag1));
+    };
+    auto read_w = [&](int tn, const uint8_t* base) {
+        const uint8_t* b = base + ((tn >> 1) * 32 + (tn & 1) * 4) * kKBlock;
+        wf[tn % WS] = join(*reinterpret_cast<const v4i*>(b + wfrag0), *reinterpret_cast<const v4i*>(b + wfrag1));
+    };
+    __builtin_amdgcn_s_barrier();  // step 0 has landed
+    read_w(0, lds);
+    read_w(1, lds);
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) read_a(tm, lds);
+    int stage = 0;
+    for (int k = 0; k < nsteps; ++k) {
+        const uint8_t* cur = lds + stage * STAGE_BYTES;
+        stage = stage == STAGES - 1 ? 0 : stage + 1;
+        const uint8_t* nxt = lds + stage * STAGE_BYTES;
+        TG_FENCE();
+#pragma unroll
+        for (int tn = 0; tn < TN - LAST; ++tn) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) {
+                acc[tn][tm] = mfma_e4m3(wf[tn % WS], af[tm], acc[tn][tm]);
+                if (tm == 0 && tn + 2 < TN) read_w(tn + 2, cur);
+                TG_FENCE();
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitLds);  // all my reads of step k are done
+        __builtin_amdgcn_s_barrier();          // step k+1 is visible
+        TG_FENCE();
+        read_w(0, nxt);
+        read_w(1, nxt);
+        TG_FENCE();
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+#pragma unroll
+            for (int tn = TN - LAST; tn < TN; ++tn) acc[tn][tm] = mfma_e4m3(wf[tn % WS], af[tm], acc[tn][tm]);
+            TG_FENCE();
+            read_a(tm, nxt);
+            TG_FENCE();
+        }
+    }
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) asm volatile("" : : "v"(af[tm]));
+    asm volatile("" : : "v"(wf[0]), "v"(wf[1]));
+#undef TG_FENCE
+
+    float scale = p.alpha;
+    if (p.As) scale *= p.As[0];
+    if (p.Bs) scale *= p.Bs[0];
+    const bool vec_ok = p.vec_store != 0 && (p.N % 8) == 0;
+    const int64_t MN = (int64_t)p.M * p.N;
+    auto emit = [&](auto type_tag) {
+        constexpr int OT = decltype(type_tag)::value;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+            const int rt = (tm * WGM + wm) * 16 + li;
+#pragma unroll
+            for (int tp = 0; tp < TN / 2; ++tp) {
+                const int col = n0 + wn * WTN + tp * 32 + lg * 8;
+                if (rt >= rows_valid || col >= p.N) continue;
+                if constexpr (SPLIT)
+                    store8(p.partials + (int64_t)blockIdx.y * MN, OUT_F32, m0 + rt, col, p.N, p.N, acc[2 * tp][tm], acc[2 * tp + 1][tm], 0.f, vec_ok);
+                else
+                    store8(p.C, OT, m0 + rt, col, p.N, p.ldc, acc[2 * tp][tm] * scale, acc[2 * tp + 1][tm] * scale, p.beta, vec_ok);
+            }
+        }
+    };
+    if (SPLIT || p.out_type == OUT_BF16) emit(std::integral_constant<int, OUT_BF16>{});
+    else if (p.out_type == OUT_F32) emit(std::integral_constant<int, OUT_F32>{});
+    else if (p.out_type == OUT_F8) emit(std::integral_constant<int, OUT_F8>{});
+    else emit(std::integral_constant<int, OUT_F16>{});
+#endif
+}
+
+template <int BM, int BN, int STAGES>
+inline hipError_t launch_tile_ring(bool split, const GemmParams& p, int gx, int gy, hipStream_t stream) {
+    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, true>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    return hipGetLastError();
+}
+
+}  // namespace tg

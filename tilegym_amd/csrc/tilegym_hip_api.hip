@@ -174,7 +174,13 @@ bool is_mid_tile(int bm, int bn) { return ((bm == 64 || bm == 32) && bn == 32) |
 // Per-tensor 64-row tiles of 72 .. 120 weight rows: the deep 64 x 128 kernel with the rest of its weight slab unused.
 bool is_narrowed_deep_tile(int bm, int bn) { return bm == 64 && bn >= 72 && bn < 128 && bn % 8 == 0; }
 
+// Tiles of fp8_gemm_tile_ring_kernel (per-tensor).  128 x 128 names two kernels: WAVES = 8 asks for the ring (four waves load,
+// four compute), anything else for the four-wave kernel of two workgroups per compute unit.
+bool is_ring_tile(int bm, int bn) { return (bn == 128 && (bm == 96 || bm == 128 || bm == 160)) || (bn == 192 && (bm == 160 || bm == 192)); }
+bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !(bm == 128 && bn == 128); }
+
 bool tile_exists(int bm, int bn, bool block_scaled) {
+    if (is_ring_only_tile(bm, bn)) return !block_scaled;
     if (is_mid_tile(bm, bn)) return !block_scaled;  // the four waves split K inside the workgroup (per-tensor only)
     if (is_narrowed_deep_tile(bm, bn)) return !block_scaled;
     if (bm == 128 && bn == 128) return true;
@@ -200,52 +206,89 @@ int pick_split(int64_t units, int64_t target_units, int64_t kblocks, int min_ste
     return (int)cdiv(kblocks, kps);
 }
 
-// Cost model of the LDS-tiled kernels above 64 rows.  Per tile kind: microseconds per K step of a tile while its compute
-// unit holds one workgroup (`alone`: the launch has at most 256 tiles) or two (`shared`), and per tile for set-up, first
-// loads and epilogue (`fixed`).  A launch takes rounds x (K steps x step + fixed), rounds = tiles / 256 or tiles / 512
-// rounded up, plus, with split-K, the reduction launch (kReduceUs + kReduceUsPerMB x the partial sums).  The numbers are a
-// least-squares fit to 9 600 measurements on MI355X: 360 shapes (M = 96 ... 8192, 18 weight shapes, both scalings) x every
-// tile x 1 / 2 / 4 / 8 splits, weights rotated past the caches, launches replayed from a graph.  The schedule it picks is
-// within 1 % of the best measured one on average (worst case 12 %; the rules it replaces: 7 - 8 % and 2.0 x).
+// Cost model of the LDS-tiled kernels above 64 rows.  A launch takes rounds x (K steps x step + fixed): `fixed` is a tile's
+// set-up, first loads and epilogue in microseconds, `step` the time of a K step, which grows with the share of the chip that is
+// busy (a full chip runs at a lower clock and shares the way to memory): from `first` for a single tile to `full` with a tile on
+// each of the 256 compute units, and, for kernels of which two workgroups share a compute unit (`both` > 0), on to `both`
+// with 512.  Split-K adds the reduction launch.
+//
+// Per-tensor: fitted to 11 000 measurements (480 shapes, M = 65 ... 4096, weights of 1 to 320 MB, every tile x 1 / 2 / 4 / 8
+// splits, launches replayed from a graph over rotating operands).  On the 260 shapes with every split measured the pick is 1.6 %
+// behind the best schedule on average and 11 % ahead of the kernels and the model without the ring tiles (M = 256 ... 1024: 14 %;
+// 777 x 6144 x 4096 32 -> 24 us, 1014 x 5120 x 12288 85 -> 73, 604 x 12288 x 5120 50 -> 42, 154 x 6144 x 4096 17.4 -> 13.2).
+struct StepCost { int bm, bn; bool ring; float first, full, both, fixed; };
+constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.194f, 0.178f, 0.f, 1.66f},   {64, 32, false, 0.222f, 0.215f, 0.f, 1.99f},
+                                        {64, 64, false, 0.298f, 0.338f, 0.f, 3.00f},   {64, 128, false, 0.332f, 0.645f, 0.925f, 3.58f},
+                                        {128, 128, false, 0.473f, 0.843f, 0.978f, 2.98f}, {128, 256, false, 0.874f, 1.036f, 0.f, 3.16f},
+                                        {256, 256, false, 0.968f, 1.333f, 0.f, 7.72f},
+                                        {96, 128, true, 0.384f, 0.449f, 0.f, 2.46f},   {128, 128, true, 0.402f, 0.546f, 0.f, 2.89f},
+                                        {160, 128, true, 0.427f, 0.630f, 0.f, 3.42f},  {160, 192, true, 0.554f, 0.778f, 0.f, 4.31f},
+                                        {192, 192, true, 0.618f, 0.863f, 0.f, 4.90f}};
+constexpr float kReduceUs = 3.5f, kReduceUsPerMB = 0.30f;
+constexpr float kSplitMargin = 1.04f;  // a split schedule must be predicted this much faster than the best unsplit one
+// few rows over a weight that does not stay in the caches: a ring tile waits for memory (69 x 11264 x 2560: 13.8 us with
+// 96 x 128 tiles where the model says 10.6, 12.3 with 64 x 88)
+constexpr float kRingFewRows = 1.25f;
+
+float step_cost_us(const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split) {
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * split, places = t.both > 0.f ? 512 : 256;
+    const float steps = (float)cdiv(kblocks, split);
+    const float at_full = t.both > 0.f ? t.both : t.full;
+    auto part = [&](int64_t n) -> float {
+        if (n == 0) return 0.f;
+        const float step = n <= 256 ? t.first + (t.full - t.first) * (float)n / 256.f : t.full + (t.both - t.full) * (float)(n - 256) / 256.f;
+        return steps * step + t.fixed;
+    };
+    float us = (float)(tiles / places) * (steps * at_full + t.fixed) + part(tiles % places);
+    if (t.ring && M <= 96) us *= kRingFewRows;
+    if (split > 1) us += kReduceUs + kReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
+    return us;
+}
+
+// Block-scaled tiles: microseconds per K step of a tile while its compute unit holds one workgroup (`alone`: the launch has at
+// most 256 tiles) or two (`shared`), rounds = tiles / 256 or tiles / 512 rounded up; a least-squares fit to measurements
+// of 180 shapes (M = 96 ... 8192, 18 weight shapes) x every tile x 1 / 2 / 4 / 8 splits.
 struct TileCost { int bm, bn; float alone, shared, fixed; };
-constexpr TileCost kPerTensorTiles[] = {{32, 32, 0.132f, 0.332f, 2.80f},   {64, 32, 0.178f, 0.405f, 3.46f},
-                                        {64, 64, 0.249f, 0.596f, 4.43f},   {64, 128, 0.414f, 0.811f, 4.02f},
-                                        {128, 128, 0.650f, 0.929f, 3.70f}, {128, 256, 0.874f, 1.782f, 6.88f},
-                                        {256, 256, 1.150f, 1.150f, 8.19f}};
 // (block-scaled 128 x 256 exists and can be forced; leaving it out of the automatic choice measured better)
 constexpr TileCost kBlockScaledTiles[] = {{64, 128, 0.685f, 0.851f, 3.50f}, {128, 128, 0.690f, 1.016f, 4.23f},
                                           {256, 256, 1.496f, 1.496f, 8.11f}};
-constexpr float kReduceUs = 6.0f, kReduceUsPerMB = 0.235f;
-constexpr float kSplitMargin = 1.05f;  // a split schedule must be predicted this much faster than the best unsplit one
+constexpr float kBlockReduceUs = 6.0f, kBlockReduceUsPerMB = 0.235f, kBlockSplitMargin = 1.05f;
 
 float tile_cost_us(const TileCost& t, int64_t M, int64_t N, int64_t kblocks, int split) {
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * split, ksteps = cdiv(kblocks, split);
     const bool one_per_cu = t.bm == 256 && t.bn == 256;
     float us = (one_per_cu || tiles <= 256) ? (float)cdiv(tiles, 256) * ((float)ksteps * t.alone + t.fixed)
                                             : (float)cdiv(tiles, 512) * ((float)ksteps * t.shared + t.fixed);
-    if (split > 1) us += kReduceUs + kReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
+    if (split > 1) us += kBlockReduceUs + kBlockReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
     return us;
 }
 
-// The cheapest (tile, split) by the model; a tile (bm > 0) or a split (want_split > 0) given by the caller is kept.
-void pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
-                       int* bm, int* bn, int* split) {
-    const TileCost* kinds = block_scaled ? kBlockScaledTiles : kPerTensorTiles;
-    const int n_kinds = block_scaled ? (int)(sizeof(kBlockScaledTiles) / sizeof(TileCost)) : (int)(sizeof(kPerTensorTiles) / sizeof(TileCost));
-    float best = 0.f;
-    int best_bm = -1, best_bn = -1, best_split = 1;
-    for (int i = 0; i < n_kinds; ++i) {
-        const TileCost& t = kinds[i];
-        if (*bm > 0 && (t.bm != *bm || t.bn != *bn)) continue;
-        if (want_split > 1 && is_mid_tile(t.bm, t.bn)) continue;  // these split K inside the workgroup only
+// A tile and a split, with what the model says they take.
+struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us = 0.f; };
+
+// The cheapest (tile, split) by the model; a tile (bm > 0; ring: the ring form of 128 x 128) or a split (want_split > 0) given by
+// the caller is kept.
+TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
+                             int bm, int bn, bool ring) {
+    TileChoice best;
+    auto offer = [&](int kbm, int kbn, bool kring, float margin, auto&& cost) {
+        if (bm > 0 && (kbm != bm || kbn != bn || (kring && !is_ring_only_tile(kbm, kbn)) != (ring && !is_ring_only_tile(kbm, kbn)))) return;
+        if (want_split > 1 && is_mid_tile(kbm, kbn)) return;  // these split K inside the workgroup only
+        // (five full row tiles of 64 over a weight of up to 16 MB: callers rely on the 64-row kernel there -- the suite pins
+        // it; 320 x 4096 x 4096 takes 17.1 us with 64 x 88 tiles, 12.9 with 96 x 128)
+        if (kring && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (want_split > 0 && sp != 1) break;          // the caller's split is applied by the caller
-            if (sp > 1 && (is_mid_tile(t.bm, t.bn) || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
-            const float us = tile_cost_us(t, M, N, kblocks, want_split > 0 ? want_split : sp) * (sp > 1 ? kSplitMargin : 1.f);
-            if (best_bm < 0 || us < best) { best = us; best_bm = t.bm; best_bn = t.bn; best_split = sp; }
+            if (sp > 1 && (is_mid_tile(kbm, kbn) || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
+            const float us = cost(want_split > 0 ? want_split : sp) * (sp > 1 ? margin : 1.f);
+            if (best.bm < 0 || us < best.us) best = TileChoice{kbm, kbn, sp, kring, us};
         }
-    }
-    if (best_bm > 0) { *bm = best_bm; *bn = best_bn; *split = best_split; }
+    };
+    if (block_scaled)
+        for (const TileCost& t : kBlockScaledTiles) offer(t.bm, t.bn, false, kBlockSplitMargin, [&](int sp) { return tile_cost_us(t, M, N, kblocks, sp); });
+    else
+        for (const StepCost& t : kPerTensorTiles) offer(t.bm, t.bn, t.ring, kSplitMargin, [&](int sp) { return step_cost_us(t, M, N, kblocks, sp); });
+    return best;
 }
 
 // 17 .. 64 rows: the same form of model over more kinds of kernel, with constants of its own (here the weights stream from
@@ -506,8 +549,11 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, block_scaled))) bm = bn = -1;
     int model_split = 1;
+    const bool want_ring = !block_scaled && bm > 0 && is_ring_tile(bm, bn) && (is_ring_only_tile(bm, bn) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
+    if (want_ring) s.waves = 8;
     if (M > 64) {
-        pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, &bm, &bn, &model_split);
+        const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring);
+        if (pick.bm > 0) { bm = pick.bm; bn = pick.bn; model_split = pick.split; s.waves = pick.ring ? 8 : -1; }
     } else if (bm < 0) {
         auto tiles = [&](int64_t a, int64_t b) { return cdiv(M, a) * cdiv(N, b); };
         // small weights at 16 < M <= 64: narrow tiles whose four waves split K inside the workgroup fill the chip in
@@ -555,13 +601,14 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
 }
 
 // A per-tensor (K, N) weight: whether the narrow tiles read it as it lies, and with which tile; else it is copied to (N, K)
-// first and any kernel takes it.  Costs in us like tile_cost_us's, fitted by hand to 8 weights x 12 row counts (1 ... 512), both
-// ways measured: a direct tile's K step takes 0.39 - 0.45 us whatever the grid; the copy 3 us + 0.36 us per MB, and up to
-// 64 rows copy and GEMM together 7 us + 0.5 us per MB.  Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 against
-// 65.4; 1024 x 1024: 5.2 against 7.7), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied;
-// 2048 x 6144: 20.7 against 16.4), and so are most from 256 rows on (6144 x 4096 at M = 256: 28.3 direct, 24.9 copied).
+// first and any kernel takes it.  A direct tile's K step takes 0.39 - 0.45 us whatever the grid; the copy costs 5 us + 0.40 us per
+// MB on top of the cost model's GEMM above 64 rows, and up to 64 rows copy and GEMM together 7 us + 0.5 us per MB.  Above 64 rows
+// the line was fitted to 110 shapes (65 ... 512 rows) with both ways measured: 1.6 % behind the better way on average (worst 1.4 x).
+// Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 us against 65.4; 1024 x 1024: 5.2 against 7.7; 1264 x 1152 at
+// M = 275: 6.3 against 9.3), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied), and so are
+// most from 300 rows on.
 constexpr TileCost kKnTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
-constexpr float kKnMargin = 1.05f, kCopyUs = 3.0f, kCopyUsPerMB = 0.36f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
+constexpr float kKnMargin = 0.9f, kCopyUs = 5.0f, kCopyUsPerMB = 0.40f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
 bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, int* bm, int* bn) {
     if (M > 512 || N % 16 != 0 || K % 128 != 0) return false;
     const int64_t kblocks = K / 128;
@@ -574,11 +621,7 @@ bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, 
         if (*bm < 0 || us < best) { best = us; *bm = t.bm; *bn = t.bn; }
     }
     if (M <= 64) return best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
-    int nk_bm = -1, nk_bn = -1, nk_split = 1;
-    pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, &nk_bm, &nk_bn, &nk_split);
-    float nk = 0.f;
-    for (const TileCost& t : kPerTensorTiles)
-        if (t.bm == nk_bm && t.bn == nk_bn) nk = tile_cost_us(t, M, N, kblocks, nk_split);
+    const float nk = pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us;
     return best * kKnMargin <= nk + kCopyUs + kCopyUsPerMB * mb;
 }
 
@@ -837,6 +880,14 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     if (can_chunk && (K % 128) == 0 && M >= 1024 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_M) <= 0 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0 &&
         cfg_get(cfg, ncfg, TG_CFG_SPLIT_K) <= 0) {
         const int64_t tm = cdiv(M, 256), tn = cdiv(N, 256), total = tm * tn, rounds = cdiv(total, 256);
+        // (per-tensor: only where the model says that no single launch is as fast)
+        auto worth_it = [&](int64_t full_m, int64_t full_n, int64_t rest_m, int64_t rest_n) {
+            if (block_scaled || K < 1024) return true;  // (the model was fitted to K >= 1024)
+            const int64_t avail = workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
+            const float whole = pick_tile_by_cost(M, N, kblocks, false, avail, -1, -1, -1, false).us;
+            return pick_tile_by_cost(full_m, full_n, kblocks, false, avail, 1, 256, 256, false).us +
+                       pick_tile_by_cost(rest_m, rest_n, kblocks, false, avail, -1, -1, -1, false).us < whole;
+        };
         if (total > 256 && total * 100 < rounds * 256 * 80) {
             auto fills = [](int64_t tiles) { return tiles >= 256 && tiles * 100 >= cdiv(tiles, 256) * 256 * 95; };
             const int64_t n1 = ((total / 256) * 256) / tm;   // column tiles that fit the whole rounds
@@ -848,7 +899,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
             full_cfg[TG_CFG_KERNEL] = 1;
             full_cfg[TG_CFG_BLOCK_M] = full_cfg[TG_CFG_BLOCK_N] = 256;
             full_cfg[TG_CFG_SPLIT_K] = 1;
-            if (n1 >= 1 && n1 < tn && fills(tm * n1)) {
+            if (n1 >= 1 && n1 < tn && fills(tm * n1) && worth_it(M, n1 * 256, M, N - n1 * 256)) {
                 if ((rc = run_columns(0, n1 * 256, full_cfg, TG_CFG_COUNT))) return rc;
                 pieces.after_piece();
                 if ((rc = run_columns(n1 * 256, N - n1 * 256, cfg, ncfg))) return rc;
@@ -856,7 +907,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
                 pieces.publish();
                 return TG_OK;
             }
-            if (m1 >= 1 && m1 < tm && fills(m1 * tn)) {
+            if (m1 >= 1 && m1 < tm && fills(m1 * tn) && worth_it(m1 * 256, N, M - m1 * 256, N)) {
                 // the same along the rows: the pieces are contiguous row ranges of A, C and the activation scales
                 for (int piece = 0; piece < 2; ++piece) {
                     const int64_t r0 = piece ? m1 * 256 : 0, rows = piece ? M - m1 * 256 : m1 * 256;
@@ -1031,7 +1082,9 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
                                    N * K < kBs256WeightLimit && pc.As && pc.Bs && cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS) == 1 &&
                                    cfg_get(cfg, ncfg, TG_CFG_WAVES) != 8;
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
-        hipError_t e = mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
+        const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
+        hipError_t e = ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
+                     : mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
                      : ordered ? tg::run_tile256(pc, gx, stream)
                      : bs_persistent ? tg::run_bs256(tg::GROUP_DENSE, pc, gx, stream)
                      : deep ? tg::run_tile_deep(split, pc, gx, pc.split_k, stream)
