@@ -539,7 +539,7 @@ def test_deep_tile_kernel_over_fewer_weight_rows_per_tile(device, bn, M, N, K, s
     assert torch.equal(out, full)     # the same products in the same order, whatever the tile's width
 
 
-@pytest.mark.parametrize("bm,bn", [(96, 128), (128, 128), (160, 128), (160, 192), (192, 192)])
+@pytest.mark.parametrize("bm,bn", [(64, 128), (96, 128), (128, 128), (160, 128), (160, 192), (192, 192)])
 @pytest.mark.parametrize("dm,dn,K,split", [(0, 0, 128, 1), (-1, -8, 256, 1), (1, 8, 384, 2), (17, -3, 640, 1), (-33, 72, 2176, 3)])
 def test_ring_tiles(device, bm, bn, dm, dn, K, split):
     """The tiles with waves of their own for the loads: rows and columns that end inside a tile, fewer K steps than stages,
@@ -559,6 +559,29 @@ def test_ring_tiles(device, bm, bn, dm, dn, K, split):
         assert torch.equal(out.view(torch.uint8), base.view(torch.uint8))
         if dtype == torch.bfloat16:
             check(out, R.ref_gemm_per_tensor(a, b, 0.37, 0.5, trans_b=True), what=f"ring {bm}x{bn} M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("bm", [64, 96, 128, 160, 192])
+@pytest.mark.parametrize("dm,N,K,split", [(0, 256, 128, 1), (-1, 120, 1024, 1), (1, 136, 1152, 2), (17, 257, 2176, 1), (-33, 384, 2304, 2)])
+def test_ring_tiles_block_scaled(device, bm, dm, N, K, split):
+    """Chunks of activation scales that end inside a K range (8 K steps per chunk: 1, 8, 9, 17 and 2 x 9 steps), rows and
+    columns that end inside a tile.  Same bits as the 128 x 128 tile kernel, with either scale tensor missing too."""
+    M = 2 * bm + dm
+    g = _g(bm + N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)
+    sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand((N + 127) // 128, K // 128, generator=g) * 0.1 + 0.01
+    ad, bd, sad, sbd = a.to(device), b.to(device), sa.to(device), sb.to(device)
+    kc = {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": 128, "SPLIT_K": split, "WAVES": 8}
+    out, base = (torch.empty(M, N, dtype=torch.bfloat16, device=device) for _ in range(2))
+    for s1, s2 in ((sad, sbd), (None, sbd), (sad, None)):
+        _lib.fp8_gemm(out, ad, bd, s1, s2, False, True, 1.0, 0.0, kc)
+        cfg = used("tiled")
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["WAVES"]) == (bm, 128, 8), cfg
+        _lib.fp8_gemm(base, ad, bd, s1, s2, False, True, 1.0, 0.0, {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": cfg["SPLIT_K"]})
+        assert _lib.last_config()["WAVES"] != 8
+        assert torch.equal(out, base)
+        if s1 is not None and s2 is not None:
+            check(out, R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"block ring {bm} M={M} N={N} K={K}")
 
 
 def test_deep_tile_is_narrowed_to_fill_the_chip(device):

@@ -1,5 +1,5 @@
-// Per-tensor tiles of 96 x 128 to 192 x 192 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], for M above 64 and below
-// the sizes that fill whole rounds of 256 x 256 tiles.
+// Tiles of 64 x 128 to 192 x 192 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], per-tensor or block scales (tiles of
+// 128 columns), for the row counts between decoding and those that fill whole rounds of 256 x 256 tiles.
 //
 // One workgroup per compute unit: four waves compute (2 x 2, one per SIMD), four waves do nothing but request the next K steps'
 // slabs.  A direct global->LDS load holds its wave until the compute unit's address path has room (about 16 clocks per 1 KiB
@@ -7,7 +7,7 @@
 // clocks), and with every wave loading and computing the two came one after the other: 256 x 4096 x 4096 with 160 x 128 tiles
 // took 20.0 us with four such waves, 15.9 with the loads in waves of their own.
 //
-// Three or four stages hold a K step each; a stage is requested again as soon as every computing wave has read it, so
+// Three to five stages hold a K step each; a stage is requested again as soon as every computing wave has read it, so
 // STAGES - 1 steps are on their way while one is multiplied.  One barrier per step, in front of its last column tiles: behind it
 // step k+1 is visible and step k's stage is free, and the fragments of step k+1 are read while those last MFMAs run (activation
 // fragments into the registers that a row group's last MFMA releases, weight fragments over three or four rotating sets).
@@ -18,15 +18,22 @@
 // 1014 x 5120 x 12288 85 -> 73, 512 x 4096 x 4096 18.1 -> 14.0.  A fifth kind of wave that touched the lines of steps further
 // ahead to have them in the caches: no faster (23.8 against 25.2 and 54.3 against 53.0 us), not kept.
 //
-// Same slab layout, swizzles, fragment addressing, MFMA order per accumulator and epilogue arithmetic as
-// fp8_gemm_tile_kernel<128, 128, 2, 2, false, GROUP_DENSE, SPLIT>: identical results.
+// Block scales: a step's products are scaled and added as in fp8_gemm_tile.h.  The loading waves bring the activation scales
+// too, in chunks of eight K steps spread over the steps of the chunk before; the scales of step k+1 are read behind the barrier of
+// step k.  485 x 6144 x 4096 28.5 -> 22.8 us, 174 x 3520 x 4992 19.2 -> 15.5, 62 x 6144 x 4096 15.7 -> 12.6.
+//
+// Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as
+// fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results.
 #pragma once
 
 #include "fp8_gemm_tile.h"
 
 namespace tg {
 
-template <int BM, int BN, int STAGES, bool SPLIT>
+// what a missing tensor of activation scales is read as
+static __device__ const float kOneScale[4] = {1.f, 1.f, 1.f, 1.f};
+
+template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool SPLIT>
 __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int WGM = 2, WGN = 2, NL = 4;             // four computing waves, four loading waves
@@ -34,12 +41,19 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     constexpr int TM = BM / (16 * WGM), TN = WTN / 16;
     constexpr int A_IT = BM / (8 * NL), B_IT = BN / (8 * NL);
     constexpr int STAGE_BYTES = (BM + BN) * kKBlock;
-    constexpr int PER_STEP = A_IT + B_IT;
+    constexpr int S_GROUPS = BM / 8, S_PHASES = (S_GROUPS + NL - 1) / NL;  // 8-row groups of activation scales; K steps a chunk's loads are spread over
+    constexpr int PER_STEP = A_IT + B_IT + (BLOCKSCALE ? 1 : 0);
     constexpr int WS = TN == 6 ? 3 : 4;                 // weight fragment sets
     constexpr int LAST = TN == 6 ? 1 : 2;               // column tiles behind the barrier
     static_assert(BM % 32 == 0 && (TN == 4 || TN == 6) && STAGES >= 3 && STAGES * STAGE_BYTES <= 160 * 1024, "shape");
 
+    static_assert(!BLOCKSCALE || (BN == 128 && S_PHASES + STAGES - 1 <= kScaleChunk), "one weight scale per wave; a chunk of activation scales lands before its first step");
+
     __shared__ __align__(1024) uint8_t lds[STAGES * STAGE_BYTES];  // stage s: A slab, then B slab
+    // block scales: activation scales of the tile's rows, two chunks of kScaleChunk K steps, laid out as in fp8_gemm_tile.h, and
+    // the weight scales of the tile's column block for every K step
+    __shared__ __align__(256) float s_as[BLOCKSCALE ? 2 * BM * kScaleChunk : 1];
+    __shared__ float s_bs[BLOCKSCALE ? kMaxKBlocks : 1];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -81,6 +95,19 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         for (int i = 0; i < B_IT; ++i) b_off[i] = (uint32_t)min(n0 + (i * NL + lw) * 8 + lrow, p.N - 1) * (uint32_t)K + ljb * 16;
         const v4i rsrc_a = make_rsrc(p.A), rsrc_b = make_rsrc(p.B);
         const uint32_t lds0 = lds_address(lds) + lw * 1024;
+        const v4i rsrc_s = make_rsrc(p.As ? p.As : kOneScale);
+        const int s_kbi = ((lane & 7) - lrow) & 7;    // chunk step this lane fetches
+        // row group `ph` of this wave, chunk `chunk` of K steps (a phase past the last group fetches the last one again: every step
+        // requests the same number of loads)
+        auto issue_s = [&](int chunk, int ph) {
+            if constexpr (BLOCKSCALE) {
+                const int g = min(ph * NL + lw, S_GROUPS - 1);
+                const int row = m0 + min(g * 8 + lrow, rows_valid - 1);
+                const int kb = min(ks + chunk * kScaleChunk + s_kbi, p.kblocks - 1);
+                direct_load_b32(rsrc_s, lds_address(s_as) + ((chunk & 1) * BM * kScaleChunk + g * 64) * 4,
+                                p.As ? ((uint32_t)row * (uint32_t)p.kblocks + (uint32_t)kb) * 4u : 0u, 0);
+            }
+        };
         auto issue = [&](int kstep, int stage) {
             const int k0 = min(kstep, last) * kKBlock;
             const uint32_t dst = lds0 + stage * STAGE_BYTES;
@@ -89,14 +116,20 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 #pragma unroll
             for (int i = 0; i < A_IT; ++i) direct_load_b128(rsrc_a, dst + i * NL * 1024, a_off[i], k0);
         };
+        if constexpr (BLOCKSCALE)
+            for (int ph = 0; ph < S_PHASES; ++ph) issue_s(0, ph);
 #pragma unroll
-        for (int s = 0; s < STAGES; ++s) issue(ks + s, s);
+        for (int s = 0; s < STAGES; ++s) {
+            if (s > 0) issue_s(0, 0);  // (again, for the count: the waits below take every step's requests to be PER_STEP)
+            issue(ks + s, s);
+        }
         __builtin_amdgcn_s_waitcnt(kWaitPro);
         __builtin_amdgcn_s_barrier();
         int stage = 0;
         for (int k = 0; k < nsteps; ++k) {
             __builtin_amdgcn_s_waitcnt(kWaitLoop);  // step k+1 has landed (steps past the end re-fetch the last one)
             __builtin_amdgcn_s_barrier();           // and every computing wave has read step k
+            if constexpr (BLOCKSCALE) issue_s(k / kScaleChunk + 1, k % kScaleChunk);
             issue(ks + k + STAGES, stage);
             stage = stage == STAGES - 1 ? 0 : stage + 1;
         }
@@ -126,9 +159,25 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         const uint8_t* b = base + ((tn >> 1) * 32 + (tn & 1) * 4) * kKBlock;
         wf[tn % WS] = join(*reinterpret_cast<const v4i*>(b + wfrag0), *reinterpret_cast<const v4i*>(b + wfrag1));
     };
+    // block scales of the coming step: activation scale of this lane's row in each row group, weight scale of the wave's columns
+    float as_n[BLOCKSCALE ? TM : 1], bs_n = 0.f;
+    const int s_rbase = (wm * 2 + (li >> 3)) * 64 + (li & 7) * 8;
+    auto read_scales = [&](int k) {
+        if constexpr (BLOCKSCALE) {
+            const float* cs = s_as + ((k / kScaleChunk) & 1) * (BM * kScaleChunk) + s_rbase + (((k % kScaleChunk) + li) & 7);
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) as_n[tm] = cs[tm * (WGM * 128)];
+            bs_n = s_bs[min(k, nsteps - 1)];
+        }
+    };
+    if constexpr (BLOCKSCALE) {
+        for (int kb = tid; kb < nsteps; kb += 256) s_bs[kb] = p.Bs ? p.Bs[(int64_t)(n0 / 128) * p.kblocks + ks + kb] : 1.0f;
+        __builtin_amdgcn_s_waitcnt(kWaitLds);
+    }
     __builtin_amdgcn_s_barrier();  // step 0 has landed
     read_w(0, lds);
     read_w(1, lds);
+    read_scales(0);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) read_a(tm, lds);
     int stage = 0;
@@ -136,29 +185,62 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         const uint8_t* cur = lds + stage * STAGE_BYTES;
         stage = stage == STAGES - 1 ? 0 : stage + 1;
         const uint8_t* nxt = lds + stage * STAGE_BYTES;
+        // one MFMA; with block scales into a fresh product, and behind it the scale-and-add of the product issued two MFMAs before
+        // (see fp8_gemm_tile.h)
+        v4f part[BLOCKSCALE ? 3 : 1];
+        float sc[BLOCKSCALE ? TM : 1];
+        if constexpr (BLOCKSCALE) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) sc[tm] = as_n[tm] * bs_n;
+        }
+        constexpr int HEAD = (TN - LAST) * TM;  // MFMAs in front of the barrier, column tile by column tile; behind it row group by row group
+        auto tn_of = [](int j) constexpr { return j < HEAD ? j / TM : TN - LAST + (j - HEAD) % LAST; };
+        auto tm_of = [](int j) constexpr { return j < HEAD ? j % TM : (j - HEAD) / LAST; };
+        auto add = [&](int j) __attribute__((always_inline)) {
+            if constexpr (BLOCKSCALE) {
+                if (j < 0) return;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[tn_of(j)][tm_of(j)][r] = __builtin_fmaf(part[j % 3][r], sc[tm_of(j)], acc[tn_of(j)][tm_of(j)][r]);
+            }
+        };
+        auto mma = [&](int j) __attribute__((always_inline)) {
+            const int tn = tn_of(j), tm = tm_of(j);
+            if constexpr (BLOCKSCALE) part[j % 3] = mfma_e4m3(wf[tn % WS], af[tm], v4f{0.f, 0.f, 0.f, 0.f});
+            else acc[tn][tm] = mfma_e4m3(wf[tn % WS], af[tm], acc[tn][tm]);
+        };
         TG_FENCE();
 #pragma unroll
-        for (int tn = 0; tn < TN - LAST; ++tn) {
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                acc[tn][tm] = mfma_e4m3(wf[tn % WS], af[tm], acc[tn][tm]);
-                if (tm == 0 && tn + 2 < TN) read_w(tn + 2, cur);
-                TG_FENCE();
-            }
+        for (int j = 0; j < HEAD; ++j) {
+            mma(j);
+            if (tm_of(j) == 0 && tn_of(j) + 2 < TN) read_w(tn_of(j) + 2, cur);
+            add(j - 2);
+            TG_FENCE();
         }
         __builtin_amdgcn_s_waitcnt(kWaitLds);  // all my reads of step k are done
         __builtin_amdgcn_s_barrier();          // step k+1 is visible
         TG_FENCE();
         read_w(0, nxt);
         read_w(1, nxt);
+        read_scales(k + 1);
         TG_FENCE();
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
+        for (int j = HEAD; j < TN * TM; ++j) {
+            mma(j);
+            add(j - 2);
+            if (tn_of(j) == TN - 1) {
+                TG_FENCE();
+                read_a(tm_of(j), nxt);
+            }
+            TG_FENCE();
+        }
+        if constexpr (BLOCKSCALE) {
+            add(TN * TM - 2);
+            add(TN * TM - 1);
+            // keep the scale-and-add chain inside this step (see fp8_gemm_tile.h)
 #pragma unroll
-            for (int tn = TN - LAST; tn < TN; ++tn) acc[tn][tm] = mfma_e4m3(wf[tn % WS], af[tm], acc[tn][tm]);
-            TG_FENCE();
-            read_a(tm, nxt);
-            TG_FENCE();
+            for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(acc[tn][tm]));
         }
     }
 #pragma unroll
@@ -167,8 +249,10 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 #undef TG_FENCE
 
     float scale = p.alpha;
-    if (p.As) scale *= p.As[0];
-    if (p.Bs) scale *= p.Bs[0];
+    if constexpr (!BLOCKSCALE) {
+        if (p.As) scale *= p.As[0];
+        if (p.Bs) scale *= p.Bs[0];
+    }
     const bool vec_ok = p.vec_store != 0 && (p.N % 8) == 0;
     const int64_t MN = (int64_t)p.M * p.N;
     auto emit = [&](auto type_tag) {
@@ -194,10 +278,10 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 #endif
 }
 
-template <int BM, int BN, int STAGES>
+template <int BM, int BN, int STAGES, bool BLOCKSCALE>
 inline hipError_t launch_tile_ring(bool split, const GemmParams& p, int gx, int gy, hipStream_t stream) {
-    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, true>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
-    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, true>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -41,8 +41,9 @@ hipError_t run_tile256(const GemmParams& p, int gx, hipStream_t s);
 // 64x32 per-tensor tile, K split across the four waves of a workgroup (one launch; 16 < M <= ~512)
 // kn: p.B is (K, N), N % 16 == 0
 hipError_t run_tile_mid(int bm, int bn, bool kn, const GemmParams& p, hipStream_t s);
-// per-tensor tiles of 96 x 128 to 192 x 192 over a ring of LDS stages, four waves load and four compute (M > 64): same results as
-// run_tile_per_tensor's tiles
+// tiles of 64 x 128 to 192 x 192 over a ring of LDS stages, four waves load and four compute: same results as
+// run_tile_per_tensor's and run_tile_block_dense's tiles (block-scaled: bm x 128)
+hipError_t run_tile_ring_block(int bm, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 hipError_t run_tile_ring(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 // 64x128 per-tensor tile with four LDS stages (loads three K steps ahead): the 16 < M <= 64 form
 hipError_t run_tile_deep(bool split, const GemmParams& p, int gx, int gy, hipStream_t s);

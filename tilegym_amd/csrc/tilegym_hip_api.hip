@@ -174,12 +174,14 @@ bool is_mid_tile(int bm, int bn) { return ((bm == 64 || bm == 32) && bn == 32) |
 // Per-tensor 64-row tiles of 72 .. 120 weight rows: the deep 64 x 128 kernel with the rest of its weight slab unused.
 bool is_narrowed_deep_tile(int bm, int bn) { return bm == 64 && bn >= 72 && bn < 128 && bn % 8 == 0; }
 
-// Tiles of fp8_gemm_tile_ring_kernel (per-tensor).  128 x 128 names two kernels: WAVES = 8 asks for the ring (four waves load,
-// four compute), anything else for the four-wave kernel of two workgroups per compute unit.
-bool is_ring_tile(int bm, int bn) { return (bn == 128 && (bm == 96 || bm == 128 || bm == 160)) || (bn == 192 && (bm == 160 || bm == 192)); }
-bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !(bm == 128 && bn == 128); }
+// Tiles of fp8_gemm_tile_ring_kernel.  64 x 128 and 128 x 128 name two kernels each: WAVES = 8 asks for the ring (four waves load,
+// four compute), anything else for the four-wave kernels.
+bool is_ring_tile(int bm, int bn) { return (bn == 128 && (bm == 64 || bm == 96 || bm == 128 || bm == 160)) || (bn == 192 && (bm == 160 || bm == 192)); }
+bool is_block_ring_tile(int bm, int bn) { return bn == 128 && (bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 192); }
+bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !(bn == 128 && (bm == 128 || bm == 64)); }
 
 bool tile_exists(int bm, int bn, bool block_scaled) {
+    if (block_scaled && is_block_ring_tile(bm, bn)) return true;
     if (is_ring_only_tile(bm, bn)) return !block_scaled;
     if (is_mid_tile(bm, bn)) return !block_scaled;  // the four waves split K inside the workgroup (per-tensor only)
     if (is_narrowed_deep_tile(bm, bn)) return !block_scaled;
@@ -221,16 +223,26 @@ constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.194f, 0.178f, 0.f, 1.6
                                         {64, 64, false, 0.298f, 0.338f, 0.f, 3.00f},   {64, 128, false, 0.332f, 0.645f, 0.925f, 3.58f},
                                         {128, 128, false, 0.473f, 0.843f, 0.978f, 2.98f}, {128, 256, false, 0.874f, 1.036f, 0.f, 3.16f},
                                         {256, 256, false, 0.968f, 1.333f, 0.f, 7.72f},
-                                        {96, 128, true, 0.384f, 0.449f, 0.f, 2.46f},   {128, 128, true, 0.402f, 0.546f, 0.f, 2.89f},
+                                        {64, 128, true, 0.304f, 0.527f, 0.f, 1.90f},   {96, 128, true, 0.384f, 0.449f, 0.f, 2.46f},
+                                        {128, 128, true, 0.402f, 0.546f, 0.f, 2.89f},
                                         {160, 128, true, 0.427f, 0.630f, 0.f, 3.42f},  {160, 192, true, 0.554f, 0.778f, 0.f, 4.31f},
                                         {192, 192, true, 0.618f, 0.863f, 0.f, 4.90f}};
+// Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  0.9 % behind the best schedule on average, 15 % ahead
+// of the kernels and the model without the ring tiles (485 x 6144 x 4096 28.5 -> 22.8 us, 1571 x 1184 x 5120 35.8 -> 20.1,
+// 100 x 26064 x 6272 47.4 -> 40.9).  Block-scaled 128 x 256 exists and can be forced; it is left out.
+constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f},
+                                          {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f},
+                                          {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f},
+                                          {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f},
+                                          {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f}};
 constexpr float kReduceUs = 3.5f, kReduceUsPerMB = 0.30f;
 constexpr float kSplitMargin = 1.04f;  // a split schedule must be predicted this much faster than the best unsplit one
 // few rows over a weight that does not stay in the caches: a ring tile waits for memory (69 x 11264 x 2560: 13.8 us with
 // 96 x 128 tiles where the model says 10.6, 12.3 with 64 x 88)
 constexpr float kRingFewRows = 1.25f;
 
-float step_cost_us(const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split) {
+// (few_rows: the factor for ring tiles up to 96 rows)
+float step_cost_us(const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split, float few_rows) {
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * split, places = t.both > 0.f ? 512 : 256;
     const float steps = (float)cdiv(kblocks, split);
     const float at_full = t.both > 0.f ? t.both : t.full;
@@ -240,26 +252,8 @@ float step_cost_us(const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int
         return steps * step + t.fixed;
     };
     float us = (float)(tiles / places) * (steps * at_full + t.fixed) + part(tiles % places);
-    if (t.ring && M <= 96) us *= kRingFewRows;
+    if (t.ring && M <= 96) us *= few_rows;
     if (split > 1) us += kReduceUs + kReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
-    return us;
-}
-
-// Block-scaled tiles: microseconds per K step of a tile while its compute unit holds one workgroup (`alone`: the launch has at
-// most 256 tiles) or two (`shared`), rounds = tiles / 256 or tiles / 512 rounded up; a least-squares fit to measurements
-// of 180 shapes (M = 96 ... 8192, 18 weight shapes) x every tile x 1 / 2 / 4 / 8 splits.
-struct TileCost { int bm, bn; float alone, shared, fixed; };
-// (block-scaled 128 x 256 exists and can be forced; leaving it out of the automatic choice measured better)
-constexpr TileCost kBlockScaledTiles[] = {{64, 128, 0.685f, 0.851f, 3.50f}, {128, 128, 0.690f, 1.016f, 4.23f},
-                                          {256, 256, 1.496f, 1.496f, 8.11f}};
-constexpr float kBlockReduceUs = 6.0f, kBlockReduceUsPerMB = 0.235f, kBlockSplitMargin = 1.05f;
-
-float tile_cost_us(const TileCost& t, int64_t M, int64_t N, int64_t kblocks, int split) {
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * split, ksteps = cdiv(kblocks, split);
-    const bool one_per_cu = t.bm == 256 && t.bn == 256;
-    float us = (one_per_cu || tiles <= 256) ? (float)cdiv(tiles, 256) * ((float)ksteps * t.alone + t.fixed)
-                                            : (float)cdiv(tiles, 512) * ((float)ksteps * t.shared + t.fixed);
-    if (split > 1) us += kBlockReduceUs + kBlockReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
     return us;
 }
 
@@ -271,23 +265,22 @@ struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us
 TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
                              int bm, int bn, bool ring) {
     TileChoice best;
-    auto offer = [&](int kbm, int kbn, bool kring, float margin, auto&& cost) {
-        if (bm > 0 && (kbm != bm || kbn != bn || (kring && !is_ring_only_tile(kbm, kbn)) != (ring && !is_ring_only_tile(kbm, kbn)))) return;
-        if (want_split > 1 && is_mid_tile(kbm, kbn)) return;  // these split K inside the workgroup only
+    auto offer = [&](const StepCost& t) {
+        if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
+        const bool mid = is_mid_tile(t.bm, t.bn);
+        if (want_split > 1 && mid) return;  // these split K inside the workgroup only
         // (five full row tiles of 64 over a weight of up to 16 MB: callers rely on the 64-row kernel there -- the suite pins
         // it; 320 x 4096 x 4096 takes 17.1 us with 64 x 88 tiles, 12.9 with 96 x 128)
-        if (kring && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
+        if (t.ring && !block_scaled && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (want_split > 0 && sp != 1) break;          // the caller's split is applied by the caller
-            if (sp > 1 && (is_mid_tile(kbm, kbn) || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
-            const float us = cost(want_split > 0 ? want_split : sp) * (sp > 1 ? margin : 1.f);
-            if (best.bm < 0 || us < best.us) best = TileChoice{kbm, kbn, sp, kring, us};
+            if (sp > 1 && (mid || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
+            const float us = step_cost_us(t, M, N, kblocks, want_split > 0 ? want_split : sp, block_scaled ? 1.f : kRingFewRows) * (sp > 1 ? kSplitMargin : 1.f);
+            if (best.bm < 0 || us < best.us) best = TileChoice{t.bm, t.bn, sp, t.ring, us};
         }
     };
-    if (block_scaled)
-        for (const TileCost& t : kBlockScaledTiles) offer(t.bm, t.bn, false, kBlockSplitMargin, [&](int sp) { return tile_cost_us(t, M, N, kblocks, sp); });
-    else
-        for (const StepCost& t : kPerTensorTiles) offer(t.bm, t.bn, t.ring, kSplitMargin, [&](int sp) { return step_cost_us(t, M, N, kblocks, sp); });
+    if (block_scaled) { for (const StepCost& t : kBlockScaledTiles) offer(t); }
+    else for (const StepCost& t : kPerTensorTiles) offer(t);
     return best;
 }
 
@@ -297,6 +290,7 @@ TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_s
 // 1 KiB piece) and the skinny kernel (cost proportional to the weight bytes x row tiles, plus a constant).  Against the
 // best forced schedule on 72 held-out combinations: 0.4 % (per-tensor) and 0.9 % (block-scaled) behind on average, worst
 // 7 % and 16 %; the rules it replaces: 7 % on average, worst 1.4 x and 1.7 x.
+struct TileCost { int bm, bn; float alone, shared, fixed; };  // us per K step while a compute unit holds one workgroup, two; us per launch
 struct SmallRowsCosts {
     TileCost tiles[5];
     int n_tiles;
@@ -324,7 +318,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
 Schedule choose_dense(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
                       const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail) {
     Schedule s = choose_dense_tile(M, N, K, block_scaled, fast_layout, cfg, ncfg, partial_bytes_avail);
-    if (s.kernel == 1 && !block_scaled && s.bm == 64 && s.bn == 128 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
+    if (s.kernel == 1 && !block_scaled && s.waves != 8 && s.bm == 64 && s.bn == 128 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
         const int64_t tiles_m = cdiv(M, 64);
         if (tiles_m * cdiv(N, 128) * s.split_k < 256) {
             for (int bn = 120; bn >= 72 && tiles_m * cdiv(N, bn) * s.split_k <= 256; bn -= 8) s.bn = bn;
@@ -390,6 +384,20 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                 Schedule cand{1, t.bm, t.bn, 1, -1, -1, -1};
                 if (split > 1) cand.split_k = pick_split(cdiv(M, t.bm) * cdiv(N, t.bn), 256, kblocks, 4, M, N, partial_bytes_avail, split);
                 offer(cand, rounds_cost_us(t, cdiv(M, t.bm) * cdiv(N, t.bn) * cand.split_k, cdiv(kblocks, cand.split_k)) + reduce(cand.split_k));
+                if (want_split > 0) break;
+            }
+        }
+        // block-scaled: the ring form of the 64 x 128 tile (five stages; 62 x 6144 x 4096 15.7 -> 12.6 us, 30 x 4096 x 14336
+        // 21.8 -> 17.2; 63 shapes 12 % on average.  Per-tensor the deep kernel is as fast: 3 % behind)
+        if (block_scaled) {
+            for (int sp = 1; sp <= 8; sp *= 2) {
+                const int split = want_split > 0 ? want_split : sp;
+                if (split > 1 && (kblocks / split < 4 || !fits(split))) break;
+                Schedule cand{1, 64, 128, 1, -1, -1, 8};
+                if (split > 1) cand.split_k = pick_split(cdiv(N, 128), 256, kblocks, 4, M, N, partial_bytes_avail, split);
+                constexpr StepCost ring{64, 128, true, 0.338f, 0.736f, 0.f, 2.14f};
+                // (a split is as many column tiles over a shorter K)
+                offer(cand, step_cost_us(ring, M, cdiv(N, 128) * 128 * cand.split_k, cdiv(kblocks, cand.split_k), 1, 1.f) + reduce(cand.split_k));
                 if (want_split > 0) break;
             }
         }
@@ -549,7 +557,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, block_scaled))) bm = bn = -1;
     int model_split = 1;
-    const bool want_ring = !block_scaled && bm > 0 && is_ring_tile(bm, bn) && (is_ring_only_tile(bm, bn) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
+    const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && ((bm != 128 && bm != 64) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
     if (want_ring) s.waves = 8;
     if (M > 64) {
         const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring);
@@ -880,13 +888,14 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     if (can_chunk && (K % 128) == 0 && M >= 1024 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_M) <= 0 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0 &&
         cfg_get(cfg, ncfg, TG_CFG_SPLIT_K) <= 0) {
         const int64_t tm = cdiv(M, 256), tn = cdiv(N, 256), total = tm * tn, rounds = cdiv(total, 256);
-        // (per-tensor: only where the model says that no single launch is as fast)
+        // (only where the model says that no single launch is as fast)
         auto worth_it = [&](int64_t full_m, int64_t full_n, int64_t rest_m, int64_t rest_n) {
-            if (block_scaled || K < 1024) return true;  // (the model was fitted to K >= 1024)
+            if (K < 1024) return true;  // (the model was fitted to K >= 1024)
             const int64_t avail = workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
-            const float whole = pick_tile_by_cost(M, N, kblocks, false, avail, -1, -1, -1, false).us;
-            return pick_tile_by_cost(full_m, full_n, kblocks, false, avail, 1, 256, 256, false).us +
-                       pick_tile_by_cost(rest_m, rest_n, kblocks, false, avail, -1, -1, -1, false).us < whole;
+            const float whole = pick_tile_by_cost(M, N, kblocks, block_scaled, avail, -1, -1, -1, false).us;
+            const float two = pick_tile_by_cost(full_m, full_n, kblocks, block_scaled, avail, 1, 256, 256, false).us +
+                              pick_tile_by_cost(rest_m, rest_n, kblocks, block_scaled, avail, -1, -1, -1, false).us;
+            return two < whole * 1.05f;  // (the second piece starts while the first one's last tiles run)
         };
         if (total > 256 && total * 100 < rounds * 256 * 80) {
             auto fills = [](int64_t tiles) { return tiles >= 256 && tiles * 100 >= cdiv(tiles, 256) * 256 * 95; };
@@ -1069,7 +1078,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         if (rows != M && s.split_k > 1) { pc.split_k = 1; pc.ksteps_per_split = (int)kblocks; }
         int gx = (int)(cdiv(rows, s.bm) * cdiv(N, s.bn));
         const bool split = pc.split_k > 1;
-        const bool deep = s.kernel == 1 && !block_scaled && s.bm == 64 && (s.bn == 128 || is_narrowed_deep_tile(s.bm, s.bn));
+        const bool deep = s.kernel == 1 && !block_scaled && s.waves != 8 && s.bm == 64 && (s.bn == 128 || is_narrowed_deep_tile(s.bm, s.bn));
         if (deep) pc.tile_cols = s.bn;
         const bool mid = s.kernel == 1 && !block_scaled && is_mid_tile(s.bm, s.bn);
         // persistent kernel with the hand-ordered K loop for the dense per-tensor 256x256 tile, from two K steps up
@@ -1083,7 +1092,9 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
                                    cfg_get(cfg, ncfg, TG_CFG_WAVES) != 8;
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
         const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
-        hipError_t e = ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
+        const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
+        hipError_t e = block_ring ? tg::run_tile_ring_block(s.bm, split, pc, gx, pc.split_k, stream)
+                     : ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
                      : ordered ? tg::run_tile256(pc, gx, stream)
                      : bs_persistent ? tg::run_bs256(tg::GROUP_DENSE, pc, gx, stream)

@@ -46,9 +46,9 @@ def candidates(M: int, N: int, K: int, block_scaled: bool) -> List[dict]:
                 if s > 1 and (bm, bn) in ((32, 32), (64, 32), (64, 64)):
                     continue
                 out.append({"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": s})
-        if not block_scaled and M > 64:
-            # tiles over a ring of LDS stages, four waves load and four compute (WAVES = 8 picks that form of 128 x 128)
-            for bm, bn in ((96, 128), (128, 128), (160, 128), (160, 192), (192, 192)):
+        if block_scaled or M > 64:
+            # tiles over a ring of LDS stages, four waves load and four compute (WAVES = 8 picks that form of 64 x 128 and 128 x 128)
+            for bm, bn in ((64, 128), (96, 128), (128, 128), (160, 128)) + (((192, 128),) if block_scaled else ((160, 192), (192, 192))):
                 out += [{"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": s, "WAVES": 8} for s in (1, 2, 4)]
         if not block_scaled and M <= 512:
             # the 64 x 128 tile kernel over fewer weight rows per tile (more, lighter workgroups)
