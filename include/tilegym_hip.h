@@ -313,6 +313,8 @@ int32_t tg_moe_sum_routed(const tg_tensor* out, const tg_tensor* x, const tg_ten
  * Layers outside these limits (more tokens than one chunk, other intermediate sizes, fp8 activations with their own scales)
  * are run call by call, as the Python layer does.
  */
+/* The row block (128 or 256) that tg_fp8_fused_moe is fastest with for a layer of these sizes. */
+int32_t tg_fp8_fused_moe_block_m(int64_t tokens, int64_t top_k, int64_t experts, int64_t inter);
 int64_t tg_fp8_fused_moe_workspace_bytes(int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t inter,
                                          int32_t block_m);
 int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg_tensor* w1, const tg_tensor* w2,

@@ -1099,6 +1099,44 @@ def test_ragged_unaligned_empty_and_single_experts(device, bm, bn):
     check(o2, R.ref_ragged_block_scaled_bmm(a, b, None, b_s, ptr))
 
 
+@pytest.mark.parametrize("K", [128, 256, 384, 1024, 1152, 2176])
+def test_ragged_tiles_of_two_workgroups_per_compute_unit(device, K):
+    """128 x 256 tiles: a ring of half weight slabs (1, 2, 3 K steps), chunks of scales that end inside K (8, 9, 17 steps), no
+    row, one row, whole and partly filled row groups per expert.  Same bits as 128 x 128 tiles."""
+    impl = tilegym_amd.backend._REGISTRY["flashinfer.gemm.ragged_block_scaled_bmm"]["hip"]
+    sizes = [0, 1, 128, 129, 77, 300, 0, 16]
+    a, b, a_s, b_s, ptr = _ragged_inputs(sizes, 392, K, K)
+    args = [t.to(device) for t in (a, b, a_s, b_s, ptr)] + [max(sizes)]
+    out = impl(*args, kernel_configs={"BLOCK_M": 128, "BLOCK_N": 256})
+    cfg = used("tiled")
+    assert (cfg["BLOCK_M"], cfg["BLOCK_N"]) == (128, 256)
+    assert torch.equal(out, impl(*args, kernel_configs={"BLOCK_M": 128, "BLOCK_N": 128}))
+    check(out, R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr), what=f"pair tiles, K={K}")
+
+
+@pytest.mark.parametrize("crowded", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_moe_layer_same_bits_with_128_and_256_row_blocks(device, dtype, crowded):
+    """Enough 128 x 256 tiles for the form of which two share a compute unit, in both GEMMs; even routing, and every token to
+    the same four experts."""
+    T, H, I, E, k = 600, 1024, 512, 64, 4
+    g = torch.Generator(device=device).manual_seed(7 + crowded)
+    x = torch.randn(T, H, generator=g, device=device).to(dtype)
+    w1, w2 = (torch.randn(E, n, kk, generator=g, device=device).to(FP8) for n, kk in ((2 * I, H), (H, I)))
+    s1, s2 = (torch.rand(E, n // 128, kk // 128, generator=g, device=device) * 0.02 + 0.001 for n, kk in ((2 * I, H), (H, I)))
+    ids = torch.rand(T, E, generator=g, device=device).topk(k, dim=1).indices.to(torch.int32)
+    if crowded:
+        ids = torch.tensor([3, 9, 41, 63], dtype=torch.int32, device=device).expand(T, k).contiguous()
+    weights = torch.rand(T, k, generator=g, device=device)
+    outs = []
+    for block_m in (128, 256):
+        out = torch.empty(T, H, dtype=dtype, device=device)
+        _lib.fp8_fused_moe(out, x, w1, w2, s1, s2, weights, ids, block_m)
+        outs.append(out)
+    assert torch.isfinite(outs[0]).all()
+    assert torch.equal(*outs)
+
+
 def test_ragged_many_experts_and_permutation(device):
     g = _g(31)
     sizes = torch.randint(0, 40, (150,), generator=g).tolist()  # > 64 experts: multi-pass expert search

@@ -69,7 +69,7 @@ class TileGymHipError(RuntimeError):
 _lib = None
 native = None  # the extension module, once load() has run (still None where it cannot be imported)
 _NATIVE_ENTRY_POINTS = ("tg_fp8_gemm", "tg_fp8_gemm_workspace_bytes", "tg_fp8_ragged_gemm", "tg_fp8_quant_group", "tg_fp8_fused_moe",
-                        "tg_fp8_fused_moe_workspace_bytes")
+                        "tg_fp8_fused_moe_block_m", "tg_fp8_fused_moe_workspace_bytes")
 
 
 def lib_path() -> str:
@@ -132,6 +132,8 @@ def load():
     L.tg_moe_sum.argtypes = [P, P, ctypes.c_int32, ctypes.c_uint64]
     L.tg_moe_sum_routed.restype = ctypes.c_int32
     L.tg_moe_sum_routed.argtypes = [P, P, P, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint64]
+    L.tg_fp8_fused_moe_block_m.restype = ctypes.c_int32
+    L.tg_fp8_fused_moe_block_m.argtypes = [ctypes.c_int64] * 4
     L.tg_fp8_fused_moe_workspace_bytes.restype = ctypes.c_int64
     L.tg_fp8_fused_moe_workspace_bytes.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int32]
     L.tg_fp8_fused_moe.restype = ctypes.c_int32
@@ -619,6 +621,11 @@ def fp8_group_gemm(cs, As, Bs, scales_a=None, scales_b=None, trans_b=True, kerne
 
 
 _moe_ws_bytes: Dict[tuple, int] = {}
+
+
+def fused_moe_block_m(tokens: int, top_k: int, experts: int, inter: int) -> int:
+    """Row block (128 or 256) of the grouped GEMMs of a MoE layer."""
+    return int(load().tg_fp8_fused_moe_block_m(tokens, top_k, experts, inter))
 
 
 def fused_moe_ok(hidden, w1, w2, block_m: int) -> bool:

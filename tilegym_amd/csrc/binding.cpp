@@ -26,6 +26,7 @@ decltype(&tg_fp8_gemm_workspace_bytes) g_gemm_workspace_bytes = nullptr;
 decltype(&tg_fp8_ragged_gemm) g_ragged_gemm = nullptr;
 decltype(&tg_fp8_quant_group) g_quant_group = nullptr;
 decltype(&tg_fp8_fused_moe) g_fused_moe = nullptr;
+decltype(&tg_fp8_fused_moe_block_m) g_fused_moe_block_m = nullptr;
 decltype(&tg_fp8_fused_moe_workspace_bytes) g_fused_moe_workspace_bytes = nullptr;
 PyObject* g_workspaces = nullptr;     // {(device, stream, under capture): [scratch tensors, newest last]}
 PyObject* g_workspace_for = nullptr;  // callable(device, bytes, index, stream) -> tensor, for a new or larger one
@@ -304,8 +305,7 @@ PyObject* py_fused_moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         w1->size(2) != H || w2->size(0) != E || w2->size(1) != H || w2->size(2) != I2 / 2 || ids->size(0) != T || tw->sizes() != ids->sizes() ||
         x->device() != w1->device() || x->device() != w2->device())
         Py_RETURN_NONE;
-    // rows per expert decide the row tile of the grouped GEMMs (as in the Python implementation)
-    const int block_m = T * k / E >= 96 ? 256 : 128;
+    const int block_m = g_fused_moe_block_m(T, k, E, I2 / 2);
     const bool inplace = args[7] == Py_True;
     at::Tensor out = inplace ? *x : new_tensor({T, H}, x->scalar_type(), *x);
     tg_tensor dout, dx, dw1, dw2, ds1, ds2, dtw, dids, dws;
@@ -341,7 +341,7 @@ PyObject* py_set_up(PyObject*, PyObject* args) {
     };
     if (!find("tg_fp8_gemm", &g_gemm) || !find("tg_fp8_gemm_workspace_bytes", &g_gemm_workspace_bytes) || !find("tg_fp8_ragged_gemm", &g_ragged_gemm) ||
         !find("tg_fp8_quant_group", &g_quant_group) || !find("tg_fp8_fused_moe", &g_fused_moe) ||
-        !find("tg_fp8_fused_moe_workspace_bytes", &g_fused_moe_workspace_bytes))
+        !find("tg_fp8_fused_moe_block_m", &g_fused_moe_block_m) || !find("tg_fp8_fused_moe_workspace_bytes", &g_fused_moe_workspace_bytes))
         return nullptr;
     for (auto [slot, o] : {std::pair{&g_workspaces, workspaces}, std::pair{&g_workspace_for, workspace_for}, std::pair{&g_check_rc, check_rc}}) {
         Py_INCREF(o);

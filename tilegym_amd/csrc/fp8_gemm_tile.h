@@ -230,7 +230,7 @@ __device__ __forceinline__ void store8(void* C, int out_type, int64_t row, int c
 
 // Body of the tiled kernel for workgroup `bid` of problem `p` (the kernels below only differ in
 // how a workgroup finds its problem).
-template <int BM, int BN, int WGM, int WGN, bool BLOCKSCALE, int GROUP, bool SPLIT>
+template <int BM, int BN, int WGM, int WGN, bool BLOCKSCALE, int GROUP, bool SPLIT, bool PAIR = false>
 __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const int bid) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body is device-only assembly; the host pass only needs the stub
     constexpr int NT = 64 * WGM * WGN;
@@ -250,10 +250,13 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
     static_assert(!ACT || (BLOCKSCALE && BN == 256 && WTN % 64 == 0 && WGN * BM <= 2 * BM * kScaleChunk),
                   "fused activation: block-scaled, 128 gate + 128 up columns per tile, each wave with as many gate as up column tiles");
 
+    // PAIR: one activation slab and a ring of three half weight slabs, 64 KiB, so that two workgroups share a compute unit
+    constexpr int HALF = BN / 2 * kKBlock;
+    static_assert(!PAIR || (BM == 128 && BN == 256 && NW == 4 && BLOCKSCALE && TN == 8), "the pair form");
     __shared__ __align__(1024) uint8_t sA0[BM * kKBlock];
-    __shared__ __align__(1024) uint8_t sA1[BM * kKBlock];
-    __shared__ __align__(1024) uint8_t sB0[BN * kKBlock];
-    __shared__ __align__(1024) uint8_t sB1[BN * kKBlock];
+    __shared__ __align__(1024) uint8_t sA1[PAIR ? 1024 : BM * kKBlock];
+    __shared__ __align__(1024) uint8_t sB0[PAIR ? 3 * HALF : BN * kKBlock];
+    __shared__ __align__(1024) uint8_t sB1[PAIR ? 1024 : BN * kKBlock];
     // activation scales of the tile rows, two chunks of kScaleChunk K steps (block-scaled kernels only)
     __shared__ __align__(256) float sTab[BLOCKSCALE ? 2 * BM * kScaleChunk : 1];
     // weight block scales of this tile's column blocks for every K step (fetched once)
@@ -337,7 +340,12 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
     uint32_t b_off[B_IT];
 #pragma unroll
     for (int i = 0; i < B_IT; ++i) {
-        const int br = (i * NL + (wave % NL)) * 8 + lrow;  // slab row
+        int br = (i * NL + (wave % NL)) * 8 + lrow;  // slab row
+        // (PAIR: half i / 4 of the slab holds, for both wave columns, the rows of column tiles 0 - 3 or 4 - 7)
+        if constexpr (PAIR) {
+            const int hr = ((i % 4) * NL + wave) * 8 + lrow;
+            br = (hr / 64) * WTN + (i / 4) * 64 + hr % 64;
+        }
         int n;
         // fused activation: wave column wn owns slab rows WTN*wn .. +WTN-1 = WTN/2 gate rows, then the WTN/2 up rows of the same columns
         if constexpr (ACT) n = ((br % WTN) / (WTN / 2)) * p.inter + n0 + (br / WTN) * (WTN / 2) + br % (WTN / 2);
@@ -356,7 +364,17 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
 #pragma unroll
         for (int i = 0; i < B_IT; ++i) issue_b1(i, kstep, dB);
     };
-    issue_b(ks, sB0);
+    // PAIR: half h of the weight slab of a K step into a slot of the ring
+    auto issue_half = [&](int h, int kstep, int slot) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) direct_load_b128(rsrc_b, lds_address(sB0) + slot * HALF + wave * 1024 + q * NL * 1024, b_off[(PAIR ? h * 4 : 0) + (PAIR ? q : 0)], kstep * kKBlock);
+    };
+    if constexpr (PAIR) {
+        issue_half(0, ks, 0);
+        issue_half(1, ks, 1);
+    } else {
+        issue_b(ks, sB0);
+    }
 
     // ---------------------------------------------------------------- row maps and scale tables
     // Both come from global memory; the slot ids are requested first and used last, so that the two
@@ -618,9 +636,77 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
     issue_a(ks, sA0);  // (the weight slab of this step is in flight since the top of the kernel)
 #pragma unroll
     for (int ph = 0; ph < S_PHASES; ++ph) issue_s(0, ph);
-    issue_a(min(ks + 1, last), sA1);
-    __builtin_amdgcn_s_waitcnt(kWaitAllButA);  // a wave without loads in flight passes at once
-    lds_barrier();
+    if constexpr (PAIR) {
+        __builtin_amdgcn_s_waitcnt(kWaitAll);
+    } else {
+        issue_a(min(ks + 1, last), sA1);
+        __builtin_amdgcn_s_waitcnt(kWaitAllButA);  // a wave without loads in flight passes at once
+        lds_barrier();
+    }
+    // PAIR: four column tiles (one half of the weight slab at `half`) of the block-scaled step, as in mma() above
+    auto mma_half = [&](auto ntm_tag, auto h_tag, const uint8_t* half) {
+        constexpr int NTM = decltype(ntm_tag)::value, H = decltype(h_tag)::value;
+        if constexpr (NTM > 0 && PAIR) {
+            constexpr int NJ = 4 * NTM;
+            v4f part[3];
+            v8i wf[2];
+            const uint8_t* base = half + wn * 64 * kKBlock;
+            auto read_w = [&](int t) {
+                const uint8_t* b = base + w_tile_row(t) * kKBlock;
+                wf[t & 1] = join(*reinterpret_cast<const v4i*>(b + wfrag0), *reinterpret_cast<const v4i*>(b + wfrag1));
+            };
+            auto add = [&](int j) {
+                const int tn = H * 4 + j / NTM, tm = j % NTM;
+                acc[tn][tm] += part[j % 3] * scale_of(tn, tm);
+            };
+            read_w(0);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int t = j / NTM, tm = j % NTM;
+                part[j % 3] = mfma_e4m3(wf[t & 1], af[tm], v4f{0.f, 0.f, 0.f, 0.f});
+                if (tm == 0 && t + 1 < 4) read_w(t + 1);
+                if (j >= 2) add(j - 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (NJ >= 2) add(NJ - 2);
+            add(NJ - 1);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int tm = 0; tm < NTM; ++tm) asm volatile("" : "+v"(acc[H * 4 + t][tm]));
+        }
+    };
+    // PAIR main loop.  Half h of step k sits in slot (2k + h) % 3 of the ring.
+    //   top of step k : wait for A(k) and H0(k);  barrier (every wave is done with H1(k-1));  request H0(k+1) into the slot H1(k-1)
+    //                   had and a row group of the next chunk of scales;  read A fragments and scales;  MFMAs of H0(k)
+    //   middle        : wait for H1(k);  barrier (every wave holds its A fragments and is done with H0(k));  request A(k+1) into
+    //                   the one A slab and H1(k+1) into the slot H0(k) had;  MFMAs of H1(k)
+    // While one workgroup of a compute unit waits, sets up or runs its epilogue, the other one multiplies.  A 64-expert gate/up
+    // tile of 16 K steps spends 7.8 k clocks in set-up, 3.3 k per step and 11.8 k in its epilogue, two at a time; the 128 x 256 form
+    // of eight waves and 111 KiB that it replaces on large launches ran one at a time.  Gate/up and down GEMM of 64 experts, us,
+    // before -> now: 1024 tokens 93 + 51 -> 88 + 46, 3000 tokens 203 + 107 -> 166 + 96.  Bound by issue and LDS traffic: with
+    // the weights in the memory-side cache a step still takes 3.1 - 3.2 k clocks (2.6 k for its MFMAs, scale-and-adds and LDS reads alone).
+    auto pair_loop = [&](auto ntm_tag) {
+        constexpr int kWaitBut4 = 0x0F70 | 4;
+        int slot = 0;
+        for (int k = ks; k < ks_end; ++k) {
+            const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot1 == 2 ? 0 : slot1 + 1;
+            const int kn = min(k + 1, last);
+            __builtin_amdgcn_s_waitcnt(kWaitBut4);  // all but the four most recent: H1(k)
+            lds_barrier();
+            issue_s((k - ks) / kScaleChunk + 1, (k - ks) % kScaleChunk);
+            issue_half(0, kn, slot2);
+            read_a(ntm_tag, sA0);
+            read_scales(ntm_tag, k);
+            mma_half(ntm_tag, std::integral_constant<int, 0>{}, sB0 + slot * HALF);
+            __builtin_amdgcn_s_waitcnt(kWaitBut4);  // all but H0(k+1)
+            lds_barrier();
+            issue_a(kn, sA0);
+            issue_half(1, kn, slot);
+            mma_half(ntm_tag, std::integral_constant<int, 1>{}, sB0 + slot1 * HALF);
+            slot = slot2;
+        }
+    };
     // The loop exists once per number of row groups a wave may have to compute (NTM = 0 .. TM): the
     // waves of a workgroup can run different copies, every copy issues the same loads and barriers.
     auto k_loop = [&](auto ntm_tag) {
@@ -658,6 +744,17 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
     int n_tm = TM;
     if constexpr (GROUP == GROUP_DENSE) {
         k_loop(std::integral_constant<int, TM>{});
+    } else if constexpr (PAIR) {
+        n_tm = 0;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+            if (__ballot(s_dst[tile_row(tm) + li] >= 0) != 0) n_tm = tm + 1;
+        n_tm = __builtin_amdgcn_readfirstlane(n_tm);
+        if (n_tm == 4) pair_loop(std::integral_constant<int, 4>{});
+        else if (n_tm == 3) pair_loop(std::integral_constant<int, 3>{});
+        else if (n_tm == 2) pair_loop(std::integral_constant<int, 2>{});
+        else if (n_tm == 1) pair_loop(std::integral_constant<int, 1>{});
+        else pair_loop(std::integral_constant<int, 0>{});
     } else {
         static_assert(TM == 4, "dispatch below");
         n_tm = 0;
@@ -815,6 +912,18 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
 template <int BM, int BN, int WGM, int WGN, bool BLOCKSCALE, int GROUP, bool SPLIT>
 __global__ void __launch_bounds__(64 * WGM * WGN, (WGM * WGN == 4 ? 2 : 1)) fp8_gemm_tile_kernel(const GemmParams p) {
     fp8_gemm_tile_body<BM, BN, WGM, WGN, BLOCKSCALE, GROUP, SPLIT>(p, (int)blockIdx.x);
+}
+
+// Two workgroups per compute unit (see PAIR in the body).
+template <int BM, int BN, int WGM, int WGN, int GROUP>
+__global__ void __launch_bounds__(64 * WGM * WGN, 2) fp8_gemm_pair_kernel(const GemmParams p) {
+    fp8_gemm_tile_body<BM, BN, WGM, WGN, true, GROUP, false, true>(p, (int)blockIdx.x);
+}
+
+template <int GROUP>
+inline hipError_t launch_pair(const GemmParams& p, int grid_x, hipStream_t stream) {
+    hipLaunchKernelGGL((fp8_gemm_pair_kernel<128, 256, 2, 2, GROUP>), dim3(grid_x, 1, 1), dim3(256, 1, 1), 0, stream, p);
+    return hipGetLastError();
 }
 
 // A list of independent per-tensor-scaled GEMMs in one launch (tilegym.ops.group_gemm,

@@ -14,15 +14,16 @@ hipError_t run_tile_block_grouped(int bm, int bn, int group, const GemmParams& p
     }
     TG_CASE(256, 256, 4, 2)
     TG_CASE(128, 128, 2, 2)
-    TG_CASE(128, 256, 2, 4)
+    if (bm == 128 && bn == 256) return group == GROUP_RAGGED ? launch_pair<GROUP_RAGGED>(p, gx, s) : launch_pair<GROUP_GATHER>(p, gx, s);
     TG_CASE(64, 128, 1, 4)
 #undef TG_CASE
     return hipErrorInvalidConfiguration;
 }
 
 // Gate/up MoE GEMM with the SiLU-multiply-quantize epilogue (a tile is 128 gate + 128 up columns; 256 or 128 rows).
-hipError_t run_tile_moe_act(int bm, const GemmParams& p, int gx, hipStream_t s) {
+hipError_t run_tile_moe_act(int bm, bool pair, const GemmParams& p, int gx, hipStream_t s) {
     if (bm == 256) return launch_tile<256, 256, 4, 2, true, GROUP_GATHER_ACT, false>(p, gx, 1, s);
+    if (bm == 128 && pair) return launch_pair<GROUP_GATHER_ACT>(p, gx, s);
     if (bm == 128) return launch_tile<128, 256, 2, 4, true, GROUP_GATHER_ACT, false>(p, gx, 1, s);
     return hipErrorInvalidConfiguration;
 }

@@ -57,7 +57,8 @@ inline bool bs256_takes_k(int kblocks) { return kblocks >= 2 && kblocks % 4 != 1
 // compute units of the current device
 int compute_units();
 hipError_t run_tile_block_dense(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
-hipError_t run_tile_moe_act(int bm, const GemmParams& p, int gx, hipStream_t s);
+// pair: the 128-row form of which two workgroups share a compute unit
+hipError_t run_tile_moe_act(int bm, bool pair, const GemmParams& p, int gx, hipStream_t s);
 hipError_t run_tile_block_grouped(int bm, int bn, int group, const GemmParams& p, int gx, hipStream_t s);
 // The two GEMMs of the decoding MoE layer: out = T(silu(gate) * up) resp. out = T(result x routed weight).  `up` selects the
 // first.  The `fits` forms say (from the sizes in p alone) whether the layer is one for these kernels: few enough rows per

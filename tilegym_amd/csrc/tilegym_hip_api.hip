@@ -2,6 +2,7 @@
 // host, schedule selection, kernel launches.  No allocation, no synchronisation, no global
 // mutable state apart from two thread-local diagnostics (last error text, last schedule).
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -633,6 +634,33 @@ bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, 
     return best * kKnMargin <= nk + kCopyUs + kCopyUsPerMB * mb;
 }
 
+// ---- expert-grouped block-scaled GEMMs: 256 x 256 tiles, or 128 x 256 tiles of which two share a compute unit (PAIR in
+// fp8_gemm_tile.h)
+// Cost of an expert's rows in whole 128-row tiles: from clock stamps of the 64-expert layer (K = 2048; 73.6 k clocks for a full
+// 128-row tile of two, 79 k for a full 256-row tile and 62 / 50 / 39 k with three, two, one of its row groups in use, 128-row
+// tiles nearly the same whatever they hold).  `rows` routed rows spread evenly but for their own noise over the experts.
+// Layer times it decides between (us, 128-row tiles / 256-row tiles): 64 experts of (2048, 1408), top 6, 512 / 1024 / 1500 / 3000
+// tokens 130 / 148 / 195 / 272 against 144 / 162 / 177 / 298; 8 experts, top 2, 4096 tokens 123 against 142.
+float grouped_cost(int64_t rows, int64_t experts, bool pair) {
+    const double mu = (double)rows / (double)experts, sigma = sqrt(mu);
+    static const double at[5] = {-1.6, -0.67, 0.0, 0.67, 1.6}, weight[5] = {0.125, 0.25, 0.25, 0.25, 0.125};
+    double cost = 0.0;
+    for (int i = 0; i < 5; ++i) {
+        const int64_t r = std::max<int64_t>((int64_t)llround(mu + at[i] * sigma), 1);
+        if (pair) { cost += weight[i] * 1.05 * (double)cdiv(r, 128); continue; }
+        const int64_t rest = r % 256;
+        cost += weight[i] * (2.15 * (double)(r / 256) + (rest == 0 ? 0.0 : rest <= 64 ? 1.05 : rest <= 128 ? 1.36 : rest <= 192 ? 1.68 : 2.15));
+    }
+    return (float)cost;
+}
+// Row tiles of 128 rows, about.
+int64_t grouped_row_tiles(int64_t rows, int64_t experts) { return rows / 128 + std::min(rows, experts) / 2; }
+// From this many 128 x 256 tiles on two of them on a compute unit are faster than one workgroup of eight waves, or 128 x 128
+// tiles (8 experts of (4096, 1536), top 2: 179 tiles 81 against 76 us, 329 tiles 109 against 131; 64 experts, 1000 tokens, ragged:
+// 88.5 against 95.5).
+constexpr int64_t kPairTiles = 200;
+bool pair_tiles(int64_t rows, int64_t experts, int64_t col_tiles) { return grouped_row_tiles(rows, experts) * col_tiles >= kPairTiles; }
+
 struct Resolved {
     int64_t M, N, K;
     bool block_scaled;
@@ -1236,11 +1264,15 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
     }
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, true))) {
-        // measured on 64 experts of (2816, 2048) weights: padding rows cost no MFMA work (the kernel skips
-        // row groups without valid rows), so 256x256 wins from ~96 rows per expert up (101 vs 106-109 us
-        // at 96, 172 vs 184-209 at 300), 128x128 down to ~40 (88 vs 102 us at 64), 64x128 below (69 vs 80 at 24)
-        if (total_m / E >= 96 && N >= 256) { bm = 256; bn = 256; }
-        else { bm = (total_m / E >= 40) ? 128 : 64; bn = 128; }
+        // 64 x 128 tiles below 40 rows per expert (69 us against 80 at 24 rows); from there on, if there are enough of them, pairs
+        // of 128 x 256 tiles or 256 x 256 tiles, whichever the padding of the experts' last tiles makes cheaper (64 experts of
+        // (2816, 2048), us, 128 x 128 / pairs / 256 x 256: 94 rows 95.5 / 88.5 / 98.1, 188 rows 132 / 119 / 115, 281 rows 183 /
+        // 159 / 171); few tiles: 128 x 128 below 96 rows, 256 x 256 above
+        const int64_t mean = total_m / E;
+        if (mean < 40) { bm = 64; bn = 128; }
+        else if (N < 256 || (mean < 96 && !pair_tiles(total_m, E, cdiv(N, 256)))) { bm = 128; bn = 128; }
+        else if (pair_tiles(total_m, E, cdiv(N, 256)) && grouped_cost(total_m, E, true) <= grouped_cost(total_m, E, false)) { bm = 128; bn = 256; }
+        else { bm = 256; bn = 256; }
     }
     s.kernel = 1; s.bm = bm; s.bn = bn;
     remember(s);
@@ -1313,7 +1345,7 @@ int32_t tg_fp8_moe_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor*
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, true) && block_m % bm == 0)) {
         if (block_m % 256 == 0 && N >= 256) { bm = 256; bn = 256; }
-        else { bm = (block_m % 128 == 0) ? 128 : (block_m % 64 == 0) ? 64 : 0; bn = 128; }
+        else { bm = (block_m % 128 == 0) ? 128 : (block_m % 64 == 0) ? 64 : 0; bn = bm == 128 && N >= 256 && pair_tiles(num_valid, E, cdiv(N, 256)) ? 256 : 128; }
     }
     const bool fast = bm > 0 && (K % 128) == 0 && K > 0 && K <= 65536 && aligned16(a->ptr) && aligned16(b->ptr) &&
                       T * K < kOffsetLimit && N * K < kOffsetLimit && cfg_get(cfg, ncfg, TG_CFG_KERNEL) != 0;
@@ -1416,7 +1448,7 @@ int32_t tg_fp8_moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, 
     remember(s);
     const int64_t gx = cdiv(EM, bm) * (I / 128);
     if (gx > INT32_MAX) return fail(TG_ERR_INVALID, "too many tiles");
-    hipError_t e = tg::run_tile_moe_act(bm, p, (int)gx, stream);
+    hipError_t e = tg::run_tile_moe_act(bm, pair_tiles(num_valid, E, I / 128), p, (int)gx, stream);
     if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "fused MoE kernel launch failed: %s", hipGetErrorString(e));
     return TG_OK;
 }
@@ -1793,6 +1825,15 @@ tg_tensor describe(uint8_t* base, int64_t offset, int32_t dtype, std::initialize
 }  // namespace
 
 extern "C" {
+
+int32_t tg_fp8_fused_moe_block_m(int64_t tokens, int64_t top_k, int64_t experts, int64_t inter) {
+    if (tokens < 1 || top_k < 1 || experts < 1 || inter < 1) return 128;
+    const int64_t rows = tokens * top_k;
+    // (one round of 128-row tiles, one on a compute unit: halving the rows of a tile halves the time -- 8 experts of (2048, 1408),
+    // 700 tokens, top 2: 48 us against 61)
+    if (grouped_row_tiles(rows, experts) * cdiv(inter, 128) <= 256) return 128;
+    return grouped_cost(rows, experts, true) <= grouped_cost(rows, experts, false) ? 128 : 256;
+}
 
 int64_t tg_fp8_fused_moe_workspace_bytes(int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t inter,
                                          int32_t block_m) {

@@ -110,9 +110,8 @@ def fused_experts_impl(
     cache1 = None
     cache3 = None
     out = hidden_states if inplace else torch.empty((num_tokens, H), device=device, dtype=out_dtype)
-    # rows per expert decide the row tile of the grouped GEMMs: 256 once an expert sees >= 96 routed
-    # rows on average (measured on the 64-expert workload; padding rows cost no MFMA work), else 128
-    config = {"BLOCK_SIZE_M": 256 if (M * top_k) // max(E, 1) >= 96 else 128}
+    # row tile of the grouped GEMMs: 128 or 256, from the rows per expert
+    config = {"BLOCK_SIZE_M": _lib.fused_moe_block_m(M, top_k, E, N // 2)}
     fuse_act = _lib.moe_gemm_silu_quant_ok(w1, config["BLOCK_SIZE_M"]) and w1_scale is not None
     # One chunk of 16-bit activations with the fused activation epilogue: the whole layer is one call into the library
     # (intermediates in the stream's scratch buffer): the host time of four bindings and nine allocations is more than the
