@@ -584,6 +584,33 @@ def test_ring_tiles_block_scaled(device, bm, dm, N, K, split):
             check(out, R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"block ring {bm} M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(256, 320, 128), (257, 352, 256), (300, 672, 1152), (511, 1024, 384), (700, 960, 2176)])
+def test_block_scaled_256_x_320_tile(device, M, N, K):
+    """The smallest problem of one tile, last row and column tiles that are moved back over their neighbours (by every distance
+    between a column block's edge and a tile's), odd numbers of K steps, chunks of scales that end inside K; beta reads the
+    output that a moved tile's neighbour writes.  Same bits as the 256 x 256 tile.  Narrower problems and N that is no
+    multiple of 32 take another tile."""
+    g = _g(M + N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)
+    sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand((N + 127) // 128, K // 128, generator=g) * 0.1 + 0.01
+    args = [t.to(device) for t in (a, b, sa, sb)]
+    old = torch.randn(M, N, generator=g).to(torch.bfloat16).to(device)
+    for beta in (0.0, 1.0):
+        out, base = old.clone(), old.clone()
+        _lib.fp8_gemm(out, *args, False, True, 0.7, beta, {"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 320, "SPLIT_K": 1})
+        cfg = used("tiled")
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"]) == (256, 320), cfg
+        _lib.fp8_gemm(base, *args, False, True, 0.7, beta, {"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 256, "SPLIT_K": 1})
+        assert torch.equal(out, base)
+    check(w8a8_block_fp8_matmul(*args, None, torch.bfloat16, kernel_configs={"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 320}),
+          R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"256 x 320, M={M} N={N} K={K}")
+    for m, n in ((255, N), (M, 312), (M, N - 8)):
+        few = [args[0][:m], args[1][:n], args[2][:m], args[3][:(n + 127) // 128]]
+        out = w8a8_block_fp8_matmul(*[t.contiguous() for t in few], None, torch.bfloat16, kernel_configs={"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 320})
+        assert used("tiled")["BLOCK_N"] != 320
+        check(out, R.ref_w8a8_block_fp8_matmul(a[:m], b[:n], sa[:m], sb[:(n + 127) // 128], None, torch.bfloat16))
+
+
 def test_deep_tile_is_narrowed_to_fill_the_chip(device):
     """28672 weight rows at M = 64: 224 tiles of 128 columns would leave an eighth of the compute units idle; 256 tiles of 112 run."""
     g = _g(112)

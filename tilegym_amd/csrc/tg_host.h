@@ -54,6 +54,9 @@ hipError_t run_bs256(int group, const GemmParams& p, int tiles_bound, hipStream_
 // K steps run_bs256 takes: at least two, and not 4c + 1 (a last chunk of scales of a single step); the weights of all
 // experts together must also stay below 4 GiB
 inline bool bs256_takes_k(int kblocks) { return kblocks >= 2 && kblocks % 4 != 1; }
+// 256 x 320 block-scaled tile, dense rows: same results as the 256 x 256 form.  Needs both scale tensors
+inline bool bs320_takes(int64_t M, int64_t N) { return M >= 256 && N >= 320 && N % 32 == 0; }
+hipError_t run_bs320(const GemmParams& p, int gx, hipStream_t s);
 // compute units of the current device
 int compute_units();
 hipError_t run_tile_block_dense(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);

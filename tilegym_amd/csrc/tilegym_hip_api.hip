@@ -190,6 +190,7 @@ bool tile_exists(int bm, int bn, bool block_scaled) {
     if (bm == 128 && bn == 256) return true;
     if (bm == 64 && bn == 128) return true;
     if (bm == 256 && bn == 256) return true;
+    if (bm == 256 && bn == 320) return block_scaled;  // (where bs320_takes the problem; else the choice is automatic)
     return false;
 }
 
@@ -232,7 +233,7 @@ constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.194f, 0.178f, 0.f, 1.6
 // of the kernels and the model without the ring tiles (485 x 6144 x 4096 28.5 -> 22.8 us, 1571 x 1184 x 5120 35.8 -> 20.1,
 // 100 x 26064 x 6272 47.4 -> 40.9).  Block-scaled 128 x 256 exists and can be forced; it is left out.
 constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f},
-                                          {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f},
+                                          {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f},  {256, 320, false, 1.66f, 2.12f, 0.f, 9.00f},
                                           {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f},
                                           {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f},
                                           {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f}};
@@ -264,18 +265,19 @@ struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us
 // The cheapest (tile, split) by the model; a tile (bm > 0; ring: the ring form of 128 x 128) or a split (want_split > 0) given by
 // the caller is kept.
 TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
-                             int bm, int bn, bool ring) {
+                             int bm, int bn, bool ring, bool takes_320 = false) {
     TileChoice best;
     auto offer = [&](const StepCost& t) {
         if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
         const bool mid = is_mid_tile(t.bm, t.bn);
         if (want_split > 1 && mid) return;  // these split K inside the workgroup only
+        if (t.bn == 320 && (want_split > 1 || !takes_320)) return;
         // (five full row tiles of 64 over a weight of up to 16 MB: callers rely on the 64-row kernel there -- the suite pins
         // it; 320 x 4096 x 4096 takes 17.1 us with 64 x 88 tiles, 12.9 with 96 x 128)
         if (t.ring && !block_scaled && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (want_split > 0 && sp != 1) break;          // the caller's split is applied by the caller
-            if (sp > 1 && (mid || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
+            if (sp > 1 && (mid || t.bn == 320 || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
             const float us = step_cost_us(t, M, N, kblocks, want_split > 0 ? want_split : sp, block_scaled ? 1.f : kRingFewRows) * (sp > 1 ? kSplitMargin : 1.f);
             if (best.bm < 0 || us < best.us) best = TileChoice{t.bm, t.bn, sp, t.ring, us};
         }
@@ -310,15 +312,15 @@ inline float rounds_cost_us(const TileCost& t, int64_t units, int64_t steps) {
 }
 
 Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
-                           const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail);
+                           const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail, bool takes_320);
 
 // The schedule of a dense problem: choose_dense_tile's, and for the per-tensor 64 x 128 tile kernel with fewer workgroups than
 // compute units the tile narrowed (120, 112, ... 72 weight rows) as far as the workgroups still fit one round: what a
 // workgroup of this weight-streaming regime takes in, (64 + columns) x K bytes, shrinks with it, and more compute units
 // take part (28672 x 4096 at M = 64: 224 tiles of 128 columns or 256 of 112).
 Schedule choose_dense(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
-                      const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail) {
-    Schedule s = choose_dense_tile(M, N, K, block_scaled, fast_layout, cfg, ncfg, partial_bytes_avail);
+                      const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail, bool takes_320) {
+    Schedule s = choose_dense_tile(M, N, K, block_scaled, fast_layout, cfg, ncfg, partial_bytes_avail, takes_320);
     if (s.kernel == 1 && !block_scaled && s.waves != 8 && s.bm == 64 && s.bn == 128 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
         const int64_t tiles_m = cdiv(M, 64);
         if (tiles_m * cdiv(N, 128) * s.split_k < 256) {
@@ -329,7 +331,7 @@ Schedule choose_dense(int64_t M, int64_t N, int64_t K, bool block_scaled, bool f
 }
 
 Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
-                           const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail) {
+                           const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail, bool takes_320) {
     Schedule s{0, -1, -1, 1, -1, -1, -1};
     const int want_kernel = cfg_get(cfg, ncfg, TG_CFG_KERNEL);
     const int64_t kblocks = cdiv(K, 128);
@@ -557,11 +559,12 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     s.kernel = 1;
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, block_scaled))) bm = bn = -1;
+    if (bm == 256 && bn == 320 && !(takes_320 && want_split <= 1)) bm = bn = -1;
     int model_split = 1;
     const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && ((bm != 128 && bm != 64) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
     if (want_ring) s.waves = 8;
     if (M > 64) {
-        const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring);
+        const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring, takes_320);
         if (pick.bm > 0) { bm = pick.bm; bn = pick.bn; model_split = pick.split; s.waves = pick.ring ? 8 : -1; }
     } else if (bm < 0) {
         auto tiles = [&](int64_t a, int64_t b) { return cdiv(M, a) * cdiv(N, b); };
@@ -920,7 +923,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         auto worth_it = [&](int64_t full_m, int64_t full_n, int64_t rest_m, int64_t rest_n) {
             if (K < 1024) return true;  // (the model was fitted to K >= 1024)
             const int64_t avail = workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
-            const float whole = pick_tile_by_cost(M, N, kblocks, block_scaled, avail, -1, -1, -1, false).us;
+            const float whole = pick_tile_by_cost(M, N, kblocks, block_scaled, avail, -1, -1, -1, false, block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit).us;
             const float two = pick_tile_by_cost(full_m, full_n, kblocks, block_scaled, avail, 1, 256, 256, false).us +
                               pick_tile_by_cost(rest_m, rest_n, kblocks, block_scaled, avail, -1, -1, -1, false).us;
             return two < whole * 1.05f;  // (the second piece starts while the first one's last tiles run)
@@ -1016,10 +1019,11 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
 
     const bool fast_layout = !trans_a && b_is_nk && (K % 16) == 0 && aligned16(a->ptr) &&
                              aligned16(reinterpret_cast<uint64_t>(Bnt)) && N * K < kOffsetLimit && (!block_scaled || std_blocks);
-    Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free);
+    const bool takes_320 = block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit;
+    Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
     if (static_scratch) {
         // same schedule as tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split
-        const Schedule full = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, INT64_MAX / 2);
+        const Schedule full = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, INT64_MAX / 2, takes_320);
         if (full.split_k != s.split_k)
             return fail(TG_ERR_INVALID, "split-K %d of this problem needs %lld bytes of partial sums, the static scratch buffer has %lld free: "
                         "call tg_fp8_gemm with a workspace, or force a smaller SPLIT_K", full.split_k,
@@ -1121,7 +1125,8 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
         const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
         const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
-        hipError_t e = block_ring ? tg::run_tile_ring_block(s.bm, split, pc, gx, pc.split_k, stream)
+        hipError_t e = block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
+                     : block_ring ? tg::run_tile_ring_block(s.bm, split, pc, gx, pc.split_k, stream)
                      : ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
                      : ordered ? tg::run_tile256(pc, gx, stream)
