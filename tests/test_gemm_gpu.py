@@ -1164,6 +1164,24 @@ def test_moe_layer_same_bits_with_128_and_256_row_blocks(device, dtype, crowded)
     assert torch.equal(*outs)
 
 
+@pytest.mark.parametrize("dtype,bits", [(torch.bfloat16, 7), (torch.float16, 10)])
+@pytest.mark.parametrize("rule,eps", [(0, 0.0), (1, 1e-10), (1, 0.3)])
+def test_quantizer_divides_as_ieee_division_does(device, dtype, bits, rule, eps):
+    """Significands of a group's maximum (all of bf16's 128, 128 spread over f16's 1024) against 127 significands of its elements,
+    at every distance in binades that leaves a code; eps above some maxima, below others.  The codes of the IEEE quotient."""
+    n = 1 << bits
+    amax = 1.0 + (torch.arange(128) * (n // 128) + (n // 256 if bits > 7 else 0)).float() / n
+    frac = 1.0 + (torch.arange(127) * (n // 128) + 1).float() / n
+    x = torch.stack([torch.cat([amax[:, None], torch.minimum(frac[None] * 2.0 ** -d, amax[:, None])], dim=1) for d in range(14)])  # (14, 128, 128)
+    x = (x * torch.where(torch.arange(128) % 2 == 1, -1.0, 1.0) * (0.25 if eps > 0.1 else 1.0)).reshape(14, 128 * 128).to(dtype)
+    q, scales = _lib.fp8_quant_group(x.to(device), 128, eps, rule)
+    f = x.float().reshape(14, 128, 128)
+    s = f.abs().amax(dim=-1).clamp(min=eps) / 448.0
+    want = (f / s[..., None]).clamp(-448.0, 448.0).to(FP8).reshape(14, -1)
+    assert torch.equal(scales.cpu(), s)
+    assert torch.equal(q.cpu().view(torch.uint8), want.view(torch.uint8))
+
+
 def test_ragged_many_experts_and_permutation(device):
     g = _g(31)
     sizes = torch.randint(0, 40, (150,), generator=g).tolist()  # > 64 experts: multi-pass expert search
