@@ -678,16 +678,19 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
     };
     // PAIR main loop.  Half h of step k sits in slot (2k + h) % 3 of the ring.
     //   top of step k : wait for A(k) and H0(k);  barrier (every wave is done with H1(k-1));  request H0(k+1) into the slot H1(k-1)
-    //                   had and a row group of the next chunk of scales;  read A fragments and scales;  MFMAs of H0(k)
-    //   middle        : wait for H1(k);  barrier (every wave holds its A fragments and is done with H0(k));  request A(k+1) into
-    //                   the one A slab and H1(k+1) into the slot H0(k) had;  MFMAs of H1(k)
+    //                   had and a row group of the next chunk of scales;  read A fragments and scales;  barrier (every wave
+    //                   holds its A fragments);  request A(k+1) into the one A slab;  MFMAs of H0(k)
+    //   middle        : wait for H1(k);  barrier (every wave is done with H0(k));  request H1(k+1) into the slot H0(k) had;
+    //                   MFMAs of H1(k)
+    // (Without the second barrier A(k+1) is requested in the middle of the step and has half a step to land: 1 - 3 % slower up to
+    // 100 rows per expert - 1000 tokens 144.8 against 140.4 us - and the same above.)
     // While one workgroup of a compute unit waits, sets up or runs its epilogue, the other one multiplies.  A 64-expert gate/up
     // tile of 16 K steps spends 7.8 k clocks in set-up, 3.3 k per step and 11.8 k in its epilogue, two at a time; the 128 x 256 form
     // of eight waves and 111 KiB that it replaces on large launches ran one at a time.  Gate/up and down GEMM of 64 experts, us,
-    // before -> now: 1024 tokens 93 + 51 -> 88 + 46, 3000 tokens 203 + 107 -> 166 + 96.  Bound by issue and LDS traffic: with
+    // before -> now: 1024 tokens 93 + 51 -> 85 + 45, 3000 tokens 203 + 107 -> 166 + 96.  Bound by issue and LDS traffic: with
     // the weights in the memory-side cache a step still takes 3.1 - 3.2 k clocks (2.6 k for its MFMAs, scale-and-adds and LDS reads alone).
     auto pair_loop = [&](auto ntm_tag) {
-        constexpr int kWaitBut4 = 0x0F70 | 4;
+        constexpr int kWaitBut4 = 0x0F70 | 4, kWaitBut8 = 0x0F70 | 8;
         int slot = 0;
         for (int k = ks; k < ks_end; ++k) {
             const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot1 == 2 ? 0 : slot1 + 1;
@@ -698,10 +701,11 @@ __device__ __forceinline__ void fp8_gemm_tile_body(const GemmParams& p, const in
             issue_half(0, kn, slot2);
             read_a(ntm_tag, sA0);
             read_scales(ntm_tag, k);
-            mma_half(ntm_tag, std::integral_constant<int, 0>{}, sB0 + slot * HALF);
-            __builtin_amdgcn_s_waitcnt(kWaitBut4);  // all but H0(k+1)
             lds_barrier();
             issue_a(kn, sA0);
+            mma_half(ntm_tag, std::integral_constant<int, 0>{}, sB0 + slot * HALF);
+            __builtin_amdgcn_s_waitcnt(kWaitBut8);  // all but H0(k+1) and A(k+1)
+            lds_barrier();
             issue_half(1, kn, slot);
             mma_half(ntm_tag, std::integral_constant<int, 1>{}, sB0 + slot1 * HALF);
             slot = slot2;
