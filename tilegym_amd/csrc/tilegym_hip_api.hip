@@ -1022,9 +1022,11 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     const bool takes_320 = block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit;
     Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
     if (static_scratch) {
-        // same schedule as tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split
+        // same schedule as tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split.  Above 16 rows a split
+        // that nobody asked for is chosen by the cost model among those that fit: the model's constants must not decide which
+        // problems are accepted.
         const Schedule full = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, INT64_MAX / 2, takes_320);
-        if (full.split_k != s.split_k)
+        if (full.split_k != s.split_k && (M <= 16 || cfg_get(cfg, ncfg, TG_CFG_SPLIT_K) > 0))
             return fail(TG_ERR_INVALID, "split-K %d of this problem needs %lld bytes of partial sums, the static scratch buffer has %lld free: "
                         "call tg_fp8_gemm with a workspace, or force a smaller SPLIT_K", full.split_k,
                         (long long)full.split_k * M * N * 4, (long long)ws_free);
