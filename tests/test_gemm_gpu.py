@@ -1278,6 +1278,37 @@ def test_moe_gather_with_holes_in_the_slot_sequence(device, block_m):
         assert torch.equal(q.view(torch.uint8)[kd], q2.view(torch.uint8)[kd]) and torch.equal(s_[kd], s2[kd])
 
 
+@pytest.mark.parametrize("bm,bn", [(96, 128), (160, 128), (192, 128), (256, 320)])
+def test_grouped_gemms_replace_an_override_by_a_tile_that_only_dense_problems_have(device, bm, bn):
+    """Tile overrides that name a dense kernel's tile: the ragged and the gather GEMM run with the tile they pick themselves."""
+    impl = tilegym_amd.backend._REGISTRY["flashinfer.gemm.ragged_block_scaled_bmm"]["hip"]
+    sizes = [300, 0, 17]
+    a, b, a_s, b_s, ptr = _ragged_inputs(sizes, 384, 256, bm)
+    args = [t.to(device) for t in (a, b, a_s, b_s, ptr)] + [max(sizes)]
+    base = impl(*args)
+    want = used("tiled")
+    out = impl(*args, kernel_configs={"BLOCK_M": bm, "BLOCK_N": bn})
+    assert used("tiled") == want
+    assert torch.equal(out, base)
+    check(out, R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr), what=f"ragged, {bm} x {bn} asked for")
+    T, E, N, K, top_k = 200, 3, 384, 256, 2
+    block_m = 192 if bm == 96 else bm                 # (a multiple of the override's rows)
+    g = _g(bm)
+    A, B = fp8_randn((T, K), g).to(device), fp8_randn((E, N, K), g, 0.5).to(device)
+    as_, bs_ = (torch.rand(T, K // 128, generator=g) + 0.1).to(device), (torch.rand(E, N // 128, K // 128, generator=g) + 0.1).to(device)
+    w, ids = W.moe_routing(T, E, top_k, seed=9)
+    sorted_ids, expert_ids, post, _, _ = moe_align_block_size(ids.to(device), block_m, E)
+    outs, cfgs = [], []
+    for kc in (None, {"BLOCK_M": bm, "BLOCK_N": bn}):
+        C = torch.zeros(T * top_k, N, dtype=torch.bfloat16, device=device)
+        _lib.fp8_moe_gemm(C, A, B, as_, bs_, w.to(device), sorted_ids, expert_ids, post, False, top_k, block_m, kc)
+        outs.append(C)
+        cfgs.append(_lib.last_config())
+    assert cfgs[0] == cfgs[1] and torch.equal(*outs)
+    ref = R.ref_fused_moe_gemm(A.cpu(), B.cpu(), as_.cpu(), bs_.cpu(), w, ids, False, top_k)
+    check(outs[1].view(T, top_k, N), ref, what=f"gather, {bm} x {bn} asked for")
+
+
 def test_moe_fc2_shape_top_k_1(device):
     """Second MoE GEMM: activations already expanded per slot (top_k = 1), routed weight applied
     (src/tilegym/ops/moe_interface.py:290-307)."""

@@ -194,6 +194,11 @@ bool tile_exists(int bm, int bn, bool block_scaled) {
     return false;
 }
 
+// Tiles of the expert-grouped block-scaled kernels (run_tile_block_grouped); any other override leaves the choice automatic.
+bool grouped_tile_exists(int bm, int bn) {
+    return (bn == 128 && (bm == 64 || bm == 128)) || (bn == 256 && (bm == 128 || bm == 256));
+}
+
 // Split-K factor: `want` if given, else enough to reach `target_units` units of parallel work;
 // at least `min_steps` K steps per split, and the partial sums must fit the workspace.
 int pick_split(int64_t units, int64_t target_units, int64_t kblocks, int min_steps, int64_t M,
@@ -1270,7 +1275,7 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
         return TG_OK;
     }
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
-    if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, true))) {
+    if (!(bm > 0 && bn > 0 && grouped_tile_exists(bm, bn))) {
         // 64 x 128 tiles below 40 rows per expert (69 us against 80 at 24 rows); from there on, if there are enough of them, pairs
         // of 128 x 256 tiles or 256 x 256 tiles, whichever the padding of the experts' last tiles makes cheaper (64 experts of
         // (2816, 2048), us, 128 x 128 / pairs / 256 x 256: 94 rows 95.5 / 88.5 / 98.1, 188 rows 132 / 119 / 115, 281 rows 183 /
@@ -1350,7 +1355,7 @@ int32_t tg_fp8_moe_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor*
     p.em_capacity = (int)EM;
 
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
-    if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, true) && block_m % bm == 0)) {
+    if (!(bm > 0 && bn > 0 && grouped_tile_exists(bm, bn) && block_m % bm == 0)) {
         if (block_m % 256 == 0 && N >= 256) { bm = 256; bn = 256; }
         else { bm = (block_m % 128 == 0) ? 128 : (block_m % 64 == 0) ? 64 : 0; bn = bm == 128 && N >= 256 && pair_tiles(num_valid, E, cdiv(N, 256)) ? 256 : 128; }
     }
