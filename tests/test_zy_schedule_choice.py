@@ -108,8 +108,12 @@ SMALL_ROW_SHAPES = [(28, 7168, 3584), (28, 3584, 7168), (44, 9216, 4608), (60, 4
                     (52, 2560, 6912), (18, 13824, 5120), (62, 20480, 2560)]
 
 
+# few row tiles above 64 rows: 64 x 64 tiles and 64-row tiles of 72 ... 120 columns against the ring tiles and their splits
+FEW_ROW_TILE_SHAPES = [(94, 9680, 3200), (133, 4096, 4096), (356, 2048, 4864)]
+
+
 @pytest.mark.parametrize("block_scaled", [False, True])
-@pytest.mark.parametrize("M,N,K", MID_SHAPES + SMALL_ROW_SHAPES)
+@pytest.mark.parametrize("M,N,K", MID_SHAPES + SMALL_ROW_SHAPES + FEW_ROW_TILE_SHAPES)
 def test_tile_cost_model_is_close_to_the_best_forced_tile(device, M, N, K, block_scaled):
     entry = tune.tune_shape(M, N, K, block_scaled, device)
     for _ in range(2):  # up to two more looks before calling it a wrong choice

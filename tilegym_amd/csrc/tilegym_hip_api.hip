@@ -215,52 +215,71 @@ int pick_split(int64_t units, int64_t target_units, int64_t kblocks, int min_ste
     return (int)cdiv(kblocks, kps);
 }
 
+// Columns of the per-tensor 64 x 128 tile kernel's tiles: with fewer workgroups than compute units 120, 112, ... 72 weight rows per
+// tile, as far as the workgroups still fit one round.  What a workgroup of this weight-streaming regime takes in, (64 + columns) x
+// K bytes, shrinks with it, and more compute units take part (28672 x 4096 at M = 64: 224 tiles of 128 columns or 256 of 112).
+int deep_tile_cols(int64_t M, int64_t N, int64_t split) {
+    int cols = 128;
+    const int64_t rows = cdiv(M, 64) * split;
+    if (rows * cdiv(N, 128) < 256)
+        for (int bn = 120; bn >= 72 && rows * cdiv(N, bn) <= 256; bn -= 8) cols = bn;
+    return cols;
+}
+
 // Cost model of the LDS-tiled kernels above 64 rows.  A launch takes rounds x (K steps x step + fixed): `fixed` is a tile's
 // set-up, first loads and epilogue in microseconds, `step` the time of a K step, which grows with the share of the chip that is
 // busy (a full chip runs at a lower clock and shares the way to memory): from `first` for a single tile to `full` with a tile on
 // each of the 256 compute units, and, for kernels of which two workgroups share a compute unit (`both` > 0), on to `both`
-// with 512.  Split-K adds the reduction launch.
+// with 512.  A step takes `memory` longer where the weights come from memory: the caches keep those of a few MB between calls, so
+// this sets in at 8 MB and is complete at 20.  Split-K adds the reduction launch.
 //
-// Per-tensor: fitted to 11 000 measurements (480 shapes, M = 65 ... 4096, weights of 1 to 320 MB, every tile x 1 / 2 / 4 / 8
-// splits, launches replayed from a graph over rotating operands).  On the 260 shapes with every split measured the pick is 1.6 %
-// behind the best schedule on average and 11 % ahead of the kernels and the model without the ring tiles (M = 256 ... 1024: 14 %;
-// 777 x 6144 x 4096 32 -> 24 us, 1014 x 5120 x 12288 85 -> 73, 604 x 12288 x 5120 50 -> 42, 154 x 6144 x 4096 17.4 -> 13.2).
-struct StepCost { int bm, bn; bool ring; float first, full, both, fixed; };
-constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.194f, 0.178f, 0.f, 1.66f},   {64, 32, false, 0.222f, 0.215f, 0.f, 1.99f},
-                                        {64, 64, false, 0.298f, 0.338f, 0.f, 3.00f},   {64, 128, false, 0.332f, 0.645f, 0.925f, 3.58f},
-                                        {128, 128, false, 0.473f, 0.843f, 0.978f, 2.98f}, {128, 256, false, 0.874f, 1.036f, 0.f, 3.16f},
-                                        {256, 256, false, 0.968f, 1.333f, 0.f, 7.72f},
-                                        {64, 128, true, 0.304f, 0.527f, 0.f, 1.90f},   {96, 128, true, 0.384f, 0.449f, 0.f, 2.46f},
-                                        {128, 128, true, 0.402f, 0.546f, 0.f, 2.89f},
-                                        {160, 128, true, 0.427f, 0.630f, 0.f, 3.42f},  {160, 192, true, 0.554f, 0.778f, 0.f, 4.31f},
-                                        {192, 192, true, 0.618f, 0.863f, 0.f, 4.90f}};
-// Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  0.9 % behind the best schedule on average, 15 % ahead
-// of the kernels and the model without the ring tiles (485 x 6144 x 4096 28.5 -> 22.8 us, 1571 x 1184 x 5120 35.8 -> 20.1,
-// 100 x 26064 x 6272 47.4 -> 40.9).  Block-scaled 128 x 256 exists and can be forced; it is left out.
-constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f},
-                                          {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f},  {256, 320, false, 1.66f, 2.12f, 0.f, 9.00f},
-                                          {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f},
-                                          {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f},
-                                          {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f}};
-constexpr float kReduceUs = 3.5f, kReduceUsPerMB = 0.30f;
-constexpr float kSplitMargin = 1.04f;  // a split schedule must be predicted this much faster than the best unsplit one
-// few rows over a weight that does not stay in the caches: a ring tile waits for memory (69 x 11264 x 2560: 13.8 us with
-// 96 x 128 tiles where the model says 10.6, 12.3 with 64 x 88)
-constexpr float kRingFewRows = 1.25f;
+// Per-tensor: fitted to 80 000 timings (1791 shapes, M = 65 ... 4096, weights of 1 to 320 MB, every tile x 1 / 2 / 4 / 8 splits,
+// launches replayed from a graph over rotating operands).  The pick is 1.0 % behind the best schedule on average, more than 10 %
+// behind on 45 shapes, at worst 1.49 x (304 x 2848 x 4096: 64 x 64 tiles 16.6 us, 64 x 128 ring 11.1).  Against the kernels and the
+// model without the ring tiles it is 11 % ahead on average, more than 5 % behind on 13 shapes, at worst 1.21 x
+// (100 x 8192 x 8192 27.6 against 22.9).  Fitted to 1461 of the shapes
+// it was 1.2 % behind the best on the other 330, at worst 1.38 x.
+struct StepCost { int bm, bn; bool ring; float first, full, both, fixed, memory; };
+constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.110f, 0.125f, 0.f, 3.394f, 0.008f},  {64, 32, false, 0.144f, 0.198f, 0.f, 3.133f, 0.f},
+                                        {64, 64, false, 0.299f, 0.268f, 0.f, 3.527f, 0.018f}, {64, 128, false, 0.434f, 0.418f, 1.733f, 4.634f, 0.f},
+                                        {128, 128, false, 0.219f, 0.458f, 0.811f, 4.588f, 0.296f}, {128, 256, false, 0.845f, 1.172f, 0.f, 4.156f, 0.260f},
+                                        {256, 256, false, 1.377f, 1.016f, 0.f, 6.470f, 0.039f},
+                                        {64, 128, true, 0.210f, 0.270f, 0.f, 3.672f, 0.145f}, {96, 128, true, 0.255f, 0.288f, 0.f, 4.403f, 0.146f},
+                                        {128, 128, true, 0.219f, 0.396f, 0.f, 4.433f, 0.160f}, {160, 128, true, 0.241f, 0.421f, 0.f, 5.001f, 0.219f},
+                                        {160, 192, true, 0.544f, 0.473f, 0.f, 5.075f, 0.218f}, {192, 192, true, 0.387f, 0.628f, 0.f, 5.953f, 0.200f}};
+// (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
+constexpr float kDeepTileRowsShare = 0.53f;
+// Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.0 % behind the best schedule on average,
+// at worst 1.29 x; 17 % ahead of the kernels and the model without the ring tiles, more than 5 % behind on five, at worst 1.08 x
+// (491 x 20400 x 7296 103.1 against 96.0 us).  Block-scaled 128 x 256 exists and can be forced; it is left out.
+constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f, 0.f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f, 0.f},
+                                          {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f, 0.f},  {256, 320, false, 1.66f, 2.12f, 0.f, 9.00f, 0.f},
+                                          {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f, 0.f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f, 0.f},
+                                          {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f, 0.f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f, 0.f},
+                                          {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f, 0.f}};
+// split_margin: a split schedule must be predicted this much faster than the best unsplit one.  odd_kib: what a ring tile's step takes
+// longer over weights from memory whose rows lie an odd number of KiB apart (224 x 5120 x 5120: 0.47 us a step with 64 x 128 tiles,
+// 0.41 at 25 MB with other K).
+struct TileModel { const StepCost* kinds; int n; float reduce_us, reduce_us_per_mb, split_margin, odd_kib; };
+constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 2.662f, 0.378f, 1.0f, 0.043f};
+constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
-// (few_rows: the factor for ring tiles up to 96 rows)
-float step_cost_us(const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split, float few_rows) {
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * split, places = t.both > 0.f ? 512 : 256;
-    const float steps = (float)cdiv(kblocks, split);
+// (cols: weight rows per tile where they are not the kind's own)
+float step_cost_us(const TileModel& m, const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split, int cols) {
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, cols) * split, places = t.both > 0.f ? 512 : 256;
+    // (the narrow tiles' four waves split K: whole groups of four steps)
+    const float steps = (float)(is_mid_tile(t.bm, t.bn) ? cdiv(kblocks, 4) * 4 : cdiv(kblocks, split));
     const float at_full = t.both > 0.f ? t.both : t.full;
+    const float narrowed = cols == t.bn ? 1.f : kDeepTileRowsShare + (1.f - kDeepTileRowsShare) * (float)cols / (float)t.bn;
+    const float from_memory = std::min(std::max(((float)(N * kblocks * 128) - 8e6f) / 12e6f, 0.f), 1.f);
+    const float memory = from_memory * (t.memory + (t.ring && kblocks % 16 == 8 ? m.odd_kib : 0.f));
     auto part = [&](int64_t n) -> float {
         if (n == 0) return 0.f;
         const float step = n <= 256 ? t.first + (t.full - t.first) * (float)n / 256.f : t.full + (t.both - t.full) * (float)(n - 256) / 256.f;
-        return steps * step + t.fixed;
+        return steps * (step * narrowed + memory) + t.fixed;
     };
-    float us = (float)(tiles / places) * (steps * at_full + t.fixed) + part(tiles % places);
-    if (t.ring && M <= 96) us *= few_rows;
-    if (split > 1) us += kReduceUs + kReduceUsPerMB * (float)(M * N * 4 * split) * 1e-6f;
+    float us = (float)(tiles / places) * (steps * (at_full * narrowed + memory) + t.fixed) + part(tiles % places);
+    if (split > 1) us += m.reduce_us + m.reduce_us_per_mb * (float)(M * N * 4 * split) * 1e-6f;
     return us;
 }
 
@@ -271,6 +290,7 @@ struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us
 // the caller is kept.
 TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
                              int bm, int bn, bool ring, bool takes_320 = false) {
+    const TileModel& m = block_scaled ? kBlockScaledModel : kPerTensorModel;
     TileChoice best;
     auto offer = [&](const StepCost& t) {
         if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
@@ -280,15 +300,17 @@ TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_s
         // (five full row tiles of 64 over a weight of up to 16 MB: callers rely on the 64-row kernel there -- the suite pins
         // it; 320 x 4096 x 4096 takes 17.1 us with 64 x 88 tiles, 12.9 with 96 x 128)
         if (t.ring && !block_scaled && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
+        const bool deep = !block_scaled && !t.ring && t.bm == 64 && t.bn == 128;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (want_split > 0 && sp != 1) break;          // the caller's split is applied by the caller
             if (sp > 1 && (mid || t.bn == 320 || kblocks / sp < 4 || (int64_t)sp * M * N * 4 > partial_bytes_avail)) break;
-            const float us = step_cost_us(t, M, N, kblocks, want_split > 0 ? want_split : sp, block_scaled ? 1.f : kRingFewRows) * (sp > 1 ? kSplitMargin : 1.f);
-            if (best.bm < 0 || us < best.us) best = TileChoice{t.bm, t.bn, sp, t.ring, us};
+            const int split = want_split > 0 ? want_split : sp;
+            const int cols = deep && bm <= 0 ? deep_tile_cols(M, N, split) : t.bn;
+            const float us = step_cost_us(m, t, M, N, kblocks, split, cols) * (sp > 1 ? m.split_margin : 1.f);
+            if (best.bm < 0 || us < best.us) best = TileChoice{t.bm, cols, sp, t.ring, us};
         }
     };
-    if (block_scaled) { for (const StepCost& t : kBlockScaledTiles) offer(t); }
-    else for (const StepCost& t : kPerTensorTiles) offer(t);
+    for (int i = 0; i < m.n; ++i) offer(m.kinds[i]);
     return best;
 }
 
@@ -319,18 +341,12 @@ inline float rounds_cost_us(const TileCost& t, int64_t units, int64_t steps) {
 Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
                            const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail, bool takes_320);
 
-// The schedule of a dense problem: choose_dense_tile's, and for the per-tensor 64 x 128 tile kernel with fewer workgroups than
-// compute units the tile narrowed (120, 112, ... 72 weight rows) as far as the workgroups still fit one round: what a
-// workgroup of this weight-streaming regime takes in, (64 + columns) x K bytes, shrinks with it, and more compute units
-// take part (28672 x 4096 at M = 64: 224 tiles of 128 columns or 256 of 112).
+// The schedule of a dense problem: choose_dense_tile's, the per-tensor 64 x 128 tile kernel's columns as deep_tile_cols has them.
 Schedule choose_dense(int64_t M, int64_t N, int64_t K, bool block_scaled, bool fast_layout,
                       const int32_t* cfg, int32_t ncfg, int64_t partial_bytes_avail, bool takes_320) {
     Schedule s = choose_dense_tile(M, N, K, block_scaled, fast_layout, cfg, ncfg, partial_bytes_avail, takes_320);
     if (s.kernel == 1 && !block_scaled && s.waves != 8 && s.bm == 64 && s.bn == 128 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
-        const int64_t tiles_m = cdiv(M, 64);
-        if (tiles_m * cdiv(N, 128) * s.split_k < 256) {
-            for (int bn = 120; bn >= 72 && tiles_m * cdiv(N, bn) * s.split_k <= 256; bn -= 8) s.bn = bn;
-        }
+        s.bn = deep_tile_cols(M, N, s.split_k);
     }
     return s;
 }
@@ -403,9 +419,9 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                 if (split > 1 && (kblocks / split < 4 || !fits(split))) break;
                 Schedule cand{1, 64, 128, 1, -1, -1, 8};
                 if (split > 1) cand.split_k = pick_split(cdiv(N, 128), 256, kblocks, 4, M, N, partial_bytes_avail, split);
-                constexpr StepCost ring{64, 128, true, 0.338f, 0.736f, 0.f, 2.14f};
+                constexpr StepCost ring{64, 128, true, 0.338f, 0.736f, 0.f, 2.14f, 0.f};
                 // (a split is as many column tiles over a shorter K)
-                offer(cand, step_cost_us(ring, M, cdiv(N, 128) * 128 * cand.split_k, cdiv(kblocks, cand.split_k), 1, 1.f) + reduce(cand.split_k));
+                offer(cand, step_cost_us(kBlockScaledModel, ring, M, cdiv(N, 128) * 128 * cand.split_k, cdiv(kblocks, cand.split_k), 1, 128) + reduce(cand.split_k));
                 if (want_split > 0) break;
             }
         }
