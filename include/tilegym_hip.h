@@ -121,7 +121,9 @@ int32_t tg_fp8_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b,
  * a (K,N) weight go to a TG_STATIC_SCRATCH_BYTES array inside the library's device image (one copy per GPU,
  * held until the process ends).  The call allocates nothing and frees nothing.  A problem whose schedule needs
  * more scratch than the array holds returns TG_ERR_INVALID (the text says how much): call tg_fp8_gemm with a
- * caller-owned workspace for it.  (Above 16 rows a split that cfg[] does not ask for is chosen among those that fit.)  All calls on one GPU share that GPU's array, whatever the stream: calls that
+ * caller-owned workspace for it.  What runs is tg_fp8_gemm's schedule, with its bits (above 64 rows an automatic split never needs
+ * more than the array).  One exception, above 16 rows: a (K,N) weight's copy takes part of the array, and a split that cfg[]
+ * does not ask for is chosen among those that fit the rest.  All calls on one GPU share that GPU's array, whatever the stream: calls that
  * overlap in time on one GPU race on it; calls on one stream never overlap.  Nothing in the array needs to start
  * at zero (no atomics are used), so nothing is cleared between calls.  The first call on a device looks the
  * array's address up (hipGetSymbolAddress); make that call outside graph capture.

@@ -7,6 +7,7 @@ shared by every call on the GPU and keeps the previous call's contents."""
 import pytest
 import torch
 
+from oracle import reference as R
 from tilegym_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +88,34 @@ def test_static_scratch_allocates_nothing(device):
     torch.cuda.synchronize()
     free1, _ = torch.cuda.mem_get_info()
     assert torch.cuda.memory_reserved() == res0 and free1 == free0
+
+
+@pytest.mark.parametrize("M,N,K,block_scaled", [(1500, 3072, 14336, False), (2200, 3072, 14336, False), (1800, 8864, 6784, True)])
+def test_static_scratch_runs_the_schedule_of_the_workspace_form(device, M, N, K, block_scaled):
+    """Problems whose split-K sums could outgrow the 32 MiB array, and one whose columns run in pieces: both entry points decide
+    with the same scratch, so they report the same schedule (number of pieces included) and give the same bits."""
+    a, b, sa, sb = _case(M, N, K, M, device)
+    if block_scaled:
+        g = torch.Generator(device=device).manual_seed(M)
+        sa = torch.rand(M, K // 128, generator=g, device=device) + 0.5
+        sb = torch.rand(-(-N // 128), K // 128, generator=g, device=device) + 0.5
+    c_ref, c_new, _ = _both(a, b, sa, sb, M, N)
+    assert torch.equal(c_ref, c_new)
+
+
+@pytest.mark.parametrize("M,N,K", [(311, 3920, 7808), (183, 1872, 13056), (44, 2880, 10752)])
+def test_static_scratch_takes_a_split_that_fits_beside_the_copy_of_a_weight(device, M, N, K):
+    """Above 16 rows a (K, N) weight's copy leaves only part of the array: an automatic split is chosen among those that fit the rest
+    (a forced one is refused)."""
+    a, b, sa, sb = _case(M, N, K, 9, device, trans_b=False)
+    c = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device)
+    _lib.fp8_gemm_static_scratch(c, a, b, sa, sb, trans_b=False)
+    split = _lib.last_config()["SPLIT_K"]
+    assert split == 1 or split * M * N * 4 + N * K <= _lib.STATIC_SCRATCH_BYTES
+    cols = torch.arange(0, N, 37)
+    ref = R.ref_gemm_per_tensor(a.cpu(), b.cpu()[:, cols].t().contiguous(), sa.cpu(), sb.cpu(), trans_b=True)
+    ok, rep = R.compare_to_oracle(c[:, cols.to(device)], ref, 8.5e-3, 8.5e-3)   # one bf16 ulp (a tie may round the other way)
+    assert ok, rep
+    with pytest.raises(_lib.TileGymHipError) as ei:
+        _lib.fp8_gemm_static_scratch(c, a, b, sa, sb, trans_b=False, kernel_configs={"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": 8})
+    assert ei.value.rc == -6 and "static scratch" in str(ei.value)

@@ -283,6 +283,11 @@ float step_cost_us(const TileModel& m, const StepCost& t, int64_t M, int64_t N, 
     return us;
 }
 
+// Partial sums of an automatic split: no more than the array of tg_fp8_gemm_static_scratch holds, so that both entry points run the
+// same schedule with the same bits.  (Ten of 1791 measured per-tensor shapes change, none of 585 block-scaled ones: eight become 5 to
+// 15 % faster -- 2048 x 4096 x 14336 113 -> 99 us, 777 x 3584 x 18944 75 -> 65 -- and two 3 % slower, 194 x 24608 x 10624 87.1 -> 89.7.)
+constexpr int64_t kAutoPartialBytes = TG_STATIC_SCRATCH_BYTES;
+
 // A tile and a split, with what the model says they take.
 struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us = 0.f; };
 
@@ -292,6 +297,7 @@ TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_s
                              int bm, int bn, bool ring, bool takes_320 = false) {
     const TileModel& m = block_scaled ? kBlockScaledModel : kPerTensorModel;
     TileChoice best;
+    if (want_split <= 0 && partial_bytes_avail > kAutoPartialBytes) partial_bytes_avail = kAutoPartialBytes;
     auto offer = [&](const StepCost& t) {
         if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
         const bool mid = is_mid_tile(t.bm, t.bn);
@@ -902,6 +908,8 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         if (!aligned16(workspace->ptr)) return fail(TG_ERR_INVALID, "workspace must be 16-byte aligned");
     }
     if (M == 0 || N == 0) return TG_OK;
+    // scratch memory of this call: the caller's workspace or the library's array
+    const int64_t scratch_bytes = static_scratch ? (int64_t)TG_STATIC_SCRATCH_BYTES : workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
 
     // ---- column chunks.  The columns of C (rows of an (N, K) weight) can be computed in pieces, each a call of its own on
     // the same stream and workspace; the pieces take C's real row stride as an argument.
@@ -943,10 +951,9 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         // (only where the model says that no single launch is as fast)
         auto worth_it = [&](int64_t full_m, int64_t full_n, int64_t rest_m, int64_t rest_n) {
             if (K < 1024) return true;  // (the model was fitted to K >= 1024)
-            const int64_t avail = workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
-            const float whole = pick_tile_by_cost(M, N, kblocks, block_scaled, avail, -1, -1, -1, false, block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit).us;
-            const float two = pick_tile_by_cost(full_m, full_n, kblocks, block_scaled, avail, 1, 256, 256, false).us +
-                              pick_tile_by_cost(rest_m, rest_n, kblocks, block_scaled, avail, -1, -1, -1, false).us;
+            const float whole = pick_tile_by_cost(M, N, kblocks, block_scaled, scratch_bytes, -1, -1, -1, false, block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit).us;
+            const float two = pick_tile_by_cost(full_m, full_n, kblocks, block_scaled, scratch_bytes, 1, 256, 256, false).us +
+                              pick_tile_by_cost(rest_m, rest_n, kblocks, block_scaled, scratch_bytes, -1, -1, -1, false).us;
             return two < whole * 1.05f;  // (the second piece starts while the first one's last tiles run)
         };
         if (total > 256 && total * 100 < rounds * 256 * 80) {
@@ -1001,12 +1008,11 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     hipStream_t stream = reinterpret_cast<hipStream_t>(hip_stream);
 
     // ---- workspace carving: [split-K partial sums ...][optional K-contiguous copy of B]
-    int64_t ws_bytes = workspace ? numel(workspace) * elem_size(workspace->dtype) : 0;
+    const int64_t ws_bytes = scratch_bytes;
     uint8_t* ws = workspace ? reinterpret_cast<uint8_t*>(workspace->ptr) : nullptr;
     if (static_scratch) {
         const hipError_t e = scratch_address(device_id, &ws);
         if (e != hipSuccess) return fail(TG_ERR_DEVICE, "cannot locate the static scratch buffer on device %d: %s", device_id, hipGetErrorString(e));
-        ws_bytes = TG_STATIC_SCRATCH_BYTES;
         const int64_t copy_bytes = (!trans_b && !trans_a && cfg_get(cfg, ncfg, TG_CFG_KERNEL) != 0) ? (N * K + 255) / 256 * 256 : 0;
         if (copy_bytes > ws_bytes)
             return fail(TG_ERR_INVALID, "the K-contiguous copy of a (K,N) weight needs %lld bytes, the static scratch buffer holds %lld: "
@@ -1043,11 +1049,13 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     const bool takes_320 = block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit;
     Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
     if (static_scratch) {
-        // same schedule as tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split.  Above 16 rows a split
-        // that nobody asked for is chosen by the cost model among those that fit: the model's constants must not decide which
-        // problems are accepted.
+        // The schedule of tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split.  (Above 64 rows an
+        // automatic split stays within the array, see kAutoPartialBytes.)  One exception, above 16 rows: a (K, N) weight's copy
+        // takes part of the array, and a split that nobody asked for is chosen among those that fit the rest -- the constants of
+        // the cost models must not decide which of these problems are accepted.
         const Schedule full = choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, INT64_MAX / 2, takes_320);
-        if (full.split_k != s.split_k && (M <= 16 || cfg_get(cfg, ncfg, TG_CFG_SPLIT_K) > 0))
+        const bool among_fitting = M > 16 && !trans_b && cfg_get(cfg, ncfg, TG_CFG_SPLIT_K) <= 0;
+        if (full.split_k != s.split_k && !among_fitting)
             return fail(TG_ERR_INVALID, "split-K %d of this problem needs %lld bytes of partial sums, the static scratch buffer has %lld free: "
                         "call tg_fp8_gemm with a workspace, or force a smaller SPLIT_K", full.split_k,
                         (long long)full.split_k * M * N * 4, (long long)ws_free);
