@@ -160,12 +160,27 @@ def test_per_tensor_mid_tiles(device, bm, bn, M, N, K):
 def test_mid_tiles_are_the_default_for_small_weights(device):
     g = _g(8)
     b = fp8_randn((4096, 4096), g, 0.02)
-    for M, want in ((32, (32, 32)), (64, (32, 32)), (128, (64, 32)), (192, (64, 64)), (256, (64, 64)), (320, (64, 88))):   # (320 rows: five row tiles x 47 tiles of 88 columns fit one round, 32 of 128 leave 96 compute units idle)
+    for M, want in ((32, (32, 32)), (64, (32, 32)), (128, (64, 32)), (192, (64, 64)), (256, (64, 64))):
         a = fp8_randn((M, 4096), g)
         out = matmul(a.to(device), b.to(device), trans_b=True, scale_a=0.01, scale_b=0.02, out_dtype=torch.bfloat16)
         cfg = used("tiled")
         assert (cfg["BLOCK_M"], cfg["BLOCK_N"]) == want, (M, cfg)
         check(out, R.ref_gemm_per_tensor(a, b, 0.01, 0.02, trans_b=True), what=f"M={M} default")
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (2048, 4096), (2048, 8192), (3072, 4096)])
+def test_a_full_last_row_tile_changes_no_schedule(device, N, K):
+    """319 and 320 rows are five row tiles of 64 either way (four of 96, three of 128, two of 160 and 192): the same kernel runs, and the
+    first 319 rows get the same bits."""
+    g = _g(320)
+    a, b = fp8_randn((320, K), g), fp8_randn((N, K), g, 0.02)
+    outs, cfgs = [], []
+    for M in (319, 320):
+        outs.append(matmul(a[:M].to(device), b.to(device), trans_b=True, scale_a=0.01, scale_b=0.02, out_dtype=torch.bfloat16))
+        cfgs.append(used("tiled"))
+    assert cfgs[0] == cfgs[1]
+    assert torch.equal(outs[0], outs[1][:319])
+    check(outs[1], R.ref_gemm_per_tensor(a, b, 0.01, 0.02, trans_b=True), what=f"320 x {N} x {K}")
 
 
 def test_weights_of_2_gib_and_more_run_in_column_chunks(device):

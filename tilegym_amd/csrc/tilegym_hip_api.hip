@@ -303,9 +303,6 @@ TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_s
         const bool mid = is_mid_tile(t.bm, t.bn);
         if (want_split > 1 && mid) return;  // these split K inside the workgroup only
         if (t.bn == 320 && (want_split > 1 || !takes_320)) return;
-        // (five full row tiles of 64 over a weight of up to 16 MB: callers rely on the 64-row kernel there -- the suite pins
-        // it; 320 x 4096 x 4096 takes 17.1 us with 64 x 88 tiles, 12.9 with 96 x 128)
-        if (t.ring && !block_scaled && bm <= 0 && M == 320 && N * kblocks * 128 <= ((int64_t)16 << 20)) return;
         const bool deep = !block_scaled && !t.ring && t.bm == 64 && t.bn == 128;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (want_split > 0 && sp != 1) break;          // the caller's split is applied by the caller
