@@ -637,28 +637,36 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
 }
 
 // A per-tensor (K, N) weight: whether the narrow tiles read it as it lies, and with which tile; else it is copied to (N, K)
-// first and any kernel takes it.  A direct tile's K step takes 0.39 - 0.45 us whatever the grid; the copy costs 5 us + 0.40 us per
-// MB on top of the cost model's GEMM above 64 rows, and up to 64 rows copy and GEMM together 7 us + 0.5 us per MB.  Above 64 rows
-// the line was fitted to 110 shapes (65 ... 512 rows) with both ways measured: 1.6 % behind the better way on average (worst 1.4 x).
-// Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 us against 65.4; 1024 x 1024: 5.2 against 7.7; 1264 x 1152 at
-// M = 275: 6.3 against 9.3), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied), and so are
-// most from 300 rows on.
-constexpr TileCost kKnTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
-constexpr float kKnMargin = 0.9f, kCopyUs = 5.0f, kCopyUsPerMB = 0.40f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
+// first and any kernel takes it.  Up to 64 rows a direct tile's K step takes 0.39 - 0.45 us whatever the grid, and copy and GEMM together
+// 7 us + 0.5 us per MB.  Above, the direct tiles have step costs like the kernels of the race, and the copy costs 5.4 us + 0.47 us per
+// MB on top of the race's GEMM: fitted to 724 shapes (65 ... 512 rows) with both ways measured, 0.9 % behind the better way on
+// average, at worst 1.29 x (96 x 2048 x 7168); with one step cost for every grid 5.6 % and 1.74 x.
+// Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 us against 65.4; 1024 x 1024: 5.2 against 7.7; 1888 x 5504 at
+// M = 91: 12.2 against 21.2), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied), and so are
+// most from 300 rows on (2672 x 7424 at M = 485: 31.8 against 46.6).
+constexpr TileCost kKnFewRowsTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
+constexpr StepCost kKnTiles[] = {{32, 32, false, 0.202f, 0.278f, 0.f, 1.484f, 0.020f}, {64, 32, false, 0.381f, 0.327f, 0.f, 1.631f, 0.006f},
+                                 {64, 64, false, 0.357f, 0.455f, 0.f, 1.815f, 0.043f}};
+constexpr float kCopyUs = 5.44f, kCopyUsPerMB = 0.471f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
 bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, int* bm, int* bn) {
     if (M > 512 || N % 16 != 0 || K % 128 != 0) return false;
     const int64_t kblocks = K / 128;
     const float mb = (float)(N * K) * 1e-6f;
     float best = 0.f;
     *bm = -1;
-    for (const TileCost& t : kKnTiles) {
-        const float tiles = (float)(cdiv(M, t.bm) * cdiv(N, t.bn));   // one workgroup per compute unit
-        const float us = (tiles > 256.f ? tiles / 256.f : 1.f) * ((float)kblocks * t.alone + t.fixed);
-        if (*bm < 0 || us < best) { best = us; *bm = t.bm; *bn = t.bn; }
+    auto offer = [&](int tile_m, int tile_n, float us) {
+        if (*bm < 0 || us < best) { best = us; *bm = tile_m; *bn = tile_n; }
+    };
+    if (M <= 64) {
+        for (const TileCost& t : kKnFewRowsTiles) {
+            const float tiles = (float)(cdiv(M, t.bm) * cdiv(N, t.bn));   // one workgroup per compute unit
+            offer(t.bm, t.bn, (tiles > 256.f ? tiles / 256.f : 1.f) * ((float)kblocks * t.alone + t.fixed));
+        }
+        return best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
     }
-    if (M <= 64) return best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
+    for (const StepCost& t : kKnTiles) offer(t.bm, t.bn, step_cost_us(kPerTensorModel, t, M, N, kblocks, 1, t.bn));
     const float nk = pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us;
-    return best * kKnMargin <= nk + kCopyUs + kCopyUsPerMB * mb;
+    return best <= nk + kCopyUs + kCopyUsPerMB * mb;
 }
 
 // ---- expert-grouped block-scaled GEMMs: 256 x 256 tiles, or 128 x 256 tiles of which two share a compute unit (PAIR in
