@@ -38,13 +38,6 @@ constexpr int64_t kQuantFewWorkgroups = 1 << 13;
 
 enum QuantRule { QUANT_ZERO_TO_ONE = 0, QUANT_EPS = 1, QUANT_EPS_POW2 = 2 };
 
-// LPG lanes per group (group size 8 * LPG).  STRIDED: the scale of group j of row r goes to
-// scales[r * s_row + j * s_col] (groups < 2^31); otherwise to scales[g].
-// I8: the destination is int8 instead of e4m3 (per_token_group_quant_8bit with dst_dtype=torch.int8,
-// tests/suites/flashinfer/test_per_token_group_quant_8bit.py:41-68): scale = amax / 127, q = the quotient clamped to
-// [-128, 127] and converted as a float -> integer cast does (toward zero).
-// (body of 256-thread block `block`, thread `tid` of it: the kernel below runs it as such, the MoE preparation kernel
-// runs four such blocks per 1024-thread workgroup)
 // Maximum over the LPG (2, 4, 8, 16) neighbouring lanes of a group, in every one of them: lane permutations inside the vector
 // instruction, no trip through the LDS crossbar.
 template <int CTRL>
@@ -78,6 +71,13 @@ __device__ __forceinline__ float short_quotient(float a, float s, float r) {
     return __builtin_fmaf(-__builtin_fmaf(s, t, -a), r, t);
 }
 
+// LPG lanes per group (group size 8 * LPG).  STRIDED: the scale of group j of row r goes to
+// scales[r * s_row + j * s_col] (groups < 2^31); otherwise to scales[g].
+// I8: the destination is int8 instead of e4m3 (per_token_group_quant_8bit with dst_dtype=torch.int8,
+// tests/suites/flashinfer/test_per_token_group_quant_8bit.py:41-68): scale = amax / 127, q = the quotient clamped to
+// [-128, 127] and converted as a float -> integer cast does (toward zero).
+// (body of 256-thread block `block`, thread `tid` of it: the kernel below runs it as such, the MoE preparation kernel
+// runs four such blocks per 1024-thread workgroup)
 template <typename T, int LPG, bool STRIDED, bool I8, int G = kQuantGroupsPerLane>
 __device__ __forceinline__ void act_quant_group_body(const T* __restrict__ x, uint8_t* __restrict__ q,
                                                      float* __restrict__ scales, int64_t groups, float eps,
