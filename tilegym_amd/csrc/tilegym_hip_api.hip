@@ -233,20 +233,21 @@ int deep_tile_cols(int64_t M, int64_t N, int64_t split) {
 // with 512.  A step takes `memory` longer where the weights come from memory: the caches keep those of a few MB between calls, so
 // this sets in at 8 MB and is complete at 20.  Split-K adds the reduction launch.
 //
-// Per-tensor: fitted to 80 000 timings (1791 shapes, M = 65 ... 4096, weights of 1 to 320 MB, every tile x 1 / 2 / 4 / 8 splits,
-// launches replayed from a graph over rotating operands).  The pick is 1.0 % behind the best schedule on average, more than 10 %
-// behind on 45 shapes, at worst 1.49 x (304 x 2848 x 4096: 64 x 64 tiles 16.6 us, 64 x 128 ring 11.1).  Against the kernels and the
-// model without the ring tiles it is 11 % ahead on average, more than 5 % behind on 13 shapes, at worst 1.21 x
-// (100 x 8192 x 8192 27.6 against 22.9).  Fitted to 1461 of the shapes
-// it was 1.2 % behind the best on the other 330, at worst 1.38 x.
+// Per-tensor: fitted to 160 000 timings (1780 shapes, M = 65 ... 4096, weights of 1 to 320 MB, every tile x 1 / 2 / 4 / 8 splits),
+// replayed from a graph once over three sets of operands, which the memory-side cache holds up to some 80 MB each, and once over
+// 768 MB of them: the constants stand for the geometric mean of the two, since the library cannot know which it is.  The pick is
+// 1.3 % behind the best schedule on average with weights from memory and 0.9 % with cached ones, more than 10 % behind on 67 and 41
+// shapes, at worst 1.43 x (75 x 1968 x 7424) and 1.38 x (233 x 3952 x 5632); fitted to three quarters of the shapes 1.5 % and 1.3 % on the
+// others.  Against the kernels and the model without the ring tiles it is 12 % and 17 % ahead on average, more than 5 % behind on 39 and
+// 13 shapes, at worst 1.17 x (320 x 3072 x 8192 22.8 against 19.5 us) and 1.18 x (133 x 1024 x 8192 10.6 against 9.0).
 struct StepCost { int bm, bn; bool ring; float first, full, both, fixed, memory; };
-constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.110f, 0.125f, 0.f, 3.394f, 0.008f},  {64, 32, false, 0.144f, 0.198f, 0.f, 3.133f, 0.f},
-                                        {64, 64, false, 0.299f, 0.268f, 0.f, 3.527f, 0.018f}, {64, 128, false, 0.434f, 0.418f, 1.733f, 4.634f, 0.f},
-                                        {128, 128, false, 0.219f, 0.458f, 0.811f, 4.588f, 0.296f}, {128, 256, false, 0.845f, 1.172f, 0.f, 4.156f, 0.260f},
-                                        {256, 256, false, 1.377f, 1.016f, 0.f, 6.470f, 0.039f},
-                                        {64, 128, true, 0.210f, 0.270f, 0.f, 3.672f, 0.145f}, {96, 128, true, 0.255f, 0.288f, 0.f, 4.403f, 0.146f},
-                                        {128, 128, true, 0.219f, 0.396f, 0.f, 4.433f, 0.160f}, {160, 128, true, 0.241f, 0.421f, 0.f, 5.001f, 0.219f},
-                                        {160, 192, true, 0.544f, 0.473f, 0.f, 5.075f, 0.218f}, {192, 192, true, 0.387f, 0.628f, 0.f, 5.953f, 0.200f}};
+constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.106f, 0.122f, 0.f, 3.296f, 0.008f}, {64, 32, false, 0.169f, 0.192f, 0.f, 2.825f, 0.002f},
+                                        {64, 64, false, 0.175f, 0.271f, 0.f, 3.494f, 0.035f}, {64, 128, false, 0.623f, 0.752f, 1.153f, 3.531f, 0.001f},
+                                        {128, 128, false, 0.215f, 0.854f, 0.944f, 5.766f, 0.081f}, {128, 256, false, 0.552f, 1.278f, 0.f, 5.713f, 0.083f},
+                                        {256, 256, false, 1.297f, 1.009f, 0.f, 11.556f, 0.012f},
+                                        {64, 128, true, 0.219f, 0.313f, 0.f, 3.087f, 0.060f}, {96, 128, true, 0.371f, 0.293f, 0.f, 3.990f, 0.102f},
+                                        {128, 128, true, 0.344f, 0.387f, 0.f, 5.394f, 0.095f}, {160, 128, true, 0.496f, 0.552f, 0.f, 4.331f, 0.075f},
+                                        {160, 192, true, 0.441f, 0.667f, 0.f, 6.211f, 0.064f}, {192, 192, true, 0.628f, 0.675f, 0.f, 8.253f, 0.061f}};
 // (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
 constexpr float kDeepTileRowsShare = 0.53f;
 // Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.0 % behind the best schedule on average,
@@ -258,10 +259,10 @@ constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879
                                           {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f, 0.f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f, 0.f},
                                           {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f, 0.f}};
 // split_margin: a split schedule must be predicted this much faster than the best unsplit one.  odd_kib: what a ring tile's step takes
-// longer over weights from memory whose rows lie an odd number of KiB apart (224 x 5120 x 5120: 0.47 us a step with 64 x 128 tiles,
-// 0.41 at 25 MB with other K).
+// longer over weights from memory whose rows lie an odd number of KiB apart (64 x 128 tiles over 5120 x 5120 from memory 0.47 - 0.50 us a
+// step, over other weights of 25 MB 0.41).
 struct TileModel { const StepCost* kinds; int n; float reduce_us, reduce_us_per_mb, split_margin, odd_kib; };
-constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 2.662f, 0.378f, 1.0f, 0.043f};
+constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 3.272f, 0.316f, 1.0f, 0.018f};
 constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
 // (cols: weight rows per tile where they are not the kind's own)
@@ -638,16 +639,16 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
 
 // A per-tensor (K, N) weight: whether the narrow tiles read it as it lies, and with which tile; else it is copied to (N, K)
 // first and any kernel takes it.  Up to 64 rows a direct tile's K step takes 0.39 - 0.45 us whatever the grid, and copy and GEMM together
-// 7 us + 0.5 us per MB.  Above, the direct tiles have step costs like the kernels of the race, and the copy costs 5.4 us + 0.47 us per
-// MB on top of the race's GEMM: fitted to 724 shapes (65 ... 512 rows) with both ways measured, 0.9 % behind the better way on
-// average, at worst 1.29 x (96 x 2048 x 7168); with one step cost for every grid 5.6 % and 1.74 x.
+// 7 us + 0.5 us per MB.  Above, the direct tiles have step costs like the kernels of the race, and the copy costs 4.1 us + 0.47 us per
+// MB on top of the race's GEMM: fitted to 718 shapes (65 ... 512 rows) with both ways measured, cached and from memory: 0.6 % behind the
+// better way on average in either, at worst 1.21 x (with one step cost for every grid 5.5 - 6.1 % and 1.75 x).
 // Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 us against 65.4; 1024 x 1024: 5.2 against 7.7; 1888 x 5504 at
 // M = 91: 12.2 against 21.2), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied), and so are
 // most from 300 rows on (2672 x 7424 at M = 485: 31.8 against 46.6).
 constexpr TileCost kKnFewRowsTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
-constexpr StepCost kKnTiles[] = {{32, 32, false, 0.202f, 0.278f, 0.f, 1.484f, 0.020f}, {64, 32, false, 0.381f, 0.327f, 0.f, 1.631f, 0.006f},
-                                 {64, 64, false, 0.357f, 0.455f, 0.f, 1.815f, 0.043f}};
-constexpr float kCopyUs = 5.44f, kCopyUsPerMB = 0.471f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
+constexpr StepCost kKnTiles[] = {{32, 32, false, 0.236f, 0.232f, 0.f, 1.174f, 0.f}, {64, 32, false, 0.358f, 0.321f, 0.f, 1.139f, 0.f},
+                                 {64, 64, false, 0.298f, 0.426f, 0.f, 1.862f, 0.024f}};
+constexpr float kCopyUs = 4.11f, kCopyUsPerMB = 0.466f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
 bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, int* bm, int* bn) {
     if (M > 512 || N % 16 != 0 || K % 128 != 0) return false;
     const int64_t kblocks = K / 128;
