@@ -4,16 +4,18 @@
 // 4096 x 5120 is 320 tiles of 256 x 256 (a full round of 256 compute units and a quarter of one) and exactly 256 of 256 x 320.
 // Schedule, slab layout, swizzles, fragment addressing and arithmetic are those of
 // fp8_gemm_tile_kernel<256, 256, 4, 2, true, GROUP_DENSE, false> (see there): identical results.  What differs:
-//   * a wave's part is 64 x 160: 160 accumulator registers.  To stay inside the
-//     register file a wave keeps one per-lane offset
-//     per operand (the pass of the loads is in the scalar offset; rows past the end of an operand read zeros through sized
-//     descriptors and are never stored);
+//   * a wave's part is 64 x 160: 160 accumulator registers.  To stay inside the register file (255 of 256) a wave keeps one per-lane
+//     offset per operand, the pass of the loads being in the scalar offset.  There is no register left to clamp the rows of a last
+//     tile, and the descriptors are not sized to the operands: what keeps every load inside them is that the last row and column
+//     tiles are moved back to end with the operands (and store only what is theirs), which takes M >= 256, N >= 320 and
+//     N % 32 == 0 (bs320_takes; a wave's edge between two weight scales lies at a multiple of 32 columns);
 //   * the two stages take 144 KiB of LDS and the activation scales the other 16.  The weight scales come through scalar loads, one
 //     step ahead.  A wave's 160 columns lie in two blocks of 128: the pairs of column tiles in front of the boundary take
 //     the first block's scale, the others the second one's.
-// Bound by power and issue like the 256 x 256 form; it moves a tenth fewer bytes to LDS per MFMA.  Quantizer and GEMM, us, before
-// (256 x 256 tiles, in two pieces where the last round was mostly empty) -> now: 4096 x 5120 x 12288 288 -> 266,
-// 4096 x 5120 x 4096 103 -> 90, 3000 x 6400 x 7168 177 -> 149, 8192 x 5120 x 5120 255 -> 238.  With whole rounds of 256 x 256 tiles
+// Bound by power and issue like the 256 x 256 form (1.8 GHz on average over the launch, 0.57 of the matrix slots: the counters in
+// profiles/ring_pair_bs320_pmc.txt); it moves a tenth fewer bytes to LDS per MFMA.  Quantizer and GEMM, us, side by side with the 256 x 256
+// tiles, in two pieces where the last round was mostly empty, and the quantizer before it: 4096 x 5120 x 12288 278 -> 250,
+// 4096 x 5120 x 4096 99 -> 85, 3000 x 6400 x 7168 168 -> 138, 8192 x 5120 x 5120 240 -> 219.  With whole rounds of 256 x 256 tiles
 // that form is ahead (4096 x 12288 x 5120: 222 against 274 for the GEMM): the cost model decides.
 #pragma once
 

@@ -12,15 +12,18 @@
 // step k+1 is visible and step k's stage is free, and the fragments of step k+1 are read while those last MFMAs run (activation
 // fragments into the registers that a row group's last MFMA releases, weight fragments over three or four rotating sets).
 //
-// Bound on a full chip by power, that is by bytes moved per MFMA: 240 tiles of 160 x 128 run at 1.3 - 1.5 GHz with 82 % of the
-// matrix pipes' slots in use, 64 of them at 2.25 GHz (clock stamps); hence the 192 x 192 tile for larger problems, which moves
-// a quarter less.  Measured (us, before -> now): 777 x 6144 x 4096 27.6 -> 20.9, 1400 x 12288 x 5120 102 -> 79,
-// 1014 x 5120 x 12288 85 -> 73, 512 x 4096 x 4096 18.1 -> 14.0.  A fifth kind of wave that touched the lines of steps further
-// ahead to have them in the caches: no faster (23.8 against 25.2 and 54.3 against 53.0 us), not kept.
+// Bound on a full chip by power, that is by bytes moved per MFMA: a 160 x 128 tile of 32 steps takes 38 thousand cycles, 0.53 of them
+// with the matrix pipes busy, whether 64 or 240 compute units work; 64 tiles take 18.2 us, 240 tiles of zeros 19.6, 240 of random data
+// 22.2 - 22.9 (2.1, 1.94 and 1.69 GHz on average: the counters in profiles/ring_pair_bs320_pmc.txt).  Hence the 192 x 192 tile for larger
+// problems, which moves a quarter less.  Measured side by side with the choice among the other kernels (us): 777 x 6144 x 4096 26.9 -> 19.9,
+// 1400 x 12288 x 5120 101 -> 78, 1014 x 5120 x 12288 83 -> 61, 512 x 4096 x 4096 17.8 -> 12.8, 185 x 6144 x 4096 16.9 -> 11.8.  A fifth kind
+// of wave that touched the lines of steps further ahead to have them in the caches: no faster (23.8 against 25.2 and 54.3 against
+// 53.0 us), not kept.
 //
 // Block scales: a step's products are scaled and added as in fp8_gemm_tile.h.  The loading waves bring the activation scales
 // too, in chunks of eight K steps spread over the steps of the chunk before; the scales of step k+1 are read behind the barrier of
-// step k.  485 x 6144 x 4096 28.5 -> 22.8 us, 174 x 3520 x 4992 19.2 -> 15.5, 62 x 6144 x 4096 15.7 -> 12.6.
+// step k.  With the quantizer 485 x 6144 x 4096 30.6 -> 23.6 us, 174 x 3520 x 4992 21.4 -> 18.0,
+// 62 x 6144 x 4096 18.4 -> 15.4.
 //
 // Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as
 // fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results.

@@ -250,7 +250,7 @@ constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.106f, 0.122f, 0.f, 3.2
                                         {160, 192, true, 0.441f, 0.667f, 0.f, 6.211f, 0.064f}, {192, 192, true, 0.628f, 0.675f, 0.f, 8.253f, 0.061f}};
 // (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
 constexpr float kDeepTileRowsShare = 0.53f;
-// Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.0 % behind the best schedule on average,
+// Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.1 % behind the best schedule on average,
 // at worst 1.29 x; 17 % ahead of the kernels and the model without the ring tiles, more than 5 % behind on five, at worst 1.08 x
 // (491 x 20400 x 7296 103.1 against 96.0 us).  Block-scaled 128 x 256 exists and can be forced; it is left out.
 constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f, 0.f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f, 0.f},
@@ -285,8 +285,8 @@ float step_cost_us(const TileModel& m, const StepCost& t, int64_t M, int64_t N, 
 }
 
 // Partial sums of an automatic split: no more than the array of tg_fp8_gemm_static_scratch holds, so that both entry points run the
-// same schedule with the same bits.  (Ten of 1791 measured per-tensor shapes change, none of 585 block-scaled ones: eight become 5 to
-// 15 % faster -- 2048 x 4096 x 14336 113 -> 99 us, 777 x 3584 x 18944 75 -> 65 -- and two 3 % slower, 194 x 24608 x 10624 87.1 -> 89.7.)
+// same schedule with the same bits.  (Six of 1780 measured per-tensor shapes change, none of 585 block-scaled ones: four become 4 to
+// 21 % faster -- 1024 x 8192 x 8192 79 -> 69 us from memory, 76 -> 60 cached -- and two 1 to 6 % slower, 194 x 24608 x 10624 87 -> 90.)
 constexpr int64_t kAutoPartialBytes = TG_STATIC_SCRATCH_BYTES;
 
 // A tile and a split, with what the model says they take.

@@ -4,7 +4,7 @@
     TILEGYM_HIP_TUNE=tune.json python my_decode_loop.py
 
 The library picks its schedules in O(1): fixed rules up to 16 rows, cost models over kernels, tiles and split-K factors
-above (``choose_dense`` in csrc/tilegym_hip_api.hip; their constants were fitted to tables this module wrote), and a test
+above (``choose_dense`` in csrc/tilegym_hip_api.hip; their constants were fitted to timings taken as this module takes them), and a test
 holds the choice within 25 % of the best forced schedule on shapes outside the fit (measured: 1 - 2 % on average).
 For a caller who wants the last few percent on the shapes of one model, this module does what the reference's
 exhaustive search does (src/tilegym/ops/cutile/matmul.py:327-418): it times the candidates on this GPU -- weights
