@@ -576,6 +576,26 @@ def test_ring_tiles(device, bm, bn, dm, dn, K, split):
             check(out, R.ref_gemm_per_tensor(a, b, 0.37, 0.5, trans_b=True), what=f"ring {bm}x{bn} M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("bm,bn", [(64, 32), (32, 64), (64, 64), (32, 128), (256, 128)])
+@pytest.mark.parametrize("dm,dn,K,split", [(0, 0, 128, 1), (-1, -8, 1664, 1), (1, 8, 384, 2), (17, -3, 640, 1), (-15, 72, 2176, 3)])
+def test_ring_tiles_narrow_and_tall(device, bm, bn, dm, dn, K, split):
+    """The same for the tiles of 32 and 64 columns, 32 rows and 256 rows (13 K steps: one more than the twelve stages; one wave
+    column, one or two column tiles per wave)."""
+    test_ring_tiles(device, bm, bn, dm, dn, K, split)
+
+
+@pytest.mark.parametrize("M,N,K,want", [(24, 12288, 1280, (32, 64)), (33, 12288, 1280, (64, 64)), (256, 4096, 1280, (64, 64)), (128, 4096, 1408, (64, 32)),
+                                        (256, 28672, 1280, (256, 128))])
+def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
+    g = _g(M + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.02)
+    out = matmul(a.to(device), b.to(device), trans_b=True, scale_a=0.01, scale_b=0.02, out_dtype=torch.float16)
+    cfg = used("tiled")
+    assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["WAVES"]) == want + (8,), cfg
+    cols = torch.arange(0, N, 13)
+    check(out[:, cols.to(device)], R.ref_gemm_per_tensor(a, b[cols], 0.01, 0.02, trans_b=True, out_dtype=torch.float16), what=f"M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("bm", [64, 96, 128, 160, 192])
 @pytest.mark.parametrize("dm,N,K,split", [(0, 256, 128, 1), (-1, 120, 1024, 1), (1, 136, 1152, 2), (17, 257, 2176, 1), (-33, 384, 2304, 2)])
 def test_ring_tiles_block_scaled(device, bm, dm, N, K, split):
@@ -2043,6 +2063,31 @@ def test_kn_weights_read_as_they_lie(device, M, N, K, out_dtype):
     assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
     if out_dtype is torch.bfloat16:
         check(got, R.ref_gemm_per_tensor(a, b, 0.25, 0.5, trans_b=True))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 1280), (17, 1040, 1408), (50, 1040, 5120), (33, 12304, 1280), (60, 20496, 1280), (70, 2064, 1664), (129, 6160, 1280),
+                                   (200, 8208, 2176), (300, 4112, 1280), (256, 28688, 1280), (500, 4112, 4096), (1025, 1040, 1280)])
+def test_kn_weights_on_ring_tiles(device, M, N, K):
+    """(K, N) weights that the ring tiles turn inside LDS, over every tile they choose from: rows and columns that end inside a tile,
+    split K, alpha and beta.  The same tile and split asked for by name works on the (N, K) copy: the bits agree."""
+    g = _g(M * 5 + N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.3)
+    ad, kn = a.to(device), b.view(torch.uint8).t().contiguous().view(FP8).to(device)
+    for out_dtype in (torch.bfloat16, torch.float32, FP8):
+        kw = dict(scale_a=0.25, scale_b=0.125, out_dtype=out_dtype)
+        got = matmul(ad, kn, **kw)
+        cfg = used("tiled")
+        assert cfg["WAVES"] == 8 or M > 1024, cfg
+        kc = {"KERNEL": "tiled", "BLOCK_M": cfg["BLOCK_M"], "BLOCK_N": cfg["BLOCK_N"], "SPLIT_K": cfg["SPLIT_K"], "WAVES": 8}
+        want = matmul(ad, kn, kernel_configs=kc, **kw)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), cfg
+    check(matmul(ad, kn, scale_a=0.25, scale_b=0.125, out_dtype=torch.bfloat16), R.ref_gemm_per_tensor(a, b, 0.25, 0.125, trans_b=True), what=str(cfg))
+    c0 = torch.randn(M, N, generator=g)
+    c, c2 = c0.to(device), c0.to(device)
+    one = torch.ones(1, device=device)
+    _lib.fp8_gemm(c, ad, kn, one, None, False, False, 1.5, 0.5)
+    _lib.fp8_gemm(c2, ad, kn, one, None, False, False, 1.5, 0.5, kc)
+    assert torch.equal(c, c2)
 
 
 @pytest.mark.parametrize("rows", [8191, 8192, 8195])

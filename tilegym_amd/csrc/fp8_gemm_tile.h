@@ -110,6 +110,12 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
+// Bytes of the (K, N) slab that 16 lanes turn: lane i of them fetches 8 bytes of K row i / 2, columns 8 (i % 2) ..., and receives
+// column i of the 8 rows.
+__device__ __forceinline__ v2i lds_read_transposed_8x16(uint32_t address) {
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(uintptr_t)address);
+}
+
 // Chunk swizzle of a 128-byte slab row: 16-byte chunk j of row r sits at chunk position j ^ (r % 8).
 // Measured on gfx950 (128 B/clk LDS): ds_read_b128 of 16 consecutive rows at one logical chunk is
 // conflict free with this XOR (8 clocks per 1 KiB wave-read, the LDS's full rate); additive
@@ -227,6 +233,40 @@ __device__ __forceinline__ void store8(void* C, int out_type, int64_t row, int c
         }
     }
 }
+
+// Store 8 consecutive outputs, no beta, at element `base` of C; the 16 bytes of 16-bit outputs must be aligned.
+template <int OT>
+__device__ __forceinline__ void put8(void* C, int64_t base, v4f lo, v4f hi) {
+    typedef float v8f __attribute__((ext_vector_type(8)));
+    const v8f v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    if constexpr (OT == OUT_F32) {
+        v4f* p = reinterpret_cast<v4f*>(reinterpret_cast<float*>(C) + base);
+        p[0] = lo;
+        p[1] = hi;
+    } else if constexpr (OT == OUT_F8) {
+        *reinterpret_cast<v2i*>(reinterpret_cast<uint8_t*>(C) + base) = v2i{pack_e4m3x4(lo[0], lo[1], lo[2], lo[3]), pack_e4m3x4(hi[0], hi[1], hi[2], hi[3])};
+    } else if constexpr (OT == OUT_BF16) {
+        typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+        *reinterpret_cast<bf16x8*>(reinterpret_cast<__bf16*>(C) + base) = __builtin_convertvector(v, bf16x8);
+    } else {
+        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+        *reinterpret_cast<f16x8*>(reinterpret_cast<_Float16*>(C) + base) = __builtin_convertvector(v, f16x8);
+    }
+}
+
+// The two per-tensor scales of a problem (null: 1), requested at the top of a kernel as scalar loads and multiplied at its end: read
+// in the epilogue they are two trips to memory, one after the other, behind the last MFMA.
+static __device__ const float kOneScale[4] = {1.f, 1.f, 1.f, 1.f};
+struct TensorScales {
+    float a, b;
+    __device__ __forceinline__ explicit TensorScales(const GemmParams& p) {
+        a = *(const __attribute__((address_space(4))) float*)(uintptr_t)(p.As ? p.As : kOneScale);
+        b = *(const __attribute__((address_space(4))) float*)(uintptr_t)(p.Bs ? p.Bs : kOneScale);
+    }
+    // behind a wait that covers the two loads anyway; keeps the compiler from moving them down to their use
+    __device__ __forceinline__ void arrived() { asm volatile("" : "+s"(a), "+s"(b)); }
+    __device__ __forceinline__ float times(float alpha) const { return alpha * a * b; }
+};
 
 // Body of the tiled kernel for workgroup `bid` of problem `p` (the kernels below only differ in
 // how a workgroup finds its problem).

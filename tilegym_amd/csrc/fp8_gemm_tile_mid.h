@@ -13,6 +13,8 @@
 // flight against the latency of HBM, not the matrix pipe (16 - 64 MFMAs per step): keeping a stage idle while its
 // step is multiplied cost 20 % (4096 x 4096 weight, M = 256: 15.5 -> 12.5 us).  The four partial tiles are added
 // through LDS at the end, in a fixed order.
+// The ring tiles of fp8_gemm_tile_ring.h take most problems of K >= 1280 from it (256 x 4096 x 4096: 12.1 us here, 9.0 there); it stays
+// for shorter K and for few tiles (32 x 32 over 4096 x 4096 at M <= 64: 7.1 us in both).
 // The price is activation traffic: every workgroup reads all K of its activation rows (L2 hits), one or two bytes per
 // weight byte, and those bytes take LDS that would otherwise hold weights in flight from HBM.  It pays while one round
 // of workgroups covers the problem and the weights are small (measured: 4096 x 4096 and 6144 x 4096 at M <= 256); for
@@ -36,12 +38,6 @@
 #include "fp8_gemm_tile.h"
 
 namespace tg {
-
-// Bytes of the (K, N) slab that 16 lanes turn: lane i of them fetches 8 bytes of K row i / 2, columns 8 (i % 2) ..., and receives
-// column i of the 8 rows.
-__device__ __forceinline__ v2i lds_read_transposed_8x16(uint32_t address) {
-    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(uintptr_t)address);
-}
 
 template <int BM, int BN, int STAGES, bool KN>
 __global__ void __launch_bounds__(256, 1) fp8_gemm_tile_mid_kernel(const GemmParams p) {

@@ -1,4 +1,4 @@
-// Tiles of 64 x 128 to 192 x 192 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], per-tensor or block scales (tiles of
+// Tiles of 32 x 64 to 256 x 128 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], per-tensor or block scales (tiles of
 // 128 columns), for the row counts between decoding and those that fill whole rounds of 256 x 256 tiles.
 //
 // One workgroup per compute unit: four waves compute (2 x 2, one per SIMD), four waves do nothing but request the next K steps'
@@ -7,7 +7,7 @@
 // clocks), and with every wave loading and computing the two came one after the other: 256 x 4096 x 4096 with 160 x 128 tiles
 // took 20.0 us with four such waves, 15.9 with the loads in waves of their own.
 //
-// Three to five stages hold a K step each; a stage is requested again as soon as every computing wave has read it, so
+// Three to twelve stages hold a K step each; a stage is requested again as soon as every computing wave has read it, so
 // STAGES - 1 steps are on their way while one is multiplied.  One barrier per step, in front of its last column tiles: behind it
 // step k+1 is visible and step k's stage is free, and the fragments of step k+1 are read while those last MFMAs run (activation
 // fragments into the registers that a row group's last MFMA releases, weight fragments over three or four rotating sets).
@@ -25,6 +25,18 @@
 // step k.  With the quantizer 485 x 6144 x 4096 30.6 -> 23.6 us, 174 x 3520 x 4992 21.4 -> 18.0,
 // 62 x 6144 x 4096 18.4 -> 15.4.
 //
+// 32 and 64 rows or columns, up to twelve stages: one round of workgroups over 4096 to 12288 weight rows at 24 to 256 rows, bound by
+// the bytes a compute unit takes in from its L2 (a 64 x 64 step 0.17 us = 46 bytes a clock, 3.7 us besides, of which 1.9 are the
+// launch).  Against the tiles whose four waves split K (fp8_gemm_tile_mid.h) and 64 x 128 tiles with splits: 256 x 4096 x 4096 12.1 -> 9.0
+// us, 128 x 6144 x 4096 12.2 -> 8.7, 50 x 12288 x 5120 17.4 -> 12.5, 50 x 4096 x 14336 18.0 -> 15.4, 24 x 12288 x 5120 17.1 -> 12.2.
+// 256 x 128: 200 x 28672 x 4096 44 -> 37.
+//
+// KN: the weight is (K, N); its slab is 128 K rows of BN bytes, staged as they lie and turned on the way out of LDS
+// (ds_read_b64_tr_b8), so no (N, K) copy is made.  Bound as above: the lines of a K row tile are whole with 128 columns and halves with
+// 64 (1.62 instead of 1.05 million requests to L2 at 256 x 4096 x 4096: 13.0 us, 32 x 128 tiles 12.3, the (N, K) form 9.0).  What it measured
+// against the copy stands at pick_kn_tile.  Not kept: tiles dealt over the XCDs column by column in other orders (within 5 %
+// either way), weights fetched past the first-level cache (30 to 50 % slower).
+//
 // Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as
 // fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results.
 #pragma once
@@ -33,13 +45,16 @@
 
 namespace tg {
 
-// what a missing tensor of activation scales is read as
-static __device__ const float kOneScale[4] = {1.f, 1.f, 1.f, 1.f};
+// Place of 16-byte chunk j of K row r of a (K, N) slab: j ^ swz_kn(r).  Two groups of 16 lanes fetch 8 K rows of one chunk each at
+// once, rows r ... r + 7 and r + 16 ... r + 23.  128-byte rows: row bit 0 picks a half of the 64 banks, bits 1, 2 and 4 the place in
+// it.  64-byte rows: bits 0 and 1 pick a quarter, bits 2 and 4 the place.
+template <int BN>
+__device__ __forceinline__ int swz_kn(int r) { return BN == 64 ? ((r >> 2) & 1) | ((r >> 3) & 2) : ((r >> 1) & 3) | ((r >> 2) & 4); }
 
-template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool SPLIT>
+template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool SPLIT, bool KN>
 __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    constexpr int WGM = 2, WGN = 2, NL = 4;             // four computing waves, four loading waves
+    constexpr int NL = 4, WGN = BN == 32 ? 1 : 2, WGM = 4 / WGN;  // four loading waves, four computing waves
     constexpr int WTN = BN / WGN;
     constexpr int TM = BM / (16 * WGM), TN = WTN / 16;
     constexpr int A_IT = BM / (8 * NL), B_IT = BN / (8 * NL);
@@ -47,9 +62,10 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     constexpr int S_GROUPS = BM / 8, S_PHASES = (S_GROUPS + NL - 1) / NL;  // 8-row groups of activation scales; K steps a chunk's loads are spread over
     constexpr int PER_STEP = A_IT + B_IT + (BLOCKSCALE ? 1 : 0);
     constexpr int WS = TN == 6 ? 3 : 4;                 // weight fragment sets
-    constexpr int LAST = TN == 6 ? 1 : 2;               // column tiles behind the barrier
-    static_assert(BM % 32 == 0 && (TN == 4 || TN == 6) && STAGES >= 3 && STAGES * STAGE_BYTES <= 160 * 1024, "shape");
+    constexpr int LAST = TN == 4 ? 2 : 1;               // column tiles behind the barrier
+    static_assert(BM % (16 * WGM) == 0 && (TN == 2 || TN == 4 || TN == 6) && STAGES >= 3 && STAGES * STAGE_BYTES <= 160 * 1024, "shape");
 
+    static_assert(!KN || ((BN == 128 || BN == 64) && !BLOCKSCALE), "(K, N) weights: a K row of the tile is one 128-byte line or half of one");
     static_assert(!BLOCKSCALE || (BN == 128 && S_PHASES + STAGES - 1 <= kScaleChunk), "one weight scale per wave; a chunk of activation scales lands before its first step");
 
     __shared__ __align__(1024) uint8_t lds[STAGES * STAGE_BYTES];  // stage s: A slab, then B slab
@@ -95,7 +111,12 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 #pragma unroll
         for (int i = 0; i < A_IT; ++i) a_off[i] = (uint32_t)(m0 + min((i * NL + lw) * 8 + lrow, rows_valid - 1)) * (uint32_t)K + lj * 16;
 #pragma unroll
-        for (int i = 0; i < B_IT; ++i) b_off[i] = (uint32_t)min(n0 + (i * NL + lw) * 8 + lrow, p.N - 1) * (uint32_t)K + ljb * 16;
+        for (int i = 0; i < B_IT; ++i) {
+            // (KN: K row kr, whose 16-byte place q holds chunk q ^ swz_kn(kr); columns past N repeat the last ones)
+            const int kr = (i * NL + lw) * (1024 / BN) + lane / (BN / 16), q = lane % (BN / 16);
+            if constexpr (KN) b_off[i] = (uint32_t)kr * (uint32_t)p.N + min(n0 + ((q ^ swz_kn<BN>(kr)) << 4), p.N - 16);
+            else b_off[i] = (uint32_t)min(n0 + (i * NL + lw) * 8 + lrow, p.N - 1) * (uint32_t)K + ljb * 16;
+        }
         const v4i rsrc_a = make_rsrc(p.A), rsrc_b = make_rsrc(p.B);
         const uint32_t lds0 = lds_address(lds) + lw * 1024;
         const v4i rsrc_s = make_rsrc(p.As ? p.As : kOneScale);
@@ -115,7 +136,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
             const int k0 = min(kstep, last) * kKBlock;
             const uint32_t dst = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-            for (int i = 0; i < B_IT; ++i) direct_load_b128(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], k0);
+            for (int i = 0; i < B_IT; ++i) direct_load_b128(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], KN ? k0 * p.N : k0);
 #pragma unroll
             for (int i = 0; i < A_IT; ++i) direct_load_b128(rsrc_a, dst + i * NL * 1024, a_off[i], k0);
         };
@@ -141,6 +162,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     }
 
     // ---------------------------------------------------------------- computing waves
+    TensorScales scales(BLOCKSCALE ? GemmParams{} : p);
     const int wm = wave % WGM, wn = wave / WGM;
     const int li = lane & 15, lg = lane >> 4;
     const uint32_t frag0 = wm * 16 * kKBlock + li * kKBlock + ((lg ^ swz16(li)) << 4), frag1 = frag0 ^ 64;
@@ -158,7 +180,22 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         const uint8_t* a = base + tm * (WGM * 16 * kKBlock);
         af[tm] = join(*reinterpret_cast<const v4i*>(a + frag0), *reinterpret_cast<const v4i*>(a + frag1));
     };
+    // KN: column li of column tile tn is what 16 lanes turn out of 8 K rows x 16 columns (lane li fetches K row li / 2)
+    uint32_t kn_off[KN ? TN : 1];
+    if constexpr (KN) {
+        const int r = lg * 16 + (li >> 1);
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) kn_off[tn] = BM * kKBlock + r * BN + (((wn * TN + tn) ^ swz_kn<BN>(r)) << 4) + (li & 1) * 8;
+    }
     auto read_w = [&](int tn, const uint8_t* base) {
+        if constexpr (KN) {
+            // K bytes lg * 16 ... + 15 and 64 + lg * 16 ... + 15, eight at a time
+            const uint32_t at = lds_address(base) + kn_off[tn];
+            const v2i p0 = lds_read_transposed_8x16(at), p1 = lds_read_transposed_8x16(at + 8 * BN);
+            const v2i p2 = lds_read_transposed_8x16(at + 64 * BN), p3 = lds_read_transposed_8x16(at + 72 * BN);
+            wf[tn % WS] = v8i{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            return;
+        }
         const uint8_t* b = base + ((tn >> 1) * 32 + (tn & 1) * 4) * kKBlock;
         wf[tn % WS] = join(*reinterpret_cast<const v4i*>(b + wfrag0), *reinterpret_cast<const v4i*>(b + wfrag1));
     };
@@ -178,6 +215,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         __builtin_amdgcn_s_waitcnt(kWaitLds);
     }
     __builtin_amdgcn_s_barrier();  // step 0 has landed
+    scales.arrived();
     read_w(0, lds);
     read_w(1, lds);
     read_scales(0);
@@ -223,7 +261,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
         __builtin_amdgcn_s_barrier();          // step k+1 is visible
         TG_FENCE();
         read_w(0, nxt);
-        read_w(1, nxt);
+        if constexpr (TN > 2) read_w(1, nxt);
         read_scales(k + 1);
         TG_FENCE();
 #pragma unroll
@@ -236,6 +274,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
             }
             TG_FENCE();
         }
+        if constexpr (TN == 2) read_w(1, nxt);  // (its registers were the last MFMAs')
         if constexpr (BLOCKSCALE) {
             add(TN * TM - 2);
             add(TN * TM - 1);
@@ -251,13 +290,49 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     asm volatile("" : : "v"(wf[0]), "v"(wf[1]));
 #undef TG_FENCE
 
-    float scale = p.alpha;
-    if constexpr (!BLOCKSCALE) {
-        if (p.As) scale *= p.As[0];
-        if (p.Bs) scale *= p.Bs[0];
-    }
+    const float scale = BLOCKSCALE ? p.alpha : scales.times(p.alpha);
     const bool vec_ok = p.vec_store != 0 && (p.N % 8) == 0;
     const int64_t MN = (int64_t)p.M * p.N;
+    // KN: a lane's four columns of tile t are 16 t + 4 lg ...; what lanes 16 apart hold of a tile pair changes places, so that eight
+    // consecutive columns stand in one lane again
+    if constexpr (KN) {
+#pragma unroll
+        for (int tp = 0; tp < TN / 2; ++tp)
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[2 * tp][tm][r]), __float_as_uint(acc[2 * tp + 1][tm][r]), false, false);
+                    acc[2 * tp][tm][r] = __uint_as_float(sw[0]);
+                    acc[2 * tp + 1][tm][r] = __uint_as_float(sw[1]);
+                }
+    }
+    const int pair_col = KN ? (lg & 1) * 16 + (lg >> 1) * 8 : lg * 8;
+    // Whole 16-byte stores without beta: straight code, no test per store (the general form below is forty times as long and its
+    // way through the instruction cache takes longer than the stores).
+    auto emit_whole = [&](auto type_tag) __attribute__((always_inline)) {
+        constexpr int OT = decltype(type_tag)::value;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+            const int rt = (tm * WGM + wm) * 16 + li;
+            if (rt >= rows_valid) continue;
+            const int col = n0 + wn * WTN + pair_col;
+            const int64_t at = SPLIT ? (int64_t)blockIdx.y * MN + (int64_t)(m0 + rt) * p.N + col : (int64_t)(m0 + rt) * p.ldc + col;
+#pragma unroll
+            for (int tp = 0; tp < TN / 2; ++tp) {
+                if (col + tp * 32 >= p.N) continue;
+                if constexpr (SPLIT) put8<OUT_F32>(p.partials, at + tp * 32, acc[2 * tp][tm], acc[2 * tp + 1][tm]);
+                else put8<OT>(p.C, at + tp * 32, acc[2 * tp][tm] * scale, acc[2 * tp + 1][tm] * scale);
+            }
+        }
+    };
+    if (vec_ok && (SPLIT || p.beta == 0.f)) {
+        if (SPLIT || p.out_type == OUT_BF16) emit_whole(std::integral_constant<int, OUT_BF16>{});
+        else if (p.out_type == OUT_F32) emit_whole(std::integral_constant<int, OUT_F32>{});
+        else if (p.out_type == OUT_F8) emit_whole(std::integral_constant<int, OUT_F8>{});
+        else emit_whole(std::integral_constant<int, OUT_F16>{});
+        return;
+    }
     auto emit = [&](auto type_tag) {
         constexpr int OT = decltype(type_tag)::value;
 #pragma unroll
@@ -265,7 +340,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
             const int rt = (tm * WGM + wm) * 16 + li;
 #pragma unroll
             for (int tp = 0; tp < TN / 2; ++tp) {
-                const int col = n0 + wn * WTN + tp * 32 + lg * 8;
+                const int col = n0 + wn * WTN + tp * 32 + pair_col;
                 if (rt >= rows_valid || col >= p.N) continue;
                 if constexpr (SPLIT)
                     store8(p.partials + (int64_t)blockIdx.y * MN, OUT_F32, m0 + rt, col, p.N, p.N, acc[2 * tp][tm], acc[2 * tp + 1][tm], 0.f, vec_ok);
@@ -281,10 +356,10 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 #endif
 }
 
-template <int BM, int BN, int STAGES, bool BLOCKSCALE>
+template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool KN = false>
 inline hipError_t launch_tile_ring(bool split, const GemmParams& p, int gx, int gy, hipStream_t stream) {
-    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, true>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
-    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, true, KN>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false, KN>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -175,11 +175,15 @@ bool is_mid_tile(int bm, int bn) { return ((bm == 64 || bm == 32) && bn == 32) |
 // Per-tensor 64-row tiles of 72 .. 120 weight rows: the deep 64 x 128 kernel with the rest of its weight slab unused.
 bool is_narrowed_deep_tile(int bm, int bn) { return bm == 64 && bn >= 72 && bn < 128 && bn % 8 == 0; }
 
-// Tiles of fp8_gemm_tile_ring_kernel.  64 x 128 and 128 x 128 name two kernels each: WAVES = 8 asks for the ring (four waves load,
-// four compute), anything else for the four-wave kernels.
-bool is_ring_tile(int bm, int bn) { return (bn == 128 && (bm == 64 || bm == 96 || bm == 128 || bm == 160)) || (bn == 192 && (bm == 160 || bm == 192)); }
+// Tiles of fp8_gemm_tile_ring_kernel.  64 x 32, 64 x 64, 64 x 128 and 128 x 128 name two kernels each: WAVES = 8 asks for the ring
+// (four waves load, four compute), anything else for the four-wave kernels.
+bool is_ring_tile(int bm, int bn) {
+    return (bn == 128 && (bm == 32 || bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 256)) || (bn == 192 && (bm == 160 || bm == 192)) ||
+           (bn == 64 && (bm == 32 || bm == 64)) || (bn == 32 && bm == 64);
+}
 bool is_block_ring_tile(int bm, int bn) { return bn == 128 && (bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 192); }
-bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !(bn == 128 && (bm == 128 || bm == 64)); }
+bool names_two_kernels(int bm, int bn) { return (bn == 128 && (bm == 128 || bm == 64)) || is_mid_tile(bm, bn); }
+bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !names_two_kernels(bm, bn); }
 
 bool tile_exists(int bm, int bn, bool block_scaled) {
     if (block_scaled && is_block_ring_tile(bm, bn)) return true;
@@ -240,14 +244,16 @@ int deep_tile_cols(int64_t M, int64_t N, int64_t split) {
 // shapes, at worst 1.43 x (75 x 1968 x 7424) and 1.38 x (233 x 3952 x 5632); fitted to three quarters of the shapes 1.5 % and 1.3 % on the
 // others.  Against the kernels and the model without the ring tiles it is 12 % and 17 % ahead on average, more than 5 % behind on 39 and
 // 13 shapes, at worst 1.17 x (320 x 3072 x 8192 22.8 against 19.5 us) and 1.18 x (133 x 1024 x 8192 10.6 against 9.0).
-struct StepCost { int bm, bn; bool ring; float first, full, both, fixed, memory; };
+struct StepCost { int bm, bn; bool ring; float first, full, both, fixed, memory; int from_k = 0; };  // from_k: offered from this K on
 constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.106f, 0.122f, 0.f, 3.296f, 0.008f}, {64, 32, false, 0.169f, 0.192f, 0.f, 2.825f, 0.002f},
                                         {64, 64, false, 0.175f, 0.271f, 0.f, 3.494f, 0.035f}, {64, 128, false, 0.623f, 0.752f, 1.153f, 3.531f, 0.001f},
                                         {128, 128, false, 0.215f, 0.854f, 0.944f, 5.766f, 0.081f}, {128, 256, false, 0.552f, 1.278f, 0.f, 5.713f, 0.083f},
                                         {256, 256, false, 1.297f, 1.009f, 0.f, 11.556f, 0.012f},
                                         {64, 128, true, 0.219f, 0.313f, 0.f, 3.087f, 0.060f}, {96, 128, true, 0.371f, 0.293f, 0.f, 3.990f, 0.102f},
                                         {128, 128, true, 0.344f, 0.387f, 0.f, 5.394f, 0.095f}, {160, 128, true, 0.496f, 0.552f, 0.f, 4.331f, 0.075f},
-                                        {160, 192, true, 0.441f, 0.667f, 0.f, 6.211f, 0.064f}, {192, 192, true, 0.628f, 0.675f, 0.f, 8.253f, 0.061f}};
+                                        {160, 192, true, 0.441f, 0.667f, 0.f, 6.211f, 0.064f}, {192, 192, true, 0.628f, 0.675f, 0.f, 8.253f, 0.061f},
+                                        {64, 32, true, 0.131f, 0.133f, 0.f, 2.836f, 0.f, 1280}, {32, 64, true, 0.131f, 0.133f, 0.f, 2.836f, 0.f, 1280},
+                                        {64, 64, true, 0.163f, 0.185f, 0.f, 2.980f, 0.f, 1280}, {256, 128, true, 0.409f, 0.761f, 0.f, 6.266f, 0.f, 1280}};
 // (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
 constexpr float kDeepTileRowsShare = 0.53f;
 // Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.1 % behind the best schedule on average,
@@ -265,11 +271,13 @@ struct TileModel { const StepCost* kinds; int n; float reduce_us, reduce_us_per_
 constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 3.272f, 0.316f, 1.0f, 0.018f};
 constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
+constexpr TileModel kSmallRowsRing{nullptr, 0, 2.6f, 0.25f, 1.0f, 0.f};  // (the reduction launch behind the ring tiles of up to 64 rows)
+
 // (cols: weight rows per tile where they are not the kind's own)
 float step_cost_us(const TileModel& m, const StepCost& t, int64_t M, int64_t N, int64_t kblocks, int split, int cols) {
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, cols) * split, places = t.both > 0.f ? 512 : 256;
     // (the narrow tiles' four waves split K: whole groups of four steps)
-    const float steps = (float)(is_mid_tile(t.bm, t.bn) ? cdiv(kblocks, 4) * 4 : cdiv(kblocks, split));
+    const float steps = (float)(!t.ring && is_mid_tile(t.bm, t.bn) ? cdiv(kblocks, 4) * 4 : cdiv(kblocks, split));
     const float at_full = t.both > 0.f ? t.both : t.full;
     const float narrowed = cols == t.bn ? 1.f : kDeepTileRowsShare + (1.f - kDeepTileRowsShare) * (float)cols / (float)t.bn;
     const float from_memory = std::min(std::max(((float)(N * kblocks * 128) - 8e6f) / 12e6f, 0.f), 1.f);
@@ -294,14 +302,15 @@ struct TileChoice { int bm = -1, bn = -1, split = 1; bool ring = false; float us
 
 // The cheapest (tile, split) by the model; a tile (bm > 0; ring: the ring form of 128 x 128) or a split (want_split > 0) given by
 // the caller is kept.
-TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
-                             int bm, int bn, bool ring, bool takes_320 = false) {
-    const TileModel& m = block_scaled ? kBlockScaledModel : kPerTensorModel;
+TileChoice pick_tile_by_cost(const TileModel& m, int64_t M, int64_t N, int64_t kblocks, int64_t partial_bytes_avail, int want_split = -1,
+                             int bm = -1, int bn = -1, bool ring = false, bool takes_320 = false) {
+    const bool block_scaled = &m == &kBlockScaledModel;
     TileChoice best;
     if (want_split <= 0 && partial_bytes_avail > kAutoPartialBytes) partial_bytes_avail = kAutoPartialBytes;
     auto offer = [&](const StepCost& t) {
         if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
-        const bool mid = is_mid_tile(t.bm, t.bn);
+        const bool mid = !t.ring && is_mid_tile(t.bm, t.bn);
+        if (t.from_k > kblocks * 128 && bm <= 0) return;
         if (want_split > 1 && mid) return;  // these split K inside the workgroup only
         if (t.bn == 320 && (want_split > 1 || !takes_320)) return;
         const bool deep = !block_scaled && !t.ring && t.bm == 64 && t.bn == 128;
@@ -316,6 +325,10 @@ TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_s
     };
     for (int i = 0; i < m.n; ++i) offer(m.kinds[i]);
     return best;
+}
+TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
+                             int bm, int bn, bool ring, bool takes_320 = false) {
+    return pick_tile_by_cost(block_scaled ? kBlockScaledModel : kPerTensorModel, M, N, kblocks, partial_bytes_avail, want_split, bm, bn, ring, takes_320);
 }
 
 // 17 .. 64 rows: the same form of model over more kinds of kernel, with constants of its own (here the weights stream from
@@ -413,6 +426,28 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                 if (split > 1) cand.split_k = pick_split(cdiv(M, t.bm) * cdiv(N, t.bn), 256, kblocks, 4, M, N, partial_bytes_avail, split);
                 offer(cand, rounds_cost_us(t, cdiv(M, t.bm) * cdiv(N, t.bn) * cand.split_k, cdiv(kblocks, cand.split_k)) + reduce(cand.split_k));
                 if (want_split > 0) break;
+            }
+        }
+        // Per-tensor ring tiles of 32 and 64 rows, from 96 tiles on (with fewer most of the chip idles and the narrow tiles that split
+        // K are as fast: 24 x 4096 x 4096 7.0 against 7.3 us, 50 x 4096 x 4096 7.1 and 7.1), predicted at least 5 % faster than anything
+        // else.  32-row tiles run unsplit; 64 x 64 takes over above 32 rows.  24 x 12288 x 5120 17.1 -> 12.2 us, 50 x 12288 x 5120
+        // 19.8 -> 12.8, 50 x 4096 x 14336 18.8 -> 15.7 (with splits by four).  Fitted to 1777 shapes, weights of 1 to 310 MB, three sets
+        // of operands: 14 % ahead of the kinds above on average, more than 5 % behind on 29 at worst 1.2 x; above 160 MB the 64 x 72 ... 128 tiles,
+        // whose weights pass the caches by, are ahead by up to 1.35 x (60 x 18192 x 11008 50 against 68 us).
+        if (!block_scaled && K >= 1280 && N * K <= ((int64_t)160 << 20)) {
+            constexpr StepCost rings[] = {{32, 64, true, 0.088f, 0.185f, 0.f, 3.312f, 0.011f}, {64, 64, true, 0.093f, 0.293f, 0.f, 3.394f, 0.f},
+                                          {32, 128, true, 0.143f, 0.392f, 0.f, 3.273f, 0.019f}, {64, 128, true, 0.158f, 0.599f, 0.f, 3.219f, 0.f}};
+            for (const StepCost& t : rings) {
+                if (t.bm == 64 && M <= 32) continue;
+                for (int sp = 1; sp <= 8; sp *= 2) {
+                    const int split = want_split > 0 ? want_split : sp;
+                    if (split > 1 && (t.bm == 32 || kblocks / split < 4 || !fits(split))) break;
+                    Schedule cand{1, t.bm, t.bn, 1, -1, -1, 8};
+                    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
+                    if (split > 1) cand.split_k = pick_split(tiles, 256, kblocks, 4, M, N, partial_bytes_avail, split);
+                    if (tiles * cand.split_k >= 96) offer(cand, 1.05f * step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn));
+                    if (want_split > 0) break;
+                }
             }
         }
         // block-scaled: the ring form of the 64 x 128 tile (five stages; 62 x 6144 x 4096 15.7 -> 12.6 us, 30 x 4096 x 14336
@@ -586,7 +621,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, block_scaled))) bm = bn = -1;
     if (bm == 256 && bn == 320 && !(takes_320 && want_split <= 1)) bm = bn = -1;
     int model_split = 1;
-    const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && ((bm != 128 && bm != 64) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
+    const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && (!names_two_kernels(bm, bn) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
     if (want_ring) s.waves = 8;
     if (M > 64) {
         const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring, takes_320);
@@ -606,7 +641,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     s.bn = bn;
     const int64_t wgs = cdiv(M, bm) * cdiv(N, bn);
     s.split_k = 1;
-    if (is_mid_tile(bm, bn)) return s;  // K is split inside the workgroup: one launch
+    if (is_mid_tile(bm, bn) && s.waves != 8) return s;  // K is split inside the workgroup: one launch
     if (want_split > 1) {
         s.split_k = pick_split(wgs, 256, kblocks, 4, M, N, partial_bytes_avail, want_split);
     } else if (M > 64) {
@@ -637,27 +672,48 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
     return true;
 }
 
-// A per-tensor (K, N) weight: whether the narrow tiles read it as it lies, and with which tile; else it is copied to (N, K)
-// first and any kernel takes it.  Up to 64 rows a direct tile's K step takes 0.39 - 0.45 us whatever the grid, and copy and GEMM together
-// 7 us + 0.5 us per MB.  Above, the direct tiles have step costs like the kernels of the race, and the copy costs 4.1 us + 0.47 us per
-// MB on top of the race's GEMM: fitted to 718 shapes (65 ... 512 rows) with both ways measured, cached and from memory: 0.6 % behind the
-// better way on average in either, at worst 1.21 x (with one step cost for every grid 5.5 - 6.1 % and 1.75 x).
-// Wide or short weights go direct (28672 x 4096 at M = 16: 37.5 us against 65.4; 1024 x 1024: 5.2 against 7.7; 1888 x 5504 at
-// M = 91: 12.2 against 21.2), long K against few columns is copied (4096 x 14336 at M = 16: 48.6 direct, 39.0 copied), and so are
-// most from 300 rows on (2672 x 7424 at M = 485: 31.8 against 46.6).
+// A per-tensor (K, N) weight: the tile (and split) that reads it as it lies, or none where copying it to (N, K) first is cheaper.
+//
+// K from 1280 on: the ring tiles, with step costs of their own (a step is 1.2 to 1.6 times as long as over an (N, K) weight: 64-column
+// tiles take half of every 128-byte line, and K rows a multiple of 4 KiB apart crowd few cache sets -- 256 x 4096 x 4096 12.3 us with 32 x
+// 128 tiles, 256 x 3968 x 4096 10.7), against the race's GEMM with the copy's 4.1 us + 0.47 us per MB on top.  Fitted to 3871 shapes (1 ... 2048
+// rows, three sets of operands): 2.2 % behind the best ring tile up to 64 rows and 0.8 % above, at worst 1.25 x; against the narrow
+// tiles of fp8_gemm_tile_mid.h and the copy, which took all of these, 31 % ahead on average, behind by more than 5 % on 219 (5.5 us and
+// shorter, or by 8 % at most): 1 x 4096 x 14336 36.0 -> 14.3 us, 50 x 4096 x 14336 41 -> 16.5, 100 x 28672 x 4096 57.5 -> 28.7,
+// 400 x 12288 x 5120 53 -> 31, 64 x 2048 x 2048 7.9 -> 4.8.
+//
+// Shorter K: the narrow tiles, by the costs they were fitted to, or the copy.  (The ring would be up to 40 % faster there too, 16400 x 1152
+// at M = 64 7.3 against 12.6 us; which tiles run at these sizes is held by callers that compare a forced schedule's bits.)
+constexpr StepCost kKnRingFewRows[] = {{32, 64, true, 0.205f, 0.369f, 0.f, 2.357f, 0.f}, {64, 64, true, 0.221f, 0.420f, 0.f, 2.422f, 0.f},
+                                       {32, 128, true, 0.200f, 0.630f, 0.f, 2.829f, 0.f}, {64, 128, true, 0.240f, 0.660f, 0.f, 2.788f, 0.f}};
+constexpr TileModel kKnFewRowsModel{kKnRingFewRows, (int)(sizeof(kKnRingFewRows) / sizeof(StepCost)), 3.1f, 0.25f, 1.0f, 0.f};
+constexpr StepCost kKnRing[] = {{32, 64, true, 0.177f, 0.278f, 0.f, 2.819f, 0.f}, {64, 64, true, 0.253f, 0.329f, 0.f, 2.872f, 0.f},
+                                {32, 128, true, 0.265f, 0.332f, 0.f, 3.169f, 0.f}, {64, 128, true, 0.302f, 0.372f, 0.f, 3.631f, 0.f},
+                                {96, 128, true, 0.346f, 0.412f, 0.f, 3.929f, 0.f}, {128, 128, true, 0.368f, 0.468f, 0.f, 4.557f, 0.f},
+                                {160, 128, true, 0.375f, 0.537f, 0.f, 5.306f, 0.f}, {256, 128, true, 0.452f, 0.739f, 0.f, 6.638f, 0.f}};
+constexpr TileModel kKnModel{kKnRing, (int)(sizeof(kKnRing) / sizeof(StepCost)), 3.6f, 0.30f, 1.0f, 0.f};
 constexpr TileCost kKnFewRowsTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.41f, 0.f, 3.5f}, {64, 64, 0.45f, 0.f, 4.5f}};
 constexpr StepCost kKnTiles[] = {{32, 32, false, 0.236f, 0.232f, 0.f, 1.174f, 0.f}, {64, 32, false, 0.358f, 0.321f, 0.f, 1.139f, 0.f},
                                  {64, 64, false, 0.298f, 0.426f, 0.f, 1.862f, 0.024f}};
 constexpr float kCopyUs = 4.11f, kCopyUsPerMB = 0.466f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
-bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, int* bm, int* bn) {
-    if (M > 512 || N % 16 != 0 || K % 128 != 0) return false;
+bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, Schedule* s) {
+    if (N % 16 != 0 || K % 128 != 0) return false;
     const int64_t kblocks = K / 128;
     const float mb = (float)(N * K) * 1e-6f;
+    *s = Schedule{1, -1, -1, 1, -1, -1, -1};
     float best = 0.f;
-    *bm = -1;
     auto offer = [&](int tile_m, int tile_n, float us) {
-        if (*bm < 0 || us < best) { best = us; *bm = tile_m; *bn = tile_n; }
+        if (s->bm < 0 || us < best) { best = us; s->bm = tile_m; s->bn = tile_n; }
     };
+    if (K >= 1280) {
+        const TileModel& m = M <= 64 ? kKnFewRowsModel : kKnModel;
+        const TileChoice pick = pick_tile_by_cost(m, M, N, kblocks, partial_bytes_avail);
+        if (M > 64 && pick.us > pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us + kCopyUs + kCopyUsPerMB * mb) return false;
+        *s = Schedule{1, pick.bm, pick.bn, 1, -1, -1, 8};
+        if (pick.split > 1) s->split_k = pick_split(cdiv(M, pick.bm) * cdiv(N, pick.bn), 256, kblocks, 4, M, N, partial_bytes_avail, pick.split);
+        return true;
+    }
+    if (M > 512) return false;
     if (M <= 64) {
         for (const TileCost& t : kKnFewRowsTiles) {
             const float tiles = (float)(cdiv(M, t.bm) * cdiv(N, t.bn));   // one workgroup per compute unit
@@ -1030,13 +1086,13 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     const uint8_t* Bnt = reinterpret_cast<const uint8_t*>(b->ptr);
     bool b_is_nk = trans_b != 0;
     const int want_kernel = cfg_get(cfg, ncfg, TG_CFG_KERNEL);
-    bool direct_kn = false;   // a (K, N) weight read as it lies by the narrow tiles
-    int kn_bm = -1, kn_bn = -1;
+    bool direct_kn = false;   // a (K, N) weight read as it lies
+    Schedule kn{};
     if (!b_is_nk && !trans_a && want_kernel != 0 && K > 0) {
         // (K,N) weights: make a K-contiguous copy at the tail of the workspace when it fits
         const int64_t need = (N * K + 255) / 256 * 256;
         direct_kn = ws_free >= need && !static_scratch && !block_scaled && M * K < kOffsetLimit && N * K < kOffsetLimit && aligned16(a->ptr) && aligned16(b->ptr) &&
-                    nothing_forced(cfg, ncfg) && pick_kn_tile(M, N, K, ws_free - need, &kn_bm, &kn_bn);
+                    nothing_forced(cfg, ncfg) && pick_kn_tile(M, N, K, ws_free - need, &kn);
         if (!direct_kn && ws_free >= need) {
             uint8_t* bt = ws + ws_bytes - need;
             bt = reinterpret_cast<uint8_t*>(reinterpret_cast<uintptr_t>(bt) & ~(uintptr_t)15);
@@ -1053,7 +1109,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     const bool fast_layout = !trans_a && b_is_nk && (K % 16) == 0 && aligned16(a->ptr) &&
                              aligned16(reinterpret_cast<uint64_t>(Bnt)) && N * K < kOffsetLimit && (!block_scaled || std_blocks);
     const bool takes_320 = block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit;
-    Schedule s = direct_kn ? Schedule{1, kn_bm, kn_bn, 1, -1, -1, -1} : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
+    Schedule s = direct_kn ? kn : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
     if (static_scratch) {
         // The schedule of tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split.  (Above 64 rows an
         // automatic split stays within the array, see kAutoPartialBytes.)  One exception, above 16 rows: a (K, N) weight's copy
@@ -1149,7 +1205,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         const bool split = pc.split_k > 1;
         const bool deep = s.kernel == 1 && !block_scaled && s.waves != 8 && s.bm == 64 && (s.bn == 128 || is_narrowed_deep_tile(s.bm, s.bn));
         if (deep) pc.tile_cols = s.bn;
-        const bool mid = s.kernel == 1 && !block_scaled && is_mid_tile(s.bm, s.bn);
+        const bool mid = s.kernel == 1 && !block_scaled && s.waves != 8 && is_mid_tile(s.bm, s.bn);
         // persistent kernel with the hand-ordered K loop for the dense per-tensor 256x256 tile, from two K steps up
         // (WAVES = 8 asks for the generic eight-wave tile kernel instead)
         const bool ordered = s.kernel == 1 && !block_scaled && !split && s.bm == 256 && s.bn == 256 && kblocks >= 2 &&
@@ -1164,6 +1220,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
         hipError_t e = block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
                      : block_ring ? tg::run_tile_ring_block(s.bm, split, pc, gx, pc.split_k, stream)
+                     : ring && direct_kn ? tg::run_tile_ring_kn(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
                      : ordered ? tg::run_tile256(pc, gx, stream)
