@@ -133,6 +133,28 @@ def test_persistent_256_walks_several_tiles_per_workgroup(device, M, N, K, out_d
     check(res[rows.to(device)], ref, what=f"persistent 256x256 M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("bm,bn", [(32, 64), (64, 64), (32, 128)])
+@pytest.mark.parametrize("dm,N,K,split", [(0, 256, 128, 1), (-1, 120, 1024, 1), (1, 136, 1152, 2), (17, 257, 2176, 1), (-15, 384, 2304, 2), (0, 192, 4096, 1)])
+def test_ring_tiles_block_scaled_narrow(device, bm, bn, dm, N, K, split):
+    """The tiles of 64 columns (half of a block of weight scales) and 32 rows, over the same edges and four chunks of scales: same bits
+    as the 128 x 128 tile kernel, with either scale tensor missing too, and the oracle's result; beta in the epilogue."""
+    M = 2 * bm + dm
+    g = _g(bm + bn + N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)
+    sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand((N + 127) // 128, K // 128, generator=g) * 0.1 + 0.01
+    ad, bd, sad, sbd = a.to(device), b.to(device), sa.to(device), sb.to(device)
+    c0 = torch.randn(M, N, generator=g)
+    for s1, s2, dtype, beta in ((sad, sbd, torch.bfloat16, 0.0), (None, sbd, torch.float32, 0.0), (sad, None, torch.float16, 0.0), (sad, sbd, torch.float32, 0.5)):
+        out, base = c0.to(device).to(dtype), c0.to(device).to(dtype)
+        _lib.fp8_gemm(out, ad, bd, s1, s2, False, True, 1.0, beta, {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": split, "WAVES": 8})
+        cfg = used("tiled")
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["WAVES"]) == (bm, bn, 8), cfg
+        _lib.fp8_gemm(base, ad, bd, s1, s2, False, True, 1.0, beta, {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": cfg["SPLIT_K"]})
+        assert torch.equal(out, base)
+        if dtype is torch.bfloat16:
+            check(out, R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"block ring {bm}x{bn} M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("bm,bn", [(32, 32), (64, 32), (64, 64)])
 @pytest.mark.parametrize("M,N,K", [(64, 512, 1024), (40, 200, 384), (17, 1000, 2560), (130, 72, 128), (33, 264, 256), (96, 4096, 4096)])
 def test_per_tensor_mid_tiles(device, bm, bn, M, N, K):

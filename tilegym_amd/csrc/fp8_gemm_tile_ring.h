@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     static_assert(BM % (16 * WGM) == 0 && (TN == 2 || TN == 4 || TN == 6) && STAGES >= 3 && STAGES * STAGE_BYTES <= 160 * 1024, "shape");
 
     static_assert(!KN || ((BN == 128 || BN == 64) && !BLOCKSCALE), "(K, N) weights: a K row of the tile is one 128-byte line or half of one");
-    static_assert(!BLOCKSCALE || (BN == 128 && S_PHASES + STAGES - 1 <= kScaleChunk), "one weight scale per wave; a chunk of activation scales lands before its first step");
+    static_assert(!BLOCKSCALE || (128 % BN == 0 && S_PHASES + STAGES - 1 <= kScaleChunk), "one weight scale per tile; a chunk of activation scales lands before its first step");
 
     __shared__ __align__(1024) uint8_t lds[STAGES * STAGE_BYTES];  // stage s: A slab, then B slab
     // block scales: activation scales of the tile's rows, two chunks of kScaleChunk K steps, laid out as in fp8_gemm_tile.h, and

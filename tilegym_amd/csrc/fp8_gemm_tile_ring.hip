@@ -39,7 +39,11 @@ hipError_t run_tile_ring_kn(int bm, int bn, bool split, const GemmParams& p, int
     return hipErrorInvalidConfiguration;
 }
 
-hipError_t run_tile_ring_block(int bm, bool split, const GemmParams& p, int gx, int gy, hipStream_t s) {
+hipError_t run_tile_ring_block(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s) {
+    if (bm == 32 && bn == 64) return launch_tile_ring<32, 64, 8, true>(split, p, gx, gy, s);
+    if (bm == 64 && bn == 64) return launch_tile_ring<64, 64, 7, true>(split, p, gx, gy, s);
+    if (bn != 128) return hipErrorInvalidConfiguration;
+    if (bm == 32) return launch_tile_ring<32, 128, 7, true>(split, p, gx, gy, s);
     if (bm == 64) return launch_tile_ring<64, 128, 5, true>(split, p, gx, gy, s);
     if (bm == 96) return launch_tile_ring<96, 128, 4, true>(split, p, gx, gy, s);
     if (bm == 128) return launch_tile_ring<128, 128, 4, true>(split, p, gx, gy, s);

@@ -42,8 +42,8 @@ hipError_t run_tile256(const GemmParams& p, int gx, hipStream_t s);
 // kn: p.B is (K, N), N % 16 == 0
 hipError_t run_tile_mid(int bm, int bn, bool kn, const GemmParams& p, hipStream_t s);
 // tiles of 64 x 128 to 192 x 192 over a ring of LDS stages, four waves load and four compute: same results as
-// run_tile_per_tensor's and run_tile_block_dense's tiles (block-scaled: bm x 128)
-hipError_t run_tile_ring_block(int bm, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
+// run_tile_per_tensor's and run_tile_block_dense's tiles (block-scaled: bm x 128 and bm x 64)
+hipError_t run_tile_ring_block(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 // p.B is (K, N): N % 16 == 0, K % 128 == 0
 hipError_t run_tile_ring_kn(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 hipError_t run_tile_ring(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);

@@ -175,13 +175,13 @@ bool is_mid_tile(int bm, int bn) { return ((bm == 64 || bm == 32) && bn == 32) |
 // Per-tensor 64-row tiles of 72 .. 120 weight rows: the deep 64 x 128 kernel with the rest of its weight slab unused.
 bool is_narrowed_deep_tile(int bm, int bn) { return bm == 64 && bn >= 72 && bn < 128 && bn % 8 == 0; }
 
-// Tiles of fp8_gemm_tile_ring_kernel.  64 x 32, 64 x 64, 64 x 128 and 128 x 128 name two kernels each: WAVES = 8 asks for the ring
+// Tiles of fp8_gemm_tile_ring_kernel.  64 x 32, 64 x 64 (per-tensor), 64 x 128 and 128 x 128 name two kernels each: WAVES = 8 asks for the ring
 // (four waves load, four compute), anything else for the four-wave kernels.
 bool is_ring_tile(int bm, int bn) {
     return (bn == 128 && (bm == 32 || bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 256)) || (bn == 192 && (bm == 160 || bm == 192)) ||
            (bn == 64 && (bm == 32 || bm == 64)) || (bn == 32 && bm == 64);
 }
-bool is_block_ring_tile(int bm, int bn) { return bn == 128 && (bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 192); }
+bool is_block_ring_tile(int bm, int bn) { return (bn == 64 && (bm == 32 || bm == 64)) || (bn == 128 && (bm == 32 || bm == 64 || bm == 96 || bm == 128 || bm == 160 || bm == 192)); }
 bool names_two_kernels(int bm, int bn) { return (bn == 128 && (bm == 128 || bm == 64)) || is_mid_tile(bm, bn); }
 bool is_ring_only_tile(int bm, int bn) { return is_ring_tile(bm, bn) && !names_two_kernels(bm, bn); }
 
@@ -257,13 +257,15 @@ constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.106f, 0.122f, 0.f, 3.2
 // (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
 constexpr float kDeepTileRowsShare = 0.53f;
 // Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.1 % behind the best schedule on average,
-// at worst 1.29 x; 17 % ahead of the kernels and the model without the ring tiles, more than 5 % behind on five, at worst 1.08 x
+// at worst 1.29 x.  The 32 x 64 and 64 x 64 tiles at the end came later (3437 shapes of 65 to 1024 rows: 6 % ahead of the others on average, more
+// than 5 % behind on four, at worst 1.08 x).  The others: 17 % ahead of the kernels and the model without the ring tiles, more than 5 % behind on five, at worst 1.08 x
 // (491 x 20400 x 7296 103.1 against 96.0 us).  Block-scaled 128 x 256 exists and can be forced; it is left out.
 constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879f, 3.42f, 0.f}, {128, 128, false, 0.610f, 0.863f, 1.064f, 4.23f, 0.f},
                                           {256, 256, false, 1.361f, 1.727f, 0.f, 7.49f, 0.f},  {256, 320, false, 1.66f, 2.12f, 0.f, 9.00f, 0.f},
                                           {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f, 0.f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f, 0.f},
                                           {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f, 0.f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f, 0.f},
-                                          {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f, 0.f}};
+                                          {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f, 0.f},
+                                          {32, 64, true, 0.171f, 0.169f, 0.f, 2.888f, 0.018f, 1280}, {64, 64, true, 0.208f, 0.218f, 0.f, 3.291f, 0.018f, 1280}};
 // split_margin: a split schedule must be predicted this much faster than the best unsplit one.  odd_kib: what a ring tile's step takes
 // longer over weights from memory whose rows lie an odd number of KiB apart (64 x 128 tiles over 5120 x 5120 from memory 0.47 - 0.50 us a
 // step, over other weights of 25 MB 0.41).
@@ -450,6 +452,24 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                 }
             }
         }
+        // block-scaled: the ring tiles of 32 and 64 rows, weights to 100 MB (above, the 64 x 128 tiles are up to 1.15 x ahead).  Fitted to 1628 shapes,
+        // 13 % ahead on average of the 64 x 128 tiles and the streaming form alone, more than 5 % behind on five, at worst 1.14 x (5.9 against 5.2 us): without the
+        // quantizer, 50 x 4096 x 4096 8.4 -> 7.5 us, 24 x 12288 x 5120 15.5 -> 12.9, 50 x 12288 x 5120 16.3 -> 13.9.
+        if (block_scaled && K >= 1280 && N * K <= ((int64_t)100 << 20)) {
+            constexpr StepCost rings[] = {{32, 64, true, 0.136f, 0.214f, 0.f, 3.408f, 0.f}, {64, 64, true, 0.169f, 0.296f, 0.f, 3.556f, 0.f},
+                                          {32, 128, true, 0.185f, 0.414f, 0.f, 3.684f, 0.f}};
+            for (const StepCost& t : rings) {
+                for (int sp = 1; sp <= 8; sp *= 2) {
+                    const int split = want_split > 0 ? want_split : sp;
+                    if (split > 1 && (kblocks / split < 4 || !fits(split))) break;
+                    Schedule cand{1, t.bm, t.bn, 1, -1, -1, 8};
+                    if (split > 1) cand.split_k = pick_split(cdiv(M, t.bm) * cdiv(N, t.bn), 256, kblocks, 4, M, N, partial_bytes_avail, split);
+                    // (a split must be predicted 10 % faster: its reduction is a launch more for the host, too)
+                    offer(cand, step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn) * (cand.split_k > 1 ? 1.1f : 1.f));
+                    if (want_split > 0) break;
+                }
+            }
+        }
         // block-scaled: the ring form of the 64 x 128 tile (five stages; 62 x 6144 x 4096 15.7 -> 12.6 us, 30 x 4096 x 14336
         // 21.8 -> 17.2; 63 shapes 12 % on average.  Per-tensor the deep kernel is as fast: 3 % behind)
         if (block_scaled) {
@@ -621,7 +641,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     if (!(bm > 0 && bn > 0 && tile_exists(bm, bn, block_scaled))) bm = bn = -1;
     if (bm == 256 && bn == 320 && !(takes_320 && want_split <= 1)) bm = bn = -1;
     int model_split = 1;
-    const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && (!names_two_kernels(bm, bn) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
+    const bool want_ring = bm > 0 && (block_scaled ? is_block_ring_tile(bm, bn) : is_ring_tile(bm, bn)) && (!names_two_kernels(bm, bn) || (block_scaled && bn == 64) || cfg_get(cfg, ncfg, TG_CFG_WAVES) == 8);
     if (want_ring) s.waves = 8;
     if (M > 64) {
         const TileChoice pick = pick_tile_by_cost(M, N, kblocks, block_scaled, partial_bytes_avail, want_split, bm, bn, want_ring, takes_320);
@@ -1219,7 +1239,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
         const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
         hipError_t e = block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
-                     : block_ring ? tg::run_tile_ring_block(s.bm, split, pc, gx, pc.split_k, stream)
+                     : block_ring ? tg::run_tile_ring_block(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : ring && direct_kn ? tg::run_tile_ring_kn(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : mid ? tg::run_tile_mid(s.bm, s.bn, direct_kn, pc, stream)
