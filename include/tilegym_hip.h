@@ -65,14 +65,16 @@ enum {
                          * 32x32, 64x32, 64x64 (K split inside the workgroup) and 64 x 72 .. 120 in steps of 8; tiles over a ring of LDS stages (four
                          * waves load, four compute): 96x128, 160x128, with WAVES = 8 also 64x128 and 128x128, per-tensor 32x64, 32x128, 256x128, 160x192 and 192x192 and with WAVES = 8 64x32 and 64x64,
                          * block-scaled 192x128; block-scaled 256x320 (M >= 256, N >= 320, N % 32 == 0, both scale tensors, no split).  Grouped
-                         * GEMMs: 64x128, 128x128, 128x256, 256x256.  Any other pair leaves the tile to the library */
+                         * GEMMs: 64x128, 128x128, 128x256, 256x256; ragged with ROW_GROUPS = 1 also the persistent ring tiles 32x128, 64x128, 64x192, 64x256,
+                         * 128x192, 128x256 (K % 128 == 0, K >= 640, 128 columns 1024; E <= 256; both scale tensors).  Any other pair leaves the tile to the library */
     TG_CFG_BLOCK_N = 2, /* tiled kernel: rows of B per workgroup (see BLOCK_M); stream kernel, wide form (ROW_GROUPS = 4,
                          * K % 128 == 0): rows of B per workgroup, a multiple of 4 up to 64 (four waves own a quarter each); narrow form: 1 .. 16 */
     TG_CFG_SPLIT_K = 3, /* K partitions reduced through the workspace (1 = none)         */
     TG_CFG_ROW_GROUPS = 4, /* skinny kernel: 16-row groups of B per wave (1/2/4); stream kernel: LDS buffers per wave (1/2);
                             * tiled 256x256 block-scaled kernels (dense and ragged): 1 = the persistent form (one workgroup per
                             * compute unit walks the tiles, three weight slabs in LDS, scales in registers); the ragged GEMM
-                            * chooses it by itself for K <= 1536 */
+                            * chooses it by itself for K <= 1536 from 192 rows per expert on; ragged ring tiles: 1 asks for them
+                            * (reported as 1) */
     TG_CFG_WAVES = 5,   /* skinny kernel: waves per workgroup splitting K (4/8/16); stream kernel: 8 = eight waves split K inside a 16-row workgroup, and with ROW_GROUPS = 4 (the wide form) 1 = one 1 KiB piece per wave in flight instead of two half pieces; tiled 256x256 kernels: 8 = the generic eight-wave tile kernel (one workgroup per tile) instead of the persistent one; tiled 64x32, 64x64, 64x128 and 128x128: 8 = the ring form of the tile (reported as 8 for every ring tile); ragged GEMM, streaming form: 4 / 6 / 8 waves (64 / 96 / 128 weight rows) per workgroup */
     TG_CFG_QUANT_BLOCK_N = 6, /* block-scaled tg_fp8_gemm: weight rows per scale (default 128) */
     TG_CFG_QUANT_BLOCK_K = 7, /* block-scaled tg_fp8_gemm: K elements per scale (default 128): the reference's

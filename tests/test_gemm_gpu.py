@@ -1266,7 +1266,112 @@ def test_ragged_fallback_for_odd_k(device):
     check(c, ref)
 
 
+@pytest.mark.parametrize("bm,bn,K", [(32, 128, 1024), (64, 128, 1152), (64, 256, 640), (64, 256, 1152), (128, 256, 640), (128, 256, 2176), (64, 192, 640), (128, 192, 1152)])
+@pytest.mark.parametrize("many", [False, True])
+def test_ragged_ring_tiles(device, bm, bn, K, many):
+    """The persistent tiles: the fewest K steps they take (5, 8), chunks of scales that end inside K or hold one step (9, 17), experts
+    without rows, with one, with more than a tile; fewer tiles than workgroups and several tiles on each; every output type, columns
+    that end inside a tile and odd ones.  Same bits as 128 x 128 tiles."""
+    g = _g(K + bm)
+    if many:   # 130 experts (the search for a tile's expert crosses 64), about nine hundred tiles of 128 columns
+        sizes, N = torch.randint(0, 2 * bm // 3, (130,), generator=g).tolist(), 904
+        sizes[64], sizes[129] = 0, bm + 1
+    else:
+        sizes, N = [0, 1, 128, 129, 77, 300, 0, 16], 392
+    a, b, a_s, b_s, ptr = _ragged_inputs(sizes, N, K, K, total_extra=3)
+    dev = [t.to(device) for t in (a, b, a_s, b_s, ptr)]
+    for dtype in (torch.bfloat16, torch.float32, torch.float16, FP8):
+        out, base = (torch.zeros(a.shape[0], N, device=device).to(dtype) for _ in range(2))
+        _lib.fp8_ragged_gemm(out, *dev, {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "ROW_GROUPS": 1})
+        cfg = used("tiled")
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["ROW_GROUPS"]) == (bm, bn, 1), cfg
+        _lib.fp8_ragged_gemm(base, *dev, {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128})
+        assert _lib.last_config()["ROW_GROUPS"] != 1
+        assert torch.equal(out.view(torch.uint8), base.view(torch.uint8)), dtype
+    if not many:
+        res = torch.zeros(a.shape[0], N, dtype=torch.bfloat16, device=device)
+        _lib.fp8_ragged_gemm(res, *dev, {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "ROW_GROUPS": 1})
+        check(res[: sum(sizes)], R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr)[: sum(sizes)], what=f"ragged ring {bm}x{bn} K={K}")
+    odd = torch.zeros(a.shape[0], N - 5, dtype=torch.bfloat16, device=device)
+    want = torch.zeros_like(odd)
+    bo, so = b[:, : N - 5].contiguous().to(device), dev[3]
+    _lib.fp8_ragged_gemm(odd, dev[0], bo, dev[2], so, dev[4], {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "ROW_GROUPS": 1})
+    _lib.fp8_ragged_gemm(want, dev[0], bo, dev[2], so, dev[4], {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128})
+    assert torch.equal(odd, want)
+
+
+@pytest.mark.parametrize("rows,want", [(40, None), (400, None), (401, (32, 128)), (1500, (64, 128)), (2000, (128, 128))])  # None: streaming
+def test_ragged_ring_tiles_are_the_default_for_few_rows_per_expert(device, rows, want):
+    g = _g(rows)
+    E, N, K = 40, 512, 2048
+    sizes = torch.bincount(torch.randint(0, E, (rows,), generator=g), minlength=E).tolist()
+    a, b, a_s, b_s, ptr = _ragged_inputs(sizes, N, K, rows)
+    out = ragged_block_scaled_bmm(a.to(device), b.to(device), a_s.to(device), b_s.to(device), ptr.to(device), max(sizes))
+    cfg = used("tiled" if want else "stream")
+    if want:
+        assert (cfg["BLOCK_M"], cfg["BLOCK_N"]) == want and (cfg["ROW_GROUPS"] == 1) == (rows <= 40 * E), cfg
+    check(out, R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr), what=f"{rows} rows")
+
+
 # ----------------------------------------------------------------------------- MoE token gather
+@pytest.mark.parametrize("block_m,K", [(64, 640), (64, 1152), (128, 640), (128, 1152)])
+def test_moe_gather_on_ring_tiles(device, block_m, K):
+    """The persistent tiles of the gather form and of the form with the activation epilogue: several tiles on a workgroup, slots masked out
+    in the middle of an expert's rows, ids beyond the output's rows, an expert without tokens, routed weights.  Same bits as the kernels of one workgroup
+    per tile and as the two steps."""
+    g = _g(block_m + K)
+    T, E, N, top_k = 300, 40, 1792, 3
+    A, B = fp8_randn((T, K), g).to(device), fp8_randn((E, N, K), g, 0.5).to(device)
+    a_s, b_s = (torch.rand(T, K // 128, generator=g) * 0.05 + 0.01).to(device), (torch.rand(E, N // 128, K // 128, generator=g) + 0.1).to(device)
+    w, ids = W.moe_routing(T, E, top_k, seed=11)
+    ids[ids == 3] = 4
+    sorted_ids, expert_ids, post, _, _ = moe_align_block_size(ids.to(device), block_m, E)
+    sorted_ids = sorted_ids.clone()
+    hole = torch.rand(sorted_ids.numel(), generator=g) < 0.2
+    hole[:40] = True
+    sorted_ids[hole.to(device)] = T * top_k
+    num_valid = T * top_k - 37
+    wd = w.to(device)
+    for dtype in (torch.bfloat16, torch.float32):
+        got, want = (torch.zeros(num_valid, N, dtype=dtype, device=device) for _ in range(2))
+        for mul in (True, False):
+            _lib.fp8_moe_gemm(got, A, B, a_s, b_s, wd, sorted_ids, expert_ids, post, mul, top_k, block_m)
+            cfg = used("tiled")
+            assert cfg["ROW_GROUPS"] == 1 and cfg["BLOCK_M"] == block_m, cfg
+            _lib.fp8_moe_gemm(want, A, B, a_s, b_s, wd, sorted_ids, expert_ids, post, mul, top_k, block_m, {"BLOCK_M": 64, "BLOCK_N": 128})
+            assert _lib.last_config()["ROW_GROUPS"] != 1
+            assert torch.equal(got, want)
+    if block_m == 128:
+        c = want.to(torch.bfloat16)
+        _lib.fp8_moe_gemm(c, A, B, a_s, b_s, wd, sorted_ids, expert_ids, post, False, top_k, block_m, {"BLOCK_M": 64, "BLOCK_N": 128})
+        q2, s2 = _lib.silu_mul_quant_1x128(c)
+        q, s = _lib.fp8_moe_gemm_silu_quant(A, B, a_s, b_s, sorted_ids, expert_ids, post, top_k, block_m, num_valid, torch.bfloat16)
+        assert _lib.last_config()["ROW_GROUPS"] == 1
+        live = sorted_ids[(sorted_ids >= 0) & (sorted_ids < num_valid)].long()
+        assert torch.equal(q.view(torch.uint8)[live], q2.view(torch.uint8)[live]) and torch.equal(s[live], s2[live])
+
+
+@pytest.mark.parametrize("T,H,I,E,k", [(200, 1024, 1024, 16, 2), (150, 1152, 640, 40, 4), (300, 640, 1024, 24, 3), (90, 1024, 512, 8, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_moe_layer_on_64_row_blocks(device, T, H, I, E, k, dtype, monkeypatch):
+    """Up to 47 rows per expert the one-call layer pads experts to 64 rows and runs on the ring tiles (GEMM2 on 64 x 128 tiles where its K
+    is too short for them); ids outside [0, E) included.  Same bits as the call-by-call layer on 128-row blocks."""
+    from tilegym_amd.ops import fused_moe, moe_interface
+
+    g = _g(T + H + I)
+    x = torch.randn(T, H, generator=g).to(dtype).to(device)
+    w1, w2 = fp8_randn((E, 2 * I, H), g, 0.5).to(device), fp8_randn((E, H, I), g, 0.5).to(device)
+    s1, s2 = (torch.rand(E, 2 * I // 128, H // 128, generator=g) * 0.02).to(device), (torch.rand(E, H // 128, I // 128, generator=g) * 0.02).to(device)
+    tw, ids = W.moe_routing(T, E, k, seed=5)
+    ids[5, 0], ids[7, k - 1] = -1, E
+    args = (x, w1, w2, tw.to(device), ids.to(device))
+    got = fused_moe(*args, w1_scale=s1, w2_scale=s2)
+    assert T * k > E * 7   # (past the decoding form)
+    monkeypatch.setattr(_lib, "native", None)
+    monkeypatch.setattr(moe_interface, "USE_ONE_CALL_LAYER", False)
+    assert torch.equal(got, fused_moe(*args, w1_scale=s1, w2_scale=s2))
+
+
 @pytest.mark.parametrize("block_m", [64, 128, 16, 256])
 @pytest.mark.parametrize("mul_w", [False, True])
 def test_moe_gather_gemm(device, block_m, mul_w):

@@ -88,6 +88,10 @@ constexpr int kTargetWaves = 4096;                  // 16 waves on each of 256 C
 // ragged GEMM: up to this many rows in all take the streaming form (config 5's weights, 64 experts: 6 rows 11.9 / 7.1 us
 // against 16.6 / 12.5 for the 64x128 tiles; 24 rows 26.0 / 16.1 against 23.0 / 16.1; 96 rows 60.6 / 35.5 against 59.9 / 32.8)
 constexpr int64_t kRaggedStreamRows = 8;
+// ... and, up to 10 rows per expert, problems that this form reads in at most 384 workgroups of 64 weight rows (every expert with rows counted): the
+// tiles leave compute units idle there (us, streaming / tiles: 8 experts of (1024, 896), 60 rows 5.5 / 9.4, 16 of (1024, 4096), 48
+// rows 14.6 / 19.7, 8 of (2816, 2432), 75 rows 12.9 / 14.7; above 384 it is up to 1.37 x behind).
+constexpr int64_t kRaggedStreamMean = 10, kRaggedStreamGroups = 384;
 constexpr int64_t kBs256WeightLimit = ((int64_t)1 << 32) - 1;  // the persistent block-scaled kernel addresses all experts' weights with one 32-bit offset
 
 // Switches to the caller's device for the lifetime of a call.
@@ -685,6 +689,13 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     return s;
 }
 
+// No tile, form or wave count asked for (a kernel family may be).
+bool nothing_forced_but_kernel(const int32_t* cfg, int32_t ncfg) {
+    for (int slot : {TG_CFG_BLOCK_M, TG_CFG_BLOCK_N, TG_CFG_ROW_GROUPS, TG_CFG_WAVES})
+        if (cfg_get(cfg, ncfg, slot) >= 0) return false;
+    return true;
+}
+
 // No kernel, tile, split or wave count asked for.
 bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
     for (int slot : {TG_CFG_KERNEL, TG_CFG_BLOCK_M, TG_CFG_BLOCK_N, TG_CFG_SPLIT_K, TG_CFG_ROW_GROUPS, TG_CFG_WAVES})
@@ -773,6 +784,66 @@ int64_t grouped_row_tiles(int64_t rows, int64_t experts) { return rows / 128 + s
 // 88.5 against 95.5).
 constexpr int64_t kPairTiles = 200;
 bool pair_tiles(int64_t rows, int64_t experts, int64_t col_tiles) { return grouped_row_tiles(rows, experts) * col_tiles >= kPairTiles; }
+
+// ---- the persistent ring tiles of the grouped GEMMs (fp8_gemm_grouped_ring.h)
+struct RingTile { int bm, bn; };  // bm 0: another kernel's problem
+bool grouped_ring_takes(const tg::GemmParams& p, int group, int bm, int bn) {
+    const bool exists = group == tg::GROUP_GATHER_ACT ? bn == 256 && (bm == 64 || bm == 128)
+                                                      : (bm == 32 && bn == 128) || (bm == 64 && (bn == 128 || bn == 192 || bn == 256)) || (bm == 128 && (bn == 192 || bn == 256));
+    return exists && p.As && p.Bs && p.K % 128 == 0 && p.kblocks >= tg::grouped_ring_steps(bn) && (group != tg::GROUP_RAGGED || p.E <= 256);
+}
+// Tiles of bm rows that `rows` rows spread evenly, but for their own noise, over E experts make.
+double expected_row_tiles(int64_t rows, int64_t E, int bm) {
+    const double mu = (double)rows / (double)E;
+    if (mu < 8.0) {  // experts with any rows, and one standard deviation more: a round of few tiles costs as much as a full one
+        const double none = exp(-mu);
+        return std::min((double)E, (double)E * (1.0 - none) + sqrt((double)E * none * (1.0 - (1.0 + mu) * none)));
+    }
+    static const double at[5] = {-1.6, -0.67, 0.0, 0.67, 1.6}, weight[5] = {0.125, 0.25, 0.25, 0.25, 0.125};
+    double tiles = 0.0;
+    for (int i = 0; i < 5; ++i) tiles += weight[i] * (double)cdiv(std::max<int64_t>((int64_t)llround(mu + at[i] * sqrt(mu)), 1), bm);
+    return tiles * (double)E;
+}
+// Weight bytes of the experts that have rows, about.
+double expected_weight_bytes(int64_t rows, int64_t E, int64_t N, int64_t K) {
+    return (double)E * (1.0 - exp(-(double)rows / (double)E)) * (double)N * (double)K;
+}
+// Up to 40 rows per expert, and up to 116 where the experts' weights (256 MB and more) come from memory anyway: while one row tile per
+// expert holds nearly all of them.  Measured over 2200 ragged problems (8 to 128 experts) against the best of all
+// the other kernels: up to one row per expert 2 % ahead on average, 1 - 10 rows 6 %, 10 - 40 5 %, 40 - 116 2 %, at best 35 % (against
+// the choice among those kernels 8 - 15 %, 3 % from 40 rows on).  With smaller weights and 40 rows the kernels of one workgroup per tile are up to 1.36 x ahead (two of
+// them multiply on a compute unit), above 116 rows up to 1.35 x.
+// Little weight to read (below 80 MB; 30 MB if all tiles of 128 columns run at once) leaves nothing for the ring to hide: 128 x 128 or pairs are
+// 1.06 - 1.2 x ahead (600 problems).
+// 32 rows to 18 per expert, 64 to 47; 128, 192 or 256 columns by the rounds that 256 workgroups need (a round costs its columns + 16).
+RingTile grouped_ring_tile(const tg::GemmParams& p, int group, int64_t rows, int block_m) {
+    const int64_t E = p.E, N = group == tg::GROUP_GATHER_ACT ? 2 * (int64_t)p.inter : (int64_t)p.N;
+    const double mu = (double)rows / (double)E, bytes = (double)E * (double)N * (double)p.K;
+    if (mu > 116.0 || (mu > 40.0 && bytes < 256e6)) return RingTile{0, 0};
+    const double touched = expected_weight_bytes(rows, E, N, p.K);
+    auto cost = [&](int bm, int bn) {
+        const double rounds = ceil(expected_row_tiles(rows, E, bm) * (double)cdiv(N, bn) / 256.0 - 0.01);
+        return (rounds < 1.0 ? 1.0 : rounds) * (double)(bn + 16);
+    };
+    RingTile best{0, 0};
+    double best_cost = 0.0;
+    auto offer = [&](int bm, int bn) {
+        if ((block_m > 0 && block_m != bm) || !grouped_ring_takes(p, group, bm, bn)) return;
+        const double c = cost(bm, bn);
+        if (group == tg::GROUP_RAGGED && touched < (bn == 128 && c <= 128.0 + 16.0 ? 30e6 : 80e6)) return;
+        if (best.bm == 0 || c < best_cost) { best = RingTile{bm, bn}; best_cost = c; }
+    };
+    if (block_m == 128 || (block_m == 0 && mu > 47.0)) {
+        offer(128, 256);
+        offer(128, 192);
+    } else {
+        if (block_m == 0) offer(mu <= 18.0 ? 32 : 64, 128);
+        else offer(block_m, 128);
+        offer(64, 256);
+        offer(64, 192);
+    }
+    return best;
+}
 
 struct Resolved {
     int64_t M, N, K;
@@ -1360,7 +1431,9 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
     // KERNEL = stream asks for it at any row count, KERNEL = tiled for the tile kernels below.
     const int want_kernel = cfg_get(cfg, ncfg, TG_CFG_KERNEL);
     const bool stream_ok = p.As && p.Bs && N * K < ((int64_t)1 << 31) && E <= 65535;
-    if (stream_ok && (want_kernel == 3 || (want_kernel < 0 && total_m <= kRaggedStreamRows))) {
+    const bool few_streams = total_m <= kRaggedStreamMean * E && std::min(total_m, E) * cdiv(N, 64) <= kRaggedStreamGroups &&
+                             nothing_forced_but_kernel(cfg, ncfg);
+    if (stream_ok && (want_kernel == 3 || (want_kernel < 0 && (total_m <= kRaggedStreamRows || few_streams)))) {
         s.kernel = 3; s.row_groups = 4; s.waves = 4;
         // Waves (16 weight rows each) per workgroup: WAVES = 4 / 6 / 8, else the fewest that give the fewest rounds of 256
         // workgroups with rows -- at most one grid row per routed row.  One token of config 5 (six experts): gate+up
@@ -1383,14 +1456,31 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
         return TG_OK;
     }
     int bm = cfg_get(cfg, ncfg, TG_CFG_BLOCK_M), bn = cfg_get(cfg, ncfg, TG_CFG_BLOCK_N);
+    // experts with few rows: the persistent ring tiles (ROW_GROUPS = 1 with one of their tiles asks for them)
+    RingTile ring = grouped_ring_tile(p, tg::GROUP_RAGGED, total_m, 0);
+    const bool ring_forced = bm > 0 && bn > 0 && cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS) == 1 && grouped_ring_takes(p, tg::GROUP_RAGGED, bm, bn);
+    if (ring_forced) ring = RingTile{bm, bn};
+    if (ring.bm > 0 && (ring_forced || nothing_forced_but_kernel(cfg, ncfg))) {
+        s.kernel = 1; s.bm = ring.bm; s.bn = ring.bn; s.row_groups = 1;
+        remember(s);
+        const hipError_t e = tg::run_grouped_ring(ring.bm, ring.bn, tg::GROUP_RAGGED, p, stream);
+        if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "grouped kernel launch failed: %s", hipGetErrorString(e));
+        return TG_OK;
+    }
     if (!(bm > 0 && bn > 0 && grouped_tile_exists(bm, bn))) {
-        // 64 x 128 tiles below 40 rows per expert (69 us against 80 at 24 rows); from there on, if there are enough of them, pairs
+        // Below 40 rows per expert, what the ring tiles leave: short K over 30 MB of weights and more in pairs of 128 x 256 tiles (two tiles'
+        // set-ups on a compute unit hide each other), else 128 x 128 (500 problems: each within 2 % of the best on average, 64 x 128
+        // 1.05 - 1.4 x behind), 64 x 128 where the weights take longest (69 us against 80 at 24 rows).  From there on, if there are enough of them, pairs
         // of 128 x 256 tiles or 256 x 256 tiles, whichever the padding of the experts' last tiles makes cheaper (64 experts of
         // (2816, 2048), us, 128 x 128 / pairs / 256 x 256: 94 rows 95.5 / 88.5 / 98.1, 188 rows 132 / 119 / 115, 281 rows 183 /
-        // 159 / 171); few tiles: 128 x 128 below 96 rows, 256 x 256 above
+        // 159 / 171); fewer than 240 tiles of 128 x 256: 128 x 128, but for the persistent form's problems (8 experts of (3072, 3072) at 192
+        // rows 27.1 against 43.9 us with 256 x 256, 16 of (1664, 1024) at 100 rows 12.4 against 20.5, 8 of (1280, 1792) at 271 rows 17.3 against
+        // 31.2; over 170 such problems 1.19 x)
         const int64_t mean = total_m / E;
-        if (mean < 40) { bm = 64; bn = 128; }
-        else if (N < 256 || (mean < 96 && !pair_tiles(total_m, E, cdiv(N, 256)))) { bm = 128; bn = 128; }
+        const double touched = expected_weight_bytes(total_m, E, N, K);
+        if (mean < 40 && p.kblocks < 8 && touched >= 30e6 && N >= 256) { bm = 128; bn = 256; }
+        else if (mean < 40) { bm = touched >= 80e6 ? 64 : 128; bn = 128; }
+        else if (N < 256 || ((mean <= 256 || p.kblocks > 12) && grouped_row_tiles(total_m, E) * cdiv(N, 256) < kPairTiles * 6 / 5)) { bm = 128; bn = 128; }
         else if (pair_tiles(total_m, E, cdiv(N, 256)) && grouped_cost(total_m, E, true) <= grouped_cost(total_m, E, false)) { bm = 128; bn = 256; }
         else { bm = 256; bn = 256; }
     }
@@ -1403,11 +1493,12 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
     // 256x256: the persistent form (one workgroup per compute unit walks the tiles, the operand rings run on across tiles)
     // hides a tile's set-up and first loads behind the previous tile, which pays for short tiles: measured on 64 experts,
     // 24576 rows, 104 vs 112 us at K = 1408 (11 steps per tile), but 215 vs 196 us at K = 2048 (16 steps), where the
-    // hardware's dispatch of one workgroup per tile balances the partly filled row tiles better than a fixed walk.
+    // hardware's dispatch of one workgroup per tile balances the partly filled row tiles better than a fixed walk.  Below 192 rows per
+    // expert it does so at any K (64 - 128 rows 1.04 - 1.2 x, 128 - 192 1.01 - 1.09 x, even from 192 on; 700 problems of K <= 1536).
     // ROW_GROUPS = 1 asks for it, WAVES = 8 for the kernel of one workgroup per tile.
     const int want_form = cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS);
     const bool persistent = bm == 256 && bn == 256 && p.As && p.Bs && tg::bs256_takes_k(p.kblocks) && E * N * K < kBs256WeightLimit &&
-                            cfg_get(cfg, ncfg, TG_CFG_WAVES) != 8 && (want_form == 1 || (want_form < 0 && p.kblocks <= 12));
+                            cfg_get(cfg, ncfg, TG_CFG_WAVES) != 8 && (want_form == 1 || (want_form < 0 && p.kblocks <= 12 && total_m / E >= 192));
     if (persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
     hipError_t e = persistent ? tg::run_bs256(tg::GROUP_RAGGED, p, (int)gx, stream)
                               : tg::run_tile_block_grouped(bm, bn, tg::GROUP_RAGGED, p, (int)gx, stream);
@@ -1482,21 +1573,24 @@ int32_t tg_fp8_moe_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor*
         if (tg::run_generic(q, stream) != hipSuccess) return fail(TG_ERR_LAUNCH, "fallback kernel launch failed");
         return TG_OK;
     }
+    const RingTile ring = nothing_forced_but_kernel(cfg, ncfg) ? grouped_ring_tile(p, tg::GROUP_GATHER, num_valid, block_m) : RingTile{0, 0};
+    if (ring.bm > 0) { bm = ring.bm; bn = ring.bn; s.row_groups = 1; }
     s.kernel = 1; s.bm = bm; s.bn = bn;
     remember(s);
     const int64_t gx = cdiv(EM, bm) * cdiv(N, bn);
     if (gx > INT32_MAX) return fail(TG_ERR_INVALID, "too many tiles");
-    hipError_t e = tg::run_tile_block_grouped(bm, bn, tg::GROUP_GATHER, p, (int)gx, stream);
+    hipError_t e = ring.bm > 0 ? tg::run_grouped_ring(bm, bn, tg::GROUP_GATHER, p, stream)
+                               : tg::run_tile_block_grouped(bm, bn, tg::GROUP_GATHER, p, (int)gx, stream);
     if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "grouped kernel launch failed: %s", hipGetErrorString(e));
     return TG_OK;
 }
 
-int32_t tg_fp8_moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, const tg_tensor* a, const tg_tensor* b,
+// Body of tg_fp8_moe_gemm_silu_quant; block_m = 64 too, for the layer that has made sure that the ring tiles take the problem.
+static int32_t moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, const tg_tensor* a, const tg_tensor* b,
                                    const tg_tensor* a_scale, const tg_tensor* b_scale,
                                    const tg_tensor* sorted_token_ids, const tg_tensor* expert_ids,
                                    const tg_tensor* num_tokens_post_padded, int32_t top_k, int32_t block_m,
                                    int32_t act_dtype, int32_t device_id, uint64_t hip_stream) {
-    g_err[0] = 0;
     int32_t rc;
     if ((rc = check_tensor(a, "a", 2)) || (rc = check_tensor(b, "b", 3)) || (rc = check_tensor(q, "q", 2)) ||
         (rc = check_tensor(scales, "scales", 2)) || (rc = check_tensor(a_scale, "a_scale", 2)) ||
@@ -1515,7 +1609,6 @@ int32_t tg_fp8_moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, 
     if (N % 2 || I % 128 || I == 0) return fail(TG_ERR_INVALID, "b must hold 2*I rows per expert with I a positive multiple of 128 (got %lld)", (long long)N);
     if (K % 128 || K == 0 || K > 65536) return fail(TG_ERR_INVALID, "K must be a multiple of 128 in [128, 65536]");
     if (top_k <= 0) return fail(TG_ERR_INVALID, "top_k must be positive");
-    if (block_m <= 0 || block_m % 128) return fail(TG_ERR_INVALID, "block_m must be a positive multiple of 128 for the fused form");
     const int64_t num_valid = q->shape[0];
     if (q->shape[1] != I) return fail(TG_ERR_INVALID, "q must have %lld columns", (long long)I);
     if (num_valid > T * top_k) return fail(TG_ERR_INVALID, "q has %lld rows but a provides only %lld slots", (long long)num_valid, (long long)(T * top_k));
@@ -1563,14 +1656,28 @@ int32_t tg_fp8_moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, 
     p.act_scales = reinterpret_cast<float*>(scales->ptr);
     p.act_is_bf16 = act_dtype == TG_BF16 ? 1 : 0;
 
-    const int bm = block_m % 256 == 0 ? 256 : 128;  // a row tile must not span two alignment blocks (experts)
-    Schedule s{1, bm, 256, 1, -1, -1, -1};
+    int bm = block_m % 256 == 0 ? 256 : 128;  // a row tile must not span two alignment blocks (experts)
+    RingTile ring = grouped_ring_tile(p, tg::GROUP_GATHER_ACT, num_valid, block_m);
+    if (ring.bm == 0 && block_m == 64) ring = RingTile{64, 256};
+    if (ring.bm > 0) bm = ring.bm;
+    Schedule s{1, bm, 256, 1, ring.bm > 0 ? 1 : -1, -1, -1};
     remember(s);
     const int64_t gx = cdiv(EM, bm) * (I / 128);
     if (gx > INT32_MAX) return fail(TG_ERR_INVALID, "too many tiles");
-    hipError_t e = tg::run_tile_moe_act(bm, pair_tiles(num_valid, E, I / 128), p, (int)gx, stream);
+    hipError_t e = ring.bm > 0 ? tg::run_grouped_ring(bm, 256, tg::GROUP_GATHER_ACT, p, stream) : tg::run_tile_moe_act(bm, pair_tiles(num_valid, E, I / 128), p, (int)gx, stream);
     if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "fused MoE kernel launch failed: %s", hipGetErrorString(e));
     return TG_OK;
+}
+
+int32_t tg_fp8_moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, const tg_tensor* a, const tg_tensor* b,
+                                   const tg_tensor* a_scale, const tg_tensor* b_scale,
+                                   const tg_tensor* sorted_token_ids, const tg_tensor* expert_ids,
+                                   const tg_tensor* num_tokens_post_padded, int32_t top_k, int32_t block_m,
+                                   int32_t act_dtype, int32_t device_id, uint64_t hip_stream) {
+    g_err[0] = 0;
+    if (block_m <= 0 || block_m % 128) return fail(TG_ERR_INVALID, "block_m must be a positive multiple of 128 for the fused form");
+    return moe_gemm_silu_quant(q, scales, a, b, a_scale, b_scale, sorted_token_ids, expert_ids, num_tokens_post_padded, top_k, block_m,
+                               act_dtype, device_id, hip_stream);
 }
 
 // argument checks of moe_align_block_size (host side only); n = number of (token, slot) pairs, cap = len(sorted_token_ids)
@@ -1909,6 +2016,7 @@ MoeDecode moe_decode(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I) {
     d.takes = tg::moe_decode_fits(d.up, true, (int)T) && tg::moe_decode_fits(d.down, false, (int)T);
     return d;
 }
+const float kAny = 1.0f, *const kNotNull = &kAny;  // (a scale tensor that is there, where only that matters)
 MoeLayout moe_layout(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I, int64_t block_m, int64_t elem16) {
     MoeLayout l{};
     auto take = [&](int64_t bytes) { const int64_t at = l.total; l.total += (bytes + 255) / 256 * 256; return at; };
@@ -1995,7 +2103,7 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
     if ((2 * I) % 256 != 0 || H % 128 != 0) return fail(TG_ERR_INVALID, "this entry point needs 2I %% 256 == 0 and H %% 128 == 0");
     if (T == 0) return TG_OK;
     const int64_t elem16 = 2;
-    const MoeLayout l = moe_layout(T, k, E, H, I, block_m, elem16);
+    MoeLayout l = moe_layout(T, k, E, H, I, block_m, elem16);
     if (l.cap > INT32_MAX) return fail(TG_ERR_INVALID, "too many (token, slot) pairs");
     if (numel(workspace) * elem_size(workspace->dtype) < l.total)
         return fail(TG_ERR_INVALID, "workspace holds %lld bytes, the layer needs %lld", (long long)(numel(workspace) * elem_size(workspace->dtype)),
@@ -2043,6 +2151,18 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
         if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "decoding MoE launch failed: %s", hipGetErrorString(e));
         return TG_OK;
     }
+    // Up to 47 rows per expert the experts are padded to 64 rows, for the ring tiles of 64 rows, if the layer's layout with such blocks fits the
+    // workspace of the caller's.
+    if (block_m == 128 && T * k <= 47 * E) {
+        tg::GemmParams up{};
+        up.As = up.Bs = kNotNull;
+        up.E = (int)E; up.N = (int)(2 * I); up.K = (int)H; up.inter = (int)I; up.kblocks = (int)(H / 128);
+        const MoeLayout narrow = moe_layout(T, k, E, H, I, 64, elem16);
+        if (narrow.total <= l.total && grouped_ring_tile(up, tg::GROUP_GATHER_ACT, T * k, 64).bm == 64) {
+            l = narrow;
+            block_m = 64;
+        }
+    }
     const tg_tensor sorted_ids = describe(ws, l.sorted_ids, TG_I32, {l.cap});
     const tg_tensor expert_ids = describe(ws, l.expert_ids, TG_I32, {l.nblk});
     const tg_tensor post = describe(ws, l.post, TG_I32, {1});
@@ -2058,7 +2178,7 @@ int32_t tg_fp8_fused_moe(const tg_tensor* out, const tg_tensor* hidden, const tg
     if ((rc = tg_moe_align_quant_1x128(topk_ids, block_m, (int32_t)E, &sorted_ids, &expert_ids, &post, &cumsum, &max_count, &xq, &xs, hidden,
                                        device_id, hip_stream)))
         return rc;
-    if ((rc = tg_fp8_moe_gemm_silu_quant(&q2, &s2, &xq, w1, &xs, w1_scale, &sorted_ids, &expert_ids, &post, (int32_t)k, block_m, hidden->dtype,
+    if ((rc = moe_gemm_silu_quant(&q2, &s2, &xq, w1, &xs, w1_scale, &sorted_ids, &expert_ids, &post, (int32_t)k, block_m, hidden->dtype,
                                          device_id, hip_stream)))
         return rc;
     if ((rc = tg_fp8_moe_gemm(&c3_rows, &q2, w2, &s2, w2_scale, &weights_flat, &sorted_ids, &expert_ids, &post, 1, 1, block_m, nullptr, 0,
