@@ -618,6 +618,49 @@ def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
     check(out[:, cols.to(device)], R.ref_gemm_per_tensor(a, b[cols], 0.01, 0.02, trans_b=True, out_dtype=torch.float16), what=f"M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("block_scaled", [False, True])
+@pytest.mark.parametrize("M,N,K,want", [(16, 25616, 4096, (32, 128)), (17, 25616, 4096, (32, 128)), (33, 32768, 4096, (64, 128)), (64, 25604, 4096, (64, 128)),
+                                        (16, 16360, 8192, (32, 64)), (50, 14728, 8192, (64, 64)), (65, 25616, 4096, (96, 128)), (128, 25616, 4096, (128, 128)),
+                                        (160, 25616, 4096, (160, 128)), (256, 25616, 4096, (256, 128)), (250, 20112, 5120, (256, 128))])
+def test_ring_tiles_over_weights_from_memory(device, block_scaled, M, N, K, want):
+    """Weights of 100 MB and more on one row tile: workgroups start at different K steps and go round, over chunks of activation scales
+    that end inside the round; N that ends inside a tile, first and last row counts of the tiles.  Small integers and scales
+    that are powers of two: every sum is exact in fp32, whatever its order."""
+    if block_scaled and M > 160:
+        pytest.skip("per-tensor tiles")
+    g = torch.Generator(device=device).manual_seed(M + N)
+    a, b = (torch.randint(-2, 3, s, generator=g, device=device).float() for s in ((M, K), (N, K)))
+    a8, b8 = a.to(FP8), b.to(FP8)
+    if block_scaled:
+        sa, sb = (2.0 ** torch.randint(-1, 2, s, generator=g, device=device).float() for s in ((M, K // 128), ((N + 127) // 128, K // 128)))
+        a *= sa.repeat_interleave(128, 1)
+        b *= sb.repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+    else:
+        sa = sb = torch.full((1,), 0.5, device=device)
+    out = torch.full((M, N), float("nan"), device=device)
+    cfg = {"KERNEL": "tiled", "BLOCK_M": want[0], "BLOCK_N": want[1], "SPLIT_K": 1, "WAVES": 8}
+    if block_scaled or 17 <= M <= 64:  # (the library's own choice there)
+        cfg = None
+    _lib.fp8_gemm(out, a8, b8, sa, sb, False, True, 1.0, 0.0, cfg)
+    got = used("tiled")
+    assert (got["BLOCK_M"], got["BLOCK_N"], got["WAVES"], got["SPLIT_K"]) == want + (8, 1), got
+    assert torch.equal(out, (a @ b.t()) * (1.0 if block_scaled else 0.25))
+
+
+@pytest.mark.parametrize("M,N,K,want", [(8, 12288, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 14336, 4224, (32, 64)),
+                                        (8, 6144, 4096, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
+def test_block_scaled_decode_on_ring_tiles(device, M, N, K, want):
+    g = _g(M + N)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)
+    sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand(N // 128, K // 128, generator=g) * 0.1 + 0.01
+    out = w8a8_block_fp8_matmul(a.to(device), b.to(device), sa.to(device), sb.to(device), None, torch.bfloat16)
+    cfg = used("tiled" if want else "stream")
+    assert not want or (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["WAVES"]) == want + (8,), cfg
+    rows = torch.arange(0, N, 128 * 5)[:, None].add(torch.arange(128)).flatten()  # (whole scale blocks)
+    rows = rows[rows < N]
+    check(out[:, rows.to(device)], R.ref_w8a8_block_fp8_matmul(a, b[rows], sa, sb[::5], None, torch.bfloat16), what=f"M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("bm", [64, 96, 128, 160, 192])
 @pytest.mark.parametrize("dm,N,K,split", [(0, 256, 128, 1), (-1, 120, 1024, 1), (1, 136, 1152, 2), (17, 257, 2176, 1), (-33, 384, 2304, 2)])
 def test_ring_tiles_block_scaled(device, bm, dm, N, K, split):

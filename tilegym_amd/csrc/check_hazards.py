@@ -51,7 +51,7 @@ VGPR_SPILL_LIMITS = {"fp8_gemm_tile256_kernel": 0, "fp8_gemm_tile_ring_kernel": 
 # 1024-byte aligned, so one static variable would take 1 KiB).
 NO_STATIC_LDS = ("moe_decode_kernel", "moe_decode_sum_kernel")
 # translation units with inline-assembly memory instructions
-DEFAULT_SOURCES = ["fp8_gemm_tile_pt.hip", "fp8_gemm_tile256.hip", "fp8_gemm_tile_ring.hip", "fp8_gemm_tile_bs.hip", "fp8_gemm_tile_bs256.hip", "fp8_gemm_tile_bs320.hip",
+DEFAULT_SOURCES = ["fp8_gemm_tile_pt.hip", "fp8_gemm_tile256.hip", "fp8_gemm_tile_ring.hip", "fp8_gemm_tile_ring_once.hip", "fp8_gemm_grouped_ring.hip", "fp8_gemm_tile_bs.hip", "fp8_gemm_tile_bs256.hip", "fp8_gemm_tile_bs320.hip",
                    "fp8_gemm_tile_grouped.hip", "fp8_gemm_tile_list.hip", "fp8_gemm_stream.hip", "fp8_moe_decode.hip"]
 
 

@@ -37,6 +37,13 @@
 // against the copy stands at pick_kn_tile.  Not kept: tiles dealt over the XCDs column by column in other orders (within 5 %
 // either way), weights fetched past the first-level cache (30 to 50 % slower).
 //
+// ONCE, for one row tile over a weight that comes from memory (100 MB and more: three sets of operands do not fit in the caches):
+// the weight loads are non-temporal, and workgroup b starts at K step b of its range and goes round -- rows a power of two apart
+// would put the requests of one moment on few memory channels.  The same products are added, in a rotated order.  28672 x 4096,
+// us before / after, per-tensor: 50 rows 27.5 / 23.4, 90 rows 30.1 / 26.2, 128 rows 32.1 / 28.8, 256 rows 40.2 / 35.6; block-scaled:
+// 16 rows 25.5 / 23.1, 50 rows 28.5 / 24.0.  Either alone 24 - 25.5 at 24 rows, both 22.3.  Smaller weights stay in the caches from one call to
+// the next and are up to 1.4 x slower with non-temporal loads; K that is no power of two is 3 - 5 % slower rotated and the same without.
+//
 // Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as
 // fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results.
 #pragma once
@@ -51,7 +58,7 @@ namespace tg {
 template <int BN>
 __device__ __forceinline__ int swz_kn(int r) { return BN == 64 ? ((r >> 2) & 1) | ((r >> 3) & 2) : ((r >> 1) & 3) | ((r >> 2) & 4); }
 
-template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool SPLIT, bool KN>
+template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool SPLIT, bool KN, bool ONCE>
 __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NL = 4, WGN = BN == 32 ? 1 : 2, WGM = 4 / WGN;  // four loading waves, four computing waves
@@ -92,6 +99,8 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
     }
     const int nsteps = ks_end - ks, last = ks_end - 1;
     if (nsteps <= 0) return;
+    // ONCE: first K step of this workgroup; step ks + k is the kth behind it, round the end of the range
+    const int turn = ONCE && (K & (K - 1)) == 0 ? pid % nsteps : 0;
 
     constexpr int kPro = (STAGES - 1) * PER_STEP, kLoop = (STAGES - 2) * PER_STEP;  // loads that may stay in flight
     static_assert(kPro < 64, "vmcnt has six bits");
@@ -127,16 +136,28 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
             if constexpr (BLOCKSCALE) {
                 const int g = min(ph * NL + lw, S_GROUPS - 1);
                 const int row = m0 + min(g * 8 + lrow, rows_valid - 1);
-                const int kb = min(ks + chunk * kScaleChunk + s_kbi, p.kblocks - 1);
+                int kb = ks + chunk * kScaleChunk + s_kbi;
+                if constexpr (ONCE) {
+                    kb += turn;
+                    if (kb > last) kb -= nsteps;
+                }
+                kb = min(kb, p.kblocks - 1);
                 direct_load_b32(rsrc_s, lds_address(s_as) + ((chunk & 1) * BM * kScaleChunk + g * 64) * 4,
                                 p.As ? ((uint32_t)row * (uint32_t)p.kblocks + (uint32_t)kb) * 4u : 0u, 0);
             }
         };
         auto issue = [&](int kstep, int stage) {
+            if constexpr (ONCE) {
+                kstep += turn;
+                if (kstep > last) kstep -= nsteps;
+            }
             const int k0 = min(kstep, last) * kKBlock;
             const uint32_t dst = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-            for (int i = 0; i < B_IT; ++i) direct_load_b128(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], KN ? k0 * p.N : k0);
+            for (int i = 0; i < B_IT; ++i) {
+                if constexpr (ONCE) direct_load_b128_nt(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], k0);
+                else direct_load_b128(rsrc_b, dst + BM * kKBlock + i * NL * 1024, b_off[i], KN ? k0 * p.N : k0);
+            }
 #pragma unroll
             for (int i = 0; i < A_IT; ++i) direct_load_b128(rsrc_a, dst + i * NL * 1024, a_off[i], k0);
         };
@@ -207,7 +228,12 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
             const float* cs = s_as + ((k / kScaleChunk) & 1) * (BM * kScaleChunk) + s_rbase + (((k % kScaleChunk) + li) & 7);
 #pragma unroll
             for (int tm = 0; tm < TM; ++tm) as_n[tm] = cs[tm * (WGM * 128)];
-            bs_n = s_bs[min(k, nsteps - 1)];
+            k = min(k, nsteps - 1);
+            if constexpr (ONCE) {
+                k += turn;
+                if (k >= nsteps) k -= nsteps;
+            }
+            bs_n = s_bs[k];
         }
     };
     if constexpr (BLOCKSCALE) {
@@ -358,8 +384,14 @@ __global__ void __launch_bounds__(512, 1) fp8_gemm_tile_ring_kernel(const GemmPa
 
 template <int BM, int BN, int STAGES, bool BLOCKSCALE, bool KN = false>
 inline hipError_t launch_tile_ring(bool split, const GemmParams& p, int gx, int gy, hipStream_t stream) {
-    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, true, KN>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
-    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false, KN>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    if (split) hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, true, KN, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false, KN, false>), dim3(gx, gy, 1), dim3(512, 1, 1), 0, stream, p);
+    return hipGetLastError();
+}
+
+template <int BM, int BN, int STAGES, bool BLOCKSCALE>
+inline hipError_t launch_tile_ring_once(const GemmParams& p, int gx, hipStream_t stream) {
+    hipLaunchKernelGGL((fp8_gemm_tile_ring_kernel<BM, BN, STAGES, BLOCKSCALE, false, false, true>), dim3(gx, 1, 1), dim3(512, 1, 1), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -256,8 +256,8 @@ constexpr StepCost kPerTensorTiles[] = {{32, 32, false, 0.106f, 0.122f, 0.f, 3.2
                                         {64, 128, true, 0.219f, 0.313f, 0.f, 3.087f, 0.060f}, {96, 128, true, 0.371f, 0.293f, 0.f, 3.990f, 0.102f},
                                         {128, 128, true, 0.344f, 0.387f, 0.f, 5.394f, 0.095f}, {160, 128, true, 0.496f, 0.552f, 0.f, 4.331f, 0.075f},
                                         {160, 192, true, 0.441f, 0.667f, 0.f, 6.211f, 0.064f}, {192, 192, true, 0.628f, 0.675f, 0.f, 8.253f, 0.061f},
-                                        {64, 32, true, 0.131f, 0.133f, 0.f, 2.836f, 0.f, 1280}, {32, 64, true, 0.131f, 0.133f, 0.f, 2.836f, 0.f, 1280},
-                                        {64, 64, true, 0.163f, 0.185f, 0.f, 2.980f, 0.f, 1280}, {256, 128, true, 0.409f, 0.761f, 0.f, 6.266f, 0.f, 1280}};
+                                        {64, 32, true, 0.131f, 0.133f, 0.f, 2.836f, 0.035f, 1280}, {32, 64, true, 0.131f, 0.133f, 0.f, 2.836f, 0.045f, 1280},
+                                        {64, 64, true, 0.163f, 0.185f, 0.f, 2.980f, 0.057f, 1280}, {256, 128, true, 0.409f, 0.761f, 0.f, 6.266f, 0.050f, 1280}};
 // (the 64 x 128 four-stage kernel's step over fewer columns: this share of it does not shrink with them)
 constexpr float kDeepTileRowsShare = 0.53f;
 // Block-scaled: fitted to 4 000 measurements (290 shapes, the same ranges).  On 585 others 1.1 % behind the best schedule on average,
@@ -269,7 +269,7 @@ constexpr StepCost kBlockScaledTiles[] = {{64, 128, false, 0.654f, 0.867f, 0.879
                                           {64, 128, true, 0.320f, 0.480f, 0.f, 2.58f, 0.f},     {96, 128, true, 0.428f, 0.492f, 0.f, 2.96f, 0.f},
                                           {128, 128, true, 0.483f, 0.595f, 0.f, 3.66f, 0.f},    {160, 128, true, 0.528f, 0.685f, 0.f, 4.37f, 0.f},
                                           {192, 128, true, 0.595f, 0.767f, 0.f, 4.59f, 0.f},
-                                          {32, 64, true, 0.171f, 0.169f, 0.f, 2.888f, 0.018f, 1280}, {64, 64, true, 0.208f, 0.218f, 0.f, 3.291f, 0.018f, 1280}};
+                                          {32, 64, true, 0.171f, 0.169f, 0.f, 2.888f, 0.040f, 1280}, {64, 64, true, 0.208f, 0.218f, 0.f, 3.291f, 0.050f, 1280}};
 // split_margin: a split schedule must be predicted this much faster than the best unsplit one.  odd_kib: what a ring tile's step takes
 // longer over weights from memory whose rows lie an odd number of KiB apart (64 x 128 tiles over 5120 x 5120 from memory 0.47 - 0.50 us a
 // step, over other weights of 25 MB 0.41).
@@ -277,6 +277,22 @@ struct TileModel { const StepCost* kinds; int n; float reduce_us, reduce_us_per_
 constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 3.272f, 0.316f, 1.0f, 0.018f};
 constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
+// The form of the ring tiles for weights that come from memory and are read once (ONCE in fp8_gemm_tile_ring.h): one row tile over
+// 100 MB or more.  K a power of two, where the rotated start pays; the 256-row tile at any K (20480 x 5120 44.9 -> 41.6 us at 256
+// rows, 14336 x 12288 70.2 -> 60.9), the others are 2 - 5 % behind the plain loads there.
+constexpr int64_t kMemoryWeight = 100000000;
+bool power_of_two(int64_t x) { return (x & (x - 1)) == 0; }
+bool read_once(int64_t M, int64_t N, int64_t K, bool block_scaled, int bm, int bn) {
+    if (M > bm || N * K < kMemoryWeight) return false;
+    if (bm == 256) return bn == 128 && !block_scaled;
+    return K >= 4096 && power_of_two(K) && (bm <= 64 ? bn == 64 || bn == 128 : bn == 128 && bm <= 160);
+}
+// ... and the columns of its tiles up to 64 rows: those that fill most of the compute units at once (0: neither does).
+int read_once_columns(int64_t N, int64_t K) {
+    if (N * K < kMemoryWeight || K < 4096 || !power_of_two(K)) return 0;
+    const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128);
+    return t128 >= 200 && t128 <= 256 ? 128 : t64 >= 230 && t64 <= 256 ? 64 : 0;
+}
 constexpr TileModel kSmallRowsRing{nullptr, 0, 2.6f, 0.25f, 1.0f, 0.f};  // (the reduction launch behind the ring tiles of up to 64 rows)
 
 // (cols: weight rows per tile where they are not the kind's own)
@@ -418,6 +434,9 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         auto fits = [&](int split) { return split == 1 || (int64_t)split * M * N * 4 <= partial_bytes_avail; };
         Schedule best{0, -1, -1, 1, -1, -1, -1};
         float best_us = 0.f;
+        // weights from memory on the ring tiles made for them (28672 x 4096, 24 rows: 28.9 -> 22.3 us per-tensor, 28.0 -> 23.1
+        // block-scaled; 16384 x 8192 26.7 -> 25.1 and 30.9 -> 24.9; 16384 x 16384 70 -> 44)
+        if (const int cols = want_split <= 1 ? read_once_columns(N, K) : 0) return Schedule{1, M <= 32 ? 32 : 64, cols, 1, -1, -1, 8};
         auto offer = [&](const Schedule& cand, float us) {
             if (best.kernel == 0 || us < best_us) { best = cand; best_us = us; }  // (no margin against splits here: measured better)
         };
@@ -434,24 +453,25 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                 if (want_split > 0) break;
             }
         }
-        // Per-tensor ring tiles of 32 and 64 rows, from 96 tiles on (with fewer most of the chip idles and the narrow tiles that split
-        // K are as fast: 24 x 4096 x 4096 7.0 against 7.3 us, 50 x 4096 x 4096 7.1 and 7.1), predicted at least 5 % faster than anything
-        // else.  32-row tiles run unsplit; 64 x 64 takes over above 32 rows.  24 x 12288 x 5120 17.1 -> 12.2 us, 50 x 12288 x 5120
-        // 19.8 -> 12.8, 50 x 4096 x 14336 18.8 -> 15.7 (with splits by four).  Fitted to 1777 shapes, weights of 1 to 310 MB, three sets
-        // of operands: 14 % ahead of the kinds above on average, more than 5 % behind on 29 at worst 1.2 x; above 160 MB the 64 x 72 ... 128 tiles,
-        // whose weights pass the caches by, are ahead by up to 1.35 x (60 x 18192 x 11008 50 against 68 us).
-        if (!block_scaled && K >= 1280 && N * K <= ((int64_t)160 << 20)) {
+        // Per-tensor ring tiles of 32 and 64 rows, predicted at least 5 % faster than anything else.  32-row tiles run unsplit; 64 x 64
+        // takes over above 32 rows.  24 x 12288 x 5120 17.1 -> 12.2 us, 50 x 12288 x 5120 19.8 -> 12.8, 50 x 4096 x 14336 18.8 -> 15.7
+        // (with splits by four).  From 150 workgroups on, 200 with a split: a weight that is not in the caches (one layer of many)
+        // asks for many workgroups that request it -- with 96 of them 50 x 6144 x 4096 takes 8.8 us against 9.9 for the tiles that split K
+        // in the workgroup if the weight was read just before, but 12.2 against 9.6 if not, 50 x 5120 x 12288 with two splits 16.9 against 19.9 and 25.2
+        // against 19.9; the shapes above 16.7 / 17.5, 21.3 / 20.7 and 18.4 / 18.9 from memory.  Short K and small weights are the other
+        // tiles' for the same reason (24 x 6144 x 2048 5.8 / 5.7 and 7.2 / 5.7), weights of 100 MB and more, too (60 x 18192 x 11008 68 / 50).
+        if (!block_scaled && K >= 1280 && N * K < kMemoryWeight) {
             constexpr StepCost rings[] = {{32, 64, true, 0.088f, 0.185f, 0.f, 3.312f, 0.011f}, {64, 64, true, 0.093f, 0.293f, 0.f, 3.394f, 0.f},
                                           {32, 128, true, 0.143f, 0.392f, 0.f, 3.273f, 0.019f}, {64, 128, true, 0.158f, 0.599f, 0.f, 3.219f, 0.f}};
             for (const StepCost& t : rings) {
-                if (t.bm == 64 && M <= 32) continue;
+                if ((t.bm == 64 && M <= 32) || (t.bm == 32 && M > 32 && (K < 4096 || K > 8192))) continue;
                 for (int sp = 1; sp <= 8; sp *= 2) {
                     const int split = want_split > 0 ? want_split : sp;
                     if (split > 1 && (t.bm == 32 || kblocks / split < 4 || !fits(split))) break;
                     Schedule cand{1, t.bm, t.bn, 1, -1, -1, 8};
                     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
                     if (split > 1) cand.split_k = pick_split(tiles, 256, kblocks, 4, M, N, partial_bytes_avail, split);
-                    if (tiles * cand.split_k >= 96) offer(cand, 1.05f * step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn));
+                    if (tiles >= 150 ? split == 1 : split >= 4 && tiles * cand.split_k >= 200) offer(cand, 1.05f * step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn));
                     if (want_split > 0) break;
                 }
             }
@@ -468,6 +488,9 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                     if (split > 1 && (kblocks / split < 4 || !fits(split))) break;
                     Schedule cand{1, t.bm, t.bn, 1, -1, -1, 8};
                     if (split > 1) cand.split_k = pick_split(cdiv(M, t.bm) * cdiv(N, t.bn), 256, kblocks, 4, M, N, partial_bytes_avail, split);
+                    // (above 25 MB fewer than 96 workgroups, above 40 MB fewer than 150 or two splits are slower from memory: 50 x 8192 x 8192 in 128 column tiles 14.5 us
+                    // against 17.8 if the weight was read just before, but 21.5 against 20.3 if not)
+                    if (N * K > 25000000 && want_split < 0 && (split == 1 ? cdiv(N, t.bn) < (N * K > 40000000 ? 150 : 96) : split == 2)) continue;
                     // (a split must be predicted 10 % faster: its reduction is a launch more for the host, too)
                     offer(cand, step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn) * (cand.split_k > 1 ? 1.1f : 1.f));
                     if (want_split > 0) break;
@@ -522,6 +545,20 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     // up to four rows against a weight of a few MB: the skinny kernel (no LDS, no barrier) is 4 - 19 % ahead of the
     // streaming one (2048 x 2048 block-scaled at M = 1: 4.17 against 4.94 us; per-tensor 4.21 against 4.53)
     if (nothing_forced && M <= 4 && N * K <= ((int64_t)5 << 20)) return skinny_schedule();
+    // block-scaled, up to 16 rows, where ring tiles of 32 rows fill the chip about once: the scale-and-adds of a row of weights are
+    // dealt out over a workgroup, where the streaming form's waves do them between two waits (us, streaming / ring, weight in the caches and from
+    // memory, 16 rows: 12288 x 5120 at 8 rows 15.6 / 12.4 and 15.6 / 15.0, 10240 x 5120 at 8 rows 15.0 / 11.1 and 14.9 / 14.1, 14336 x 4224 13.8 / 12.2 and 13.9 / 13.5,
+    // 20480 x 2048 14.4 / 10.0 and 14.3 / 10.9, 18432 x 7168 35.2 / 30.2, 28672 x 4096 25.5 / 23.1; more than eight rows also
+    // 6144 x 4096 11.6 / 8.8 and 11.3 / 11.2).  Outside the streaming form is ahead from memory: 8192 x 8192 13.8 for 17.0 but 18.5 for
+    // 16.9, and from K = 5120 on with more than eight rows (10240 x 5120 at 16 rows 17.1 for 15.7).
+    if (nothing_forced && block_scaled && tile_ok && M <= 16 && K >= 1280 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_M) <= 0 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
+        const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128), bytes = N * K;
+        int cols = read_once_columns(N, K);
+        if (cols == 0 && t64 >= 150 && t64 <= 256 && bytes <= 75000000 && (M <= 8 || K < 5120)) cols = 64;
+        if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 2048 && K < 5120 && bytes <= 40000000) cols = 64;
+        if (cols == 0 && t64 > 256 && t128 <= 256 && K <= 8192 && !(bytes >= kMemoryWeight && power_of_two(K))) cols = 128;
+        if (cols > 0) return Schedule{1, 32, cols, 1, -1, -1, 8};
+    }
     if (skinny && want_kernel != 2 && (want_kernel == 3 || K >= 1024)) {
         // weight streaming through LDS, 1 KiB of a row per load instruction
         s.kernel = 3;
@@ -1310,7 +1347,9 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
         const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
         const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
-        hipError_t e = block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
+        const bool once = (ring || block_ring) && !split && rows == M && trans_b && read_once(M, N, K, block_scaled, s.bm, s.bn);
+        hipError_t e = once ? tg::run_tile_ring_once(block_scaled, s.bm, s.bn, pc, gx, stream)
+                     : block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
                      : block_ring ? tg::run_tile_ring_block(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : ring && direct_kn ? tg::run_tile_ring_kn(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
                      : ring ? tg::run_tile_ring(s.bm, s.bn, split, pc, gx, pc.split_k, stream)
