@@ -647,7 +647,39 @@ def test_ring_tiles_over_weights_from_memory(device, block_scaled, M, N, K, want
     assert torch.equal(out, (a @ b.t()) * (1.0 if block_scaled else 0.25))
 
 
-@pytest.mark.parametrize("M,N,K,want", [(8, 12288, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 14336, 4224, (32, 64)),
+@pytest.mark.parametrize("block_scaled", [False, True])
+@pytest.mark.parametrize("M,N,K,form", [(1, 8208, 1024, 4), (8, 8208, 1152, 4), (3, 8192, 1024, 1), (3, 6160, 9344, 1), (1, 4096, 9344, 1)])
+def test_decode_streams_narrow_or_wide(device, block_scaled, M, N, K, form):
+    """Either side of 512 workgroups of 16 weight rows (from there on the wide form); over ten pieces of K with more workgroups than
+    compute units (one buffer per wave) and as many (eight waves)."""
+    g = _g(N + K)
+    a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.2)
+    rows = torch.arange(128 * 3)
+    if block_scaled:
+        sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand((N + 127) // 128, K // 128, generator=g) * 0.1 + 0.01
+        out = w8a8_block_fp8_matmul(a.to(device), b.to(device), sa.to(device), sb.to(device), None, torch.bfloat16)
+        ref = [R.ref_w8a8_block_fp8_matmul(a, b[:384], sa, sb[:3], None, torch.bfloat16)]
+    else:
+        out = matmul(a.to(device), b.to(device), trans_b=True, scale_a=0.01, scale_b=0.02, out_dtype=torch.bfloat16)
+        ref = [R.ref_gemm_per_tensor(a, r, 0.01, 0.02, trans_b=True, out_dtype=torch.bfloat16) for r in (b[:384], b[-40:])]
+    cfg = used("stream")
+    assert (cfg["ROW_GROUPS"] == 4) == (form == 4) or (block_scaled and K > 2048), cfg
+    check(out[:, rows.to(device)], ref[0], what=f"M={M} N={N} K={K}")
+    if not block_scaled:
+        check(out[:, -40:], ref[1], what=f"M={M} N={N} K={K}, last rows")
+
+
+def test_block_scaled_skinny_to_sixteen_rows(device):
+    for M, N, K, want in ((8, 4096, 1280, "skinny"), (9, 2048, 1280, "skinny"), (16, 2048, 1536, "skinny"), (8, 1024, 2176, "stream"), (9, 4096, 1024, "stream")):
+        g = _g(M + N)
+        a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.2)
+        sa, sb = torch.rand(M, K // 128, generator=g) * 0.1 + 0.01, torch.rand(N // 128, K // 128, generator=g) * 0.1 + 0.01
+        out = w8a8_block_fp8_matmul(a.to(device), b.to(device), sa.to(device), sb.to(device), None, torch.bfloat16)
+        used(want)
+        check(out, R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M,N,K,want", [(8, 10240, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 11008, 4096, (32, 64)),
                                         (8, 6144, 4096, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
 def test_block_scaled_decode_on_ring_tiles(device, M, N, K, want):
     g = _g(M + N)

@@ -544,17 +544,20 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     const bool nothing_forced = want_kernel < 0 && want_split < 0 && cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS) < 0 && cfg_get(cfg, ncfg, TG_CFG_WAVES) < 0;
     // up to four rows against a weight of a few MB: the skinny kernel (no LDS, no barrier) is 4 - 19 % ahead of the
     // streaming one (2048 x 2048 block-scaled at M = 1: 4.17 against 4.94 us; per-tensor 4.21 against 4.53)
-    if (nothing_forced && M <= 4 && N * K <= ((int64_t)5 << 20)) return skinny_schedule();
+    // block-scaled over short rows to eight (5 MB) and sixteen rows (3 MB; 8 rows, 2016 x 1024 3.7 against 5.2 us, 3984 x 1024 3.9 against
+    // 5.3; from K = 2560 on the streaming kernel is ahead again: 8 x 1200 x 3712 5.8 against 6.7)
+    const int64_t skinny_mb = M <= 4 ? 5 : block_scaled && K <= 2048 ? (M <= 8 ? 5 : M <= 16 ? 3 : 0) : 0;
+    if (nothing_forced && N * K <= skinny_mb << 20) return skinny_schedule();
     // block-scaled, up to 16 rows, where ring tiles of 32 rows fill the chip about once: the scale-and-adds of a row of weights are
     // dealt out over a workgroup, where the streaming form's waves do them between two waits (us, streaming / ring, weight in the caches and from
-    // memory, 16 rows: 12288 x 5120 at 8 rows 15.6 / 12.4 and 15.6 / 15.0, 10240 x 5120 at 8 rows 15.0 / 11.1 and 14.9 / 14.1, 14336 x 4224 13.8 / 12.2 and 13.9 / 13.5,
+    // memory, 16 rows: 10240 x 5120 at 8 rows 15.0 / 11.1 and 14.9 / 14.1, 12288 x 2048 8.0 / 7.4 and 8.0 / 7.6,
     // 20480 x 2048 14.4 / 10.0 and 14.3 / 10.9, 18432 x 7168 35.2 / 30.2, 28672 x 4096 25.5 / 23.1; more than eight rows also
     // 6144 x 4096 11.6 / 8.8 and 11.3 / 11.2).  Outside the streaming form is ahead from memory: 8192 x 8192 13.8 for 17.0 but 18.5 for
-    // 16.9, and from K = 5120 on with more than eight rows (10240 x 5120 at 16 rows 17.1 for 15.7).
+    // 16.9, 12288 x 5120 12.7 for 16.4 but 17.1 for 16.4, and from K = 5120 on with more than eight rows (10240 x 5120 at 16 rows 17.1 for 15.7).
     if (nothing_forced && block_scaled && tile_ok && M <= 16 && K >= 1280 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_M) <= 0 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
         const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128), bytes = N * K;
         int cols = read_once_columns(N, K);
-        if (cols == 0 && t64 >= 150 && t64 <= 256 && bytes <= 75000000 && (M <= 8 || K < 5120)) cols = 64;
+        if (cols == 0 && t64 >= 150 && t64 <= 256 && bytes <= 55000000 && (M <= 8 || K < 5120)) cols = 64;
         if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 2048 && K < 5120 && bytes <= 40000000) cols = 64;
         if (cols == 0 && t64 > 256 && t128 <= 256 && K <= 8192 && !(bytes >= kMemoryWeight && power_of_two(K))) cols = 128;
         if (cols > 0) return Schedule{1, 32, cols, 1, -1, -1, 8};
@@ -580,13 +583,15 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         if (wide_split > pieces) wide_split = pieces;
         if (wide_split > 16) wide_split = 16;
         if (wide_wgs >= 112 && pieces < 6) wide_split = 1;  // (8192 x 3072 at M = 16: 7.9 us unsplit, 9.5 with two splits)
-        // The wide form wins from 136 row blocks on (11008 x 4096 at M = 16: 11.1 us against 14.3 for the narrow form), and
+        // The wide form wins where the narrow one takes more than two workgroups of 16 rows per compute unit (11008 x 4096 at M = 16: 11.1
+        // us against 14.3 for the narrow form; at M = 1 8512 x 4352 14.9 against 9.9, 11632 x 1024 8.4 and 5.5, block-scaled 14416 x 1152 10.0 and
+        // 7.0), and
         // with fewer once the weight is large enough that the reduction launch is paid back: ~32 MB, ~24 MB at more than
         // eight rows where every narrow workgroup's own activation loads weigh more (6144 x 4096 at M = 16: 9.3 against
         // 9.6; 1536 x 24576: 10.4 - 11.9 against 13.5 - 19.4).  One to four rows over 96 - 135 row blocks stay narrow: its
         // 384 - 540 workgroups fill the chip without a reduction (8192 x 8192 at M = 1: 13.6 against 15.7).
-        bool wide_auto = N >= 16384 || (wide_wgs >= 136 && K >= 2048) ||
-                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= 176 && !(M <= 4 && wide_wgs >= 96));
+        bool wide_auto = N >= 16384 || N > 8192 ||
+                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= 160 && !(M <= 4 && wide_wgs >= 96));
         // Weight rows per workgroup of the two-piece wide form.  64 rows leave compute units idle when N / 64 is well below 256 or a little above it; fewer rows per
         // workgroup fill the chip in one launch where split-K needed a second one.  Cost of a choice ~ rounds of 256
         // workgroups x (rows + 16): 12288 x 5120 at M = 16 takes 12.6 us with 48 rows (256 workgroups) against 13.2 with
@@ -1298,8 +1303,10 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         const int64_t per_wave = cdiv(s.split_k > 1 ? p.ksteps_per_split : pieces, 4);
         int nbuf = cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS);  // stream kernel: LDS buffers per wave
         // measured: one 16 KiB buffer per wave and two workgroups per compute unit beat two buffers and
-        // one workgroup, except for long K where they tie
-        if (nbuf != 1 && nbuf != 2) nbuf = (per_wave >= 3 && s.mt == 1 && !block_scaled) ? 2 : 1;
+        // one workgroup, except for long K where they tie as long as there is no second workgroup (463 of them over 5552 x 11264 at three
+        // rows 20.7 us with two buffers, 14.6 with one; 415 over 6640 x 9600 20.7 and 15.1)
+        const int64_t narrow_wgs = cdiv(N, s.bn > 0 ? s.bn : 16) * s.split_k;
+        if (nbuf != 1 && nbuf != 2) nbuf = (per_wave >= 3 && s.mt == 1 && !block_scaled && narrow_wgs <= 256) ? 2 : 1;
         if (s.mt != 1 || s.waves == 8) nbuf = 1;
         if (s.row_groups == 4 && s.waves == 4 && s.bn > 0) p.wave_rows = s.bn / 4;
         if (s.row_groups != 4 && s.bn > 0) p.wave_rows = s.bn;  // narrow form: weight rows per workgroup
@@ -2045,6 +2052,10 @@ struct MoeDecode {
 MoeDecode moe_decode(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I) {
     MoeDecode d{};
     if (T <= 0 || T * k > tg::kMoeDecodeSlots || E > 512 || H % 128 != 0 || I % 128 != 0 || H > 65536 || I > 65536) return d;
+    // From 5.5 rows per expert on the ring tiles are as fast over 400 MB of weights and more when the rows are spread evenly, and ahead
+    // when they are not (64 experts of (2048, 1408), top 6, streaming / ring tiles: 64 tokens 106.7 / 107.9 us, half of them alike 125.8 / 106.6;
+    // 40 tokens 100.7 / 105.1 and 101.4 / 101.1).  Smaller layers fill fewer of the ring's rounds (24 of (3072, 1536), 7 rows 72.8 / 90.4).
+    if (2 * T * k > 11 * E && 3 * E * H * I >= 400000000) return d;
     d.up.slots = d.down.slots = (int)(T * k);
     d.up.top_k = d.down.top_k = (int)k;
     d.up.E = d.down.E = (int)E;
