@@ -2106,6 +2106,26 @@ def test_ragged_stream_form_is_the_default_for_one_token(device):
     used("tiled")
 
 
+@pytest.mark.parametrize("kc", [None, {"KERNEL": "stream"}, {"KERNEL": "tiled"}])
+@pytest.mark.parametrize("ptr", [[0, 7, 7, 18, 29], [0, 20, 24, 24, 29], [-5, 7, 7, 18, 20]])
+def test_ragged_segments_past_the_rows_are_contained(device, ptr, kc):
+    """An m_indptr that gives rows outside the 20 that A and C have: rows inside come out as documented (none of a segment that starts
+    below 0), and nothing is written past C.  Operands and result lie inside larger buffers, so that a missing clamp shows as a value."""
+    M, N, K, slack = 20, 256, 1024, 32
+    a, b, a_s, b_s, _ = _ragged_inputs([M + 2 * slack, 0, 0, 0], N, K, M)
+    big = torch.full((M + 2 * slack, N), 3.0, dtype=torch.bfloat16, device=device)
+    out = big[slack:slack + M]
+    _lib.fp8_ragged_gemm(out, a.to(device)[slack:slack + M], b.to(device), a_s.to(device)[slack:slack + M], b_s.to(device),
+                         torch.tensor(ptr, dtype=torch.int32, device=device), kc)
+    used("stream" if kc is None else kc["KERNEL"])
+    assert bool((big[:slack] == 3).all()) and bool((big[slack + M:] == 3).all())
+    a, a_s = a[slack:slack + M], a_s[slack:slack + M]
+    for e in range(4):
+        lo, hi = ptr[e], min(ptr[e + 1], M)
+        if 0 <= lo < hi:
+            check(out[lo:hi], R.ref_w8a8_block_fp8_matmul(a[lo:hi], b[e], a_s[lo:hi], b_s[e], None, torch.bfloat16), what=f"{ptr} expert {e}")
+
+
 @pytest.mark.parametrize("T", [1, 16, 64])
 @pytest.mark.parametrize("which", ["gate_up", "down"])
 def test_config5_moe_decode_regime(device, which, T):

@@ -623,8 +623,9 @@ __global__ void __launch_bounds__(64 * NW) fp8_gemm_stream_ragged_kernel(const G
     const int li = lane & 15, lg = lane >> 4;
     const int K = p.K, N = p.N;
     const int e = blockIdx.y;
-    const int row_lo = __builtin_amdgcn_readfirstlane(p.m_indptr[e]), row_hi = __builtin_amdgcn_readfirstlane(p.m_indptr[e + 1]);
-    if (row_hi <= row_lo) return;
+    // (rows outside the M that A and C have are nobody's, whatever m_indptr holds)
+    const int row_lo = __builtin_amdgcn_readfirstlane(p.m_indptr[e]), row_hi = min(__builtin_amdgcn_readfirstlane(p.m_indptr[e + 1]), p.M);
+    if (row_lo < 0 || row_hi <= row_lo) return;
     const int n_base = blockIdx.x * (16 * NW) + wave * 16;
     const int npieces = (K + PIECE - 1) / PIECE;
     const int tail_steps = (K % PIECE) / kKBlock;  // 0: every piece is whole
