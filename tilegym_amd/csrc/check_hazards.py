@@ -44,7 +44,8 @@ EARLY_USE_KNOWN = ("fp8_gemm_bs256_kernelILi0ELb1E", "fp8_gemm_bs256_kernelILi1E
 # Third check, of speed rather than correctness: vector registers spilled by the kernels whose loops are hand-scheduled.
 # A source change that looks harmless can push one of them over the register file (the TAIL forms went from 0 to
 # 129 / 216 spilled registers, and 2.7 times the run time, when their second K step was made unconditional).
-VGPR_SPILL_LIMITS = {"fp8_gemm_tile256_kernel": 0, "fp8_gemm_tile_ring_kernel": 0, "fp8_gemm_pair_kernel": 0, "fp8_gemm_bs320_kernel": 0,
+VGPR_SPILL_LIMITS = {"fp8_gemm_tile256_kernel": 0, "fp8_gemm_tile_ring_kernel": 0, "fp8_gemm_grouped_ring_kernel": 0,
+                     "fp8_gemm_pair_kernel": 0, "fp8_gemm_bs320_kernel": 0,
                      "fp8_gemm_bs256_kernelILi0ELb0E": 52, "fp8_gemm_bs256_kernelILi0ELb1E": 0,
                      "fp8_gemm_bs256_kernelILi1ELb0E": 17, "fp8_gemm_bs256_kernelILi1ELb1E": 0}
 # Kernels that are launched with as much dynamic LDS as a compute unit has: no static LDS beside it (the dynamic array is

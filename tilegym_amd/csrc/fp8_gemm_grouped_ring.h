@@ -278,9 +278,13 @@ __global__ void __launch_bounds__(64 * (NC + 4), 1) fp8_gemm_grouped_ring_kernel
     for (int i = 0; i < ntiles; ++i) {
         int dst[TM];
         float rw[TM];
+        // (worked out per tile: kept over the loop, the address is the one register too many of the 128 x 256 activation form)
+        int here = lane;
+        asm volatile("" : "+v"(here));
+        const int row0 = wm * 16 + (here & 15);
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm) {
-            dst[tm] = s_dst[i & 1][(tm * WGM + wm) * 16 + li];
+            dst[tm] = s_dst[i & 1][tm * (WGM * 16) + row0];
             rw[tm] = 1.0f;
             if constexpr (GROUP == GROUP_GATHER)
                 if (p.row_weight && dst[tm] >= 0) rw[tm] = p.row_weight[dst[tm]];
