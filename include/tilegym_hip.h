@@ -108,12 +108,13 @@ enum {
  *     (both must be of the same kind; block form requires the NT layout.)
  * workspace: NULL, or a 16-byte-aligned scratch buffer (any dtype, contents irrelevant) of at
  *     least tg_fp8_gemm_workspace_bytes() bytes.  It holds split-K partial sums, for
- *     (K,N) weights a K-contiguous copy of b, and for a K that the MFMA kernels cannot step
+ *     (K,N) weights that are not read as they lie a K-contiguous copy of b, and for a K that the MFMA kernels cannot step
  *     through (K % 16 != 0; K % 128 != 0 above 64 rows) copies of a and b with every row
  *     zero-padded to the next multiple of 128.  Calls that share a workspace must not overlap
- *     in time (calls on one stream never do).  Without a workspace the split-K schedules, the
- *     (K,N) fast path and the padded copies are not used (such a K then runs on the fallback
- *     kernel).
+ *     in time (calls on one stream never do).  Without a workspace the split-K schedules and the
+ *     copies are not used: a (K,N) weight is read as it lies if it is per-tensor scaled, K % 128 == 0,
+ *     N % 16 == 0 and cfg[] asks for nothing, else it runs on the fallback kernel, and so does a K that
+ *     would be padded.
  */
 int32_t tg_fp8_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b,
                     const tg_tensor* scale_a, const tg_tensor* scale_b, int32_t trans_a,
@@ -128,8 +129,8 @@ int32_t tg_fp8_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b,
  * held until the process ends).  The call allocates nothing and frees nothing.  A problem whose schedule needs
  * more scratch than the array holds returns TG_ERR_INVALID (the text says how much): call tg_fp8_gemm with a
  * caller-owned workspace for it.  What runs is tg_fp8_gemm's schedule, with its bits (above 64 rows an automatic split never needs
- * more than the array).  One exception, above 16 rows: a (K,N) weight's copy takes part of the array, and a split that cfg[]
- * does not ask for is chosen among those that fit the rest.  All calls on one GPU share that GPU's array, whatever the stream: calls that
+ * more than the array).  One exception, above 16 rows: for a (K,N) weight, a split that cfg[] does not ask for is chosen among
+ * those that fit beside a copy of the weight.  All calls on one GPU share that GPU's array, whatever the stream: calls that
  * overlap in time on one GPU race on it; calls on one stream never overlap.  Nothing in the array needs to start
  * at zero (no atomics are used), so nothing is cleared between calls.  The first call on a device looks the
  * array's address up (hipGetSymbolAddress); make that call outside graph capture.

@@ -119,3 +119,23 @@ def test_static_scratch_takes_a_split_that_fits_beside_the_copy_of_a_weight(devi
     with pytest.raises(_lib.TileGymHipError) as ei:
         _lib.fp8_gemm_static_scratch(c, a, b, sa, sb, trans_b=False, kernel_configs={"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": 8})
     assert ei.value.rc == -6 and "static scratch" in str(ei.value)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1040, 5120), (16, 2048, 4096), (5, 4096, 7168), (16, 656, 14336), (9, 16384, 1280), (16, 400, 1152)])
+def test_static_scratch_reads_a_kn_weight_as_the_workspace_form_does(device, M, N, K):
+    """Up to 16 rows the two entry points run one schedule on a (K, N) weight, too: read as it lies, with or without splits, or copied."""
+    a, b, sa, sb = _case(M, N, K, M + N, device, trans_b=False)
+    c_ref, c_new, _ = _both(a, b, sa, sb, M, N, trans_b=False)
+    assert torch.equal(c_ref, c_new)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 2048, 4096), (200, 1040, 1408), (600, 208, 1024)])
+def test_kn_weight_without_room_for_its_copy_is_read_as_it_lies(device, M, N, K):
+    a, b, sa, sb = _case(M, N, K, M + N, device, trans_b=False)
+    c = torch.empty(M, N, dtype=torch.bfloat16, device=device)
+    _lib.fp8_gemm(c, a, b, sa, sb, trans_b=False, use_workspace=False)
+    assert _lib.last_config()["KERNEL_NAME"] == "tiled" and _lib.last_config()["SPLIT_K"] == 1
+    cols = torch.arange(0, N, 7)
+    ref = R.ref_gemm_per_tensor(a.cpu(), b.cpu()[:, cols].t().contiguous(), sa.cpu(), sb.cpu(), trans_b=True)
+    ok, rep = R.compare_to_oracle(c[:, cols.to(device)], ref, 8.5e-3, 8.5e-3)   # one bf16 ulp (a tie may round the other way)
+    assert ok, rep

@@ -769,7 +769,7 @@ constexpr TileCost kKnFewRowsTiles[] = {{32, 32, 0.39f, 0.f, 3.6f}, {64, 32, 0.4
 constexpr StepCost kKnTiles[] = {{32, 32, false, 0.236f, 0.232f, 0.f, 1.174f, 0.f}, {64, 32, false, 0.358f, 0.321f, 0.f, 1.139f, 0.f},
                                  {64, 64, false, 0.298f, 0.426f, 0.f, 1.862f, 0.024f}};
 constexpr float kCopyUs = 4.11f, kCopyUsPerMB = 0.466f, kCopiedFewRowsUs = 7.0f, kCopiedFewRowsUsPerMB = 0.5f;
-bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, Schedule* s) {
+bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, bool can_copy, Schedule* s) {
     if (N % 16 != 0 || K % 128 != 0) return false;
     const int64_t kblocks = K / 128;
     const float mb = (float)(N * K) * 1e-6f;
@@ -782,22 +782,22 @@ bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, 
         const TileModel& m = M <= 64 ? kKnFewRowsModel : kKnModel;
         const TileChoice pick = pick_tile_by_cost(m, M, N, kblocks, partial_bytes_avail);
         // (predicted 5 % faster, at least: beyond the rows of the fit the two are close; 2974 x 28672 x 4096 339 us as it lies, 332 copied)
-        if (M > 64 && 1.05f * pick.us > pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us + kCopyUs + kCopyUsPerMB * mb) return false;
+        if (can_copy && M > 64 && 1.05f * pick.us > pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us + kCopyUs + kCopyUsPerMB * mb) return false;
         *s = Schedule{1, pick.bm, pick.bn, 1, -1, -1, 8};
         if (pick.split > 1) s->split_k = pick_split(cdiv(M, pick.bm) * cdiv(N, pick.bn), 256, kblocks, 4, M, N, partial_bytes_avail, pick.split);
         return true;
     }
-    if (M > 512) return false;
+    if (can_copy && M > 512) return false;
     if (M <= 64) {
         for (const TileCost& t : kKnFewRowsTiles) {
             const float tiles = (float)(cdiv(M, t.bm) * cdiv(N, t.bn));   // one workgroup per compute unit
             offer(t.bm, t.bn, (tiles > 256.f ? tiles / 256.f : 1.f) * ((float)kblocks * t.alone + t.fixed));
         }
-        return best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
+        return !can_copy || best <= kCopiedFewRowsUs + kCopiedFewRowsUsPerMB * mb;
     }
     for (const StepCost& t : kKnTiles) offer(t.bm, t.bn, step_cost_us(kPerTensorModel, t, M, N, kblocks, 1, t.bn));
     const float nk = pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us;
-    return best <= nk + kCopyUs + kCopyUsPerMB * mb;
+    return !can_copy || best <= nk + kCopyUs + kCopyUsPerMB * mb;
 }
 
 // ---- expert-grouped block-scaled GEMMs: 256 x 256 tiles, or 128 x 256 tiles of which two share a compute unit (PAIR in
@@ -1223,10 +1223,13 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
     bool direct_kn = false;   // a (K, N) weight read as it lies
     Schedule kn{};
     if (!b_is_nk && !trans_a && want_kernel != 0 && K > 0) {
-        // (K,N) weights: make a K-contiguous copy at the tail of the workspace when it fits
+        // (K,N) weights: read as they lie, or make a K-contiguous copy at the tail of the workspace when it fits.  The choice sees no
+        // more room for partial sums than the static array has, so that it is the same from both entry points (above 16 rows the
+        // static array's room beside a copy: the exception below).
         const int64_t need = (N * K + 255) / 256 * 256;
-        direct_kn = ws_free >= need && !static_scratch && !block_scaled && M * K < kOffsetLimit && N * K < kOffsetLimit && aligned16(a->ptr) && aligned16(b->ptr) &&
-                    nothing_forced(cfg, ncfg) && pick_kn_tile(M, N, K, ws_free - need, &kn);
+        const int64_t room = std::min(static_scratch && M > 16 ? ws_free - need : ws_free, kAutoPartialBytes);
+        direct_kn = !block_scaled && M * K < kOffsetLimit && N * K < kOffsetLimit && aligned16(a->ptr) && aligned16(b->ptr) &&
+                    nothing_forced(cfg, ncfg) && pick_kn_tile(M, N, K, room, ws_free >= need, &kn);
         if (!direct_kn && ws_free >= need) {
             uint8_t* bt = ws + ws_bytes - need;
             bt = reinterpret_cast<uint8_t*>(reinterpret_cast<uintptr_t>(bt) & ~(uintptr_t)15);
@@ -1244,7 +1247,7 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
                              aligned16(reinterpret_cast<uint64_t>(Bnt)) && N * K < kOffsetLimit && (!block_scaled || std_blocks);
     const bool takes_320 = block_scaled && scale_a && scale_b && tg::bs320_takes(M, N) && M * K < kOffsetLimit;
     Schedule s = direct_kn ? kn : choose_dense(M, N, K, block_scaled, fast_layout, cfg, ncfg, ws_free, takes_320);
-    if (static_scratch) {
+    if (static_scratch && !direct_kn) {
         // The schedule of tg_fp8_gemm with a full-size workspace, or an error: never a silently smaller split.  (Above 64 rows an
         // automatic split stays within the array, see kAutoPartialBytes.)  One exception, above 16 rows: a (K, N) weight's copy
         // takes part of the array, and a split that nobody asked for is chosen among those that fit the rest -- the constants of
