@@ -2106,6 +2106,19 @@ def test_ragged_stream_form_is_the_default_for_one_token(device):
     used("tiled")
 
 
+@pytest.mark.parametrize("waves", [4, 6, 8])
+@pytest.mark.parametrize("sizes", [[0, 16, 17, 1, 32, 33, 0, 5], [0] * 70 + [49, 0, 15, 64] + [0] * 60 + [31], [200], [3] * 5 + [400]])
+def test_ragged_stream_form_with_crowded_experts(device, sizes, waves):
+    """Experts whose rows end at, before and behind a multiple of 16, on either side of 64 experts, with most of the rows and with all."""
+    N, K = 392, 1152
+    a, b, a_s, b_s, ptr = _ragged_inputs(sizes, N, K, len(sizes) + sum(sizes), total_extra=7)
+    out = torch.zeros(a.shape[0], N, dtype=torch.bfloat16, device=device)
+    _lib.fp8_ragged_gemm(out, *[t.to(device) for t in (a, b, a_s, b_s, ptr)], {"KERNEL": "stream", "WAVES": waves})
+    assert used("stream")["WAVES"] == waves
+    check(out[: sum(sizes)], R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr)[: sum(sizes)], what=f"{sizes}")
+    assert not out[sum(sizes):].any()
+
+
 @pytest.mark.parametrize("kc", [None, {"KERNEL": "stream"}, {"KERNEL": "tiled"}])
 @pytest.mark.parametrize("ptr", [[0, 7, 7, 18, 29], [0, 20, 24, 24, 29], [-5, 7, 7, 18, 20]])
 def test_ragged_segments_past_the_rows_are_contained(device, ptr, kc):
