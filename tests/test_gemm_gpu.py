@@ -1388,6 +1388,31 @@ def test_ragged_ring_tiles_are_the_default_for_few_rows_per_expert(device, rows,
     check(out, R.ref_ragged_block_scaled_bmm(a, b, a_s, b_s, ptr), what=f"{rows} rows")
 
 
+@pytest.mark.parametrize("routing", ["even", "one expert", "a third on two experts", "two thirds of the experts"])
+def test_ragged_ring_tiles_take_their_columns_from_the_routing(device, routing):
+    """32 row tiles over 1536 columns: 192 columns are one round of 256 workgroups; a row tile more and 256 columns are, a third of the experts
+    without rows and 128 are.  Crowded experts walk several row tiles over the same columns.  Same bits as 128 x 128 tiles."""
+    E, N, K, rows = 32, 1536, 2048, 640
+    gen = torch.Generator(device=device).manual_seed(7)
+    ids = torch.arange(rows, device=device) % E
+    if routing.startswith("one"):
+        ids[:] = 5
+    elif routing.startswith("a third"):
+        ids[::6], ids[1::6] = 0, E - 1
+    elif routing.startswith("two"):
+        ids %= 2 * E // 3
+    ptr = torch.zeros(E + 1, dtype=torch.int32, device=device)
+    ptr[1:] = torch.cumsum(torch.bincount(ids, minlength=E), 0)
+    a, b = (torch.randint(0, 0x70, s, generator=gen, dtype=torch.uint8, device=device).view(FP8) for s in ((rows, K), (E, N, K)))
+    sa, sb = (torch.rand(*s, generator=gen, device=device) for s in ((rows, K // 128), (E, N // 128, K // 128)))
+    out = ragged_block_scaled_bmm(a, b, sa, sb, ptr, rows)
+    cfg = used("tiled")
+    assert (cfg["BLOCK_M"], cfg["BLOCK_N"], cfg["ROW_GROUPS"]) == (64, 256, 1), cfg
+    want = torch.empty_like(out)
+    _lib.fp8_ragged_gemm(want, a, b, sa, sb, ptr, {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128})
+    assert torch.equal(out, want)
+
+
 # ----------------------------------------------------------------------------- MoE token gather
 @pytest.mark.parametrize("block_m,K", [(64, 640), (64, 1152), (128, 640), (128, 1152)])
 def test_moe_gather_on_ring_tiles(device, block_m, K):

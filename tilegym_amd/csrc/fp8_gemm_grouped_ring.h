@@ -17,7 +17,11 @@
 //
 // Eight computing waves for 256 columns (four of 64 x 128 were no faster than the kernels of one workgroup per tile: two waves on a SIMD take
 // turns at the scale-and-add), non-temporal weight loads (8 - 11 % over plain ones), 192 columns where 256 would leave a round half empty
-// (32 experts of (1536, 4096): 46 us with 256, 43.7 with 192).  Measured, us before / after (floor at 6.5 TB/s), 64 experts of (2816, 2048)
+// (32 experts of (1536, 4096): 46 us with 256, 43.7 with 192).  Rows that are not spread evenly: a crowded expert's row tiles go over the same
+// columns one after the other, and the columns of a tile are chosen on the device.  Over 3900 problems ahead of the kernels of one
+// workgroup per tile by 1.12 x with the rows spread evenly, 1.17 on an eighth of the experts, 1.12 with half and 1.19 with all of them on one, 1.11 by
+// Zipf's law (without the two 1.13, 1.07, 1.08, 1.02, 1.09); it stays behind where few experts have hundreds of rows each and the mean
+// says 30 (120 experts of (2304, 2560), 5032 rows on 15 of them: 96 us, pairs of 128 x 256 tiles 47).  Measured, us before / after (floor at 6.5 TB/s), 64 experts of (2816, 2048)
 // top 6: 40 tokens 61.6 / 56.8 (56.0), 200 tokens 65.2 / 61.7 (58.2), 1000 tokens 87.0 / 80.8 (64.0); 128 experts of (1536, 2048) top 8:
 // 8 tokens 38.8 / 31.1 (25.0), 1000 tokens 94.1 / 81.8 (68.3); 16 experts of (2048, 2048) top 2: 40 tokens 17.4 / 14.0 (10.4).  A layer of
 // the first size (align, quantize, two GEMMs, sum): 200 tokens 122 / 108.
@@ -58,29 +62,10 @@ __global__ void __launch_bounds__(64 * (NC + 4), 1) fp8_gemm_grouped_ring_kernel
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = p.K, nsteps = p.kblocks;
-    // columns of a tile: BN, or fewer so that the tiles come out even over the compute units.  The weight rows that a tile leaves out
-    // are requested from beyond the descriptor's range (no memory request) and not stored.
-    const int cols = ACT ? 128 : p.tile_cols;
-    const int tiles_n = ACT ? p.inter / 128 : (p.N + cols - 1) / cols;
-
-    // ---- the workgroup's tiles: first, first + stride, ... of its XCD's range
+    // ---- the workgroup's tiles: first, first + stride, ... of its XCD's range.  Columns of a tile: BN, or fewer so that the tiles come out
+    // even over the compute units; the weight rows that a tile leaves out are requested from beyond the descriptor's range (no memory request)
+    // and not stored.
     int post_pad = 0, total_mt;
-    // (no more row tiles than M rows in E segments can have, whatever m_indptr holds)
-    if constexpr (GROUP == GROUP_RAGGED) total_mt = min(ragged_count_tiles(p.m_indptr, p.E, BM, lane), p.M / BM + p.E);
-    else {
-        post_pad = min(p.num_post_pad[0], p.em_capacity);
-        total_mt = (post_pad + BM - 1) / BM;
-    }
-    total_mt = __builtin_amdgcn_readfirstlane(total_mt);
-    const int nblk = total_mt * tiles_n;
-    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8;  // (the grid is a multiple of eight)
-    const int share = nblk / 8, rest = nblk % 8;
-    const int first = xcd * share + min(xcd, rest) + (int)blockIdx.x / 8;
-    const int end = xcd * share + min(xcd, rest) + share + (xcd < rest ? 1 : 0);
-    const int ntiles = first < end ? (end - first - 1) / stride + 1 : 0;
-    if (ntiles == 0) return;
-    const int total_steps = ntiles * nsteps;
-
     if constexpr (GROUP == GROUP_RAGGED) {
         int base = 0;
         for (int e0 = 0; e0 < p.E; e0 += 64) {
@@ -99,37 +84,77 @@ __global__ void __launch_bounds__(64 * (NC + 4), 1) fp8_gemm_grouped_ring_kernel
             if (wave == 0 && e < p.E) s_end[e] = incl;
             base = __shfl(incl, 63);
         }
+        total_mt = min(base, p.M / BM + p.E);  // (no more row tiles than M rows in E segments can have, whatever m_indptr holds)
         __syncthreads();
+    } else {
+        post_pad = min(p.num_post_pad[0], p.em_capacity);
+        total_mt = (post_pad + BM - 1) / BM;
     }
+    total_mt = __builtin_amdgcn_readfirstlane(total_mt);
+    int cols = ACT ? 128 : p.tile_cols;
+    if constexpr (BN == 256 && !ACT) {
+        // tile_cols 0: by the rounds that the tiles make (a round costs its columns + 16).  Decided here, where the row tiles are known: an
+        // expert with more rows than the others is a tile or two more, and those may be a round more.
+        if (cols == 0) {
+            const float places = __builtin_amdgcn_rcpf((float)gridDim.x);  // (an integer division would delay the first loads by 0.2 us)
+            float best = 1e30f;
+#pragma unroll
+            for (int c = 256; c >= (BM == 128 ? 192 : 128); c -= 64) {
+                const float cost = __builtin_ceilf((float)(total_mt * ((p.N + c - 1) / c)) * places - 1e-3f) * (float)(c + 16);
+                if (cost < best) { best = cost; cols = c; }
+            }
+        }
+    }
+    const int tiles_n = ACT ? p.inter / 128 : (p.N + cols - 1) / cols;
+    const int nblk = total_mt * tiles_n;
+    const int xcd = blockIdx.x % 8, stride = gridDim.x / 8;  // (the grid is a multiple of eight)
+    const int share = nblk / 8, rest = nblk % 8;
+    const int first = xcd * share + min(xcd, rest) + (int)blockIdx.x / 8;
+    const int end = xcd * share + min(xcd, rest) + share + (xcd < rest ? 1 : 0);
+    const int ntiles = first < end ? (end - first - 1) / stride + 1 : 0;
+    if (ntiles == 0) return;
+    const int total_steps = ntiles * nsteps;
 
     // ---- a tile's expert, first column and rows.  find() requests what publish() looks at two K steps later: nothing in between waits.
     struct Tile { int expert, n0, lo, hi; };  // lo, hi: ragged, the thread's row and the end of the expert's; gather, the thread's slot
     auto find = [&](int i) {
         const int t = first + i * stride;
-        const int tile_m = t / tiles_n, tile_n = t % tiles_n;
+        const int tile_m = t / tiles_n;
+        int tile_n = t % tiles_n;
         Tile f;
-        f.n0 = tile_n * cols;
         f.lo = f.hi = 0;
         if constexpr (GROUP == GROUP_RAGGED) {
-            int e = 0, before = 0;
+            int e = 0, before = 0, upto = 0;  // row tiles in front of the expert, and with it
             for (int e0 = 0; e0 < p.E; e0 += 64) {
-                const int mine = e0 + lane < p.E ? s_end[e0 + lane] : 0x7FFFFFFF;
-                const unsigned long long hit = __ballot(mine > tile_m);
+                const int ends = e0 + lane < p.E ? s_end[e0 + lane] : 0x7FFFFFFF;
+                const unsigned long long hit = __ballot(ends > tile_m);
                 if (hit) {
-                    e = e0 + __ffsll((long long)hit) - 1;
+                    const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+                    e = e0 + l;
+                    upto = __builtin_amdgcn_readlane(ends, l);
+                    if (l > 0) before = __builtin_amdgcn_readlane(ends, l - 1);
                     break;
                 }
+                before = __builtin_amdgcn_readlane(ends, 63);
             }
-            e = __builtin_amdgcn_readfirstlane(e);
-            before = e > 0 ? s_end[e - 1] : 0;
+            // a crowded expert's row tiles one after the other over the same columns: the compute units of an XCD that work on it at one time
+            // share its weight in their L2 (with two row tiles the weight is read once more either way, and column by column is 0.8 % ahead)
+            const int mine = upto - before;
+            int row_tile = tile_m - before;
+            if (mine > 2) {
+                const int at = t - before * tiles_n;
+                tile_n = at / mine;
+                row_tile = at - tile_n * mine;
+            }
             f.expert = e;
-            f.lo = p.m_indptr[e] + (tile_m - before) * BM + tid;
+            f.lo = p.m_indptr[e] + row_tile * BM + tid;
             f.hi = p.m_indptr[e + 1];
         } else {
             const int m0 = tile_m * BM;  // position in the sorted slot sequence
             f.expert = p.expert_ids[m0 / p.block_m];
             f.lo = tid < BM && m0 + tid < post_pad ? p.sorted_ids[m0 + tid] : p.num_valid;
         }
+        f.n0 = tile_n * cols;
         return f;
     };
     auto publish = [&](Tile& f, int buf) {
@@ -280,7 +305,7 @@ __global__ void __launch_bounds__(64 * (NC + 4), 1) fp8_gemm_grouped_ring_kernel
         float rw[TM];
         // (worked out per tile: kept over the loop, the address is the one register too many of the 128 x 256 activation form)
         int here = lane;
-        asm volatile("" : "+v"(here));
+        if constexpr (ACT && BM == 128) asm volatile("" : "+v"(here));
         const int row0 = wm * 16 + (here & 15);
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm) {

@@ -5,7 +5,7 @@
 namespace tg {
 
 hipError_t run_grouped_ring(int bm, int cols, int group, GemmParams p, hipStream_t s) {
-    const int bn = cols == 192 ? 256 : cols;
+    const int bn = cols == 192 || cols == 0 ? 256 : cols;
     p.tile_cols = cols;
     if (p.kblocks < grouped_ring_steps(bn) || p.K % kKBlock != 0 || !p.As || !p.Bs || (group == GROUP_RAGGED && p.E > kGroupedRingExperts) ||
         (group != GROUP_RAGGED && p.block_m % bm != 0)) return hipErrorInvalidValue;

@@ -69,8 +69,8 @@ hipError_t run_tile_block_dense(int bm, int bn, bool split, const GemmParams& p,
 hipError_t run_tile_moe_act(int bm, bool pair, const GemmParams& p, int gx, hipStream_t s);
 // persistent tiles of 32, 64 or 128 rows x 128, 192 or 256 weight rows for experts with few rows: same results as the others of the
 // group mode.  Needs both scale tensors, K a multiple of 128 with at least grouped_ring_steps steps, at most 256 experts if ragged, and
-// an alignment block that bm divides if gathered.  GROUP_GATHER_ACT: 256 weight rows
-constexpr int grouped_ring_steps(int cols) { return cols > 128 ? 5 : 8; }  // the ring's stages and two
+// an alignment block that bm divides if gathered.  GROUP_GATHER_ACT: 256 weight rows.  cols 0: 128, 192 or 256, chosen on the device
+constexpr int grouped_ring_steps(int cols) { return cols != 128 ? 5 : 8; }  // the ring's stages and two
 hipError_t run_grouped_ring(int bm, int cols, int group, GemmParams p, hipStream_t s);
 hipError_t run_tile_block_grouped(int bm, int bn, int group, const GemmParams& p, int gx, hipStream_t s);
 // The two GEMMs of the decoding MoE layer: out = T(silu(gate) * up) resp. out = T(result x routed weight).  `up` selects the

@@ -859,15 +859,21 @@ double expected_weight_bytes(int64_t rows, int64_t E, int64_t N, int64_t K) {
 // them multiply on a compute unit), above 116 rows up to 1.35 x.
 // Little weight to read (below 80 MB; 30 MB if all tiles of 128 columns run at once) leaves nothing for the ring to hide: 128 x 128 or pairs are
 // 1.06 - 1.2 x ahead (600 problems).
-// 32 rows to 18 per expert, 64 to 47; 128, 192 or 256 columns by the rounds that 256 workgroups need (a round costs its columns + 16).
+// 32 rows to 18 per expert, 64 to 47; tiles of 128 columns or the ones that take up to 256 by the rounds that 256 workgroups need (a round
+// costs its columns + 16).  How many columns the latter take is decided on the device, where the rows per expert are known (tile_cols 0).
 RingTile grouped_ring_tile(const tg::GemmParams& p, int group, int64_t rows, int block_m) {
     const int64_t E = p.E, N = group == tg::GROUP_GATHER_ACT ? 2 * (int64_t)p.inter : (int64_t)p.N;
     const double mu = (double)rows / (double)E, bytes = (double)E * (double)N * (double)p.K;
     if (mu > 116.0 || (mu > 40.0 && bytes < 256e6)) return RingTile{0, 0};
     const double touched = expected_weight_bytes(rows, E, N, p.K);
     auto cost = [&](int bm, int bn) {
-        const double rounds = ceil(expected_row_tiles(rows, E, bm) * (double)cdiv(N, bn) / 256.0 - 0.01);
-        return (rounds < 1.0 ? 1.0 : rounds) * (double)(bn + 16);
+        double least = 0.0;
+        for (int c = bn; c >= (bm == 128 ? 192 : 128); c -= 64) {
+            const double rounds = ceil(expected_row_tiles(rows, E, bm) * (double)cdiv(N, c) / 256.0 - 0.01);
+            const double us = (rounds < 1.0 ? 1.0 : rounds) * (double)(c + 16);
+            if (c == bn || us < least) least = us;
+        }
+        return least;
     };
     RingTile best{0, 0};
     double best_cost = 0.0;
@@ -879,12 +885,10 @@ RingTile grouped_ring_tile(const tg::GemmParams& p, int group, int64_t rows, int
     };
     if (block_m == 128 || (block_m == 0 && mu > 47.0)) {
         offer(128, 256);
-        offer(128, 192);
     } else {
         if (block_m == 0) offer(mu <= 18.0 ? 32 : 64, 128);
         else offer(block_m, 128);
         offer(64, 256);
-        offer(64, 192);
     }
     return best;
 }
@@ -1514,7 +1518,7 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
     if (ring.bm > 0 && (ring_forced || nothing_forced_but_kernel(cfg, ncfg))) {
         s.kernel = 1; s.bm = ring.bm; s.bn = ring.bn; s.row_groups = 1;
         remember(s);
-        const hipError_t e = tg::run_grouped_ring(ring.bm, ring.bn, tg::GROUP_RAGGED, p, stream);
+        const hipError_t e = tg::run_grouped_ring(ring.bm, ring_forced || ring.bn == 128 ? ring.bn : 0, tg::GROUP_RAGGED, p, stream);
         if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "grouped kernel launch failed: %s", hipGetErrorString(e));
         return TG_OK;
     }
@@ -1630,7 +1634,7 @@ int32_t tg_fp8_moe_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tensor*
     remember(s);
     const int64_t gx = cdiv(EM, bm) * cdiv(N, bn);
     if (gx > INT32_MAX) return fail(TG_ERR_INVALID, "too many tiles");
-    hipError_t e = ring.bm > 0 ? tg::run_grouped_ring(bm, bn, tg::GROUP_GATHER, p, stream)
+    hipError_t e = ring.bm > 0 ? tg::run_grouped_ring(bm, bn == 128 ? bn : 0, tg::GROUP_GATHER, p, stream)
                                : tg::run_tile_block_grouped(bm, bn, tg::GROUP_GATHER, p, (int)gx, stream);
     if (e != hipSuccess) return fail(TG_ERR_LAUNCH, "grouped kernel launch failed: %s", hipGetErrorString(e));
     return TG_OK;
