@@ -1523,9 +1523,10 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
         return TG_OK;
     }
     if (!(bm > 0 && bn > 0 && grouped_tile_exists(bm, bn))) {
-        // Below 40 rows per expert, what the ring tiles leave: short K over 30 MB of weights and more in pairs of 128 x 256 tiles (two tiles'
-        // set-ups on a compute unit hide each other), else 128 x 128 (500 problems: each within 2 % of the best on average, 64 x 128
-        // 1.05 - 1.4 x behind), 64 x 128 where the weights take longest (69 us against 80 at 24 rows).  From there on, if there are enough of them, pairs
+        // Below 40 rows per expert, what the ring tiles leave: 128 x 128 (500 problems: within 2 % of the best on average, 64 x 128
+        // 1.05 - 1.4 x behind), 64 x 128 where the weights take longest (69 us against 80 at 24 rows).  Over 30 MB and more of K below 1024 pairs of
+        // 128 x 256 tiles are 8 % ahead of 128 x 128 if the rows are spread evenly, 1 - 2 % by Zipf's law or with half of them on one
+        // expert, but 14 and 21 % behind with all of them on an eighth of the experts or on one (207 problems).  From there on, if there are enough of them, pairs
         // of 128 x 256 tiles or 256 x 256 tiles, whichever the padding of the experts' last tiles makes cheaper (64 experts of
         // (2816, 2048), us, 128 x 128 / pairs / 256 x 256: 94 rows 95.5 / 88.5 / 98.1, 188 rows 132 / 119 / 115, 281 rows 183 /
         // 159 / 171); fewer than 240 tiles of 128 x 256: 128 x 128, but for the persistent form's problems (8 experts of (3072, 3072) at 192
@@ -1533,8 +1534,7 @@ int32_t tg_fp8_ragged_gemm(const tg_tensor* c, const tg_tensor* a, const tg_tens
         // 31.2; over 170 such problems 1.19 x)
         const int64_t mean = total_m / E;
         const double touched = expected_weight_bytes(total_m, E, N, K);
-        if (mean < 40 && p.kblocks < 8 && touched >= 30e6 && N >= 256) { bm = 128; bn = 256; }
-        else if (mean < 40) { bm = touched >= 80e6 ? 64 : 128; bn = 128; }
+        if (mean < 40) { bm = touched >= 80e6 && p.kblocks >= 8 ? 64 : 128; bn = 128; }
         else if (N < 256 || ((mean <= 256 || p.kblocks > 12) && grouped_row_tiles(total_m, E) * cdiv(N, 256) < kPairTiles * 6 / 5)) { bm = 128; bn = 128; }
         else if (pair_tiles(total_m, E, cdiv(N, 256)) && grouped_cost(total_m, E, true) <= grouped_cost(total_m, E, false)) { bm = 128; bn = 256; }
         else { bm = 256; bn = 256; }
