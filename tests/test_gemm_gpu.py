@@ -618,6 +618,21 @@ def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
     check(out[:, cols.to(device)], R.ref_gemm_per_tensor(a, b[cols], 0.01, 0.02, trans_b=True, out_dtype=torch.float16), what=f"M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("kind,M,N,K,ring", [
+    ("nk", 88, 1520, 5248, False), ("nk", 90, 4096, 4096, True), ("nk", 128, 4096, 4096, False), ("nk", 256, 4096, 4096, True), ("nk", 482, 9216, 3072, False),
+    ("block", 100, 1120, 8320, False)])
+def test_narrow_ring_tiles_are_chosen_where_they_hold_from_memory(device, kind, M, N, K, ring):
+    """Either side of the lines between the narrow ring tiles (and 256 x 128), and the kernels that are ahead of them when the weight is not in the caches."""
+    zeros = lambda *shape: torch.zeros(*shape, dtype=torch.uint8, device=device).view(FP8)  # noqa: E731
+    c = torch.empty(M, N, dtype=torch.bfloat16, device=device)
+    one = torch.ones(1, device=device)
+    sa, sb = (torch.ones(M, K // 128, device=device), torch.ones(-(-N // 128), K // 128, device=device)) if kind == "block" else (one, one)
+    _lib.fp8_gemm(c, zeros(M, K), zeros(K, N) if kind == "kn" else zeros(N, K), sa, sb, trans_b=kind != "kn")
+    cfg = _lib.last_config()
+    narrow = cfg["WAVES"] == 8 and (cfg["BLOCK_N"] <= 64 or cfg["BLOCK_M"] in (32, 256))
+    assert (cfg["KERNEL_NAME"] == "tiled" and narrow) == ring, cfg
+
+
 @pytest.mark.parametrize("block_scaled", [False, True])
 @pytest.mark.parametrize("M,N,K,want", [(16, 25616, 4096, (32, 128)), (17, 25616, 4096, (32, 128)), (33, 32768, 4096, (64, 128)), (64, 25604, 4096, (64, 128)),
                                         (16, 16360, 8192, (32, 64)), (50, 14728, 8192, (64, 64)), (65, 25616, 4096, (96, 128)), (128, 25616, 4096, (128, 128)),

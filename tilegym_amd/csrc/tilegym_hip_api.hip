@@ -295,6 +295,19 @@ int read_once_columns(int64_t N, int64_t K) {
     const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128);
     return t128 >= 200 && t128 <= 256 ? 128 : t64 >= 230 && t64 <= 256 ? 64 : 0;
 }
+// Whether a tile with `from_k` keeps what it gains over cached weights when the weight comes from memory.  The compute units' requests are
+// then what counts: few workgroups over a long K (above 44 x their number) ask for too little at once, and so do tiles of 32 rows or columns with
+// fewer than 160 or 128 workgroups, or (64 x 32 above 96 rows) a full round of them over long K, and 256 x 128 with fewer than 192.  Of 5500
+// choices of 65 to 700 rows that these tiles took the line keeps those that gain 1.29 x per-tensor and 1.28 x block-scaled cached, 1.21 and
+// 1.31 x from memory, and gives up 1.15 and 1.16 x cached, 0.97 (at worst 0.72) and 1.02 x (0.80) from memory: 4096 x 8192 at 88 rows and the like.
+bool holds_from_memory(const StepCost& t, bool block_scaled, int64_t M, int64_t N, int64_t K, int split) {
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
+    if (t.bm == 256) return tiles >= 192;
+    if (split > 1) return true;
+    if (K > 44 * tiles) return false;
+    if (block_scaled) return true;
+    return t.bm == 32 ? tiles >= 160 : t.bn == 32 ? tiles >= 128 && (tiles <= 250 || K < 4096 || M <= 96) : true;
+}
 constexpr TileModel kSmallRowsRing{nullptr, 0, 2.6f, 0.25f, 1.0f, 0.f};  // (the reduction launch behind the ring tiles of up to 64 rows)
 
 // (cols: weight rows per tile where they are not the kind's own)
@@ -330,6 +343,7 @@ TileChoice pick_tile_by_cost(const TileModel& m, int64_t M, int64_t N, int64_t k
                              int bm = -1, int bn = -1, bool ring = false, bool takes_320 = false) {
     const bool block_scaled = &m == &kBlockScaledModel;
     TileChoice best;
+    const StepCost* kind = nullptr;
     if (want_split <= 0 && partial_bytes_avail > kAutoPartialBytes) partial_bytes_avail = kAutoPartialBytes;
     auto offer = [&](const StepCost& t) {
         if (bm > 0 && (t.bm != bm || t.bn != bn || t.ring != ring)) return;
@@ -344,10 +358,15 @@ TileChoice pick_tile_by_cost(const TileModel& m, int64_t M, int64_t N, int64_t k
             const int split = want_split > 0 ? want_split : sp;
             const int cols = deep && bm <= 0 ? deep_tile_cols(M, N, split) : t.bn;
             const float us = step_cost_us(m, t, M, N, kblocks, split, cols) * (sp > 1 ? m.split_margin : 1.f);
-            if (best.bm < 0 || us < best.us) best = TileChoice{t.bm, cols, sp, t.ring, us};
+            if (best.bm < 0 || us < best.us) { best = TileChoice{t.bm, cols, sp, t.ring, us}; kind = &t; }
         }
     };
     for (int i = 0; i < m.n; ++i) offer(m.kinds[i]);
+    if (bm <= 0 && kind && kind->from_k > 0 && !holds_from_memory(*kind, block_scaled, M, N, kblocks * 128, want_split > 0 ? want_split : best.split)) {
+        best = TileChoice{};
+        for (int i = 0; i < m.n; ++i)
+            if (m.kinds[i].from_k == 0) offer(m.kinds[i]);
+    }
     return best;
 }
 TileChoice pick_tile_by_cost(int64_t M, int64_t N, int64_t kblocks, bool block_scaled, int64_t partial_bytes_avail, int want_split,
