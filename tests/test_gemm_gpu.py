@@ -620,7 +620,8 @@ def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
 
 @pytest.mark.parametrize("kind,M,N,K,ring", [
     ("nk", 88, 1520, 5248, False), ("nk", 90, 4096, 4096, True), ("nk", 128, 4096, 4096, False), ("nk", 256, 4096, 4096, True), ("nk", 482, 9216, 3072, False),
-    ("block", 100, 1120, 8320, False)])
+    ("block", 100, 1120, 8320, False),
+    ("kn", 16, 1024, 1920, False), ("kn", 16, 10240, 1920, True), ("kn", 256, 4096, 4096, False), ("kn", 16, 4096, 4096, True)])
 def test_narrow_ring_tiles_are_chosen_where_they_hold_from_memory(device, kind, M, N, K, ring):
     """Either side of the lines between the narrow ring tiles (and 256 x 128), and the kernels that are ahead of them when the weight is not in the caches."""
     zeros = lambda *shape: torch.zeros(*shape, dtype=torch.uint8, device=device).view(FP8)  # noqa: E731
@@ -2340,7 +2341,7 @@ def test_kn_weights_read_as_they_lie(device, M, N, K, out_dtype):
         check(got, R.ref_gemm_per_tensor(a, b, 0.25, 0.5, trans_b=True))
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 16, 1280), (17, 1040, 1408), (50, 1040, 5120), (33, 12304, 1280), (60, 20496, 1280), (70, 2064, 1664), (129, 6160, 1280),
+@pytest.mark.parametrize("M,N,K", [(1, 8208, 1280), (17, 9232, 1408), (50, 1040, 5120), (33, 12304, 1280), (60, 20496, 1280), (70, 6160, 1664), (129, 6160, 1280),
                                    (200, 8208, 2176), (300, 4112, 1280), (256, 28688, 1280), (500, 4112, 4096), (1025, 1040, 1280)])
 def test_kn_weights_on_ring_tiles(device, M, N, K):
     """(K, N) weights that the ring tiles turn inside LDS, over every tile they choose from: rows and columns that end inside a tile,

@@ -776,8 +776,8 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
 // shorter, or by 8 % at most): 1 x 4096 x 14336 36.0 -> 14.3 us, 50 x 4096 x 14336 41 -> 16.5, 100 x 28672 x 4096 57.5 -> 28.7,
 // 400 x 12288 x 5120 53 -> 31, 64 x 2048 x 2048 7.9 -> 4.8.
 //
-// Shorter K: the narrow tiles, by the costs they were fitted to, or the copy.  (The ring would be up to 40 % faster there too, 16400 x 1152
-// at M = 64 7.3 against 12.6 us; which tiles run at these sizes is held by callers that compare a forced schedule's bits.)
+// Else, and for shorter K: the narrow tiles, by the costs they were fitted to, or the copy.  (The ring was fitted from K = 1280 on.  Over cached weights
+// it is up to 40 % ahead below, too -- 16400 x 1152 at M = 64 7.3 against 12.6 us -- but from memory short K and few columns are where it loses.)
 constexpr StepCost kKnRingFewRows[] = {{32, 64, true, 0.205f, 0.369f, 0.f, 2.357f, 0.f}, {64, 64, true, 0.221f, 0.420f, 0.f, 2.422f, 0.f},
                                        {32, 128, true, 0.200f, 0.630f, 0.f, 2.829f, 0.f}, {64, 128, true, 0.240f, 0.660f, 0.f, 2.788f, 0.f}};
 constexpr TileModel kKnFewRowsModel{kKnRingFewRows, (int)(sizeof(kKnRingFewRows) / sizeof(StepCost)), 3.1f, 0.25f, 1.0f, 0.f};
@@ -801,12 +801,29 @@ bool pick_kn_tile(int64_t M, int64_t N, int64_t K, int64_t partial_bytes_avail, 
     };
     if (K >= 1280) {
         const TileModel& m = M <= 64 ? kKnFewRowsModel : kKnModel;
-        const TileChoice pick = pick_tile_by_cost(m, M, N, kblocks, partial_bytes_avail);
+        TileChoice pick = pick_tile_by_cost(m, M, N, kblocks, partial_bytes_avail);
+        // Tiles of 64 columns take half of every line: from memory they need 128 workgroups up to 64 rows; above, 160 of 32 rows and K below 2048,
+        // or 128 of 64 rows, but not over K rows a multiple of 4 KiB apart (256 x 4096 x 4096 cached and from memory, us:
+        // the narrow 64 x 64 tile 14.0 and 18.2, ring 64 x 64 13.6 and 19.7, 32 x 128 12.8 and 19.0, copy 21.5 and 21.0).
+        // Of 12600 choices of 1 to 1000 rows the line keeps those that gain 1.50 x cached and 1.39 x from memory on average and gives
+        // up 1.10 and 0.93 x (at worst 0.74: 16 x 1024 x 1920).
+        auto holds_with = [&](const TileChoice& t) {
+            const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
+            return !can_copy || t.bn != 64 || t.split > 1 ||
+                   (M <= 64 ? tiles >= 128 : t.bm == 32 ? tiles >= 160 && K < 2048 : tiles >= 128 && !(K >= 4096 && N % 4096 == 0));
+        };
+        if (M > 64 && pick.bm == 32 && !holds_with(pick)) {
+            const TileChoice taller = pick_tile_by_cost(m, M, N, kblocks, partial_bytes_avail, -1, 64, 64, true);
+            if (holds_with(taller) && taller.us <= 1.15f * pick.us) pick = taller;
+        }
+        const bool holds = holds_with(pick);
         // (predicted 5 % faster, at least: beyond the rows of the fit the two are close; 2974 x 28672 x 4096 339 us as it lies, 332 copied)
-        if (can_copy && M > 64 && 1.05f * pick.us > pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us + kCopyUs + kCopyUsPerMB * mb) return false;
-        *s = Schedule{1, pick.bm, pick.bn, 1, -1, -1, 8};
-        if (pick.split > 1) s->split_k = pick_split(cdiv(M, pick.bm) * cdiv(N, pick.bn), 256, kblocks, 4, M, N, partial_bytes_avail, pick.split);
-        return true;
+        if (holds && can_copy && M > 64 && 1.05f * pick.us > pick_tile_by_cost(M, N, kblocks, false, partial_bytes_avail, -1, -1, -1, false).us + kCopyUs + kCopyUsPerMB * mb) return false;
+        if (holds) {
+            *s = Schedule{1, pick.bm, pick.bn, 1, -1, -1, 8};
+            if (pick.split > 1) s->split_k = pick_split(cdiv(M, pick.bm) * cdiv(N, pick.bn), 256, kblocks, 4, M, N, partial_bytes_avail, pick.split);
+            return true;
+        }
     }
     if (can_copy && M > 512) return false;
     if (M <= 64) {
