@@ -623,7 +623,8 @@ def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
     ("block", 100, 1120, 8320, False),
     ("kn", 16, 1024, 1920, False), ("kn", 16, 10240, 1920, True), ("kn", 256, 4096, 4096, False), ("kn", 16, 4096, 4096, True),
     ("nk", 24, 12288, 5120, True), ("nk", 30, 17072, 5120, False), ("nk", 40, 12288, 5120, True), ("nk", 64, 12288, 5120, False), ("nk", 64, 6144, 4096, False),
-    ("nk", 50, 4096, 14336, True), ("nk", 50, 2048, 5120, False), ("nk", 24, 22032, 2560, False)])
+    ("nk", 50, 4096, 14336, True), ("nk", 50, 2048, 5120, False), ("nk", 24, 22032, 2560, False),
+    ("block", 24, 12288, 5120, True), ("block", 20, 18576, 2944, False), ("block", 28, 3520, 4864, False), ("block", 17, 1520, 2304, False), ("block", 17, 8192, 8192, False)])
 def test_narrow_ring_tiles_are_chosen_where_they_hold_from_memory(device, kind, M, N, K, ring):
     """Either side of the lines between the narrow ring tiles (and 256 x 128), and the kernels that are ahead of them when the weight is not in the caches."""
     zeros = lambda *shape: torch.zeros(*shape, dtype=torch.uint8, device=device).view(FP8)  # noqa: E731

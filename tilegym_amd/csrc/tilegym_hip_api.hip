@@ -486,8 +486,9 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         // worst 0.75: 30 x 17072 x 5120).
         Schedule ring{0, -1, -1, 1, -1, -1, -1};
         float ring_us = 0.f;
-        auto offer_ring = [&](const Schedule& cand, float us) {
-            if (ring.kernel == 0 || us < ring_us) { ring = cand; ring_us = us; }
+        bool ring_holds = true;
+        auto offer_ring = [&](const Schedule& cand, float us, bool holds = true) {
+            if (ring.kernel == 0 || us < ring_us) { ring = cand; ring_us = us; ring_holds = holds; }
         };
         if (!block_scaled && K >= 1280 && N * K < kMemoryWeight) {
             constexpr StepCost rings[] = {{32, 64, true, 0.088f, 0.185f, 0.f, 3.312f, 0.011f}, {64, 64, true, 0.093f, 0.293f, 0.f, 3.394f, 0.f}};
@@ -523,8 +524,16 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                     // (above 25 MB fewer than 96 workgroups, above 40 MB fewer than 150 or two splits are slower from memory: 50 x 8192 x 8192 in 128 column tiles 14.5 us
                     // against 17.8 if the weight was read just before, but 21.5 against 20.3 if not)
                     if (N * K > 25000000 && want_split < 0 && (split == 1 ? cdiv(N, t.bn) < (N * K > 40000000 ? 150 : 96) : split == 2)) continue;
+                    // More than one round over 45 MB and more, 128 columns with splits there (17 x 8192 x 8192 17.5 -> 18.7), and one row tile of 32 rows over a long K in fewer than 128 workgroups, are slower
+                    // from memory (20 x 18576 x 2944 14.3 -> 17.9 us, cached 12.1 -> 16.0; 28 x 3520 x 4864 10.9 -> 12.7), and so are all of them where the skinny kernel is the
+                    // best of the others (17 x 1520 x 2304 5.3 against 6.9; cached they are even).  Of 10270 choices the line keeps those that gain 1.20 x
+                    // cached and 1.21 x from memory and gives up 1.04 and 0.87 x (at worst 0.77).
+                    const int64_t cols = cdiv(N, t.bn);
+                    const bool holds = want_split > 0 ||
+                                       (!(N * K > 45000000 && (cdiv(M, t.bm) * cols * cand.split_k > 256 || (t.bn == 128 && split > 1))) &&
+                                        !(split == 1 && t.bm == 32 && t.bn == 64 && cols < 128 && K > (M <= 32 ? 4096 : cols < 64 ? 4992 : 6144)));
                     // (a split must be predicted 10 % faster: its reduction is a launch more for the host, too)
-                    offer(cand, step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn) * (cand.split_k > 1 ? 1.1f : 1.f));
+                    offer_ring(cand, step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn) * (cand.split_k > 1 ? 1.1f : 1.f), holds);
                     if (want_split > 0) break;
                 }
             }
@@ -561,7 +570,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
             const Schedule cand = skinny_schedule();
             offer(cand, (float)cdiv(N, 16) / 256.f * (float)kblocks * c.skinny_step * (float)cand.mt + c.skinny_fixed + reduce(cand.split_k));
         }
-        if (ring.kernel != 0 && ring_us < best_us) best = ring;
+        if (ring.kernel != 0 && ring_us < best_us && ring_holds && !(block_scaled && best.kernel == 2 && ring.split_k == 1)) best = ring;
         // the wide form, unsplit: weight rows per workgroup so that the workgroups fill the chip, as for up to 16 rows
         if (best.kernel == 3 && best.row_groups == 4 && best.split_k == 1) {
             int64_t best_cost = 0;
