@@ -698,8 +698,8 @@ def test_block_scaled_skinny_to_sixteen_rows(device):
         check(out, R.ref_w8a8_block_fp8_matmul(a, b, sa, sb, None, torch.bfloat16), what=f"M={M} N={N} K={K}")
 
 
-@pytest.mark.parametrize("M,N,K,want", [(8, 10240, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 11008, 4096, (32, 64)),
-                                        (8, 6144, 4096, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
+@pytest.mark.parametrize("M,N,K,want", [(8, 10240, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 11008, 4096, None),
+                                        (8, 6144, 4096, None), (16, 6400, 3072, None), (4, 20864, 4096, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
 def test_block_scaled_decode_on_ring_tiles(device, M, N, K, want):
     g = _g(M + N)
     a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)

@@ -592,16 +592,19 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     if (nothing_forced && N * K <= skinny_mb << 20) return skinny_schedule();
     // block-scaled, up to 16 rows, where ring tiles of 32 rows fill the chip about once: the scale-and-adds of a row of weights are
     // dealt out over a workgroup, where the streaming form's waves do them between two waits (us, streaming / ring, weight in the caches and from
-    // memory, 16 rows: 10240 x 5120 at 8 rows 15.0 / 11.1 and 14.9 / 14.1, 12288 x 2048 8.0 / 7.4 and 8.0 / 7.6,
-    // 20480 x 2048 14.4 / 10.0 and 14.3 / 10.9, 18432 x 7168 35.2 / 30.2, 28672 x 4096 25.5 / 23.1; more than eight rows also
-    // 6144 x 4096 11.6 / 8.8 and 11.3 / 11.2).  Outside the streaming form is ahead from memory: 8192 x 8192 13.8 for 17.0 but 18.5 for
-    // 16.9, 12288 x 5120 12.7 for 16.4 but 17.1 for 16.4, and from K = 5120 on with more than eight rows (10240 x 5120 at 16 rows 17.1 for 15.7).
+    // memory: 10240 x 5120 at 8 rows 14.9 / 11.2 and 14.8 / 14.2, 12288 x 2048 at 16 rows 7.7 / 7.5 and 7.6 / 7.5, 6144 x 4096 at 16 rows 11.5 / 8.8
+    // and 11.2 / 10.5, 28672 x 4096 at 16 rows 24.9 / 23.6 and 25.7 / 24.8; boxes differ by 5 % from memory).  Not where it is behind from memory: 64 columns over more than 44 MB whose K is a power of two (rows 4096 bytes
+    // apart; 11008 x 4096 11.7 / 10.2 and 11.8 / 12.2) or of 240 workgroups on, fewer than 150 workgroups below K = 3584
+    // (6416 x 3072 at 10 rows 9.2 / 7.5 and 8.8 / 9.8), 128 columns over 80 MB with K a power of two (20880 x 4096 at 4 rows 21.1 / 16.4 and 21.2 / 22.2) or from 200 workgroups over
+    // 120 MB (27232 x 6528 at 5 rows 33.8 / 37.4 and 34.6 / 37.9); from K = 5120 on with more than eight rows (12288 x 5120 at 16 rows 17.1 for 16.4).  Of 4480 choices
+    // up to 16 rows (the streaming form's own lines below included) the line keeps those that gain 1.29 x cached and 1.20 x from memory
+    // and gives up 1.11 and 1.03 x (a quarter of them more than 3 % behind from memory, at worst 0.82).
     if (nothing_forced && block_scaled && tile_ok && M <= 16 && K >= 1280 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_M) <= 0 && cfg_get(cfg, ncfg, TG_CFG_BLOCK_N) <= 0) {
         const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128), bytes = N * K;
         int cols = read_once_columns(N, K);
-        if (cols == 0 && t64 >= 150 && t64 <= 256 && bytes <= 55000000 && (M <= 8 || K < 5120)) cols = 64;
-        if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 2048 && K < 5120 && bytes <= 40000000) cols = 64;
-        if (cols == 0 && t64 > 256 && t128 <= 256 && K <= 8192 && !(bytes >= kMemoryWeight && power_of_two(K))) cols = 128;
+        if (cols == 0 && t64 >= 150 && t64 <= 256 && (bytes <= 44000000 || (bytes <= 55000000 && t64 < 240 && !power_of_two(K))) && (M <= 8 || K < 5120)) cols = 64;
+        if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 3584 && K < 5120 && bytes <= 40000000) cols = 64;
+        if (cols == 0 && t64 > 256 && t128 <= 256 && K <= 8192 && !(bytes >= 80000000 && power_of_two(K)) && !(bytes >= 120000000 && t128 >= 200)) cols = 128;
         if (cols > 0) return Schedule{1, 32, cols, 1, -1, -1, 8};
     }
     if (skinny && want_kernel != 2 && (want_kernel == 3 || K >= 1024)) {
@@ -632,8 +635,10 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         // eight rows where every narrow workgroup's own activation loads weigh more (6144 x 4096 at M = 16: 9.3 against
         // 9.6; 1536 x 24576: 10.4 - 11.9 against 13.5 - 19.4).  One to four rows over 96 - 135 row blocks stay narrow: its
         // 384 - 540 workgroups fill the chip without a reduction (8192 x 8192 at M = 1: 13.6 against 15.7).
-        bool wide_auto = N >= 16384 || N > 8192 ||
-                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= 160 && !(M <= 4 && wide_wgs >= 96));
+        // (block-scaled with long K and up to four rows the narrow form keeps a little more: 5536 x 6912 at two rows 11.5 us narrow, 13.9 with two splits;
+        // 8368 x 10240 at one 25.5 and 27.5)
+        bool wide_auto = (N > 8192 && !(block_scaled && K > 8192 && wide_wgs < 136)) ||
+                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= (block_scaled && M <= 4 ? 176 : 160) && !(M <= 4 && wide_wgs >= 96));
         // Weight rows per workgroup of the two-piece wide form.  64 rows leave compute units idle when N / 64 is well below 256 or a little above it; fewer rows per
         // workgroup fill the chip in one launch where split-K needed a second one.  Cost of a choice ~ rounds of 256
         // workgroups x (rows + 16): 12288 x 5120 at M = 16 takes 12.6 us with 48 rows (256 workgroups) against 13.2 with
