@@ -74,7 +74,9 @@ enum {
                             * tiled 256x256 block-scaled kernels (dense and ragged): 1 = the persistent form (one workgroup per
                             * compute unit walks the tiles, three weight slabs in LDS, scales in registers); the ragged GEMM
                             * chooses it by itself for K <= 1536 from 192 rows per expert on; ragged ring tiles: 1 asks for them
-                            * (reported as 1) */
+                            * (reported as 1); dense ring tiles of one row tile over a weight of 100 MB and more: 1 asks for the form that reads the
+                            * weight past the caches (K a power of two from 4096 on, or 256x128) and, if K is a power of two, sums over K in a
+                            * rotated order -- not the bits of the other kernels.  The library uses it where no tile is asked for (reported as 1) */
     TG_CFG_WAVES = 5,   /* skinny kernel: waves per workgroup splitting K (4/8/16); stream kernel: 8 = eight waves split K inside a 16-row workgroup, and with ROW_GROUPS = 4 (the wide form) 1 = one 1 KiB piece per wave in flight instead of two half pieces; tiled 256x256 kernels: 8 = the generic eight-wave tile kernel (one workgroup per tile) instead of the persistent one; tiled 64x32, 64x64, 64x128 and 128x128: 8 = the ring form of the tile (reported as 8 for every ring tile); ragged GEMM, streaming form: 4 / 6 / 8 waves (64 / 96 / 128 weight rows) per workgroup */
     TG_CFG_QUANT_BLOCK_N = 6, /* block-scaled tg_fp8_gemm: weight rows per scale (default 128) */
     TG_CFG_QUANT_BLOCK_K = 7, /* block-scaled tg_fp8_gemm: K elements per scale (default 128): the reference's

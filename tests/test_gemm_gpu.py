@@ -657,13 +657,45 @@ def test_ring_tiles_over_weights_from_memory(device, block_scaled, M, N, K, want
     else:
         sa = sb = torch.full((1,), 0.5, device=device)
     out = torch.full((M, N), float("nan"), device=device)
-    cfg = {"KERNEL": "tiled", "BLOCK_M": want[0], "BLOCK_N": want[1], "SPLIT_K": 1, "WAVES": 8}
+    cfg = {"KERNEL": "tiled", "BLOCK_M": want[0], "BLOCK_N": want[1], "SPLIT_K": 1, "WAVES": 8, "ROW_GROUPS": 1}
     if block_scaled or 17 <= M <= 64:  # (the library's own choice there)
         cfg = None
     _lib.fp8_gemm(out, a8, b8, sa, sb, False, True, 1.0, 0.0, cfg)
     got = used("tiled")
-    assert (got["BLOCK_M"], got["BLOCK_N"], got["WAVES"], got["SPLIT_K"]) == want + (8, 1), got
+    assert (got["BLOCK_M"], got["BLOCK_N"], got["WAVES"], got["SPLIT_K"], got["ROW_GROUPS"]) == want + (8, 1, 1), got
     assert torch.equal(out, (a @ b.t()) * (1.0 if block_scaled else 0.25))
+
+
+@pytest.mark.parametrize("block_scaled", [False, True])
+@pytest.mark.parametrize("M,bm,bn,K", [(30, 32, 128, 4096), (61, 64, 64, 8192), (150, 160, 128, 4096)])
+def test_rotated_sums_are_asked_for_and_named(device, block_scaled, M, bm, bn, K):
+    """A tile asked for by name alone sums in the order of every other kernel (the bits of 128 x 128 tiles), with ROW_GROUPS = 1 in the
+    rotated one; either within the oracle's tolerance on operands of ordinary values, with either scale tensor missing and with beta."""
+    N = 100000000 // K // 128 * 128 + 128
+    g = torch.Generator(device=device).manual_seed(M + K)
+    a, b = torch.randn(M, K, generator=g, device=device).to(FP8), (torch.randn(N, K, generator=g, device=device) * 0.5).to(FP8)
+    if block_scaled:
+        sa, sb = torch.rand(M, K // 128, generator=g, device=device) * 0.1 + 0.01, torch.rand(N // 128, K // 128, generator=g, device=device) * 0.1 + 0.01
+    else:
+        sa, sb = torch.full((1,), 0.5, device=device), torch.full((1,), 0.25, device=device)
+    kc = {"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": 1, "WAVES": 8}
+    blocks = torch.arange(0, N // 128, 97)
+    cols = (blocks[:, None] * 128 + torch.arange(128)).flatten()
+    c0 = torch.randn(M, N, generator=g, device=device)
+    for s1, s2, dtype, beta in ((sa, sb, torch.bfloat16, 0.0), (None, sb, torch.float32, 0.0), (sa, None, torch.float16, 0.0), (sa, sb, torch.float32, 0.5)):
+        plain, turned, base = (c0.to(dtype, copy=True) for _ in range(3))
+        _lib.fp8_gemm(plain, a, b, s1, s2, False, True, 1.0, beta, kc)
+        assert _lib.last_config()["ROW_GROUPS"] != 1 and _lib.last_config()["BLOCK_M"] == bm
+        _lib.fp8_gemm(base, a, b, s1, s2, False, True, 1.0, beta, {"KERNEL": "tiled", "BLOCK_M": 128, "BLOCK_N": 128, "SPLIT_K": 1})
+        assert torch.equal(plain, base)
+        _lib.fp8_gemm(turned, a, b, s1, s2, False, True, 1.0, beta, {**kc, "ROW_GROUPS": 1})
+        assert _lib.last_config()["ROW_GROUPS"] == 1 and _lib.last_config()["BLOCK_M"] == bm
+        f = lambda t, scale: t.cpu().double() if scale is None else t.cpu().double() * (scale.cpu().double() if scale.numel() == 1 else scale.cpu().double().repeat_interleave(128, 1))  # noqa: E731
+        bs = s2 if s2 is None or not block_scaled else s2[blocks.to(device)].repeat_interleave(128, 0)
+        ref = f(a.float(), s1) @ f(b[cols.to(device)].float(), bs).t() + beta * c0[:, cols.to(device)].cpu().double()
+        err = (turned[:, cols.to(device)].cpu().double() - ref).norm() / ref.norm()
+        # about twice what is measured: f32 sums of the matrix unit 2.8e-5, the outputs' rounding 1.7e-3 (bf16) and 2.1e-4 (f16)
+        assert err < {torch.float32: 6e-5, torch.float16: 6e-4, torch.bfloat16: 4e-3}[dtype], err
 
 
 @pytest.mark.parametrize("block_scaled", [False, True])

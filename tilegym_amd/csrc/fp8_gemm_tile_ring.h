@@ -1,5 +1,5 @@
 // Tiles of 32 x 64 to 256 x 128 over a ring of LDS stages: C[m,n] = sum_k A[m,k] * B[n,k], per-tensor or block scales (tiles of
-// 128 columns), for the row counts between decoding and those that fill whole rounds of 256 x 256 tiles.
+// 64 and 128 columns), for the row counts between decoding and those that fill whole rounds of 256 x 256 tiles.
 //
 // One workgroup per compute unit: four waves compute (2 x 2, one per SIMD), four waves do nothing but request the next K steps'
 // slabs.  A direct global->LDS load holds its wave until the compute unit's address path has room (about 16 clocks per 1 KiB
@@ -39,13 +39,15 @@
 //
 // ONCE, for one row tile over a weight that comes from memory (100 MB and more: three sets of operands do not fit in the caches):
 // the weight loads are non-temporal, and workgroup b starts at K step b of its range and goes round -- rows a power of two apart
-// would put the requests of one moment on few memory channels.  The same products are added, in a rotated order.  28672 x 4096,
+// would put the requests of one moment on few memory channels.  The same products are added, in a rotated order: not the bits of
+// the other forms.  Hence only where the library chooses the tile, or ROW_GROUPS = 1 asks for it.  28672 x 4096,
 // us before / after, per-tensor: 50 rows 27.5 / 23.4, 90 rows 30.1 / 26.2, 128 rows 32.1 / 28.8, 256 rows 40.2 / 35.6; block-scaled:
 // 16 rows 25.5 / 23.1, 50 rows 28.5 / 24.0.  Either alone 24 - 25.5 at 24 rows, both 22.3.  Smaller weights stay in the caches from one call to
 // the next and are up to 1.4 x slower with non-temporal loads; K that is no power of two is 3 - 5 % slower rotated and the same without.
 //
 // Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as
-// fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results.
+// fp8_gemm_tile_kernel<128, 128, 2, 2, BLOCKSCALE, GROUP_DENSE, SPLIT>: identical results but for ONCE's order over a K that is a power
+// of two.
 #pragma once
 
 #include "fp8_gemm_tile.h"

@@ -48,7 +48,8 @@ hipError_t run_tile_ring_block(int bm, int bn, bool split, const GemmParams& p, 
 hipError_t run_tile_ring_kn(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 hipError_t run_tile_ring(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 // The same tiles (32 or 64 rows x 64 or 128, 96, 128 or 160 rows x 128, per-tensor 256 x 128) for one row tile over a weight from
-// memory; K range unsplit; the sum over K starts at another step in each workgroup if K is a power of two
+// memory; K range unsplit.  If K is a power of two the sum over K starts at another step in each workgroup: the same products, added in
+// another order than by the other kernels
 hipError_t run_tile_ring_once(bool block_scaled, int bm, int bn, const GemmParams& p, int gx, hipStream_t s);
 // 64x128 per-tensor tile with four LDS stages (loads three K steps ahead): the 16 < M <= 64 form
 hipError_t run_tile_deep(bool split, const GemmParams& p, int gx, int gy, hipStream_t s);

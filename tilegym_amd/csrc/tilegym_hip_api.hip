@@ -279,8 +279,8 @@ struct TileModel { const StepCost* kinds; int n; float reduce_us, reduce_us_per_
 constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTiles) / sizeof(StepCost)), 3.272f, 0.316f, 1.0f, 0.018f};
 constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
-// The form of the ring tiles for weights that come from memory and are read once (ONCE in fp8_gemm_tile_ring.h): one row tile over
-// 100 MB or more.  K a power of two, where the rotated start pays; the 256-row tile at any K (20480 x 5120 44.9 -> 41.6 us at 256
+// The form of the ring tiles for weights that come from memory and are read once (ONCE in fp8_gemm_tile_ring.h; reported, and asked for
+// beside a tile, as ROW_GROUPS = 1): one row tile over 100 MB or more.  K a power of two, where the rotated start pays; the 256-row tile at any K (20480 x 5120 44.9 -> 41.6 us at 256
 // rows, 14336 x 12288 70.2 -> 60.9), the others are 2 - 5 % behind the plain loads there.
 constexpr int64_t kMemoryWeight = 100000000;
 bool power_of_two(int64_t x) { return (x & (x - 1)) == 0; }
@@ -1425,7 +1425,10 @@ int32_t fp8_gemm_impl(const tg_tensor* c, const tg_tensor* a, const tg_tensor* b
         if (bs_persistent) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
         const bool ring = s.kernel == 1 && !block_scaled && s.waves == 8 && is_ring_tile(s.bm, s.bn);
         const bool block_ring = s.kernel == 1 && block_scaled && s.waves == 8 && is_block_ring_tile(s.bm, s.bn);
-        const bool once = (ring || block_ring) && !split && rows == M && trans_b && read_once(M, N, K, block_scaled, s.bm, s.bn);
+        // (sums in another order than every other kernel: a schedule asked for by name means that order only with ROW_GROUPS = 1)
+        const bool once = (ring || block_ring) && !split && rows == M && trans_b && read_once(M, N, K, block_scaled, s.bm, s.bn) &&
+                          (cfg_get(cfg, ncfg, TG_CFG_ROW_GROUPS) == 1 || nothing_forced_but_kernel(cfg, ncfg));
+        if (once) g_last_cfg[TG_CFG_ROW_GROUPS] = 1;
         hipError_t e = once ? tg::run_tile_ring_once(block_scaled, s.bm, s.bn, pc, gx, stream)
                      : block_scaled && s.bm == 256 && s.bn == 320 ? tg::run_bs320(pc, gx, stream)
                      : block_ring ? tg::run_tile_ring_block(s.bm, s.bn, split, pc, gx, pc.split_k, stream)

@@ -50,6 +50,8 @@ def candidates(M: int, N: int, K: int, block_scaled: bool) -> List[dict]:
             out.append({"KERNEL": "tiled", "BLOCK_M": 256, "BLOCK_N": 320, "SPLIT_K": 1})
         for bm, bn in ((32, 64), (64, 64), (32, 128)) + (() if block_scaled else ((64, 32), (256, 128)) if M > 64 else ((64, 32),)):
             out += [{"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": s, "WAVES": 8} for s in (1, 2, 4)]
+            if N * K >= 100_000_000 and M <= bm:  # the form for one row tile over a weight from memory
+                out.append({"KERNEL": "tiled", "BLOCK_M": bm, "BLOCK_N": bn, "SPLIT_K": 1, "WAVES": 8, "ROW_GROUPS": 1})
         if block_scaled or M > 64:
             # tiles over a ring of LDS stages, four waves load and four compute (WAVES = 8 picks that form of 64 x 128 and 128 x 128)
             for bm, bn in ((64, 128), (96, 128), (128, 128), (160, 128)) + (((192, 128),) if block_scaled else ((160, 192), (192, 192))):
