@@ -12,7 +12,8 @@
 // tile's end (so K has at least five steps with 256 columns, eight with 128).  A workgroup's tiles all lie in its XCD's share of the tile sequence.
 //
 // Activation scales travel with the slabs: a chunk of eight K steps is requested right in front of the slab of its first step, into
-// one of three chunk buffers (two would be enough but for a last chunk of a single step).  Weight scales are scalar loads, one
+// one of three chunk buffers (two would be enough but for last chunks shorter than the ring: the next tile's first chunk is
+// then requested while the one before the last is read).  Weight scales are scalar loads, one
 // step ahead.  Rows that a tile does not have are requested from beyond the descriptor's range: no memory request.
 //
 // Eight computing waves for 256 columns (four of 64 x 128 were no faster than the kernels of one workgroup per tile: two waves on a SIMD take

@@ -16,7 +16,7 @@ hipError_t run_grouped_ring(int bm, int cols, int group, GemmParams p, hipStream
         if (group == GROUP_RAGGED) return launch_grouped_ring<BM, BN, STAGES, NC, GROUP_RAGGED>(p, grid, s);          \
         if (group == GROUP_GATHER) return launch_grouped_ring<BM, BN, STAGES, NC, GROUP_GATHER>(p, grid, s);          \
     }
-    TG_CASE(32, 128, 6, 4)
+    if (bm == 32 && bn == 128 && group == GROUP_RAGGED) return launch_grouped_ring<32, 128, 6, 4, GROUP_RAGGED>(p, grid, s);
     TG_CASE(64, 128, 6, 4)
     TG_CASE(64, 256, 3, 8)
     TG_CASE(128, 256, 3, 8)

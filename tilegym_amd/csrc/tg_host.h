@@ -68,7 +68,7 @@ int compute_units();
 hipError_t run_tile_block_dense(int bm, int bn, bool split, const GemmParams& p, int gx, int gy, hipStream_t s);
 // pair: the 128-row form of which two workgroups share a compute unit
 hipError_t run_tile_moe_act(int bm, bool pair, const GemmParams& p, int gx, hipStream_t s);
-// persistent tiles of 32, 64 or 128 rows x 128, 192 or 256 weight rows for experts with few rows: same results as the others of the
+// persistent tiles of 32 (ragged), 64 or 128 rows x 128, 192 or 256 weight rows for experts with few rows: same results as the others of the
 // group mode.  Needs both scale tensors, K a multiple of 128 with at least grouped_ring_steps steps, at most 256 experts if ragged, and
 // an alignment block that bm divides if gathered.  GROUP_GATHER_ACT: 256 weight rows.  cols 0: 128, 192 or 256, chosen on the device
 constexpr int grouped_ring_steps(int cols) { return cols != 128 ? 5 : 8; }  // the ring's stages and two

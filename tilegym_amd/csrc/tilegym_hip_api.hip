@@ -895,7 +895,7 @@ bool pair_tiles(int64_t rows, int64_t experts, int64_t col_tiles) { return group
 struct RingTile { int bm, bn; };  // bm 0: another kernel's problem
 bool grouped_ring_takes(const tg::GemmParams& p, int group, int bm, int bn) {
     const bool exists = group == tg::GROUP_GATHER_ACT ? bn == 256 && (bm == 64 || bm == 128)
-                                                      : (bm == 32 && bn == 128) || (bm == 64 && (bn == 128 || bn == 192 || bn == 256)) || (bm == 128 && (bn == 192 || bn == 256));
+                                                      : (bm == 32 && bn == 128 && group == tg::GROUP_RAGGED) || (bm == 64 && (bn == 128 || bn == 192 || bn == 256)) || (bm == 128 && (bn == 192 || bn == 256));
     return exists && p.As && p.Bs && p.K % 128 == 0 && p.kblocks >= tg::grouped_ring_steps(bn) && (group != tg::GROUP_RAGGED || p.E <= 256);
 }
 // Tiles of bm rows that `rows` rows spread evenly, but for their own noise, over E experts make.
@@ -1778,7 +1778,7 @@ static int32_t moe_gemm_silu_quant(const tg_tensor* q, const tg_tensor* scales, 
 
     int bm = block_m % 256 == 0 ? 256 : 128;  // a row tile must not span two alignment blocks (experts)
     RingTile ring = grouped_ring_tile(p, tg::GROUP_GATHER_ACT, num_valid, block_m);
-    if (ring.bm == 0 && block_m == 64) ring = RingTile{64, 256};
+    if (ring.bm == 0 && block_m % 128) return fail(TG_ERR_INVALID, "block_m must be a positive multiple of 128 for the fused form");
     if (ring.bm > 0) bm = ring.bm;
     Schedule s{1, bm, 256, 1, ring.bm > 0 ? 1 : -1, -1, -1};
     remember(s);
