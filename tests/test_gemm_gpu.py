@@ -714,7 +714,7 @@ def test_decode_streams_narrow_or_wide(device, block_scaled, M, N, K, form):
         out = matmul(a.to(device), b.to(device), trans_b=True, scale_a=0.01, scale_b=0.02, out_dtype=torch.bfloat16)
         ref = [R.ref_gemm_per_tensor(a, r, 0.01, 0.02, trans_b=True, out_dtype=torch.bfloat16) for r in (b[:384], b[-40:])]
     cfg = used("stream")
-    assert (cfg["ROW_GROUPS"] == 4) == (form == 4) or (block_scaled and K > 2048), cfg
+    assert (cfg["ROW_GROUPS"] == 4) == (form == 4), cfg
     check(out[:, rows.to(device)], ref[0], what=f"M={M} N={N} K={K}")
     if not block_scaled:
         check(out[:, -40:], ref[1], what=f"M={M} N={N} K={K}, last rows")
@@ -1502,10 +1502,10 @@ def test_moe_gather_on_ring_tiles(device, block_m, K):
         assert torch.equal(q.view(torch.uint8)[live], q2.view(torch.uint8)[live]) and torch.equal(s[live], s2[live])
 
 
-@pytest.mark.parametrize("T,H,I,E,k", [(200, 1024, 1024, 16, 2), (150, 1152, 640, 40, 4), (300, 640, 1024, 24, 3), (90, 1024, 512, 8, 4)])
+@pytest.mark.parametrize("T,H,I,E,k", [(200, 1024, 1024, 16, 2), (150, 1152, 640, 40, 4), (300, 640, 1024, 24, 3), (90, 1024, 512, 8, 4), (75, 1024, 512, 8, 4)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_moe_layer_on_64_row_blocks(device, T, H, I, E, k, dtype, monkeypatch):
-    """Up to 47 rows per expert the one-call layer pads experts to 64 rows and runs on the ring tiles (GEMM2 on 64 x 128 tiles where its K
+    """Up to 40 rows per expert (47 over 256 MB) the one-call layer pads experts to 64 rows and runs on the ring tiles (GEMM2 on 64 x 128 tiles where its K
     is too short for them); ids outside [0, E) included.  Same bits as the call-by-call layer on 128-row blocks."""
     from tilegym_amd.ops import fused_moe, moe_interface
 
@@ -1517,6 +1517,9 @@ def test_moe_layer_on_64_row_blocks(device, T, H, I, E, k, dtype, monkeypatch):
     ids[5, 0], ids[7, k - 1] = -1, E
     args = (x, w1, w2, tw.to(device), ids.to(device))
     got = fused_moe(*args, w1_scale=s1, w2_scale=s2)
+    cfg = _lib.last_config()  # (of the second GEMM, over the same blocks as the first, which runs on 64-row blocks on ring tiles only)
+    assert (cfg["BLOCK_M"] == 64) == (T * k <= 40 * E), cfg  # (more rows only over 256 MB)
+    assert cfg["BLOCK_M"] != 64 or (cfg["ROW_GROUPS"] == 1) == (I >= 640), cfg
     assert T * k > E * 7   # (past the decoding form)
     monkeypatch.setattr(_lib, "native", None)
     monkeypatch.setattr(moe_interface, "USE_ONE_CALL_LAYER", False)
