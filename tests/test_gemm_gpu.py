@@ -624,7 +624,7 @@ def test_narrow_and_tall_ring_tiles_are_chosen(device, M, N, K, want):
     ("kn", 16, 1024, 1920, False), ("kn", 16, 10240, 1920, True), ("kn", 256, 4096, 4096, False), ("kn", 16, 4096, 4096, True),
     ("nk", 24, 12288, 5120, True), ("nk", 30, 17072, 5120, False), ("nk", 40, 12288, 5120, True), ("nk", 64, 12288, 5120, False), ("nk", 64, 6144, 4096, False),
     ("nk", 50, 4096, 14336, True), ("nk", 50, 2048, 5120, False), ("nk", 24, 22032, 2560, False),
-    ("block", 24, 12288, 5120, True), ("block", 20, 18576, 2944, False), ("block", 28, 3520, 4864, False), ("block", 17, 1520, 2304, False), ("block", 17, 8192, 8192, False)])
+    ("block", 24, 12288, 5120, True), ("block", 20, 18576, 2944, False), ("block", 28, 3520, 4864, False), ("block", 17, 1520, 2304, False), ("block", 17, 8192, 8192, False), ("block", 21, 5120, 5120, False)])
 def test_narrow_ring_tiles_are_chosen_where_they_hold_from_memory(device, kind, M, N, K, ring):
     """Either side of the lines between the narrow ring tiles (and 256 x 128), and the kernels that are ahead of them when the weight is not in the caches."""
     zeros = lambda *shape: torch.zeros(*shape, dtype=torch.uint8, device=device).view(FP8)  # noqa: E731
@@ -731,7 +731,7 @@ def test_block_scaled_skinny_to_sixteen_rows(device):
 
 
 @pytest.mark.parametrize("M,N,K,want", [(8, 10240, 5120, (32, 64)), (9, 6144, 4096, (32, 64)), (16, 20480, 2048, (32, 128)), (16, 11008, 4096, None),
-                                        (8, 6144, 4096, None), (16, 6400, 3072, None), (4, 20864, 4096, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
+                                        (8, 6144, 4096, None), (16, 6400, 3072, None), (12, 7168, 3584, None), (4, 20864, 4096, None), (2, 5504, 6912, None), (9, 12288, 5120, None), (16, 8192, 8192, None)])  # None: streaming
 def test_block_scaled_decode_on_ring_tiles(device, M, N, K, want):
     g = _g(M + N)
     a, b = fp8_randn((M, K), g), fp8_randn((N, K), g, 0.5)

@@ -33,7 +33,7 @@
 //
 // KN: the weight is (K, N); its slab is 128 K rows of BN bytes, staged as they lie and turned on the way out of LDS
 // (ds_read_b64_tr_b8), so no (N, K) copy is made.  Bound as above: the lines of a K row tile are whole with 128 columns and halves with
-// 64 (1.62 instead of 1.05 million requests to L2 at 256 x 4096 x 4096: 13.0 us, 32 x 128 tiles 12.3, the (N, K) form 9.0).  What it measured
+// 64 (1.62 instead of 1.05 million requests to L2 at 256 x 4096 x 4096: 13.6 us, 32 x 128 tiles 12.8, the (N, K) form 9.0; from memory 19.7 and 19.0).  What it measured
 // against the copy stands at pick_kn_tile.  Not kept: tiles dealt over the XCDs column by column in other orders (within 5 %
 // either way), weights fetched past the first-level cache (30 to 50 % slower).
 //

@@ -524,13 +524,13 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
                     // (above 25 MB fewer than 96 workgroups, above 40 MB fewer than 150 or two splits are slower from memory: 50 x 8192 x 8192 in 128 column tiles 14.5 us
                     // against 17.8 if the weight was read just before, but 21.5 against 20.3 if not)
                     if (N * K > 25000000 && want_split < 0 && (split == 1 ? cdiv(N, t.bn) < (N * K > 40000000 ? 150 : 96) : split == 2)) continue;
-                    // More than one round over 45 MB and more, 128 columns with splits there (17 x 8192 x 8192 17.5 -> 18.7), and one row tile of 32 rows over a long K in fewer than 128 workgroups, are slower
+                    // More than one round over 45 MB and more, 128 columns with splits (17 x 8192 x 8192 17.5 -> 18.7, 21 x 5120 x 5120 13.0 -> 14.2), and one row tile of 32 rows over a long K in fewer than 128 workgroups, are slower
                     // from memory (20 x 18576 x 2944 14.3 -> 17.9 us, cached 12.1 -> 16.0; 28 x 3520 x 4864 10.9 -> 12.7), and so are all of them where the skinny kernel is the
                     // best of the others (17 x 1520 x 2304 5.3 against 6.9; cached they are even).  Of 10270 choices the line keeps those that gain 1.20 x
                     // cached and 1.21 x from memory and gives up 1.04 and 0.87 x (at worst 0.77).
                     const int64_t cols = cdiv(N, t.bn);
                     const bool holds = want_split > 0 ||
-                                       (!(N * K > 45000000 && (cdiv(M, t.bm) * cols * cand.split_k > 256 || (t.bn == 128 && split > 1))) &&
+                                       (!(N * K > 45000000 && cdiv(M, t.bm) * cols * cand.split_k > 256) && !(t.bn == 128 && split > 1) &&
                                         !(split == 1 && t.bm == 32 && t.bn == 64 && cols < 128 && K > (M <= 32 ? 4096 : cols < 64 ? 4992 : 6144)));
                     // (a split must be predicted 10 % faster: its reduction is a launch more for the host, too)
                     offer_ring(cand, step_cost_us(kSmallRowsRing, t, M, N, kblocks, cand.split_k, t.bn) * (cand.split_k > 1 ? 1.1f : 1.f), holds);
@@ -594,8 +594,8 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     // dealt out over a workgroup, where the streaming form's waves do them between two waits (us, streaming / ring, weight in the caches and from
     // memory: 10240 x 5120 at 8 rows 14.9 / 11.2 and 14.8 / 14.2, 12288 x 2048 at 16 rows 7.7 / 7.5 and 7.6 / 7.5, 6144 x 4096 at 16 rows 11.5 / 8.8
     // and 11.2 / 10.5, 28672 x 4096 at 16 rows 24.9 / 23.6 and 25.7 / 24.8; boxes differ by 5 % from memory).  Not where it is behind from memory: 64 columns over more than 44 MB whose K is a power of two (rows 4096 bytes
-    // apart; 11008 x 4096 11.7 / 10.2 and 11.8 / 12.2) or of 240 workgroups on, fewer than 150 workgroups below K = 3584
-    // (6416 x 3072 at 10 rows 9.2 / 7.5 and 8.8 / 9.8), 128 columns over 80 MB with K a power of two (20880 x 4096 at 4 rows 21.1 / 16.4 and 21.2 / 22.2) or from 200 workgroups over
+    // apart; 11008 x 4096 11.7 / 10.2 and 11.8 / 12.2) or of 240 workgroups on, fewer than 150 workgroups below K = 4096
+    // (6416 x 3072 at 10 rows 9.2 / 7.5 and 8.8 / 9.8, 7216 x 3584 at 12 rows 10.3 / 8.1 and 10.1 / 11.5), 128 columns over 80 MB with K a power of two (20880 x 4096 at 4 rows 21.1 / 16.4 and 21.2 / 22.2) or from 200 workgroups over
     // 120 MB (27232 x 6528 at 5 rows 33.8 / 37.4 and 34.6 / 37.9); from K = 5120 on with more than eight rows (12288 x 5120 at 16 rows 17.1 for 16.4).  Of 4480 choices
     // up to 16 rows (the streaming form's own lines below included) the line keeps those that gain 1.29 x cached and 1.20 x from memory
     // and gives up 1.11 and 1.03 x (a quarter of them more than 3 % behind from memory, at worst 0.82).
@@ -603,7 +603,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         const int64_t t64 = cdiv(N, 64), t128 = cdiv(N, 128), bytes = N * K;
         int cols = read_once_columns(N, K);
         if (cols == 0 && t64 >= 150 && t64 <= 256 && (bytes <= 44000000 || (bytes <= 55000000 && t64 < 240 && !power_of_two(K))) && (M <= 8 || K < 5120)) cols = 64;
-        if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 3584 && K < 5120 && bytes <= 40000000) cols = 64;
+        if (cols == 0 && t64 >= 96 && t64 < 150 && M > 8 && K >= 4096 && K < 5120 && bytes <= 40000000) cols = 64;
         if (cols == 0 && t64 > 256 && t128 <= 256 && K <= 8192 && !(bytes >= 80000000 && power_of_two(K)) && !(bytes >= 120000000 && t128 >= 200)) cols = 128;
         if (cols > 0) return Schedule{1, 32, cols, 1, -1, -1, 8};
     }
@@ -635,10 +635,10 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
         // eight rows where every narrow workgroup's own activation loads weigh more (6144 x 4096 at M = 16: 9.3 against
         // 9.6; 1536 x 24576: 10.4 - 11.9 against 13.5 - 19.4).  One to four rows over 96 - 135 row blocks stay narrow: its
         // 384 - 540 workgroups fill the chip without a reduction (8192 x 8192 at M = 1: 13.6 against 15.7).
-        // (block-scaled with long K and up to four rows the narrow form keeps a little more: 5536 x 6912 at two rows 11.5 us narrow, 13.9 with two splits;
-        // 8368 x 10240 at one 25.5 and 27.5)
+        // (to eight pieces, and block-scaled with long K and up to four rows, the narrow form keeps a little more: 5472 x 6272 at two rows 9.6 us narrow,
+        // 11.6 wide; block-scaled 5536 x 6912 at two rows 11.5 and, with two splits, 13.9, 8368 x 10240 at one 25.5 and 27.5)
         bool wide_auto = (N > 8192 && !(block_scaled && K > 8192 && wide_wgs < 136)) ||
-                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= (block_scaled && M <= 4 ? 176 : 160) && !(M <= 4 && wide_wgs >= 96));
+                         (N * K >= ((int64_t)(M > 8 || pieces >= 12 ? 24 : 32) << 20) && wide_wgs * wide_split >= (pieces <= 8 || (block_scaled && M <= 4) ? 176 : 160) && !(M <= 4 && wide_wgs >= 96));
         // Weight rows per workgroup of the two-piece wide form.  64 rows leave compute units idle when N / 64 is well below 256 or a little above it; fewer rows per
         // workgroup fill the chip in one launch where split-K needed a second one.  Cost of a choice ~ rounds of 256
         // workgroups x (rows + 16): 12288 x 5120 at M = 16 takes 12.6 us with 48 rows (256 workgroups) against 13.2 with
@@ -795,8 +795,8 @@ bool nothing_forced(const int32_t* cfg, int32_t ncfg) {
 // A per-tensor (K, N) weight: the tile (and split) that reads it as it lies, or none where copying it to (N, K) first is cheaper.
 //
 // K from 1280 on: the ring tiles, with step costs of their own (a step is 1.2 to 1.6 times as long as over an (N, K) weight: 64-column
-// tiles take half of every 128-byte line, and K rows a multiple of 4 KiB apart crowd few cache sets -- 256 x 4096 x 4096 12.3 us with 32 x
-// 128 tiles, 256 x 3968 x 4096 10.7), against the race's GEMM with the copy's 4.1 us + 0.47 us per MB on top.  Fitted to 3871 shapes (1 ... 2048
+// tiles take half of every 128-byte line, and K rows a multiple of 4 KiB apart crowd few cache sets -- 256 x 4096 x 4096 12.8 us with 32 x
+// 128 tiles, 256 x 3968 x 4096 10.7; the model has 13.8 for them and 13.4 for 64 x 64, which take 13.6), against the race's GEMM with the copy's 4.1 us + 0.47 us per MB on top.  Fitted to 3871 shapes (1 ... 2048
 // rows, three sets of operands): 2.2 % behind the best ring tile up to 64 rows and 0.8 % above, at worst 1.25 x; against the narrow
 // tiles of fp8_gemm_tile_mid.h and the copy, which took all of these, 31 % ahead on average, behind by more than 5 % on 219 (5.5 us and
 // shorter, or by 8 % at most): 1 x 4096 x 14336 36.0 -> 14.3 us, 50 x 4096 x 14336 41 -> 16.5, 100 x 28672 x 4096 57.5 -> 28.7,
