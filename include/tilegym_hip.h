@@ -63,8 +63,8 @@ enum {
     TG_CFG_KERNEL = 0,  /* 0 fallback (no MFMA), 1 LDS-tiled MFMA kernel, 2 skinny (direct weight streaming), 3 stream (weight streaming through LDS) */
     TG_CFG_BLOCK_M = 1, /* tiled kernel: rows of A per workgroup.  BLOCK_M x BLOCK_N of the dense GEMM: 64x128, 128x128, 128x256, 256x256; per-tensor only
                          * 32x32, 64x32, 64x64 (K split inside the workgroup) and 64 x 72 .. 120 in steps of 8; tiles over a ring of LDS stages (four
-                         * waves load, four compute): 96x128, 160x128, with WAVES = 8 also 64x128 and 128x128, per-tensor 32x64, 32x128, 256x128, 160x192 and 192x192 and with WAVES = 8 64x32 and 64x64,
-                         * block-scaled 192x128; block-scaled 256x320 (M >= 256, N >= 320, N % 32 == 0, both scale tensors, no split).  Grouped
+                         * waves load, four compute): 32x64, 32x128, 96x128, 160x128, with WAVES = 8 also 64x128 and 128x128; per-tensor also 256x128, 160x192
+                         * and 192x192 and with WAVES = 8 64x32 and 64x64; block-scaled also 64x64 and 192x128; block-scaled 256x320 (M >= 256, N >= 320, N % 32 == 0, both scale tensors, no split).  Grouped
                          * GEMMs: 64x128, 128x128, 128x256, 256x256; ragged with ROW_GROUPS = 1 also the persistent ring tiles 32x128, 64x128, 64x192, 64x256,
                          * 128x192, 128x256 (K % 128 == 0, K >= 640, 128 columns 1024; E <= 256; both scale tensors).  Any other pair leaves the tile to the library */
     TG_CFG_BLOCK_N = 2, /* tiled kernel: rows of B per workgroup (see BLOCK_M); stream kernel, wide form (ROW_GROUPS = 4,

@@ -593,7 +593,7 @@ Schedule choose_dense_tile(int64_t M, int64_t N, int64_t K, bool block_scaled, b
     // block-scaled, up to 16 rows, where ring tiles of 32 rows fill the chip about once: the scale-and-adds of a row of weights are
     // dealt out over a workgroup, where the streaming form's waves do them between two waits (us, streaming / ring, weight in the caches and from
     // memory: 10240 x 5120 at 8 rows 14.9 / 11.2 and 14.8 / 14.2, 12288 x 2048 at 16 rows 7.7 / 7.5 and 7.6 / 7.5, 6144 x 4096 at 16 rows 11.5 / 8.8
-    // and 11.2 / 10.5, 28672 x 4096 at 16 rows 24.9 / 23.6 and 25.7 / 24.8; boxes differ by 5 % from memory).  Not where it is behind from memory: 64 columns over more than 44 MB whose K is a power of two (rows 4096 bytes
+    // and 11.2 / 10.5, 28672 x 4096 at 16 rows 24.9 / 23.6 and 25.7 / 24.8; machines differ by 5 % from memory).  Not where it is behind from memory: 64 columns over more than 44 MB whose K is a power of two (rows 4096 bytes
     // apart; 11008 x 4096 11.7 / 10.2 and 11.8 / 12.2) or of 240 workgroups on, fewer than 150 workgroups below K = 4096
     // (6416 x 3072 at 10 rows 9.2 / 7.5 and 8.8 / 9.8, 7216 x 3584 at 12 rows 10.3 / 8.1 and 10.1 / 11.5), 128 columns over 80 MB with K a power of two (20880 x 4096 at 4 rows 21.1 / 16.4 and 21.2 / 22.2) or from 200 workgroups over
     // 120 MB (27232 x 6528 at 5 rows 33.8 / 37.4 and 34.6 / 37.9); from K = 5120 on with more than eight rows (12288 x 5120 at 16 rows 17.1 for 16.4).  Of 4480 choices
