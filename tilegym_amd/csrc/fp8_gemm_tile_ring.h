@@ -41,8 +41,9 @@
 // the weight loads are non-temporal, and workgroup b starts at K step b of its range and goes round -- rows a power of two apart
 // would put the requests of one moment on few memory channels.  The same products are added, in a rotated order: not the bits of
 // the other forms.  Hence only where the library chooses the tile, or ROW_GROUPS = 1 asks for it.  28672 x 4096,
-// us before / after, per-tensor: 50 rows 27.5 / 23.4, 90 rows 30.1 / 26.2, 128 rows 32.1 / 28.8, 256 rows 40.2 / 35.6; block-scaled:
-// 16 rows 25.5 / 23.1, 50 rows 28.5 / 24.0.  Either alone 24 - 25.5 at 24 rows, both 22.3.  Smaller weights stay in the caches from one call to
+// us before / after over three sets of operands and over 1 GB of weights, per-tensor: 50 rows 26.1 / 23.4 and 28.6 / 24.4, 90 rows 29.3 / 25.7
+// and 31.1 / 26.8, 128 rows 31.0 / 28.6 and 32.8 / 29.2, 256 rows 44.0 / 35.7 and 44.6 / 36.0; block-scaled: 16 rows 26.2 / 25.3 and 26.6 / 26.4,
+// 50 rows 29.8 / 26.5 and 31.6 / 26.9.  Either alone 24 - 25.5 at 24 rows, both 22.3.  Smaller weights stay in the caches from one call to
 // the next and are up to 1.4 x slower with non-temporal loads; K that is no power of two is 3 - 5 % slower rotated and the same without.
 //
 // Same slab layout, swizzles, fragment addressing, arithmetic per accumulator and epilogue as

@@ -280,8 +280,9 @@ constexpr TileModel kPerTensorModel{kPerTensorTiles, (int)(sizeof(kPerTensorTile
 constexpr TileModel kBlockScaledModel{kBlockScaledTiles, (int)(sizeof(kBlockScaledTiles) / sizeof(StepCost)), 3.5f, 0.30f, 1.04f, 0.f};
 
 // The form of the ring tiles for weights that come from memory and are read once (ONCE in fp8_gemm_tile_ring.h; reported, and asked for
-// beside a tile, as ROW_GROUPS = 1): one row tile over 100 MB or more.  K a power of two, where the rotated start pays; the 256-row tile at any K (20480 x 5120 44.9 -> 41.6 us at 256
-// rows, 14336 x 12288 70.2 -> 60.9), the others are 2 - 5 % behind the plain loads there.
+// beside a tile, as ROW_GROUPS = 1): one row tile over 100 MB or more.  K a power of two, where the rotated start pays; the 256-row tile at any K (chosen from 192
+// workgroups on, where it is 1.17 x ahead from memory: 28672 x 4096 at 256 rows 44.6 -> 36.0 us; with fewer 160 x 192 and 128 x 128 tiles are,
+// 20480 x 5120 41.4 / 41.2 but 14336 x 12288 69.5 / 82.8), the others are 2 - 5 % behind the plain loads there.
 constexpr int64_t kMemoryWeight = 100000000;
 bool power_of_two(int64_t x) { return (x & (x - 1)) == 0; }
 bool read_once(int64_t M, int64_t N, int64_t K, bool block_scaled, int bm, int bn) {
@@ -299,7 +300,7 @@ int read_once_columns(int64_t N, int64_t K) {
 // then what counts: few workgroups over a long K (above 44 x their number) ask for too little at once, and so do tiles of 32 rows or columns with
 // fewer than 160 or 128 workgroups, or (64 x 32 above 96 rows) a full round of them over long K, and 256 x 128 with fewer than 192.  Of 5500
 // choices of 65 to 700 rows that these tiles took the line keeps those that gain 1.29 x per-tensor and 1.28 x block-scaled cached, 1.21 and
-// 1.31 x from memory, and gives up 1.15 and 1.16 x cached, 0.97 (at worst 0.72) and 1.02 x (0.80) from memory: 4096 x 8192 at 88 rows and the like.
+// 1.31 x from memory, and gives up 1.15 and 1.16 x cached, 0.97 (at worst 0.72) and 1.02 x (0.80) from memory: 1520 x 5248 at 88 rows 8.4 and 11.5 us for 8.6 and 8.2.
 bool holds_from_memory(const StepCost& t, bool block_scaled, int64_t M, int64_t N, int64_t K, int split) {
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
     if (t.bm == 256) return tiles >= 192;
